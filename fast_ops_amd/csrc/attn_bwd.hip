@@ -18,7 +18,7 @@
 //      computed untransposed, S = Q K^T and dP = dO V^T (A operands = Q / dO rows from LDS, B operands = K^T / V^T
 //      held in registers), so a lane owns one key and P, dS are the B operands of dV^T = dO^T P and dK^T = Q^T dS
 //      (A operands via the transposing LDS read of the dO and Q tiles); per-row LSE and delta come from LDS.
-//      Without dropout and bias this runs as attn_bwd_dkdv_pipe_kernel, the same computation laid out by hand as a
+//      Without a bias that has a query stride this runs as attn_bwd_dkdv_pipe_kernel, the same computation laid out by hand as a
 //      software pipeline (described there); attn_bwd_dkdv_kernel is the plain, compiler-scheduled form.
 // Both recompute the scores (seven GEMMs in total instead of the five of an atomics-based single pass). softmax_scale
 // is applied once to the finished dQ and dK accumulators rather than to every dS.
@@ -40,7 +40,7 @@ constexpr int kBwdTile = 64;               // rows of a streamed tile
 struct AttnBwdParams {
   const void *q, *k, *v, *o, *d_o;
   const float* lse;
-  float* delta;
+  float* delta;       // [B, H, Sq]: -rowsum(dO O) (1 - dropout_p), written by the dQ kernel
   float* nlse;        // [B, H, Sq]: -LSE / softmax_scale, written by the dQ kernel beside delta (see there)
   void *dq, *dk, *dv;
   int B, H, Sq, Sk;
@@ -371,6 +371,9 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
       for (int e = 0; e < 8; ++e) delta -= (float)ov[e] * (float)gf[ks][e];
     }
     delta += half_swap(delta);
+    // dropout: with Z = 0 or 1 per element and k = 1 / (1 - p), dS = P (k Z dP - delta) = k P (Z dP - delta (1 - p)); the
+    // factor k is applied to the finished gradients
+    if constexpr (DROP) delta *= prm.drop.keep_prob;
     if (hh == 0 && q0w + l32 < Sq) prm.delta[(int64_t)bh * Sq + q0w + l32] = delta;
   }
   // (consumed here so that the compiler waits for these loads before the loop: a vmcnt wait inside the loop would
@@ -384,7 +387,8 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
   for (int i = 0; i < DBLK; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
-  const float c = prm.scale_log2e, scale = prm.scale;
+  const float c = prm.scale_log2e, scale = DROP ? prm.scale * prm.drop.keep_scale : prm.scale;
+  DropRows<1> drop;
 
   for (int tile = 0; tile < n_tiles; ++tile) {
     const int buf = tile & 1;
@@ -404,6 +408,9 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
       if (wave_s == 0) key_bias_next = load_bias<T>(prm.bias, key_bias_row + min((tile + 2) * kBwdTile + lane, Sk - 1));
     }
     if (CAUSAL && key0 > q0w + 31) continue;
+    if constexpr (DROP) {
+      drop.look(prm.drop, bh, Sq, Sk, q0 + wave_s * 32, tile);
+    }
     FO_LDS const char* kt = smem + buf * TILE_BYTES;
     FO_LDS const char* vt = smem + (2 + buf) * TILE_BYTES;
 
@@ -432,8 +439,10 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
     // register r of block kb holds key key0 + 32*kb + 4*hh + koff(r), koff(r) = (r & 3) + 8 * (r >> 2); dead iff
     // key > q or key >= Sk
     vec8 dsf[4];
-    // dropout (flash_attention_triton.py:524-532,599): dP reaches only the kept probabilities, scaled by 1 / (1 - p_drop)
-    const uint32_t drop_row = DROP ? prm.drop.offset + ((uint32_t)bh * (uint32_t)Sq + (uint32_t)(q0w + l32)) * (uint32_t)Sk + (uint32_t)key0 : 0u;
+    // dropout (flash_attention_triton.py:524-532,599): dP reaches only the kept probabilities
+    if constexpr (DROP) {
+      if (__builtin_expect(drop.state != kKeepAll, 0)) drop.apply(dpacc);
+    }
     // bias row of this lane's query (flash_attention_triton.py:497-509); keys past the end re-read the last one
     const int64_t bias_row = BIAS ? b * prm.bias.strides[0] + h * prm.bias.strides[1] + (int64_t)qrow * prm.bias.strides[2] : 0;
     // (the factor softmax_scale of dS is applied once, to the finished accumulators; tiles that no mask touches - most -
@@ -453,12 +462,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
             float shift = -lse2;
             if constexpr (BIAS) shift = __builtin_fmaf(b4[u], kLog2e, -lse2);
             const float p = dead ? 0.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][r], c, shift));
-            float dp = dpacc[kb][r];
-            if constexpr (DROP) {
-              const uint32_t idx = drop_row + (uint32_t)(32 * kb + 4 * hh + u + 8 * j);
-              dp = dropout_keep(idx, prm.drop.seed, prm.drop.threshold) ? dp * prm.drop.keep_scale : 0.0f;
-            }
-            dsf[kb * 2 + (r >> 3)][r & 7] = (T)(p * (dp + delta));
+            dsf[kb * 2 + (r >> 3)][r & 7] = (T)(p * (dpacc[kb][r] + delta));
           }
         };
         // The bias of four keys at a time (few values in flight: this kernel has no registers to spare). From the
@@ -642,7 +646,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_kernel(const Att
   for (int i = 0; i < DBLK; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) { dkacc[i][r] = 0.0f; dvacc[i][r] = 0.0f; }
-  const float c = prm.scale_log2e, scale = prm.scale;
+  const float c = prm.scale_log2e, scale = DROP ? prm.scale * prm.drop.keep_scale : prm.scale;
 
   for (int qt = qt0; qt < n_qt; ++qt) {
     const int buf = (qt - qt0) & 1;
@@ -654,6 +658,13 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_kernel(const Att
     FO_LDS const char* gtile = smem + (2 + buf) * TILE_BYTES;
     FO_LDS const float* lse_t = rowvals + buf * kBwdTile;
     FO_LDS const float* del_t = rowvals + (2 + buf) * kBwdTile;
+    // dropout: a lane looks at one of the tile's 64 rows, the wave's 32 keys of it as a whole (dropout_run)
+    uint64_t rows_keep = ~0ull, rows_mixed = 0;
+    if constexpr (DROP) {
+      const int run = dropout_run<5>(DropRows<1>::index(prm.drop, bh, Sq, Sk, q0t + lane, k0w), 32, prm.drop.seed, prm.drop.threshold);
+      rows_keep = __builtin_amdgcn_ballot_w64(run == kKeepAll);
+      rows_mixed = __builtin_amdgcn_ballot_w64(run == kDropMixed);
+    }
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
       if (CAUSAL && q0t + 32 * qb + 31 < k0w) continue;   // every query of the block is before every key of this wave
@@ -696,13 +707,29 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_kernel(const Att
       const int lim = CAUSAL ? key - (q0t + 32 * qb + 4 * hh) : 0;
       const int lim_end = Sq - (q0t + 32 * qb + 4 * hh);
       vec8 pf[2], dsf[2];
-      // dropout index of (first query of this lane's register set, this lane's key); consecutive queries are Sk apart
-      const uint32_t drop_base = DROP ? prm.drop.offset + ((uint32_t)bh * (uint32_t)Sq + (uint32_t)(q0t + 32 * qb + 4 * hh)) * (uint32_t)Sk + (uint32_t)key : 0u;
+      // dropout (flash_attention_triton.py:524-532,551-552): dV sees the kept probabilities, dP reaches them only. Where all
+      // or none of the block's elements are kept (nearly always) that is one factor, else a bit per register.
+      uint32_t keep_bits = 0xFFFFFFFFu;
+      float keep_all = 1.0f;
+      bool keep_each = false;
+      if constexpr (DROP) {
+        const uint32_t k32 = (uint32_t)(rows_keep >> (32 * qb)), m32 = (uint32_t)(rows_mixed >> (32 * qb));
+        keep_each = m32 != 0 || (k32 != 0 && k32 != 0xFFFFFFFFu);
+        keep_all = k32 != 0 ? 1.0f : 0.0f;
+        if (keep_each) {
+          const uint32_t first = DropRows<1>::index(prm.drop, bh, Sq, Sk, q0t + 32 * qb + 4 * hh, key);
+          keep_bits = 0;
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            keep_bits |= (dropout_keep(first + (uint32_t)((r & 3) + 8 * (r >> 2)) * (uint32_t)Sk, prm.drop.seed, prm.drop.threshold) ? 1u : 0u) << r;
+        }
+      }
       // bias column of this lane's key; queries past the end re-read the last one
       const int64_t bias_col = BIAS ? b * prm.bias.strides[0] + h * prm.bias.strides[1] + krow : 0;
       // where the bias comes from: 0 global memory, element by element; 1 the lane's own value; 2 the staged tile
-      auto softmax_grad = [&](auto masked, auto bias_mode) {
+      auto softmax_grad_of = [&](auto masked, auto bias_mode, auto each) {
       constexpr int BM = decltype(bias_mode)::value;
+      constexpr bool EACH = decltype(each)::value;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const f32x4 l4 = *(FO_LDS const f32x4*)(lse_t + 32 * qb + 8 * j + 4 * hh);
@@ -721,14 +748,20 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_kernel(const Att
           const float p = dead ? 0.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[r], c, shift));
           float pd = p, dp = dpacc[r];
           if constexpr (DROP) {
-            const bool keep = dropout_keep(drop_base + (uint32_t)(u + 8 * j) * (uint32_t)Sk, prm.drop.seed, prm.drop.threshold);
-            pd = keep ? p * prm.drop.keep_scale : 0.0f;       // dV sees the dropped, rescaled probabilities (:551-552)
-            dp = keep ? dp * prm.drop.keep_scale : 0.0f;
+            const float z = EACH ? (float)((keep_bits >> r) & 1u) : keep_all;
+            pd = p * z;
+            dp = dp * z;
           }
           pf[r >> 3][r & 7] = (T)pd;
           dsf[r >> 3][r & 7] = (T)(p * (dp + d4[u]));   // (d4 = -delta) softmax_scale is applied to the finished dK
         }
       }
+      };
+      auto softmax_grad = [&](auto masked, auto bias_mode) {
+        if constexpr (DROP) {
+          if (keep_each) { softmax_grad_of(masked, bias_mode, std::true_type{}); return; }
+        }
+        softmax_grad_of(masked, bias_mode, std::false_type{});
       };
       const bool needs_mask = q0t + 32 * qb + 32 > Sq || (CAUSAL && k0w + 31 > q0t + 32 * qb);
       typedef std::integral_constant<int, 0> BM0;
@@ -760,7 +793,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_kernel(const Att
     FO_LDS char* stage = smem + wave_s * stage_bytes(D);
     const int k0w_s = k0 + wave_s * 32;
     store_rows_via_lds<T, D>(dkacc, scale, stage, (T*)prm.dk + b * prm.dks[0] + h * prm.dks[1], prm.dks[2], k0w_s, Sk, prm.d, lane);
-    store_rows_via_lds<T, D>(dvacc, 1.0f, stage, (T*)prm.dv + b * prm.dvs[0] + h * prm.dvs[1], prm.dvs[2], k0w_s, Sk, prm.d, lane);
+    store_rows_via_lds<T, D>(dvacc, DROP ? prm.drop.keep_scale : 1.0f, stage, (T*)prm.dv + b * prm.dvs[0] + h * prm.dvs[1], prm.dvs[2], k0w_s, Sk, prm.d, lane);
   }
 }
 
@@ -805,7 +838,7 @@ constexpr bool softmax_grad_jobs_fit(int nmf) {
 static_assert(softmax_grad_jobs_fit(16) && softmax_grad_jobs_fit(8), "head_dim 128 and 64");
 
 // ---------------------------------------------------------------------------------------------------------------------
-// dK/dV without dropout and bias, as a software pipeline. The accumulators of dK and dV, the K^T and V^T fragments and
+// dK/dV without a bias that has a query stride, as a software pipeline. The accumulators of dK and dV, the K^T and V^T fragments and
 // two blocks of scores leave room for one wave per SIMD only, and a lone wave issues in order: whatever arithmetic sits
 // between two MFMAs keeps the matrix pipe waiting unless it is laid out to run beside them. A 64-query tile is two
 // 32-query blocks and four phases of NMF MFMAs each:
@@ -817,7 +850,18 @@ static_assert(softmax_grad_jobs_fit(16) && softmax_grad_jobs_fit(8), "head_dim 1
 // are two multiplications and the exponential.
 // KBIAS: with a bias that is the same for every query (query stride 0): a lane owns a key, so the bias is one value per
 // lane for the whole kernel, and P = exp2(S c + b log2 e) is a fused multiply-add where the form without bias multiplies.
-template <typename T, int D, bool CAUSAL, bool KBIAS = false>
+// DROP (flash_attention_triton.py:524-532,551-552): dV sees the kept probabilities only, and dP reaches only them: where a
+// query's elements of the workgroup's 128 keys are all dropped, its row of the dO tile in LDS is set to zero, which is both
+// (dP = dO V^T and dV = dO^T P), and where they are all kept there is nothing to do; 1 / (1 - p) is applied to the finished
+// gradients (delta comes multiplied by 1 - p, see the dQ kernel). Each lane looks at one of the next tile's 64 rows as a
+// whole (dropout_run) in the first groups of a tile, which carry no other arithmetic. A row that is neither (a few in a
+// million) counts as dropped at first. At the end the workgroup's rows of this kind, up to 64 at a time, are gathered into
+// one tile, which goes through the body once more with P of dropped elements set to zero and dP taken without delta: that
+// adds just what is missing. (A tile for each of them: 232 us at 12 heads x 4096 keys, of which 30 us were waited for.)
+// Whole backward at p = 0.1, with every element hashed in the plain kernel -> this: 12 heads x 4096 keys at head_dim 128
+// 631 -> 391 us (no dropout 387), x 8192 1957 -> 1290 (1209), x 2048 causal 187 -> 119 (105); head_dim 64, 8 x 12 heads x
+// 1024 causal 139 -> 74 (71).
+template <typename T, int D, bool CAUSAL, bool KBIAS = false, bool DROP = false>
 __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(const AttnBwdParams prm) {
   typedef typename Ops<T>::vec8 vec8;
   constexpr int TILE_BYTES = kBwdTile * D * 2;
@@ -865,8 +909,37 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   // since everyone is past phase 3 of tile j nobody reads tile j-1 any more, whose buffer - the third one - takes the
   // copy of tile j+2. Phase 4 still reads tile j, and already fetches the first fragments of tile j+1, so the fragment
   // pipeline never drains. Every wave runs hand-overs qt0-1 .. n_qt-2, each exactly once.
+  // Dropout: the rows of tile j+1 that are kept (one bit each) when tile j is handed over, and the tiles that have rows
+  // which are neither kept nor dropped, one bit for every 2^again_shift tiles.
+  uint64_t next_keep = ~0ull, next_mixed = 0, again = 0;
+  int again_shift = 0;
+  if constexpr (DROP) { while ((n_qt >> again_shift) >= 64) ++again_shift; }
+  auto drop_verdict = [&](int a, int b) {
+    next_keep = __builtin_amdgcn_ballot_w64(a == kKeepAll && b == kKeepAll);
+    next_mixed = ~(next_keep | __builtin_amdgcn_ballot_w64(a == kDropAll && b == kDropAll));
+  };
+  auto drop_index = [&](int j) -> uint32_t { return DropRows<1>::index(prm.drop, bh, Sq, Sk, j * kBwdTile + lane, k0); };
+  auto drop_look = [&](int j) {          // (outside the tile bodies)
+    const uint32_t first = drop_index(j);
+    drop_verdict(dropout_block<7>(first, prm.drop.seed, prm.drop.threshold), dropout_block<7>(first + 127u, prm.drop.seed, prm.drop.threshold));
+  };
+  // this wave's pieces of tile j+1 (in buffer `buf`) have landed, nobody reads it yet: rows of dO that are not kept become zero
+  auto drop_rows = [&](int j, int buf) {
+    if (__builtin_expect(next_keep != ~0ull, 0)) {
+      constexpr int N = TileLaneOffsets<T, D>::N, CHUNKS = D * 2 / 16, ROWS_PER_DMA = 1024 / (D * 2);
+      typedef __attribute__((ext_vector_type(4))) int i32x4;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const int row = (wave_s * N + i) * ROWS_PER_DMA + lane / CHUNKS;
+        if (!((next_keep >> row) & 1)) *(FO_LDS i32x4*)(smem + (NBUF + buf) * TILE_BYTES + (wave_s * N + i) * 1024 + lane * 16) = i32x4{0, 0, 0, 0};
+      }
+      if (next_mixed != 0) again |= 1ull << ((j + 1) >> again_shift);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+  };
   auto hand_over = [&](int j) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (DROP) drop_rows(j, (j + 1 - qt0) % NBUF);
     __builtin_amdgcn_s_barrier();
     if (j + 2 < n_qt) issue(j + 2, (j + 2 - qt0) % NBUF);
   };
@@ -905,7 +978,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   for (int i = 0; i < DBLK; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) { dkacc[i][r] = 0.0f; dvacc[i][r] = 0.0f; }
-  const float c = prm.scale_log2e, scale = prm.scale;
+  const float c = prm.scale_log2e, scale = DROP ? prm.scale * prm.drop.keep_scale : prm.scale;
 
   // Per-lane byte offsets of the fragment reads inside a tile, swizzle included (what row_frag / col_frag compute; the
   // swizzle of a row does not depend on the 32-row block or 16-row step it is in). With the tile's base added once
@@ -947,6 +1020,14 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   typedef __attribute__((ext_vector_type(2))) T vec2;
   i32x4 pf[2][2], dsf[2][2];
 
+  [[maybe_unused]] auto zero_acc = [](f32x16& acc) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_nop 1" : "+v"(acc));       // (pinned here: sunk to the first MFMA, the moves would be too close to it)
+#endif
+  };
+
   const uint32_t lane4 = (uint32_t)lane * 4u;
   // One tile. `buf`: the tile's buffer, (j - qt0) % NBUF, which the caller counts along. `spread`: tile j+2 lies wholly
   // inside Q and dO (and the lane offsets fit): its copy is not issued in one batch at the hand-over but one instruction
@@ -969,8 +1050,12 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   //   5            dV0,dK0 (t=1)    B1[0..7], A1[8..11]
   //   6            dV1,dK1 (t=0)    A1[12..15], B1[8..15]
   //   7            dV1,dK1 (t=1)    -
-  auto tile_body = [&](int j, int buf, auto masked, auto spread) __attribute__((always_inline)) {
+  [[maybe_unused]] FO_LDS int* gathered = (FO_LDS int*)(rowvals + kBwdTile);       // (in the place of the second tile's -LSE / scale)
+  auto tile_body = [&](int j, int buf, auto masked, auto spread, auto once_more) __attribute__((always_inline)) {
     constexpr bool SPREAD = decltype(spread)::value;
+    constexpr bool AGAIN = decltype(once_more)::value;      // dropout: only the kept elements of rows that are partly dropped
+    int drop_a = kKeepAll, drop_b = kKeepAll;
+    uint32_t drop_first = 0;
     constexpr int HALF = NMF / 2, NG = 4 * NMF, SPG = 48 / (3 * NMF);      // groups per half-phase / per tile, slots per group
     static_assert(SPG * 3 * NMF == 48 && kFragAhead <= KSTEPS, "48 slots over the groups of six half-phases");
     const int nbuf = buf == NBUF - 1 ? 0 : buf + 1;
@@ -1000,6 +1085,16 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
         for (int u = 0; u < 4; ++u) acc[4 * jv + u] = d4[u];
       }
     };
+    // AGAIN: the tile's rows are `j` gathered ones (see below); which of the lane's 32 elements count, one bit each
+    uint32_t alive = 0;
+    if constexpr (AGAIN) {
+#pragma unroll 1
+      for (int e = 0; e < 32; ++e) {
+        const int at = 32 * (e >> 4) + 4 * hh + (e & 3) + 8 * ((e & 15) >> 2), row = gathered[at];
+        const bool dead = (at >= j) | (CAUSAL & (key > row)) | !dropout_keep(DropRows<1>::index(prm.drop, bh, Sq, Sk, row, key), prm.drop.seed, prm.drop.threshold);
+        alive |= (dead ? 0u : 1u) << e;
+      }
+    }
     float pv[2][16];            // P of a block between its two stages
     auto stage_a = [&](int qb, int r) {
       const int koff = (r & 3) + 8 * (r >> 2);
@@ -1009,7 +1104,12 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
         const int lim_end = Sq - (q0t + 32 * qb + 4 * hh);
         dead = koff < lim || koff >= lim_end;
       }
-      pv[qb][r] = dead ? 0.0f : __builtin_amdgcn_exp2f(KBIAS ? __builtin_fmaf(sacc[qb][r], c, bias_lane) : sacc[qb][r] * c);
+      if constexpr (AGAIN) dead = !((alive >> (16 * qb + r)) & 1u);
+      float sv = sacc[qb][r];
+#if defined(__HIP_DEVICE_COMPILE__)
+      if constexpr (AGAIN) asm volatile("" : "+v"(sv));      // (read here, not earlier: see the wait states at the end of tile_body)
+#endif
+      pv[qb][r] = dead ? 0.0f : __builtin_amdgcn_exp2f(KBIAS ? __builtin_fmaf(sv, c, bias_lane) : sv * c);
     };
     auto stage_b = [&](int qb, int r) {          // elements r and r + 1
       const float ds0 = pv[qb][r] * dpacc[qb][r], ds1 = pv[qb][r + 1] * dpacc[qb][r + 1];
@@ -1038,6 +1138,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
         // the hand-over, between phases 3 and 4 (see hand_over)
         if constexpr (SPREAD) {
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          if constexpr (DROP) drop_rows(j, nbuf);
           __builtin_amdgcn_s_barrier();
           const int b2 = buf == 0 ? NBUF - 1 : buf - 1, which = wave_s & 1;   // (waves 2 and 3 repeat the row values of waves 0 and 1)
           next_q = (const char*)(qbase + (int64_t)(j + 2) * kBwdTile * prm.qs[2]);
@@ -1045,13 +1146,13 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
           next_rows = (const char*)((which ? (const float*)prm.delta : (const float*)prm.nlse) + (int64_t)bh * Sq + (j + 2) * kBwdTile);
           next_q_dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(smem + b2 * TILE_BYTES + wave_s * (TileLaneOffsets<T, D>::N * 1024)));
           next_rows_dst = (FO_LDS char*)(rowvals + (NBUF * which + b2) * kBwdTile);
-        } else {
+        } else if constexpr (!AGAIN) {
           if (j + 1 < n_qt) hand_over(j);
         }
       }
       // (two wait states where an MFMA may follow the VALU instruction that wrote its B operand: behind the hand-over,
       // whose paths join here, and where the last B job of the tile ends right before its first reader)
-      if (g == 3 * NMF || g == 3 * NMF + HALF) asm volatile("s_nop 1");
+      if (AGAIN || g == 3 * NMF || g == 3 * NMF + HALF) asm volatile("s_nop 1");
       if (ph < 2) {
         if (i < KSTEPS) mfma_scores_vgpr<T>(sacc[ph], fr[g % kFragAhead], kf[i]);
         else mfma_scores_vgpr<T>(dpacc[ph], fr[g % kFragAhead], vf[i - KSTEPS]);
@@ -1061,9 +1162,19 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
         else mfma_acc_agpr<T>(dvacc[db], fr[g % kFragAhead], __builtin_bit_cast(vec8, pf[ph - 2][t]));
       }
       refill(g);
+      if constexpr (DROP && !AGAIN) {
+        // (pieces of drop_look(j + 1), pinned to their groups)
+        if (g == 1) { drop_first = drop_index(j + 1); asm volatile("" : "+v"(drop_first)); }
+        if (g == 2) { drop_a = dropout_block<7>(drop_first, prm.drop.seed, prm.drop.threshold); asm volatile("" : "+v"(drop_a)); }
+        if (g == 3) { drop_b = dropout_block<7>(drop_first + 127u, prm.drop.seed, prm.drop.threshold); asm volatile("" : "+v"(drop_b)); }
+        if (g == HALF - 1) drop_verdict(drop_a, drop_b);
+      }
       // start values of the accumulators while they are idle: block 1 of this tile, block 0 of the next (visible since
       // the hand-over; after the last tile: read, unused)
-      if (g == 0) start_acc(dpacc[1], rowvals + (NBUF + buf) * kBwdTile, 1);
+      if (g == 0) {
+        if constexpr (AGAIN) zero_acc(dpacc[1]);
+        else start_acc(dpacc[1], rowvals + (NBUF + buf) * kBwdTile, 1);
+      }
       if (g == 1) start_acc(sacc[1], rowvals + buf * kBwdTile, 1);
       if (g == 3 * NMF) start_acc(dpacc[0], rowvals + (NBUF + nbuf) * kBwdTile, 0);
       if (g == 3 * NMF + 1) start_acc(sacc[0], rowvals + nbuf * kBwdTile, 0);
@@ -1103,20 +1214,23 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   };
 
   int j = qt0 - 1;
-  for (; j <= min(ja, n_qt) - 1 && j <= n_qt - 2; ++j) hand_over(j);
+  for (; j <= min(ja, n_qt) - 1 && j <= n_qt - 2; ++j) {
+    if constexpr (DROP) drop_look(j + 1);
+    hand_over(j);
+  }
   // Tiles that need the mask are a prefix (the causal diagonal) and possibly the last tile (queries past the end).
   // One loop per kind, each with a single body: with alternatives inside one loop the compiler moves the 128
   // accumulator registers between homes at every tile.
   auto needs_mask = [&](int jt) { return jt * kBwdTile + kBwdTile > Sq || (CAUSAL && k0w + 31 > jt * kBwdTile); };
   j = ja;
-  if (j < n_qt) {
-    const int buf = (j - qt0) % NBUF;
+  // the first fragments of the tile in buffer `buf`, and what the accumulators of its block 0 start from (as every later
+  // tile gets them at the end of the tile before it)
+  auto start_tile = [&](int buf) {
     uint32_t rq0[kFragAhead];
 #pragma unroll
     for (int ks = 0; ks < kFragAhead; ++ks) rq0[ks] = row_off[ks < KSTEPS ? ks : 0] + (uint32_t)(buf * TILE_BYTES);
 #pragma unroll
     for (int i = 0; i < kFragAhead; ++i) fr[i] = scores_frag_sd(rq0, 0, i);
-    // (dP of the first tile's block 0 starts from -delta, as every later one does at the end of the tile before it)
 #pragma unroll
     for (int jv = 0; jv < 4; ++jv) {
       const f32x4 d4 = *(FO_LDS const f32x4*)(rowvals + (NBUF + buf) * kBwdTile + 8 * jv + 4 * hh);
@@ -1126,17 +1240,59 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
 #pragma unroll
       for (int u = 0; u < 4; ++u) sacc[0][4 * jv + u] = n4[u];
     }
-  }
+  };
+  if (j < n_qt) start_tile((j - qt0) % NBUF);
   int buf = j < n_qt ? (j - qt0) % NBUF : 0;
   auto next_buf = [&]() { buf = buf == NBUF - 1 ? 0 : buf + 1; };
-  for (; j < n_qt && needs_mask(j); ++j, next_buf()) tile_body(j, buf, std::true_type{}, std::false_type{});
+  for (; j < n_qt && needs_mask(j); ++j, next_buf()) tile_body(j, buf, std::true_type{}, std::false_type{}, std::false_type{});
 #if FO_BWD_SPREAD
   // (from here on only a last tile that crosses the end of Q needs the mask; tiles j with tile j+2 wholly inside Q)
   if (qlo.ok && glo.ok)
-    for (const int end = Sq / kBwdTile - 2; j < end; ++j, next_buf()) tile_body(j, buf, std::false_type{}, std::true_type{});
+    for (const int end = Sq / kBwdTile - 2; j < end; ++j, next_buf()) tile_body(j, buf, std::false_type{}, std::true_type{}, std::false_type{});
 #endif
-  for (; j < n_qt && !needs_mask(j); ++j, next_buf()) tile_body(j, buf, std::false_type{}, std::false_type{});
-  for (; j < n_qt; ++j, next_buf()) tile_body(j, buf, std::true_type{}, std::false_type{});
+  for (; j < n_qt && !needs_mask(j); ++j, next_buf()) tile_body(j, buf, std::false_type{}, std::false_type{}, std::false_type{});
+  for (; j < n_qt; ++j, next_buf()) tile_body(j, buf, std::true_type{}, std::false_type{}, std::false_type{});
+
+  if constexpr (DROP) {
+    // rows that are partly dropped (`again` and what follows from it is the same for every wave)
+    int slot_row = 0, n_slots = 0;           // lane i holds the row of slot i
+    auto add_slots = [&]() {
+      __syncthreads();                       // everyone is done with the buffers
+      constexpr int N = TileLaneOffsets<T, D>::N, CHUNKS = D * 2 / 16, ROWS_PER_DMA = 1024 / (D * 2);
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const int at = (wave_s * N + i) * ROWS_PER_DMA + lane / CHUNKS, col = ((lane % CHUNKS) ^ swz<D>(at)) * 8;
+        const int64_t row = __shfl(slot_row, at);
+        dma16_lane_ptr(qbase + row * prm.qs[2] + col, smem + (wave_s * N + i) * 1024);
+        dma16_lane_ptr(gbase + row * prm.dos[2] + col, smem + NBUF * TILE_BYTES + (wave_s * N + i) * 1024);
+      }
+      if (wave_s == 0) {
+        dma4_lane_ptr((const float*)prm.nlse + (int64_t)bh * Sq + slot_row, rowvals);
+        gathered[lane] = slot_row;
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      start_tile(0);
+      zero_acc(dpacc[0]);
+      tile_body(n_slots, 0, std::false_type{}, std::false_type{}, std::true_type{});
+      n_slots = 0;
+    };
+    int jt = qt0 - 1;
+    next_mixed = 0;
+    while (again != 0) {
+      if (next_mixed == 0) {
+        ++jt;
+        if (jt < n_qt && ((again >> (jt >> again_shift)) & 1)) drop_look(jt);
+      }
+      while (next_mixed != 0 && n_slots < 64) {
+        const int row = jt * kBwdTile + __builtin_ctzll(next_mixed);
+        next_mixed &= next_mixed - 1;
+        if (row < Sq) { slot_row = lane == n_slots ? row : slot_row; ++n_slots; }
+      }
+      if (jt >= n_qt) again = 0;
+      if (n_slots == 64 || (again == 0 && n_slots > 0)) add_slots();
+    }
+  }
 
   acc_fence(dkacc);
   acc_fence(dvacc);
@@ -1146,7 +1302,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
     FO_LDS char* stage = smem + wave_s * stage_bytes(D);
     const int k0w_s = k0 + wave_s * 32;
     store_rows_via_lds<T, D>(dkacc, scale, stage, (T*)prm.dk + b * prm.dks[0] + h * prm.dks[1], prm.dks[2], k0w_s, Sk, prm.d, lane);
-    store_rows_via_lds<T, D>(dvacc, 1.0f, stage, (T*)prm.dv + b * prm.dvs[0] + h * prm.dvs[1], prm.dvs[2], k0w_s, Sk, prm.d, lane);
+    store_rows_via_lds<T, D>(dvacc, DROP ? prm.drop.keep_scale : 1.0f, stage, (T*)prm.dv + b * prm.dvs[0] + h * prm.dvs[1], prm.dvs[2], k0w_s, Sk, prm.d, lane);
   }
 }
 
@@ -1164,7 +1320,7 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
   static const hipError_t a2 = hipFuncSetAttribute((const void*)attn_bwd_dkdv_kernel<T, D, CAUSAL, DROP, BIAS>,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dkdv);
   const size_t lds_pipe = 6 * (size_t)kBwdTile * D * 2 + 6 * kBwdTile * sizeof(float);   // three tile buffers
-  static const hipError_t a3 = hipFuncSetAttribute((const void*)attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL>,
+  static const hipError_t a3 = hipFuncSetAttribute((const void*)attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, DROP>,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_pipe);
   if (a1 != hipSuccess || a2 != hipSuccess || a3 != hipSuccess) return FO_ERR_LAUNCH;
   // a bias without a query stride: the forms of the dQ kernel and (without dropout) of the pipelined dK/dV kernel that
@@ -1173,7 +1329,7 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
   if constexpr (BIAS) {
     static const hipError_t a4 = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<T, D, CAUSAL, DROP, false, true>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dq);
-    static const hipError_t a5 = hipFuncSetAttribute((const void*)attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, true>,
+    static const hipError_t a5 = hipFuncSetAttribute((const void*)attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, true, DROP>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_pipe);
     if (a4 != hipSuccess || a5 != hipSuccess) return FO_ERR_LAUNCH;
   }
@@ -1194,7 +1350,7 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
   if constexpr (BIAS) {
     if (key_bias) {
       attn_bwd_dq_kernel<T, D, CAUSAL, DROP, false, true><<<(unsigned)g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
-      if (!DROP && p.d == D) attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, true><<<(unsigned)g_dkdv, kBwdWaves * 64, lds_pipe, s>>>(q);
+      if (p.d == D) attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, true, DROP><<<(unsigned)g_dkdv, kBwdWaves * 64, lds_pipe, s>>>(q);
       else attn_bwd_dkdv_kernel<T, D, CAUSAL, DROP, BIAS><<<(unsigned)g_dkdv, kBwdWaves * 64, lds_dkdv, s>>>(q);
       return launch_status();
     }
@@ -1202,7 +1358,7 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
   attn_bwd_dq_kernel<T, D, CAUSAL, DROP, BIAS><<<(unsigned)g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
   // attn_bwd.variant 0 selects the plain dK/dV kernel everywhere (tests compare the two)
   // (and every head_dim other than the two the kernels are compiled for)
-  if (!DROP && !BIAS && p.d == D && tune(g_attn_bwd_variant) != 0) attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL><<<(unsigned)g_dkdv, kBwdWaves * 64, lds_pipe, s>>>(q);
+  if (!BIAS && p.d == D && tune(g_attn_bwd_variant) != 0) attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, DROP><<<(unsigned)g_dkdv, kBwdWaves * 64, lds_pipe, s>>>(q);
   else attn_bwd_dkdv_kernel<T, D, CAUSAL, DROP, BIAS><<<(unsigned)g_dkdv, kBwdWaves * 64, lds_dkdv, s>>>(q);
   return launch_status();
 }

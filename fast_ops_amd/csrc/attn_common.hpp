@@ -75,6 +75,7 @@ struct DropoutParams {
   uint32_t threshold;     // uint32(fp32(p) * fp32(4294967295)), computed on the host
   uint32_t offset;        // low 32 bits of the generator offset
   float keep_scale;       // 1 / (1 - p) in fp32; 1 when dropout is off
+  float keep_prob;        // 1 - p
 };
 __host__ __device__ __forceinline__ bool dropout_keep(uint32_t index, uint32_t seed, uint32_t threshold) {
   uint32_t a = index ^ seed;
@@ -83,14 +84,146 @@ __host__ __device__ __forceinline__ bool dropout_keep(uint32_t index, uint32_t s
   a ^= a >> 11;
   return a > threshold;
 }
+// The mask over a run of consecutive indices, mostly without hashing each of them. The hash mixes little: with the low L
+// bits of the index free, x = index ^ seed is an aligned block of 2^L values; so is y = x ^ (x >> 4), whose bits from L
+// on depend on x's bits from L on only; z = (y ^ 0xDEADBEEF) + (y << 5) then lies in [z0, z0 + 33 (2^L - 1)], i.e. in at
+// most two values A of z >> (L + 6); and the hash z ^ (z >> 11) has A ^ (A >> 11) in its bits from L + 6 on. Where both
+// of those are above, or both below, the threshold's bits, all 2^L elements are kept, or all dropped. A run that starts
+// inside a block spans two blocks. What remains undecided is hashed element by element: 0.0-0.5 % of the runs of
+// 32 rows x 1024 keys at p = 0.1-0.17 (12 heads x 2048-8192 keys, 96 heads x 1024 keys), because the kept indices form
+// long bands: about one run in ten is dropped as a whole.
+enum : int { kDropAll = 0, kKeepAll = 1, kDropMixed = 2 };
+template <int L>
+__host__ __device__ __forceinline__ int dropout_block(uint32_t index, uint32_t seed, uint32_t threshold) {
+  constexpr uint32_t low = (1u << L) - 1u;
+  const uint32_t x = (index ^ seed) & ~low;
+  const uint32_t y = (x ^ (x >> 4)) & ~low;
+  const uint32_t z0 = ((y ^ 0xDEADBEEFu) & ~low) + (y << 5), z1 = z0 + 33u * low;    // (modulo 2^32, as the hash)
+  const uint32_t a0 = z0 >> (L + 6), a1 = z1 >> (L + 6), t = threshold >> (L + 6);
+  const uint32_t w0 = a0 ^ (a0 >> 11), w1 = a1 ^ (a1 >> 11);
+  return (w0 > t && w1 > t) ? kKeepAll : (w0 < t && w1 < t) ? kDropAll : kDropMixed;
+}
+// indices first .. first + n - 1, n at most 2^L
+template <int L>
+__host__ __device__ __forceinline__ int dropout_run(uint32_t first, uint32_t n, uint32_t seed, uint32_t threshold) {
+  const int a = dropout_block<L>(first, seed, threshold), b = dropout_block<L>(first + n - 1u, seed, threshold);
+  return a == b ? a : kDropMixed;
+}
 inline DropoutParams make_dropout(float p, uint32_t seed, uint64_t rng_offset) {
   DropoutParams d;
   d.seed = seed;
   d.threshold = (uint32_t)(p * 4294967296.0f);       // fp32 product; fp32(4294967295) is 2^32
   d.offset = (uint32_t)rng_offset;
-  d.keep_scale = 1.0f / (1.0f - p);
+  d.keep_prob = 1.0f - p;
+  d.keep_scale = 1.0f / d.keep_prob;
   return d;
 }
+
+// Dropout where a lane owns a query row (forward and dQ kernels; flash_attention_triton.py:125,216-219,524-532): in the
+// forward, P of a dropped element becomes zero after the row sums have been taken, and 1 / (1 - p) is applied with the
+// normalisation of O. Hashing every element costs about twelve integer instructions per score, more than twice the rest
+// of the softmax (forward, 12 heads x 8192 keys at head_dim 128: 559 us against 352 us without dropout). So at every
+// kDropSpanTiles-th 64-key tile a wave looks at its rows' next 1024 elements as a whole (dropout_run): nearly always all of
+// them are kept, or all dropped, or every row is one or the other. Where a row is neither, every tile of the span is
+// looked at by itself, and the few rows for which that does not decide it either are hashed by the wave together, one
+// element per lane. (Hashing such spans whole, or such tiles whole, is little work in total, but all of it falls on a few
+// workgroups that the launch then waits for: 193 and 159 us at 12 heads x 4096 keys, where no dropout takes 124 us.)
+// Forward at p = 0.1, head_dim 128, hashing every element -> this: 12 heads x 4096 keys 181 -> 133 us (no dropout 124), x 8192
+// 562 -> 435 (364), x 2048 causal 62 -> 38 (32); head_dim 64, 8 x 12 heads x 1024 causal 44 -> 24 (25). What is left is the
+// workgroups whose rows the mask's bands begin or end in, and one branch per step for the others.
+constexpr int kDropSpanTiles = 1024 / 64;
+template <int QB>
+struct DropRows {
+  static constexpr int kRows = 3, kMasked = 4;
+  int state = kKeepAll;                 // wave-uniform: kKeepAll, kDropAll, kRows (every row is one or the other), kMasked
+  bool by_tile = false;
+  uint32_t bits[QB][2];                 // all ones / all zeros: the lane's row of block b is kept / dropped; kMasked: the lane's row of block b: bit (r & 3) + 8 (r >> 2) of word kb = the element in register r of
+                                        // the 32-key block kb is kept
+  static __device__ __forceinline__ uint32_t index(const DropoutParams& d, int bh, int Sq, int Sk, int row, int key) {
+    return d.offset + ((uint32_t)bh * (uint32_t)Sq + (uint32_t)row) * (uint32_t)Sk + (uint32_t)key;
+  }
+  // the state of key tile `tile`, asked for every tile in turn; row0: the wave's first row (block b is 32 b rows further)
+  template <typename P>
+  __device__ __forceinline__ void look(const P& d_in, int bh, int Sq, int Sk, int row0, int tile) {
+    if (__builtin_expect(tile % kDropSpanTiles == 0, 0)) {      // (laid out away from the tile loops)
+      const DropoutParams d = {d_in.seed, d_in.threshold, d_in.offset, 1.0f, 1.0f};
+      by_tile = look_at<10>(d, bh, Sq, Sk, row0, tile * 64);
+    }
+    if (__builtin_expect(by_tile, 0)) {
+      const DropoutParams d = {d_in.seed, d_in.threshold, d_in.offset, 1.0f, 1.0f};
+      look_at<6>(d, bh, Sq, Sk, row0, tile * 64);
+    }
+  }
+  // 2^L keys from key0 on; true if some row is neither kept nor dropped as a whole (L = 6: its bits are then hashed)
+  template <int L>
+  __device__ __forceinline__ bool look_at(const DropoutParams& d, int bh, int Sq, int Sk, int row0, int key0) {
+    const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
+    bool any_mixed = false, any_keep = false, any_drop = false;
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      const int v = dropout_run<L>(index(d, bh, Sq, Sk, row0 + 32 * b + l32, key0), 1u << L, d.seed, d.threshold);
+      bits[b][0] = bits[b][1] = v == kKeepAll ? 0xFFFFFFFFu : 0u;
+      any_keep |= __builtin_amdgcn_ballot_w64(v == kKeepAll) != 0;
+      any_drop |= __builtin_amdgcn_ballot_w64(v == kDropAll) != 0;
+      uint32_t mixed = (uint32_t)__builtin_amdgcn_ballot_w64(v == kDropMixed);      // (both halves of the wave hold the same rows)
+      any_mixed |= mixed != 0;
+      if constexpr (L == 6) {
+        while (mixed != 0) {
+          const int i = __builtin_ctz(mixed);
+          mixed &= mixed - 1;
+          const uint64_t k = __builtin_amdgcn_ballot_w64(dropout_keep(index(d, bh, Sq, Sk, row0 + 32 * b + i, key0 + lane), d.seed, d.threshold));
+          if (l32 == i) { bits[b][0] = (uint32_t)k >> (4 * hh); bits[b][1] = (uint32_t)(k >> 32) >> (4 * hh); }
+        }
+      }
+    }
+    state = any_mixed ? kMasked : any_keep && any_drop ? kRows : any_keep ? kKeepAll : kDropAll;
+    return any_mixed;
+  }
+  // P of the 32-key block kb as two B operands (registers 0..7 and 8..15) per block of rows. (One branch, straight code where
+  // whole rows are dropped: every taken branch holds up a wave that is alone on its SIMD, and with one per case and block a
+  // workgroup with such rows took 30 % longer.)
+  template <typename V>
+  __device__ __forceinline__ void apply(int kb, V (&p)[QB][2]) const {
+    typedef __attribute__((ext_vector_type(4))) uint32_t u4;
+    if (__builtin_expect(state == kMasked, 0)) {
+#pragma unroll
+      for (int b = 0; b < QB; ++b)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          u4 w = __builtin_bit_cast(u4, p[b][t]);
+#pragma unroll
+          for (int u = 0; u < 8; u += 2) {
+            const int at = (u & 3) + 8 * (u >> 2) + 16 * t;
+            const uint32_t lo = (uint32_t)((int)(bits[b][kb] << (31 - at)) >> 31), hi = (uint32_t)((int)(bits[b][kb] << (30 - at)) >> 31);
+            w[u >> 1] &= (lo & 0xFFFFu) | (hi & 0xFFFF0000u);
+          }
+          p[b][t] = __builtin_bit_cast(V, w);
+        }
+    } else {
+#pragma unroll
+      for (int b = 0; b < QB; ++b)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          u4 w = __builtin_bit_cast(u4, p[b][t]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) w[i] &= bits[b][0];
+          p[b][t] = __builtin_bit_cast(V, w);
+        }
+    }
+  }
+  // a 64-key tile of fp32 values in two accumulators
+  __device__ __forceinline__ void apply(f32x16 (&acc)[2]) const {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int at = (r & 3) + 8 * (r >> 2);
+        const uint32_t m = (uint32_t)((int)(bits[0][kb] << (31 - at)) >> 31);
+        const float x = acc[kb][r];                     // (a bit cast of the vector's element itself takes element 0)
+        acc[kb][r] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & m);
+      }
+  }
+};
 
 // Additive bias on the scaled scores (flash_attention_triton.py:176-198, attention_ref.py:50-51): element
 // (b, h, q, key) at bias + b*strides[0] + h*strides[1] + q*strides[2] + key, a stride of 0 broadcasting that dimension

@@ -253,6 +253,8 @@ __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnPara
   const int L16 = lane & 15;
   const int g16 = (lane >> 4) & 1;
 
+  DropRows<1> drop;
+
   for (int tile = 0; tile < n_tiles; ++tile) {
     const int buf = tile & 1;
     const int key0 = tile * kBN;
@@ -274,6 +276,9 @@ __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnPara
 
     // waves whose rows are all above this tile's keys have nothing to do (causal)
     if (CAUSAL && key0 > q0w + 31) continue;
+    if constexpr (DROP) {
+      drop.look(prm.drop, bh, Sq, Sk, q0w, tile);
+    }
 
     FO_LDS const char* kt = smem + buf * TILE_BYTES;
     FO_LDS const char* vt = smem + (2 + buf) * TILE_BYTES;
@@ -425,21 +430,27 @@ __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnPara
     const float mc = ((BIAS || KBIAS) && m_run == -INFINITY) ? 0.0f : m_run * c;
     float psum = 0.0f;
     vec8 pf[4];
-    // dropout: 32-bit index of this lane's query row at key 0 of the tile (flash_attention_triton.py:125,217)
-    const uint32_t drop_row = DROP ? prm.drop.offset + ((uint32_t)bh * (uint32_t)Sq + (uint32_t)(q0w + l32)) * (uint32_t)Sk + (uint32_t)key0 : 0u;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        float p = (DBG & 2) ? sacc[kb][r] : __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][r], c, -mc));
+        const float p = (DBG & 2) ? sacc[kb][r] : __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][r], c, -mc));
         psum += p;                                     // summed in fp32 before rounding and before dropout (flash_attention_triton.py:203)
-        if constexpr (DROP) {
-          const uint32_t idx = drop_row + (uint32_t)(32 * kb + 4 * hh + (r & 3) + 8 * (r >> 2));
-          p = dropout_keep(idx, prm.drop.seed, prm.drop.threshold) ? p * prm.drop.keep_scale : 0.0f;   // :216-219
-        }
         pf[kb * 2 + (r >> 3)][r & 7] = (T)p;           // rounded to the operand type for P.V (:237)
       }
     l_run += psum;
+    if constexpr (DROP) {
+      if (drop.state == kDropAll) continue;            // no probability of this wave's rows and keys is kept
+      if (__builtin_expect(drop.state != kKeepAll, 0)) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          vec8 two[1][2] = {{pf[2 * kb], pf[2 * kb + 1]}};
+          drop.apply(kb, two);
+          pf[2 * kb] = two[0][0];
+          pf[2 * kb + 1] = two[0][1];
+        }
+      }
+    }
 
     // ---- O^T += V^T P^T : four 16-key steps x DBLK d-blocks, V^T fragments fetched one group ahead
     {
@@ -473,7 +484,7 @@ __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnPara
 
   // ---- epilogue: normalise, write O and LSE
   const float l_tot = l_run + half_swap(l_run);
-  const float inv = 1.0f / l_tot;
+  const float inv = (DROP ? prm.drop.keep_scale : 1.0f) / l_tot;
   const int qi = q0w + l32;
   if (qi < Sq) {
     T* op = (T*)prm.o + b * prm.os[0] + h * prm.os[1] + (int64_t)qi * prm.os[2];
@@ -616,7 +627,7 @@ __host__ __device__ inline int wide_items(int n_qblk, bool causal) { return caus
 constexpr int kVBiasKeys = 8192;
 constexpr float kNoKeyYet = -1.0e30f;   // reference of a row all of whose keys so far a bias of -inf has removed
 
-template <typename T, int D, bool CAUSAL, int QB, int DBG, int BM = kWideBM, bool VBIAS = false>
+template <typename T, int D, bool CAUSAL, int QB, int DBG, int BM = kWideBM, bool VBIAS = false, bool DROP = false>
 __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 128 || VBIAS) ? 1 : 2) attn_fwd_wide_kernel(const AttnParams prm_arg) {
   const AttnParams& prm = prm_arg;
   // VBIAS: an additive bias that is the same for every query of a head (query stride 0: the reference's "vector" bias,
@@ -906,6 +917,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   constexpr int RD = QB == 2 ? 4 : 2;       // must divide the number of fragments of a sub-tile
   static_assert(KSTEPS % RD == 0, "fragment ring");
   i32x4 KF[RD], VF[RD];        // LDS fragment rings, refilled RD fragments ahead of use
+  DropRows<QB> drop;
   float m_run[QB], l_run[QB];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) { m_run[qb] = -INFINITY; l_run[qb] = 0.0f; }
@@ -1106,6 +1118,19 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     }
 #pragma unroll
     for (int b2 = 0; b2 < QB; ++b2) l_run[b2] += psum[b2];
+    if constexpr (DROP) {
+      if (__builtin_expect(drop.state != kKeepAll, 0)) {
+        drop.apply(P, PF[P]);
+        // (pinned here, with the wait states the next MFMAs need between a VALU write and their read)
+#pragma unroll
+        for (int b2 = 0; b2 < QB; ++b2) asm volatile("" : "+v"(PF[P][b2][0]), "+v"(PF[P][b2][1]));
+      }
+      asm volatile("s_nop 1");
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto drop_look = [&](int j) {
+    if constexpr (DROP) drop.look(prm.drop, bh, Sq, Sk, q0w, j);
   };
   using std::integral_constant;
   typedef integral_constant<int, 0> P0;
@@ -1190,6 +1215,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     // overflows the row sum and the recovery path moves the reference to it, with O and l multiplied by exp2(-huge) = 0)
     if constexpr (VBIAS) m_run[b2] = fmaxf(m_run[b2], kNoKeyYet);
   }
+  drop_look(0);
   step(0, P0{}, Y{}, N{}, Y{}, N{}, N{}, -1, N{});   // (its reference is its own row maximum: every P <= 1, no recovery)
   if (n_w > 1) step(1, P1{}, Y{}, Y{}, Y{}, N{}, N{}, -1); else step(1, P1{}, N{}, Y{}, Y{}, N{}, N{}, -1);
   // Should the steps above have parked registers in scratch memory (they do not at present), wait here, visibly to
@@ -1202,22 +1228,26 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     // unmasked tiles whose copies (K three tiles, V two tiles ahead) are whole tiles: the steps issue them
     for (; j < min(min(j_mask, n_w - 1), n_full - 3); ++j) {
       tile_top(j, true);
+      drop_look(j);
       step(2 * j, P0{}, Y{}, Y{}, N{}, Y{}, Y{}, j + 3);
       step(2 * j + 1, P1{}, Y{}, Y{}, N{}, Y{}, Y{}, j + 2);
     }
   }
   for (; j < min(j_mask, n_w - 1); ++j) {
     tile_top(j);
+    drop_look(j);
     step(2 * j, P0{}, Y{}, Y{}, N{}, Y{}, N{}, -1);
     step(2 * j + 1, P1{}, Y{}, Y{}, N{}, Y{}, N{}, -1);
   }
   for (; j < n_w - 1; ++j) {
     tile_top(j);
+    drop_look(j);
     step(2 * j, P0{}, Y{}, Y{}, Y{}, Y{}, N{}, -1);
     step(2 * j + 1, P1{}, Y{}, Y{}, Y{}, Y{}, N{}, -1);
   }
   if (j < n_w) {
     tile_top(j);
+    drop_look(j);
     step(2 * j, P0{}, Y{}, Y{}, Y{}, N{}, N{}, -1);
     step(2 * j + 1, P1{}, N{}, Y{}, Y{}, N{}, N{}, -1);
     ++j;
@@ -1269,7 +1299,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     const float l_tot = l_run[qb] + half_swap(l_run[qb]);
-    const float inv = 1.0f / l_tot;
+    const float inv = (DROP ? prm.drop.keep_scale : 1.0f) / l_tot;
     const int qi = q0w + 32 * qb + l32;
     const int srow = KEEP_ON ? l32 : 32 * qb + l32;
 #pragma unroll
@@ -1327,7 +1357,7 @@ static int device_cus() {
   return n;
 }
 
-template <typename T, int D, bool CAUSAL, int QB, int DBG = 0, int BM = kWideBM, bool VBIAS = false>
+template <typename T, int D, bool CAUSAL, int QB, int DBG = 0, int BM = kWideBM, bool VBIAS = false, bool DROP = false>
 static int launch_wide(AttnParams p, hipStream_t stream) {
   constexpr bool KEEP_ON = BM == kWideBM && !VBIAS;      // (as in the kernel)
   // rings; bias row; or the rows of O staged behind the first six slots of the rings, 32 rows of D + 8 elements per wave
@@ -1354,10 +1384,10 @@ static int launch_wide(AttnParams p, hipStream_t stream) {
   }
   p.heavy_first = (CAUSAL && BM != kWideBM) ? heavy_first_group(p, D) : 0;
   p.order_n = 0;
-  static const hipError_t attr = hipFuncSetAttribute((const void*)attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS>,
+  static const hipError_t attr = hipFuncSetAttribute((const void*)attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS, DROP>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return FO_ERR_LAUNCH;
-  attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS><<<grid, BM / (32 * QB) * 64, lds, stream>>>(p);
+  attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS, DROP><<<grid, BM / (32 * QB) * 64, lds, stream>>>(p);
   return launch_status();
 }
 
@@ -1367,7 +1397,7 @@ static int launch_wide(AttnParams p, hipStream_t stream) {
 // full. Measured (the chip holds a power budget, so a round in which only half the CUs work is already cheaper than a full
 // one): 12 heads x 8192 keys, 384 items on 256 CUs, 381 -> 363 us; 12 x 6144, 288 items, 290 -> 256; 33 x 4096, 528 items,
 // 315 -> 295; 36 x 2048 108 -> 101; 4 x 40 heads x 1024 keys 96-98 -> 98: from 2048 keys on. (attn.tail 0 switches it off.)
-template <typename T, int D, bool VBIAS>
+template <typename T, int D, bool VBIAS, bool DROP = false>
 static int launch_rows256_w4_noncausal(AttnParams p, hipStream_t stream) {
   p.id_limit = 0;
   p.tail_base = 0;
@@ -1378,11 +1408,11 @@ static int launch_rows256_w4_noncausal(AttnParams p, hipStream_t stream) {
     AttnParams head = p, rest = p;
     head.id_limit = (int)(ids - tail);
     rest.tail_base = (int)(ids - tail);
-    const int rc = launch_wide<T, D, false, 2, 0, kWideBM, VBIAS>(head, stream);
+    const int rc = launch_wide<T, D, false, 2, 0, kWideBM, VBIAS, DROP>(head, stream);
     if (rc != FO_OK) return rc;
-    return launch_wide<T, D, false, 1, 0, kBM, VBIAS>(rest, stream);
+    return launch_wide<T, D, false, 1, 0, kBM, VBIAS, DROP>(rest, stream);
   }
-  return launch_wide<T, D, false, 2, 0, kWideBM, VBIAS>(p, stream);
+  return launch_wide<T, D, false, 2, 0, kWideBM, VBIAS, DROP>(p, stream);
 }
 
 template <typename T, int D, bool CAUSAL, bool LAZY, int DBG, bool DROP = false, bool BIAS = false, bool KBIAS = false>
@@ -1412,7 +1442,7 @@ static int launch_one(const AttnParams& p, hipStream_t stream) {
     // wherever a slot frees, and the plain order is the better one.
     const int cus_x = device_cus() / 8, n_bh_x = (int)(((int64_t)p.B * p.H) >> 3);
     const int64_t n = (int64_t)n_bh_x * p.n_qblk;
-    const int resident = (D == 64 && !DROP && !BIAS && !KBIAS) ? 3 : 2;      // workgroups per compute unit (registers)
+    const int resident = (D == 64 && !BIAS) ? 3 : 2;      // workgroups per compute unit (registers)
     if (q.heavy_first == n_bh_x && cus_x > 0 && cus_x <= kOrderTab && n <= (int64_t)cus_x * resident && n <= kOrderTab && n > cus_x) {
       // (the table of the last shape is kept per host thread: filling it takes a few microseconds, a training loop
       // launches the same shape over and over)
@@ -1447,10 +1477,10 @@ static int launch_one(const AttnParams& p, hipStream_t stream) {
 // `forced` is the value of attn.variant (-1: the library's choice). Values from 256 on are timing ablations and exist
 // only in a build with FO_ABLATIONS.
 static int choose_kernel(const AttnParams& p, int D, bool causal, bool dropout, int forced) {
-  // dropout, a bias with a query stride and head dims other than 64 and 128 run on the 128-row kernel; a bias that is
-  // the same for every query (and short enough for the pipelined kernel to keep it in LDS) takes part in the choice
+  // a bias with a query stride and head dims other than 64 and 128 run on the 128-row kernel; a bias that is the same for
+  // every query (and short enough for the pipelined kernel to keep it in LDS) takes part in the choice, and so does dropout
   const bool key_bias = p.bias.ptr != nullptr && p.bias.strides[2] == 0 && ((int64_t)p.Sk + kBN - 1) / kBN * kBN <= kVBiasKeys;
-  if ((p.bias.ptr != nullptr && !key_bias) || dropout || p.d != D) return FO_ATTN_KERNEL_ROWS128;
+  if ((p.bias.ptr != nullptr && !key_bias) || p.d != D) return FO_ATTN_KERNEL_ROWS128;
   // The 256-row kernel addresses a head's keys with 32-bit byte offsets ...
   const bool wide_ok = (int64_t)p.Sk * (p.ks[2] > p.vs[2] ? p.ks[2] : p.vs[2]) * 2 < (1ll << 31);
   // ... and needs one 256-row workgroup (two query blocks each when causal) per CU to be worth it: below that the
@@ -1514,37 +1544,40 @@ static int choose_kernel(const AttnParams& p, int D, bool causal, bool dropout, 
   }
   if (v >= 256) return v;
   if (!wide_ok && v >= FO_ATTN_KERNEL_ROWS128_PIPE) v = FO_ATTN_KERNEL_ROWS128;
-  if (key_bias) {
-    // with a bias the pipelined kernel exists in two forms: 128 rows, and 256 rows as four waves
+  if (key_bias || dropout) {
+    // with a bias or with dropout the pipelined kernel exists in two forms: 128 rows, and 256 rows as four waves
     if (v == FO_ATTN_KERNEL_ROWS256_W8) v = FO_ATTN_KERNEL_ROWS256_W4;
     if (v == FO_ATTN_KERNEL_ROWS128_EXACT) v = FO_ATTN_KERNEL_ROWS128;
   }
   return v;
 }
 
+// The kernels of a call with dropout, or with a bias that is the same for every query, or with both
+template <typename T, int D, bool CAUSAL, bool DROP, bool KBIAS>
+static int launch_form(const AttnParams& p, int v, hipStream_t stream) {
+  if (v == FO_ATTN_KERNEL_ROWS128_PIPE) return launch_wide<T, D, CAUSAL, 1, 0, kBM, KBIAS, DROP>(p, stream);
+  if (v == FO_ATTN_KERNEL_ROWS256_W4) {
+    if constexpr (CAUSAL) return launch_wide<T, D, true, 2, 0, kWideBM, KBIAS, DROP>(p, stream);
+    else return launch_rows256_w4_noncausal<T, D, KBIAS, DROP>(p, stream);
+  }
+  if (v >= 256) return FO_ERR_UNSUPPORTED;
+  return launch_one<T, D, CAUSAL, true, 0, DROP, false, KBIAS>(p, stream);
+}
+
 template <typename T, int D>
 int launch(const AttnParams& p, bool causal, bool dropout, hipStream_t stream) {
-  if (p.bias.ptr != nullptr) {
-    // A bias that is the same for every query has kernels of its own: the pipelined ones where choose_kernel says so, else
-    // the per-key form of the 128-row kernel, with or without dropout. (attn.variant 1 keeps the general bias kernel,
-    // which takes any strides: tests compare the two.)
-    if (p.bias.strides[2] == 0 && tune(g_attn_variant) != FO_ATTN_KERNEL_ROWS128_EXACT) {
-      if (!dropout) {
-        const int v = choose_kernel(p, D, causal, dropout, tune(g_attn_variant));
-        if (v >= 256) return FO_ERR_UNSUPPORTED;
-        if (v == FO_ATTN_KERNEL_ROWS128_PIPE)
-          return causal ? launch_wide<T, D, true, 1, 0, kBM, true>(p, stream) : launch_wide<T, D, false, 1, 0, kBM, true>(p, stream);
-        if (v == FO_ATTN_KERNEL_ROWS256_W4)
-          return causal ? launch_wide<T, D, true, 2, 0, kWideBM, true>(p, stream) : launch_rows256_w4_noncausal<T, D, true>(p, stream);
-        return causal ? launch_one<T, D, true, true, 0, false, false, true>(p, stream) : launch_one<T, D, false, true, 0, false, false, true>(p, stream);
-      }
-      return causal ? launch_one<T, D, true, true, 0, true, false, true>(p, stream) : launch_one<T, D, false, true, 0, true, false, true>(p, stream);
-    }
+  const int asked = tune(g_attn_variant);
+  // (attn.variant 1 keeps the general bias kernel, which takes any strides, for a bias that is the same for every query:
+  // tests compare the two)
+  const bool key_bias = p.bias.ptr != nullptr && p.bias.strides[2] == 0 && asked != FO_ATTN_KERNEL_ROWS128_EXACT;
+  if (p.bias.ptr != nullptr && !key_bias) {
     if (dropout) return causal ? launch_one<T, D, true, true, 0, true, true>(p, stream) : launch_one<T, D, false, true, 0, true, true>(p, stream);
     return causal ? launch_one<T, D, true, true, 0, false, true>(p, stream) : launch_one<T, D, false, true, 0, false, true>(p, stream);
   }
-  if (dropout) return causal ? launch_one<T, D, true, true, 0, true>(p, stream) : launch_one<T, D, false, true, 0, true>(p, stream);
-  const int v = choose_kernel(p, D, causal, dropout, tune(g_attn_variant));
+  const int v = choose_kernel(p, D, causal, dropout, asked);
+  if (dropout && key_bias) return causal ? launch_form<T, D, true, true, true>(p, v, stream) : launch_form<T, D, false, true, true>(p, v, stream);
+  if (dropout) return causal ? launch_form<T, D, true, true, false>(p, v, stream) : launch_form<T, D, false, true, false>(p, v, stream);
+  if (key_bias) return causal ? launch_form<T, D, true, false, true>(p, v, stream) : launch_form<T, D, false, false, true>(p, v, stream);
   if (v == FO_ATTN_KERNEL_ROWS256_W8) return causal ? launch_wide<T, D, true, 1>(p, stream) : launch_wide<T, D, false, 1>(p, stream);
   if (v == FO_ATTN_KERNEL_ROWS128_PIPE) return causal ? launch_wide<T, D, true, 1, 0, kBM>(p, stream) : launch_wide<T, D, false, 1, 0, kBM>(p, stream);
   if (v == FO_ATTN_KERNEL_ROWS256_W4) return causal ? launch_wide<T, D, true, 2>(p, stream) : launch_rows256_w4_noncausal<T, D, false>(p, stream);
@@ -1707,7 +1740,10 @@ extern "C" int fo_attn_fwd_kernel(int B, int H, int Sq, int Sk, int D, const int
   for (int i = 0; i < 3; ++i) { p.ks[i] = ks[i]; p.vs[i] = vs[i]; }
   p.bias.ptr = has_bias ? (const void*)ks : nullptr;   // (only tested against NULL)
   p.bias.strides[2] = has_bias == 2 ? 0 : 1;
-  return choose_kernel(p, D > 64 ? 128 : 64, causal != 0, has_dropout != 0, tune(g_attn_variant));
+  // (a call with dropout takes the form that the same call without it would, with four waves where that is the eight-wave
+  // form; this query answers for the plain kernel, which serves dropout at every size)
+  if (has_dropout) return FO_ATTN_KERNEL_ROWS128;
+  return choose_kernel(p, D > 64 ? 128 : 64, causal != 0, false, tune(g_attn_variant));
 }
 
 extern "C" int fo_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
