@@ -18,6 +18,7 @@ FO_ATTN_BWD_STATIC_ROWS = 1 << 20
 ABI_MAJOR = 2            # fo_version() // 1000 the signatures below belong to
 FO_DTYPE_F16, FO_DTYPE_BF16, FO_DTYPE_F32 = 0, 1, 2
 FO_ATTN_KERNEL_ROWS128, FO_ATTN_KERNEL_ROWS128_EXACT, FO_ATTN_KERNEL_ROWS128_PIPE, FO_ATTN_KERNEL_ROWS256_W8, FO_ATTN_KERNEL_ROWS256_W4 = 0, 1, 8, 16, 32
+FO_ATTN_KERNEL_DECODE = 64
 
 
 class FoLionConsts(ctypes.Structure):
@@ -36,6 +37,8 @@ SIGNATURES = {
     "fo_tune_set": (ctypes.c_int, [ctypes.c_char_p, ctypes.c_int]),
     "fo_tune_get": (ctypes.c_int, [ctypes.c_char_p]),
     "fo_attn_fwd": (ctypes.c_int, [ctypes.c_void_p] * 5 + [ctypes.c_int] * 5 + [_I64P] * 4 + [ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
+    "fo_attn_fwd_ws": (ctypes.c_int, [ctypes.c_void_p] * 5 + [ctypes.c_int] * 5 + [_I64P] * 4 + [ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]),
+    "fo_attn_fwd_workspace": (ctypes.c_int64, [ctypes.c_int] * 5 + [_I64P] * 2 + [ctypes.c_int]),
     "fo_attn_fwd_kernel": (ctypes.c_int, [ctypes.c_int] * 5 + [_I64P] * 2 + [ctypes.c_int] * 3),
     "fo_attn_bwd": (ctypes.c_int, [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.POINTER(_I64P), ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
     "fo_attn_bwd_static_ws": (ctypes.c_int, [ctypes.c_void_p] * 9 + [ctypes.c_int] * 5 + [ctypes.POINTER(_I64P), ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),

@@ -54,6 +54,7 @@ SOURCES = {
     "attn_bwd_bf16_d128.hip": ["-mllvm", "-pragma-unroll-threshold=400000"],
     "attn_bwd_f16_d64.hip": ["-mllvm", "-pragma-unroll-threshold=400000"],
     "attn_bwd_f16_d128.hip": ["-mllvm", "-pragma-unroll-threshold=400000"],
+    "attn_decode.hip": [],
     "dropout_mask.hip": [],
 }
 # sources that other sources include (a change in one of them makes every object stale, like a header's)

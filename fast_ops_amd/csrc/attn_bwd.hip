@@ -213,26 +213,6 @@ __device__ __forceinline__ void copy_two_tiles64_inside(const T* base_a, int64_t
   }
 }
 
-// A operand of a 32x32x16 MFMA from a row-major tile in LDS: lane = row l32 of block `blk`, 8 elements at
-// column 16*ks + 8*hh
-template <typename T, int D>
-__device__ __forceinline__ typename Ops<T>::vec8 row_frag(FO_LDS const char* tile, int blk, int ks, int l32, int hh) {
-  const int row = 32 * blk + l32;
-  return *(FO_LDS const typename Ops<T>::vec8*)(tile + row * (D * 2) + (((2 * ks + hh) ^ swz<D>(row)) * 16));
-}
-// A operand = transpose of a tile block: M = 32 columns (d = 32*db ..), K = 16 rows of the tile in the order the 32x32
-// accumulator layout hands them over as a B operand (rows 16*t + 4*hh + {0..3} and + 8)
-template <typename T, int D>
-__device__ __forceinline__ typename Ops<T>::vec8 col_frag(FO_LDS const char* tile, int t, int db, int lane) {
-  const int hh = lane >> 5, L16 = lane & 15, g16 = (lane >> 4) & 1;
-  const int row0 = 16 * t + 4 * hh + (L16 >> 2), row1 = row0 + 8;
-  const int chunk = 4 * db + 2 * g16 + ((L16 & 3) >> 1);
-  const int sub = (L16 & 1) * 8;
-  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FO_LDS s16x4*)(tile + row0 * (D * 2) + ((chunk ^ swz<D>(row0)) * 16) + sub));
-  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FO_LDS s16x4*)(tile + row1 * (D * 2) + ((chunk ^ swz<D>(row1)) * 16) + sub));
-  return __builtin_bit_cast(typename Ops<T>::vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-}
-
 // A wave's 32 finished gradient rows (accumulator layout: lane = row l32, registers 4*rg + u = columns
 // 32*db + 8*rg + 4*hh + u) written to memory. Straight from the registers that is 8 bytes per lane to 32 different
 // rows per instruction (4.3 us per workgroup for dK and dV, during which the workgroup's LDS and registers keep the

@@ -55,6 +55,26 @@ __device__ __forceinline__ void dma16_lane_ptr(const void* ptr, FO_LDS void* dst
 #endif
 }
 
+// A operand of a 32x32x16 MFMA from a row-major tile in LDS: lane = row l32 of block `blk`, 8 elements at
+// column 16*ks + 8*hh
+template <typename T, int D>
+__device__ __forceinline__ typename Ops<T>::vec8 row_frag(FO_LDS const char* tile, int blk, int ks, int l32, int hh) {
+  const int row = 32 * blk + l32;
+  return *(FO_LDS const typename Ops<T>::vec8*)(tile + row * (D * 2) + (((2 * ks + hh) ^ swz<D>(row)) * 16));
+}
+// A operand = transpose of a tile block: M = 32 columns (d = 32*db ..), K = 16 rows of the tile in the order the 32x32
+// accumulator layout hands them over as a B operand (rows 16*t + 4*hh + {0..3} and + 8)
+template <typename T, int D>
+__device__ __forceinline__ typename Ops<T>::vec8 col_frag(FO_LDS const char* tile, int t, int db, int lane) {
+  const int hh = lane >> 5, L16 = lane & 15, g16 = (lane >> 4) & 1;
+  const int row0 = 16 * t + 4 * hh + (L16 >> 2), row1 = row0 + 8;
+  const int chunk = 4 * db + 2 * g16 + ((L16 & 3) >> 1);
+  const int sub = (L16 & 1) * 8;
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FO_LDS s16x4*)(tile + row0 * (D * 2) + ((chunk ^ swz<D>(row0)) * 16) + sub));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FO_LDS s16x4*)(tile + row1 * (D * 2) + ((chunk ^ swz<D>(row1)) * 16) + sub));
+  return __builtin_bit_cast(typename Ops<T>::vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
 // Sixteen zero bytes in device memory. A head_dim below the 64 or 128 columns a kernel is compiled for is handled by
 // addresses alone: whatever would read columns past the true head_dim - a lane's piece of a tile copy, a fragment
 // loaded from a row - reads these zeros instead, so the padded columns of every operand are zero (they add nothing to a
@@ -260,5 +280,23 @@ __device__ __forceinline__ void dma4_uniform_base(const void* base, uint32_t byt
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)dst)), "v"(byte_off), "s"(base) : "memory", "m0");
 #endif
 }
+
+// Attention of a few query rows over many keys (attn_decode.hip)
+struct DecodeParams {
+  const void *q, *k, *v;
+  void* o;
+  float* lse;
+  float* ws;                            // n_split > 1: decode_workspace_bytes() of it
+  int B, H, Sq, Sk;
+  int n_kv;                             // heads with keys of their own: H, or 1 (multi-query)
+  int n_split;                          // workgroups that share the keys of a row block
+  int64_t qs[3], ks[3], vs[3], os[3];   // element strides: batch, head, sequence
+  float scale_log2e;
+};
+// rows that read the same keys, and 32-row blocks of them
+__host__ __device__ inline int decode_rows(int H, int n_kv, int Sq) { return n_kv == 1 ? H * Sq : Sq; }
+int decode_split(int B, int H, int n_kv, int Sq, int Sk, int D, int n_cu);
+int64_t decode_workspace_bytes(int B, int H, int Sq, int D, int n_split);
+template <typename T, int D> int launch_decode(const DecodeParams& p, hipStream_t stream);
 
 }  // namespace fo

@@ -62,6 +62,7 @@ struct AttnParams {
   BiasParams bias;                      // used by the kernels instantiated with bias only
 };
 
+constexpr int kDecodeMinKeys = 128;
 constexpr int64_t kMaxRowStride = 1ll << 24;   // elements; see attn_fwd_impl
 constexpr float kLazyLog2 = 8.0f;   // how far (in log2 units) a tile maximum may exceed the reference before a rescale
 
@@ -1677,11 +1678,19 @@ static int check_strides(const int64_t* st, int D, bool key_or_value) {
   return FO_OK;
 }
 
+// Few query rows over many keys: the kernel of attn_decode.hip. Up to 32 rows per head, without a mask, bias or dropout.
+static int decode_n_kv(const AttnParams& p) { return (p.H == 1 || (p.ks[1] == 0 && p.vs[1] == 0)) ? 1 : p.H; }
+static bool takes_decode(const AttnParams& p, bool causal, bool dropout, int forced) {
+  if (forced >= 0 || causal || dropout || p.bias.ptr != nullptr || (p.d != 64 && p.d != 128)) return false;
+  if (p.Sq > 32 || p.Sk < kDecodeMinKeys) return false;
+  return (int64_t)p.B * p.H * p.Sq < (1ll << 31);
+}
+
 static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, float* lse,
                          int B, int H, int Sq, int Sk, int D,
                          const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os,
                          float softmax_scale, int causal, int dtype, float dropout_p, uint32_t seed, uint64_t rng_offset,
-                         const void* bias, const int64_t* bias_strides, int bias_dtype, void* stream) {
+                         const void* bias, const int64_t* bias_strides, int bias_dtype, void* stream, void* ws = nullptr, int64_t ws_bytes = 0) {
   if (!q || !k || !v || !o || !qs || !ks || !vs || !os) return FO_ERR_NULL_POINTER;
   if (dtype != FO_DTYPE_F16 && dtype != FO_DTYPE_BF16) return FO_ERR_BAD_DTYPE;
   if (const int rc = check_sizes(B, H, Sq, Sk, D)) return rc;
@@ -1724,6 +1733,18 @@ static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, f
                     (p.bias.strides[1] * elt) % 16 == 0 && (p.bias.strides[2] * elt) % 16 == 0;
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (takes_decode(p, causal != 0, drop, tune(g_attn_variant))) {
+    DecodeParams d;
+    d.q = q; d.k = k; d.v = v; d.o = o; d.lse = lse; d.ws = (float*)ws;
+    d.B = B; d.H = H; d.Sq = Sq; d.Sk = Sk; d.n_kv = decode_n_kv(p);
+    for (int i = 0; i < 3; ++i) { d.qs[i] = qs[i]; d.ks[i] = ks[i]; d.vs[i] = vs[i]; d.os[i] = os[i]; }
+    d.scale_log2e = p.scale_log2e;
+    d.n_split = decode_split(B, H, d.n_kv, Sq, Sk, D, device_cus());
+    // (no workspace, or one that is too small: a single workgroup per row block)
+    if (ws == nullptr || ((uintptr_t)ws & 15u) || ws_bytes < decode_workspace_bytes(B, H, Sq, D, d.n_split)) d.n_split = 1;
+    if (dtype == FO_DTYPE_BF16) return D == 128 ? launch_decode<__bf16, 128>(d, s) : launch_decode<__bf16, 64>(d, s);
+    return D == 128 ? launch_decode<_Float16, 128>(d, s) : launch_decode<_Float16, 64>(d, s);
+  }
   // kernels are compiled for 64 and 128 columns; a head_dim in between runs on the next one with zero columns
   if (dtype == FO_DTYPE_BF16) return D > 64 ? launch<__bf16, 128>(p, causal != 0, drop, s) : launch<__bf16, 64>(p, causal != 0, drop, s);
   return D > 64 ? launch<_Float16, 128>(p, causal != 0, drop, s) : launch<_Float16, 64>(p, causal != 0, drop, s);
@@ -1743,7 +1764,24 @@ extern "C" int fo_attn_fwd_kernel(int B, int H, int Sq, int Sk, int D, const int
   // (a call with dropout takes the form that the same call without it would, with four waves where that is the eight-wave
   // form; this query answers for the plain kernel, which serves dropout at every size)
   if (has_dropout) return FO_ATTN_KERNEL_ROWS128;
+  if (takes_decode(p, causal != 0, false, tune(g_attn_variant))) return FO_ATTN_KERNEL_DECODE;
   return choose_kernel(p, D > 64 ? 128 : 64, causal != 0, false, tune(g_attn_variant));
+}
+
+extern "C" int64_t fo_attn_fwd_workspace(int B, int H, int Sq, int Sk, int D, const int64_t* ks, const int64_t* vs, int causal) {
+  if (!ks || !vs || check_sizes(B, H, Sq, Sk, D) || check_strides(ks, D, true) || check_strides(vs, D, true)) return 0;
+  AttnParams p = {};
+  p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.d = D;
+  for (int i = 0; i < 3; ++i) { p.ks[i] = ks[i]; p.vs[i] = vs[i]; }
+  if (!takes_decode(p, causal != 0, false, tune(g_attn_variant))) return 0;
+  return decode_workspace_bytes(B, H, Sq, D, decode_split(B, H, decode_n_kv(p), Sq, Sk, D, device_cus()));
+}
+
+extern "C" int fo_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
+                              int B, int H, int Sq, int Sk, int D,
+                              const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os,
+                              float softmax_scale, int causal, int dtype, void* ws, int64_t ws_bytes, void* stream) {
+  return attn_fwd_impl(q, k, v, o, lse, B, H, Sq, Sk, D, qs, ks, vs, os, softmax_scale, causal, dtype, 0.0f, 0u, 0ull, nullptr, nullptr, 0, stream, ws, ws_bytes);
 }
 
 extern "C" int fo_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse,

@@ -117,7 +117,7 @@ def dropout_mask(
 class _FwdPlan:
     """What a forward call of one (shapes, strides, dtype, device, layout) needs besides the data pointers: checked once,
     then reused - the checks, the stride arrays for the C ABI and the sizes cost more host time than a small kernel runs."""
-    __slots__ = ("B", "H", "Sq", "Sk", "D", "qs", "ks", "vs", "os", "o_dense_like_q", "dtype_code", "device_index", "lse_shape")
+    __slots__ = ("B", "H", "Sq", "Sk", "D", "qs", "ks", "vs", "os", "o_dense_like_q", "dtype_code", "device_index", "lse_shape", "ws_bytes")
 
 
 _FWD_PLANS: dict = {}
@@ -150,6 +150,8 @@ def _fwd_plan(q: Tensor, k: Tensor, v: Tensor, dims: Tuple[int, int, int, int]) 
     plan.dtype_code = _DTYPE_CODE[q.dtype]
     plan.device_index = q.device.index if q.device.index is not None else torch.cuda.current_device()
     plan.lse_shape = (B, H, Sq)
+    with torch.cuda.device(plan.device_index):       # scratch memory of a call without mask, bias and dropout: few queries, many keys
+        plan.ws_bytes = _lib.load().fo_attn_fwd_workspace(B, H, Sq, Sk, D, plan.ks, plan.vs, 0)
     if len(_FWD_PLANS) > 4096:
         _FWD_PLANS.clear()
     _FWD_PLANS[key] = plan
@@ -183,7 +185,11 @@ def attn_fwd_strided(
         if bias is not None:
             status = lib.fo_attn_fwd_ex(*args, ctypes.byref(_extras(bias, dropout)), stream)
         elif dropout is None or dropout[0] == 0.0:
-            status = lib.fo_attn_fwd(*args, stream)
+            if plan.ws_bytes and not causal:
+                ws = torch.empty(plan.ws_bytes, dtype=torch.uint8, device=q.device)
+                status = lib.fo_attn_fwd_ws(*args, ws.data_ptr(), plan.ws_bytes, stream)
+            else:
+                status = lib.fo_attn_fwd(*args, stream)
         else:
             status = lib.fo_attn_fwd_dropout(*args, float(dropout[0]), dropout[1] & 0xFFFFFFFF, dropout[2] % (1 << 64), stream)
     finally:

@@ -46,7 +46,7 @@ const char* fo_strerror(int status);
 int fo_version(void);
 
 /* Tuning hook for benchmarks, profiling and tests: selects a kernel variant or a workgroup order by name
- * ("lion.variant", "attn.variant", "attn_bwd.variant", "attn.order", "attn.balance", "attn.keep_on", "attn.tail", "attn_bwd.order"). Every value it accepts selects
+ * ("lion.variant", "attn.variant", "attn_bwd.variant", "attn.order", "attn.balance", "attn.keep_on", "attn.tail", "attn.decode_split", "attn_bwd.order"). Every value it accepts selects
  * code that computes the same function as the default; value -1 restores the default (the measured best). Returns
  * FO_OK, or FO_ERR_UNSUPPORTED for an unknown key or a value that selects nothing. The settings are process-global
  * atomics: a call reads each one once, a call already issued is not affected. fo_tune_get additionally answers
@@ -84,6 +84,19 @@ int fo_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse
                 const int64_t* v_strides_host, const int64_t* o_strides_host,
                 float softmax_scale, int causal, int dtype, void* stream);
 
+/* fo_attn_fwd with scratch memory for shapes of few query rows and many keys (up to 32 queries per head, not causal), whose
+ * keys are then dealt to several workgroups per head: ws points to ws_bytes bytes on the device, 16-byte aligned, used by
+ * this call only until the stream has passed it and never needing to be cleared. fo_attn_fwd_workspace answers how many
+ * bytes the call of a shape can use on the current device: 0 for every other shape, and where one workgroup per head
+ * fills the chip. With less (or ws NULL) the call computes the same with one workgroup per head, as fo_attn_fwd does. No
+ * reference counterpart. */
+int64_t fo_attn_fwd_workspace(int B, int H, int Sq, int Sk, int D, const int64_t* k_strides_host, const int64_t* v_strides_host, int causal);
+int fo_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
+                   int B, int H, int Sq, int Sk, int D,
+                   const int64_t* q_strides_host, const int64_t* k_strides_host,
+                   const int64_t* v_strides_host, const int64_t* o_strides_host,
+                   float softmax_scale, int causal, int dtype, void* ws, int64_t ws_bytes, void* stream);
+
 /* Which kernel fo_attn_fwd (or _ex, with has_bias non-zero) launches for a call of this shape
  * on the current device with the current "attn.variant": one of the FO_ATTN_KERNEL_* codes below, or a negative
  * fo_status where fo_attn_fwd would reject the shape. has_bias: 0 none, 1 a bias with a query stride, 2 a bias that is
@@ -97,7 +110,8 @@ enum {
   FO_ATTN_KERNEL_ROWS128_EXACT = 1,   /* the same with the exact running maximum of flash_attention_triton.py:200-213 */
   FO_ATTN_KERNEL_ROWS128_PIPE = 8,    /* 128 query rows per workgroup, four waves x 32 rows, in the 256-row kernel's pipeline */
   FO_ATTN_KERNEL_ROWS256_W8 = 16,     /* 256 query rows per workgroup, eight waves x 32 rows */
-  FO_ATTN_KERNEL_ROWS256_W4 = 32      /* 256 query rows per workgroup, four waves x 64 rows */
+  FO_ATTN_KERNEL_ROWS256_W4 = 32,     /* 256 query rows per workgroup, four waves x 64 rows */
+  FO_ATTN_KERNEL_DECODE = 64          /* up to 32 query rows per workgroup, the keys dealt to its waves and to several workgroups */
 };
 int fo_attn_fwd_kernel(int B, int H, int Sq, int Sk, int D, const int64_t* k_strides_host, const int64_t* v_strides_host,
                        int causal, int has_bias, int has_dropout);

@@ -1,0 +1,45 @@
+"""The forward of few query rows over many keys: the keys of a row block dealt to waves and workgroups. Sizes at the edges of
+the 32-key tiles and the 32-row blocks, keys in slices of a larger cache, multi-query K/V, one and several workgroups per
+row block; against the oracle with the forward's tolerances."""
+import pytest
+import torch
+
+from fast_ops.flash_attention.flash_attention import multi_head_attention
+from fast_ops_amd import _lib
+from fast_ops_amd.flash_attention import flash_attention as surface
+from oracle.attention_oracle import attention_fwd_oracle
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+O_ATOL, O_RTOL, LSE_ATOL = 2e-2, 1e-2, 1e-3
+
+
+@pytest.mark.parametrize("split", [-1, 1, 2, 7])
+@pytest.mark.parametrize("B,H,Sq,Sk,D,dtype,multi_query", [
+    (1, 3, 1, 128, 64, torch.float16, False), (2, 5, 1, 129, 128, torch.bfloat16, False), (1, 2, 32, 1000, 64, torch.bfloat16, False),
+    (3, 4, 17, 545, 128, torch.float16, False), (2, 8, 1, 4097, 128, torch.bfloat16, True), (1, 12, 5, 700, 64, torch.float16, True),
+    (9, 1, 2, 300, 128, torch.bfloat16, False)])
+def test_decode_against_oracle(B, H, Sq, Sk, D, dtype, multi_query, split):
+    g = torch.Generator().manual_seed(Sk + D)
+    Hk = 1 if multi_query else H
+    q = torch.randn(B, H, Sq, D, generator=g).to(dtype)
+    # what lies behind the filled part of the cache must not count
+    cache = [torch.cat([torch.randn(B, Hk, Sk, D, generator=g), torch.full((B, Hk, 40, D), float("nan"))], dim=2).to(dtype) for _ in range(2)]
+    # moving row maxima: the last keys score far above the others
+    cache[0][:, :, Sk - 3:Sk] *= 6
+    k, v = (t[:, :, :Sk].expand(B, H, Sk, D) for t in cache)
+    o_ref, lse_ref = attention_fwd_oracle(q, k, v)
+    kd, vd = (t.to(DEV)[:, :, :Sk].expand(B, H, Sk, D) for t in cache)
+    surface._FWD_PLANS.clear()                       # (a plan remembers the workspace of its shape)
+    assert _lib.tune_set("attn.decode_split", split) is None
+    try:
+        o, lse = multi_head_attention(q.to(DEV), kd, vd, return_lse=True)
+        I3 = lambda t: (_lib.ctypes.c_int64 * 3)(*t.stride()[:3])
+        assert _lib.load().fo_attn_fwd_kernel(B, H, Sq, Sk, D, I3(kd), I3(vd), 0, 0, 0) == _lib.FO_ATTN_KERNEL_DECODE
+        torch.cuda.synchronize()
+    finally:
+        _lib.tune_set("attn.decode_split", -1)
+        surface._FWD_PLANS.clear()
+    err = (o.float().cpu() - o_ref).abs()
+    assert float((err - (O_ATOL + O_RTOL * o_ref.abs())).max()) <= 0, f"O: max abs err {float(err.max()):.3e}"
+    assert float((lse.cpu() - lse_ref).abs().max()) <= LSE_ATOL
