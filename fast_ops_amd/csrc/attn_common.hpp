@@ -49,6 +49,13 @@ __device__ __forceinline__ void dma16_uniform_base_lds_imm(const void* base, uin
   asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(byte_off), "s"(base), "n"(IMM) : "memory", "m0", "scc");
 #endif
 }
+// ... by the lanes of `lanes` only: the others' 16 bytes of LDS stay as they are. (For wave-uniform code: every lane is
+// active before and after. The write of EXEC is also the wait state that M0 needs.)
+__device__ __forceinline__ void dma16_uniform_base_of_lanes(const void* base, uint32_t byte_off, uint32_t dst, uint64_t lanes) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1" ::"s"(dst), "v"(byte_off), "s"(base), "s"(lanes) : "memory", "m0");
+#endif
+}
 __device__ __forceinline__ void dma16_lane_ptr(const void* ptr, FO_LDS void* dst) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)dst)), "v"(ptr) : "memory", "m0");
@@ -84,6 +91,10 @@ template <typename T>
 __device__ __forceinline__ const T* live_or_zero(const T* ptr, int col, int d) {
   return col < d ? ptr : (const T*)kZero16;
 }
+
+// Column count a kernel computes with, for a head_dim d on kernels laid out for D columns: the products leave out what
+// lies past the next multiple of 32.
+constexpr int live_columns(int D, int d) { return D == 128 ? (d <= 96 ? 96 : 128) : (d <= 32 ? 32 : 64); }
 
 // Dropout of attention probabilities, as the reference defines it (flash_attention_triton.py:38-50,125,216-219): element
 // (b*H + h, q, key) has the 32-bit index  offset + (b*H + h)*Sq*Sk + q*Sk + key  (all arithmetic modulo 2^32); the index,
