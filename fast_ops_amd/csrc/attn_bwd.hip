@@ -18,8 +18,9 @@
 //      computed untransposed, S = Q K^T and dP = dO V^T (A operands = Q / dO rows from LDS, B operands = K^T / V^T
 //      held in registers), so a lane owns one key and P, dS are the B operands of dV^T = dO^T P and dK^T = Q^T dS
 //      (A operands via the transposing LDS read of the dO and Q tiles); per-row LSE and delta come from LDS.
-//      Without a bias that has a query stride this runs as attn_bwd_dkdv_pipe_kernel, the same computation laid out by hand as a
-//      software pipeline (described there); attn_bwd_dkdv_kernel is the plain, compiler-scheduled form.
+//      Mostly this runs as attn_bwd_dkdv_pipe_kernel, the same computation laid out by hand as a software pipeline (described
+//      there); attn_bwd_dkdv_kernel is the plain, compiler-scheduled form for what that one does not take: a bias with a query
+//      stride whose tiles cannot be copied or that comes with dropout, other head dims with dropout or a bias.
 // Both recompute the scores (seven GEMMs in total instead of the five of an atomics-based single pass). softmax_scale
 // is applied once to the finished dQ and dK accumulators rather than to every dS.
 // Tiles of 64 rows go global -> LDS with the direct-to-LDS loads, double buffered (three buffers in the pipelined
@@ -277,9 +278,11 @@ constexpr int stage_bytes(int D) { return 32 * (D * 2 + 16); }   // per wave and
 // t+1 and puts them into LDS, where every wave reads them after the next barrier.
 // PAD: a head_dim below D. The products run over LIVE columns, the next multiple of 32 (live_columns); the columns of a
 // tile from head_dim on are zeroed by the copies of the first two tiles, and the later ones leave them alone.
-template <typename T, int D, bool CAUSAL, bool DROP, bool BIAS, bool KBIAS = false, bool PAD = false, int LIVE = D>
+// TBIAS: a bias with a query stride, of so many bytes per element, whose tiles can be copied (BiasRows): it too is what the
+// score accumulators start from.
+template <typename T, int D, bool CAUSAL, bool DROP, bool BIAS, bool KBIAS = false, bool PAD = false, int LIVE = D, int TBIAS = 0>
 __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const AttnBwdParams prm) {
-  static_assert(!(KBIAS && BIAS), "one bias form at a time");
+  static_assert(KBIAS + BIAS + (TBIAS != 0) <= 1, "one bias form at a time");
   typedef typename Ops<T>::vec8 vec8;
   constexpr int TILE_BYTES = kBwdTile * D * 2;
   constexpr int KSTEPS = LIVE / 16;
@@ -303,7 +306,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
 
   // (one register per piece where the kernel has them - head_dim 64, and the plain causal form at head_dim 128, which
   // were 0.4-0.6 % faster that way - and two per matrix where it would otherwise park some in scratch memory)
-  constexpr bool ROOMY = D == 64 || PAD || (CAUSAL && !DROP && !BIAS && !KBIAS);
+  constexpr bool ROOMY = D == 64 || PAD || (CAUSAL && !DROP && !BIAS && !KBIAS && TBIAS == 0);
   typename std::conditional<ROOMY, TileLaneOffsets<T, D>, TileLaneOffsetsCompact<T, D>>::type klo, vlo;
   klo.init(prm.ks[2], PAD ? D : prm.d, wave_s, lane);
   vlo.init(prm.vs[2], PAD ? D : prm.d, wave_s, lane);
@@ -348,14 +351,17 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
   FO_LDS float* key_bias = (FO_LDS float*)(smem + 4 * TILE_BYTES);      // KBIAS: [2][64], bias / scale of the keys of a tile
   float key_bias_next = 0.0f;                                           // (wave 0) this lane's key of the tile after next
   // (wave-uniform, and told so: this kernel has no vector register to spare)
-  const float per_scale = KBIAS ? __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, kLog2e / prm.scale_log2e))) : 0.0f;
-  const int64_t key_bias_row = KBIAS ? b * prm.bias.strides[0] + h * prm.bias.strides[1] : 0;
+  const float per_scale = KBIAS || TBIAS ? __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, kLog2e / prm.scale_log2e))) : 0.0f;
+  const int64_t key_bias_row = KBIAS || TBIAS ? b * prm.bias.strides[0] + h * prm.bias.strides[1] : 0;
   if constexpr (KBIAS) {
     if (wave_s == 0) {
       key_bias[lane] = load_bias<T>(prm.bias, key_bias_row + min(lane, Sk - 1)) * per_scale;
       key_bias_next = load_bias<T>(prm.bias, key_bias_row + min(kBwdTile + lane, Sk - 1));
     }
   }
+  typedef BiasRows<T, TBIAS == 4 ? 4 : 2> BR;
+  FO_LDS char* row_bias = smem + 4 * TILE_BYTES + wave_s * BR::BYTES;      // TBIAS: the wave's own
+  if constexpr (TBIAS != 0) BR::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, 0, row_bias, lane);
 
   // B operands held for the whole kernel: Q^T and dO^T fragments of this lane's query row; its LSE and delta
   const int qrow = min(q0w + l32, Sq - 1);
@@ -440,6 +446,12 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
 #pragma unroll
           for (int u = 0; u < 4; ++u) sacc[kb][4 * jv + u] = b4[u];
         }
+    }
+    if constexpr (TBIAS != 0) {
+      BR::each(row_bias, 0, l32, hh, [&](int r, float v) { sacc[0][r] = v * per_scale; });
+      BR::each(row_bias, 1, l32, hh, [&](int r, float v) { sacc[1][r] = v * per_scale; });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read: the buffer is free for the next tile's
+      if (tile + 1 < n_tiles) BR::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, key0 + kBwdTile, row_bias, lane);
     }
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks)
@@ -853,7 +865,7 @@ constexpr bool softmax_grad_jobs_fit(int nmf) {
 static_assert(softmax_grad_jobs_fit(16) && softmax_grad_jobs_fit(12) && softmax_grad_jobs_fit(8), "128, 96 and 64 columns");
 
 // ---------------------------------------------------------------------------------------------------------------------
-// dK/dV without a bias that has a query stride, as a software pipeline. The accumulators of dK and dV, the K^T and V^T fragments and
+// dK/dV as a software pipeline. The accumulators of dK and dV, the K^T and V^T fragments and
 // two blocks of scores leave room for one wave per SIMD only, and a lone wave issues in order: whatever arithmetic sits
 // between two MFMAs keeps the matrix pipe waiting unless it is laid out to run beside them. A 64-query tile is two
 // 32-query blocks and four phases of NMF MFMAs each:
@@ -877,8 +889,13 @@ static_assert(softmax_grad_jobs_fit(16) && softmax_grad_jobs_fit(12) && softmax_
 // 631 -> 391 us (no dropout 387), x 8192 1957 -> 1290 (1209), x 2048 causal 187 -> 119 (105); head_dim 64, 8 x 12 heads x
 // 1024 causal 139 -> 74 (71).
 // PAD, LIVE: a head_dim below D, as in the dQ kernel (96 columns: the phases are 12 groups long, with one or two slots each).
-template <typename T, int D, bool CAUSAL, bool KBIAS = false, bool DROP = false, bool PAD = false, int LIVE = D>
+// TBIAS: a bias with a query stride, of so many bytes per element (2, or 4 at head_dim 64, where two fp32 tiles per wave fit
+// into LDS beside the rings). The wave's 64 queries x 32 keys of tile j+2 are copied into LDS with that tile, two buffers; a
+// block's values, read transposed (a lane owns a key), are added to the start of its S accumulators in groups that carry
+// little else: S + (b - LSE) / scale then comes out of the MFMAs.
+template <typename T, int D, bool CAUSAL, bool KBIAS = false, bool DROP = false, bool PAD = false, int LIVE = D, int TBIAS = 0>
 __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(const AttnBwdParams prm) {
+  static_assert(TBIAS == 0 || !(KBIAS || DROP || PAD), "not combined");
   static_assert(!(PAD && (DROP || KBIAS)), "the second visit of dropout's rows copies whole rows");
   typedef typename Ops<T>::vec8 vec8;
   constexpr int TILE_BYTES = kBwdTile * D * 2;
@@ -911,7 +928,31 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   // (PAD: the first tile, and the K and V rows that go through the other two buffers below, zero the columns past head_dim)
   TileLiveLanes<T, D> live;
   if constexpr (PAD) live.init(prm.d, wave_s, lane);
+  // TBIAS: the wave's tile of the bias, 64 rows x 32 keys, as it lies in memory; needs what BiasRows needs
+  constexpr int BELT = TBIAS == 4 ? 4 : 2, BROW = 32 * BELT, BTILE = kBwdTile * BROW, BPIECES = BTILE / 1024, BROWS = 1024 / BROW, BLANES = BROW / 16;
+  FO_LDS char* bias_lds = (FO_LDS char*)(rowvals + 2 * NBUF * kBwdTile) + wave_s * 2 * BTILE;
+  const char* bias_lane_ptr = nullptr;       // the lane's piece of row lane / BLANES
+  int64_t bias_row_bytes = 0;
+  if constexpr (TBIAS != 0) {
+    bias_row_bytes = prm.bias.strides[2] * BELT;
+    const int col = min(k0w + (lane % BLANES) * (16 / BELT), Sk - 16 / BELT);
+    bias_lane_ptr = (const char*)prm.bias.ptr + (b * prm.bias.strides[0] + h * prm.bias.strides[1] + col) * BELT + (lane / BLANES) * bias_row_bytes;
+  }
+  auto issue_bias = [&](int qt) {
+    if (qt < ja) return;                     // (causal: this wave's keys start later)
+    FO_LDS char* dst = bias_lds + (qt & 1) * BTILE;
+    if (qt * kBwdTile + kBwdTile <= Sq) {
+#pragma unroll
+      for (int i = 0; i < BPIECES; ++i) dma16_lane_ptr(bias_lane_ptr + (int64_t)(qt * kBwdTile + i * BROWS) * bias_row_bytes, dst + i * 1024);
+    } else {
+      // (queries past the end re-read the last one; masked)
+#pragma unroll
+      for (int i = 0; i < BPIECES; ++i)
+        dma16_lane_ptr(bias_lane_ptr + (int64_t)(min(qt * kBwdTile + i * BROWS + lane / BLANES, Sq - 1) - lane / BLANES) * bias_row_bytes, dst + i * 1024);
+    }
+  };
   auto issue = [&](int qt, int buf) {
+    if constexpr (TBIAS != 0) issue_bias(qt);
     if (PAD && qt > qt0 && qt * kBwdTile + kBwdTile <= Sq && qlo.ok && glo.ok) {
       copy_tile64_inside<T, D>(qbase, prm.qs[2], qt * kBwdTile, qlo, live, smem + buf * TILE_BYTES, wave_s);
       copy_tile64_inside<T, D>(gbase, prm.dos[2], qt * kBwdTile, glo, live, smem + (NBUF + buf) * TILE_BYTES, wave_s);
@@ -1051,6 +1092,37 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
 #endif
   };
 
+  // TBIAS: the lane's 16 values of a block, then, times 1 / softmax_scale, added to the block's S accumulator one by one
+  const float per_scale = TBIAS ? __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, 1.0f / prm.scale))) : 0.0f;
+  s16x4 bias16[4];
+  f32x16 bias32;
+  auto bias_read = [&](int jt, int qb) {
+    FO_LDS const char* src = bias_lds + (jt & 1) * BTILE + qb * 32 * BROW;
+#pragma unroll
+    for (int jv = 0; jv < 4; ++jv) {
+      if constexpr (BELT == 2) {
+        bias16[jv] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FO_LDS s16x4*)(src + (8 * jv + 4 * hh + ((lane & 15) >> 2)) * BROW + ((lane >> 4) & 1) * 32 + (lane & 3) * 8));
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) bias32[4 * jv + u] = *(FO_LDS const float*)(src + (8 * jv + 4 * hh + u) * BROW + l32 * 4);
+      }
+    }
+  };
+  auto bias_add = [&](f32x16& acc, int e) {
+    float v;
+    if constexpr (BELT == 2) {
+      const short raw = bias16[e >> 2][e & 3];
+      v = (float)__builtin_bit_cast(T, raw);
+    } else {
+      v = bias32[e];
+    }
+    float sum = __builtin_fmaf(v, per_scale, acc[e]);
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(sum));            // (pinned to its group, see stage_b)
+#endif
+    acc[e] = sum;
+  };
+
   const uint32_t lane4 = (uint32_t)lane * 4u;
   // One tile. `buf`: the tile's buffer, (j - qt0) % NBUF, which the caller counts along. `spread`: tile j+2 lies wholly
   // inside Q and dO (and the lane offsets fit): its copy is not issued in one batch at the hand-over but one instruction
@@ -1151,6 +1223,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
     const char* next_q = nullptr;
     const char* next_g = nullptr;
     const char* next_rows = nullptr;
+    const char* next_bias = nullptr;
     uint32_t next_q_dst = 0;
     FO_LDS char* next_rows_dst = nullptr;
     __builtin_amdgcn_sched_barrier(0);
@@ -1169,6 +1242,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
           next_rows = (const char*)((which ? (const float*)prm.delta : (const float*)prm.nlse) + (int64_t)bh * Sq + (j + 2) * kBwdTile);
           next_q_dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(smem + b2 * TILE_BYTES + wave_s * (TileLaneOffsets<T, D>::N * 1024)));
           next_rows_dst = (FO_LDS char*)(rowvals + (NBUF * which + b2) * kBwdTile);
+          if constexpr (TBIAS != 0) next_bias = bias_lane_ptr + (int64_t)(j + 2) * kBwdTile * bias_row_bytes;
         } else if constexpr (!AGAIN) {
           if (j + 1 < n_qt) hand_over(j);
         }
@@ -1201,6 +1275,18 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       if (g == 1) start_acc(sacc[1], rowvals + buf * kBwdTile, 1);
       if (g == 3 * NMF) start_acc(dpacc[0], rowvals + (NBUF + nbuf) * kBwdTile, 0);
       if (g == 3 * NMF + 1) start_acc(sacc[0], rowvals + nbuf * kBwdTile, 0);
+      if constexpr (TBIAS != 0) {
+        // (block 1: from group 2 to two groups before its first MFMA; block 0 of the next tile: in the last half-phase but
+        // for its last group - the groups without, or with the least, softmax-gradient arithmetic)
+        constexpr int N1 = NMF - 4, N0 = HALF - 1;
+        if (g == 1) bias_read(j, 1);
+        if (g == 3 * NMF + 1) bias_read(j + 1, 0);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          if (g == 2 + e * N1 / 16) bias_add(sacc[1], e);
+          if (g == 3 * NMF + HALF + e * N0 / 16) bias_add(sacc[0], e);
+        }
+      }
       if constexpr (SPREAD) {
         if (ph == 3) {
           constexpr int N = TileLaneOffsets<T, D>::N;
@@ -1227,6 +1313,13 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
             }
           }
           if (i == 0) dma4_uniform_base(next_rows, lane4, next_rows_dst);
+          if constexpr (TBIAS != 0) {
+            // (two buffers: tile j's values have been read in the first groups)
+            constexpr int EVERY = BPIECES == NMF ? 1 : 2;
+            static_assert(BPIECES * EVERY <= NMF, "at most one piece per micro-group");
+            if (i % EVERY == 0 && i / EVERY < BPIECES)
+              dma16_lane_ptr(next_bias + (i / EVERY) * BROWS * bias_row_bytes, bias_lds + (j & 1) * BTILE + (i / EVERY) * 1024);
+          }
         }
       }
       if (g >= HALF && g < NG - HALF) {
@@ -1267,6 +1360,11 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       const f32x4 n4 = *(FO_LDS const f32x4*)(rowvals + buf * kBwdTile + 8 * jv + 4 * hh);
 #pragma unroll
       for (int u = 0; u < 4; ++u) sacc[0][4 * jv + u] = n4[u];
+    }
+    if constexpr (TBIAS != 0) {
+      bias_read(ja, 0);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) bias_add(sacc[0], e);
     }
   };
   if (j < n_qt) start_tile((j - qt0) % NBUF);
@@ -1350,6 +1448,24 @@ static int launch_bwd_pad(const AttnBwdParams& q, unsigned g_dq, unsigned g_dkdv
   return launch_status();
 }
 
+// A bias with a query stride whose tiles can be copied, without dropout: what the score accumulators start from in both
+// kernels. (An fp32 bias at head_dim 128 leaves no room for two workgroups of the dQ kernel per compute unit, nor for its tiles
+// beside the rings of the dK/dV kernel: that runs on the kernels of the general form.) General form -> this, bias [1, H, S, S]:
+// 12 heads x 3072 causal at head_dim 128 bf16 bias: dQ 156 -> 111 us, dK/dV 147 -> 90; whole backward not causal 540 -> 320;
+// at head_dim 64 235 -> 131 causal, 347 -> 209 not, with an fp32 bias 258 -> 151 and 384 -> 270.
+template <typename T, int D, bool CAUSAL, int ELT>
+static int launch_bwd_tile_bias(const AttnBwdParams& q, unsigned g_dq, unsigned g_dkdv, size_t lds_tiles, size_t lds_pipe, hipStream_t s) {
+  const size_t lds_dq = lds_tiles + kBwdWaves * BiasRows<T, ELT>::BYTES, lds_kv = lds_pipe + kBwdWaves * 2 * kBwdTile * 32 * ELT;
+  static const hipError_t a1 = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<T, D, CAUSAL, false, false, false, false, D, ELT>,
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dq);
+  static const hipError_t a2 = hipFuncSetAttribute((const void*)attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, false, false, D, ELT>,
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_kv);
+  if (a1 != hipSuccess || a2 != hipSuccess) return FO_ERR_LAUNCH;
+  attn_bwd_dq_kernel<T, D, CAUSAL, false, false, false, false, D, ELT><<<g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
+  attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, false, false, D, ELT><<<g_dkdv, kBwdWaves * 64, lds_kv, s>>>(q);
+  return launch_status();
+}
+
 template <typename T, int D, bool CAUSAL, bool DROP, bool BIAS>
 static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
   const int64_t n_bh = (int64_t)p.B * p.H;
@@ -1397,6 +1513,13 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
       if (p.d == D) attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, true, DROP><<<(unsigned)g_dkdv, kBwdWaves * 64, lds_pipe, s>>>(q);
       else attn_bwd_dkdv_kernel<T, D, CAUSAL, DROP, BIAS><<<(unsigned)g_dkdv, kBwdWaves * 64, lds_dkdv, s>>>(q);
       return launch_status();
+    }
+  }
+  if constexpr (BIAS && !DROP) {
+    // (dma_ok: base and strides are multiples of 16 bytes, the query stride is not zero)
+    if (p.d == D && p.bias.dma_ok && p.Sk % (p.bias.is_f32 ? 4 : 8) == 0 && tune(g_attn_bwd_variant) != 0) {
+      if (!p.bias.is_f32) return launch_bwd_tile_bias<T, D, CAUSAL, 2>(q, (unsigned)g_dq, (unsigned)g_dkdv, lds_tiles, lds_pipe, s);
+      if constexpr (D == 64) return launch_bwd_tile_bias<T, D, CAUSAL, 4>(q, (unsigned)g_dq, (unsigned)g_dkdv, lds_tiles, lds_pipe, s);
     }
   }
   if constexpr (!DROP && !BIAS) {

@@ -292,6 +292,47 @@ __device__ __forceinline__ void dma4_uniform_base(const void* base, uint32_t byt
 #endif
 }
 
+// A bias with a query stride where a lane owns a query row (forward and dQ kernels): the wave's 32 rows x 64 keys of a key tile,
+// copied straight into LDS, ELT bytes per element, ROW bytes per row; 16-byte piece s of a row holds the row's piece
+// s ^ (row mod pieces), so that 32 rows' reads of the same piece are spread over the banks. One buffer per wave: once a
+// tile's values are read (they start or join its score accumulators) the next tile's copy begins. Needs the
+// 16-byte alignment of dma_ok and a number of keys that is a multiple of a piece: pieces past the end then re-read the
+// last one, rows past the end the last row, and both are masked by the kernels.
+template <typename T, int ELT>
+struct BiasRows {
+  static constexpr int PIECE_KEYS = 16 / ELT, ROW = 64 * ELT, PIECES = ROW / 16, ROWS_PER_DMA = 64 / PIECES, BYTES = 32 * ROW;
+  // `row0`: element (b, h, 0, 0); q0w: the wave's first row
+  static __device__ __forceinline__ void copy(const BiasParams& bp, int64_t row0, int q0w, int Sq, int Sk, int key0, FO_LDS char* dst, int lane_in) {
+    int lane = lane_in;
+    asm volatile("" : "+v"(lane));           // (computed anew per tile: no registers held across the loop)
+#pragma unroll
+    for (int i = 0; i < 32 / ROWS_PER_DMA; ++i) {
+      const int row = i * ROWS_PER_DMA + lane / PIECES, piece = (lane % PIECES) ^ (row & (PIECES - 1));
+      const int64_t at = row0 + (int64_t)min(q0w + row, Sq - 1) * bp.strides[2] + min(key0 + piece * PIECE_KEYS, Sk - PIECE_KEYS);
+      dma16_lane_ptr((const char*)bp.ptr + at * ELT, dst + i * 1024);
+    }
+  }
+  // f(r, value) for registers 0..15 (four times four consecutive keys) of 32-key block kb of the lane's row
+  template <typename F>
+  static __device__ __forceinline__ void each(FO_LDS const char* src, int kb, int l32_in, int hh, F f) {
+    int l32 = l32_in;
+    asm volatile("" : "+v"(l32));            // (as in copy)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if constexpr (ELT == 4) {
+        const f32x4 v = *(FO_LDS const f32x4*)(src + l32 * ROW + (((8 * kb + 2 * j + hh) ^ (l32 & 15)) * 16));
+#pragma unroll
+        for (int u = 0; u < 4; ++u) f(4 * j + u, v[u]);
+      } else {
+        typedef __attribute__((ext_vector_type(4))) T vec4;
+        const vec4 v = *(FO_LDS const vec4*)(src + l32 * ROW + (((4 * kb + j) ^ (l32 & 7)) * 16) + hh * 8);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) f(4 * j + u, (float)v[u]);
+      }
+    }
+  }
+};
+
 // Attention of a few query rows over many keys (attn_decode.hip)
 struct DecodeParams {
   const void *q, *k, *v;

@@ -71,13 +71,17 @@ constexpr float kLazyLog2 = 8.0f;   // how far (in log2 units) a tile maximum ma
 // depends on r and the half of the wave only), so the MFMAs deliver S + b / scale and the rest is the code without bias.
 // Wave 0 fetches the values of tile t+2 while tile t is worked on (a plain load, waited for at the top of the next tile,
 // where every copy in flight is waited for anyway), converts those of tile t+1 and puts them into LDS for everyone.
+// TBIAS: a bias with a query stride, of so many bytes per element, whose tiles can be copied into one buffer per wave
+// (BiasRows), where the general form (BIAS) keeps two of the size an fp32 bias needs: the same arithmetic, with room for two
+// workgroups per compute unit at head_dim 128 (operand type). General form -> this, 12 heads x 3072, head_dim 128: bf16 bias
+// 187 -> 118 us, causal 92 -> 82; fp32 188 -> 178 and 107 -> 88; head_dim 64: 133 -> 83, 70 -> 63, 150 -> 118, 74 -> 74.
 // PAD: a head_dim below D. The products run over LIVE columns, the next multiple of 32 (live_columns). The copies of the first
 // two tiles zero the columns of their buffers from head_dim on (live_or_zero: a 64-bit address per lane and piece); those of
 // later tiles are made by the lanes of the live columns only, at the cost they have at head_dim D. (B=4 H=16, 777 x 1250,
 // head_dim 80, bf16: 49.1 -> 39.4 us.)
-template <typename T, int D, bool CAUSAL, bool LAZY, int DBG, bool DROP = false, bool BIAS = false, bool KBIAS = false, bool PAD = false, int LIVE = D>
+template <typename T, int D, bool CAUSAL, bool LAZY, int DBG, bool DROP = false, bool BIAS = false, bool KBIAS = false, bool PAD = false, int LIVE = D, int TBIAS = 0>
 __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnParams prm) {
-  static_assert(!(KBIAS && BIAS), "one bias form at a time");
+  static_assert(KBIAS + BIAS + (TBIAS != 0) <= 1, "one bias form at a time");
   typedef typename Ops<T>::vec8 vec8;
   constexpr int ROW_BYTES = D * 2;
   constexpr int CHUNKS = ROW_BYTES / 16;            // 16-byte chunks per row
@@ -227,13 +231,16 @@ __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnPara
   FO_LDS float* key_bias = (FO_LDS float*)(smem + 4 * TILE_BYTES);      // KBIAS: [2][64], bias / scale of the keys of a tile
   float key_bias_next = 0.0f;                                           // (wave 0) this lane's key of the tile after next
   const float per_scale = KBIAS ? 1.4426950408889634f / prm.scale_log2e : 0.0f;
-  const int64_t key_bias_row = KBIAS ? b * prm.bias.strides[0] + h * prm.bias.strides[1] : 0;
+  const int64_t key_bias_row = KBIAS || TBIAS ? b * prm.bias.strides[0] + h * prm.bias.strides[1] : 0;
   if constexpr (KBIAS) {
     if (wave_s == 0) {
       key_bias[lane] = load_bias<T>(prm.bias, key_bias_row + min(lane, Sk - 1)) * per_scale;
       key_bias_next = load_bias<T>(prm.bias, key_bias_row + min(kBN + lane, Sk - 1));
     }
   }
+  typedef BiasRows<T, TBIAS == 4 ? 4 : 2> BR;
+  FO_LDS char* row_bias = smem + 4 * TILE_BYTES + wave_s * BR::BYTES;      // TBIAS: the wave's own
+  if constexpr (TBIAS != 0) BR::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, 0, row_bias, lane);
 
   // ---- Q^T fragments (B operand): lane holds query row q0w + l32, d = 16*ks + 8*hh .. +7
   vec8 qf[KSTEPS];
@@ -257,7 +264,7 @@ __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnPara
   float l_run = 0.0f;        // running sum of this lane's half of the keys
   // with a bias the scores are turned into base-2 logits (score * scale * log2e + bias * log2e) right after the mask, and
   // everything downstream sees a scale of 1
-  const float c = BIAS ? 1.0f : prm.scale_log2e;
+  const float c = BIAS || TBIAS ? 1.0f : prm.scale_log2e;
 
   // per-lane LDS read offsets that do not depend on the tile
   //  K (ds_read_b128): row = 32*kb + l32, logical chunk = 2*ks + hh
@@ -353,8 +360,15 @@ __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnPara
       }
     }
 
+    // qk * softmax_scale + bias (flash_attention_triton.py:198)
+    if constexpr (TBIAS != 0) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+        BR::each(row_bias, kb, l32, hh, [&](int r, float v) { sacc[kb][r] = __builtin_fmaf(sacc[kb][r], prm.scale_log2e, v * 1.4426950408889634f); });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read: the buffer is free for the next tile's
+      if (tile + 1 < n_tiles) BR::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, key0 + kBN, row_bias, lane);
+    }
     if constexpr (BIAS) {
-      // qk * softmax_scale + bias (flash_attention_triton.py:198)
       if (prm.bias.dma_ok && key0 + kBN <= Sk) {
         // from the tile copied into LDS: register r = 4 j + u of block kb is key 32 kb + 8 j + 4 hh + u of row l32
         FO_LDS const char* bt = bias_lds + buf * kWaves * kBiasWaveBytes;
@@ -430,7 +444,7 @@ __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnPara
     const bool raise = LAZY ? (mloc * c > m_run * c + kLazyLog2) : (mloc > m_run);
     if (__builtin_amdgcn_ballot_w64(raise) != 0) {
       const float m_new = fmaxf(m_run, mloc);          // finite from the first tile on: key 0 is never masked
-      const float alpha = ((BIAS || KBIAS) && m_new == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f((m_run - m_new) * c);
+      const float alpha = ((BIAS || KBIAS || TBIAS) && m_new == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f((m_run - m_new) * c);
       m_run = m_new;
       l_run *= alpha;
 #pragma unroll
@@ -439,7 +453,7 @@ __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnPara
         for (int r = 0; r < 16; ++r) oacc[i][r] *= alpha;
     }
     // a bias may mask every key seen so far (-inf, e.g. left padding): the reference then stays 0 until a key counts
-    const float mc = ((BIAS || KBIAS) && m_run == -INFINITY) ? 0.0f : m_run * c;
+    const float mc = ((BIAS || KBIAS || TBIAS) && m_run == -INFINITY) ? 0.0f : m_run * c;
     float psum = 0.0f;
     vec8 pf[4];
 #pragma unroll
@@ -1427,12 +1441,12 @@ static int launch_rows256_w4_noncausal(AttnParams p, hipStream_t stream) {
   return launch_wide<T, D, false, 2, 0, kWideBM, VBIAS, DROP>(p, stream);
 }
 
-template <typename T, int D, bool CAUSAL, bool LAZY, int DBG, bool DROP = false, bool BIAS = false, bool KBIAS = false, bool PAD = false, int LIVE = D>
+template <typename T, int D, bool CAUSAL, bool LAZY, int DBG, bool DROP = false, bool BIAS = false, bool KBIAS = false, bool PAD = false, int LIVE = D, int TBIAS = 0>
 static int launch_one(const AttnParams& p, hipStream_t stream) {
-  const size_t lds_max = 4 * (size_t)kBN * D * 2 + (BIAS ? 2 * kWaves * 32 * kBN * 4 : 0) + (KBIAS ? 2 * kBN * 4 : 0);   // K, V tiles; bias tiles
-  const size_t lds = 4 * (size_t)kBN * D * 2 + (BIAS && p.bias.dma_ok ? 2 * kWaves * 32 * kBN * 4 : 0) + (KBIAS ? 2 * kBN * 4 : 0);
+  const size_t lds_max = 4 * (size_t)kBN * D * 2 + (BIAS ? 2 * kWaves * 32 * kBN * 4 : 0) + (KBIAS ? 2 * kBN * 4 : 0) + kWaves * 32 * kBN * TBIAS;   // K, V tiles; bias tiles
+  const size_t lds = 4 * (size_t)kBN * D * 2 + (BIAS && p.bias.dma_ok ? 2 * kWaves * 32 * kBN * 4 : 0) + (KBIAS ? 2 * kBN * 4 : 0) + kWaves * 32 * kBN * TBIAS;
   const unsigned grid = (unsigned)(p.n_qblk * p.B * p.H);
-  static const hipError_t attr = hipFuncSetAttribute((const void*)attn_fwd_kernel<T, D, CAUSAL, LAZY, DBG, DROP, BIAS, KBIAS, PAD, LIVE>,
+  static const hipError_t attr = hipFuncSetAttribute((const void*)attn_fwd_kernel<T, D, CAUSAL, LAZY, DBG, DROP, BIAS, KBIAS, PAD, LIVE, TBIAS>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max);
   if (attr != hipSuccess) return FO_ERR_LAUNCH;
   // Order of the workgroups of one XCD when causal: the heaviest query blocks of all its heads first, then the next
@@ -1454,7 +1468,7 @@ static int launch_one(const AttnParams& p, hipStream_t stream) {
     // wherever a slot frees, and the plain order is the better one.
     const int cus_x = device_cus() / 8, n_bh_x = (int)(((int64_t)p.B * p.H) >> 3);
     const int64_t n = (int64_t)n_bh_x * p.n_qblk;
-    const int resident = (D == 64 && !BIAS) ? 3 : 2;      // workgroups per compute unit (registers)
+    const int resident = (D == 64 && !BIAS && TBIAS != 4) ? 3 : 2;      // workgroups per compute unit (registers)
     if (q.heavy_first == n_bh_x && cus_x > 0 && cus_x <= kOrderTab && n <= (int64_t)cus_x * resident && n <= kOrderTab && n > cus_x) {
       // (the table of the last shape is kept per host thread: filling it takes a few microseconds, a training loop
       // launches the same shape over and over)
@@ -1480,7 +1494,7 @@ static int launch_one(const AttnParams& p, hipStream_t stream) {
       q.order_n = (int)n;
     }
   }
-  attn_fwd_kernel<T, D, CAUSAL, LAZY, DBG, DROP, BIAS, KBIAS, PAD, LIVE><<<grid, kWaves * 64, lds, stream>>>(q);
+  attn_fwd_kernel<T, D, CAUSAL, LAZY, DBG, DROP, BIAS, KBIAS, PAD, LIVE, TBIAS><<<grid, kWaves * 64, lds, stream>>>(q);
   return launch_status();
 }
 
@@ -1583,6 +1597,13 @@ int launch(const AttnParams& p, bool causal, bool dropout, hipStream_t stream) {
   // tests compare the two)
   const bool key_bias = p.bias.ptr != nullptr && p.bias.strides[2] == 0 && asked != FO_ATTN_KERNEL_ROWS128_EXACT;
   if (p.bias.ptr != nullptr && !key_bias) {
+    // tiles that can be copied (dma_ok: base and strides are multiples of 16 bytes) and start the score accumulators
+    if (!dropout && p.d == D && p.bias.dma_ok && p.Sk % (p.bias.is_f32 ? 4 : 8) == 0 && asked != FO_ATTN_KERNEL_ROWS128_EXACT) {
+      if (p.bias.is_f32) return causal ? launch_one<T, D, true, true, 0, false, false, false, false, D, 4>(p, stream)
+                                       : launch_one<T, D, false, true, 0, false, false, false, false, D, 4>(p, stream);
+      return causal ? launch_one<T, D, true, true, 0, false, false, false, false, D, 2>(p, stream)
+                    : launch_one<T, D, false, true, 0, false, false, false, false, D, 2>(p, stream);
+    }
     if (dropout) return causal ? launch_one<T, D, true, true, 0, true, true>(p, stream) : launch_one<T, D, false, true, 0, true, true>(p, stream);
     return causal ? launch_one<T, D, true, true, 0, false, true>(p, stream) : launch_one<T, D, false, true, 0, false, true>(p, stream);
   }

@@ -1,0 +1,36 @@
+"""A bias with a query stride whose tiles are copied into LDS (rows on 16-byte boundaries, a whole number of 16-byte pieces):
+several whole tiles and ragged last ones, rows longer than the keys with NaN behind them, keys masked with -inf at either
+end, broadcasting over batch and heads, and calls next to the rule's lines that the general kernels take. Against the
+oracle; tolerances as in test_attention_bias_gpu.py."""
+import pytest
+import torch
+
+from fast_ops.flash_attention.flash_attention import flash_attn
+from oracle.attention_oracle import attention_bwd_oracle, attention_fwd_oracle
+from test_attention_bias_gpu import DEV, _bshd, _check
+
+pytestmark = pytest.mark.gpu
+
+
+# (the last two: keys that are no whole number of pieces)
+@pytest.mark.parametrize("B,H,Sq,Sk", [(2, 2, 449, 456), (1, 3, 577, 584), (1, 2, 640, 640), (1, 2, 130, 8), (1, 1, 333, 1030), (2, 1, 300, 333)])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bias_f32", [False, True])
+@pytest.mark.parametrize("causal,dtype", [(False, torch.float16), (True, torch.bfloat16), (False, torch.bfloat16)])
+def test_tile_bias(B, H, Sq, Sk, D, bias_f32, causal, dtype):
+    g = torch.Generator().manual_seed(Sq + Sk + D)
+    q, k, v, go = (torch.randn(B, H, n, D, generator=g).to(dtype) for n in (Sq, Sk, Sk, Sq))
+    bias = (2.0 * torch.randn(1 if B == 2 else B, H, Sq, Sk, generator=g)).to(torch.float32 if bias_f32 else dtype)
+    if not causal:
+        bias[:, :, Sq // 2:, :Sk // 3] = float("-inf")        # whole tiles and parts of one, left ...
+    bias[:, :, ::3, Sk - Sk // 4:] = float("-inf")            # ... and right padding
+    o_ref, lse_ref = attention_fwd_oracle(q, k, v, causal=causal, bias=bias)
+    ref = attention_bwd_oracle(q, k, v, go, causal=causal, bias=bias)
+    pad = -Sk % 8 + 8
+    wide = torch.full(bias.shape[:-1] + (Sk + pad,), float("nan"), dtype=bias.dtype, device=DEV)
+    wide[..., :Sk] = bias.to(DEV)
+    t = [_bshd(x.to(DEV)).requires_grad_(True) for x in (q, k, v)]
+    o, lse = flash_attn(*t, bias=wide[..., :Sk], causal=causal, return_lse=True)
+    got = torch.autograd.grad(o, t, _bshd(go.to(DEV)))
+    torch.cuda.synchronize()
+    _check(_bshd(o), lse, [_bshd(x) for x in got], o_ref, lse_ref, ref)
