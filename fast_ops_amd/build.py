@@ -56,6 +56,7 @@ SOURCES = {
     "attn_bwd_f16_d128.hip": ["-mllvm", "-pragma-unroll-threshold=400000"],
     "attn_decode.hip": [],
     "dropout_mask.hip": [],
+    "bias_rows.hip": [],
 }
 # sources that other sources include (a change in one of them makes every object stale, like a header's)
 INCLUDED_SOURCES = ["attn_fwd.hip", "attn_bwd.hip"]

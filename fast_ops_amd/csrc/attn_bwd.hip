@@ -935,7 +935,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   int64_t bias_row_bytes = 0;
   if constexpr (TBIAS != 0) {
     bias_row_bytes = prm.bias.strides[2] * BELT;
-    const int col = min(k0w + (lane % BLANES) * (16 / BELT), Sk - 16 / BELT);
+    const int col = min(k0w + (lane % BLANES) * (16 / BELT), (Sk - 1) / (16 / BELT) * (16 / BELT));
     bias_lane_ptr = (const char*)prm.bias.ptr + (b * prm.bias.strides[0] + h * prm.bias.strides[1] + col) * BELT + (lane / BLANES) * bias_row_bytes;
   }
   auto issue_bias = [&](int qt) {
@@ -1517,7 +1517,7 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
   }
   if constexpr (BIAS && !DROP) {
     // (dma_ok: base and strides are multiples of 16 bytes, the query stride is not zero)
-    if (p.d == D && p.bias.dma_ok && p.Sk % (p.bias.is_f32 ? 4 : 8) == 0 && tune(g_attn_bwd_variant) != 0) {
+    if (p.d == D && p.bias.dma_ok && tune(g_attn_bwd_variant) != 0) {
       if (!p.bias.is_f32) return launch_bwd_tile_bias<T, D, CAUSAL, 2>(q, (unsigned)g_dq, (unsigned)g_dkdv, lds_tiles, lds_pipe, s);
       if constexpr (D == 64) return launch_bwd_tile_bias<T, D, CAUSAL, 4>(q, (unsigned)g_dq, (unsigned)g_dkdv, lds_tiles, lds_pipe, s);
     }

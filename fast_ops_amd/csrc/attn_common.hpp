@@ -296,8 +296,9 @@ __device__ __forceinline__ void dma4_uniform_base(const void* base, uint32_t byt
 // copied straight into LDS, ELT bytes per element, ROW bytes per row; 16-byte piece s of a row holds the row's piece
 // s ^ (row mod pieces), so that 32 rows' reads of the same piece are spread over the banks. One buffer per wave: once a
 // tile's values are read (they start or join its score accumulators) the next tile's copy begins. Needs the
-// 16-byte alignment of dma_ok and a number of keys that is a multiple of a piece: pieces past the end then re-read the
-// last one, rows past the end the last row, and both are masked by the kernels.
+// 16-byte alignment of dma_ok. Pieces past the end re-read the last one that holds a key - of which the part behind the last
+// key is read too, up to the next 16-byte boundary, and may hold anything - and rows past the end the last row; the kernels
+// mask both after the bias has been applied.
 template <typename T, int ELT>
 struct BiasRows {
   static constexpr int PIECE_KEYS = 16 / ELT, ROW = 64 * ELT, PIECES = ROW / 16, ROWS_PER_DMA = 64 / PIECES, BYTES = 32 * ROW;
@@ -308,7 +309,7 @@ struct BiasRows {
 #pragma unroll
     for (int i = 0; i < 32 / ROWS_PER_DMA; ++i) {
       const int row = i * ROWS_PER_DMA + lane / PIECES, piece = (lane % PIECES) ^ (row & (PIECES - 1));
-      const int64_t at = row0 + (int64_t)min(q0w + row, Sq - 1) * bp.strides[2] + min(key0 + piece * PIECE_KEYS, Sk - PIECE_KEYS);
+      const int64_t at = row0 + (int64_t)min(q0w + row, Sq - 1) * bp.strides[2] + min(key0 + piece * PIECE_KEYS, (Sk - 1) / PIECE_KEYS * PIECE_KEYS);
       dma16_lane_ptr((const char*)bp.ptr + at * ELT, dst + i * 1024);
     }
   }

@@ -345,7 +345,17 @@ __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnPara
       }
     }
 
-    // ---- mask: causal diagonal and keys past the end. Register r of block kb holds key
+    // qk * softmax_scale + bias (flash_attention_triton.py:198)
+    if constexpr (TBIAS != 0) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+        BR::each(row_bias, kb, l32, hh, [&](int r, float v) { sacc[kb][r] = __builtin_fmaf(sacc[kb][r], prm.scale_log2e, v * 1.4426950408889634f); });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read: the buffer is free for the next tile's
+      if (tile + 1 < n_tiles) BR::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, key0 + kBN, row_bias, lane);
+    }
+
+    // ---- mask: causal diagonal and keys past the end (after the values of TBIAS, which may be anything there). Register r of
+    //      block kb holds key
     //      key0 + 32*kb + 4*hh + koff(r), koff(r) = (r & 3) + 8 * (r >> 2); it is dead iff key > q or key >= Sk,
     //      i.e. iff lim + koff(r) > 0 with lim = max(key_base - q, key_base - Sk + 1): one compare against a constant.
     const bool need_mask = (CAUSAL && key0 + kBN - 1 > q0w) || (key0 + kBN > Sk);
@@ -360,15 +370,8 @@ __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnPara
       }
     }
 
-    // qk * softmax_scale + bias (flash_attention_triton.py:198)
-    if constexpr (TBIAS != 0) {
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-        BR::each(row_bias, kb, l32, hh, [&](int r, float v) { sacc[kb][r] = __builtin_fmaf(sacc[kb][r], prm.scale_log2e, v * 1.4426950408889634f); });
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read: the buffer is free for the next tile's
-      if (tile + 1 < n_tiles) BR::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, key0 + kBN, row_bias, lane);
-    }
     if constexpr (BIAS) {
+      // qk * softmax_scale + bias
       if (prm.bias.dma_ok && key0 + kBN <= Sk) {
         // from the tile copied into LDS: register r = 4 j + u of block kb is key 32 kb + 8 j + 4 hh + u of row l32
         FO_LDS const char* bt = bias_lds + buf * kWaves * kBiasWaveBytes;
@@ -1598,7 +1601,7 @@ int launch(const AttnParams& p, bool causal, bool dropout, hipStream_t stream) {
   const bool key_bias = p.bias.ptr != nullptr && p.bias.strides[2] == 0 && asked != FO_ATTN_KERNEL_ROWS128_EXACT;
   if (p.bias.ptr != nullptr && !key_bias) {
     // tiles that can be copied (dma_ok: base and strides are multiples of 16 bytes) and start the score accumulators
-    if (!dropout && p.d == D && p.bias.dma_ok && p.Sk % (p.bias.is_f32 ? 4 : 8) == 0 && asked != FO_ATTN_KERNEL_ROWS128_EXACT) {
+    if (!dropout && p.d == D && p.bias.dma_ok && asked != FO_ATTN_KERNEL_ROWS128_EXACT) {
       if (p.bias.is_f32) return causal ? launch_one<T, D, true, true, 0, false, false, false, false, D, 4>(p, stream)
                                        : launch_one<T, D, false, true, 0, false, false, false, false, D, 4>(p, stream);
       return causal ? launch_one<T, D, true, true, 0, false, false, false, false, D, 2>(p, stream)

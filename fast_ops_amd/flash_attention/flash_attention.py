@@ -69,6 +69,44 @@ def _expand_bias(bias: Tensor, q: Tensor, B: int, H: int, Sq: int, Sk: int) -> T
     return bias.expand(B, H, Sq, Sk)
 
 
+# When _aligned_bias copies: from so many (query, key) pairs on, by the bytes of an element - below, the copy's launch and its host
+# time cost more than it gains (12 heads, forward + backward, bf16 bias / fp32 bias: 333 keys 135 -> 153 / 135 -> 152 us, 515 keys 173 -> 149
+# / 138 -> 151, 1021 keys 465 -> 146 / 237 -> 186, 3071 keys 2418 -> 507 / 1321 -> 1000) - and up to a copy of so many bytes, without
+# and with a backward to come. The forward alone gains only while the memory-side cache (256 MiB) holds the copy: 12 heads x 3071 bf16
+# (226 MB) 332 -> 206 us and causal 210 -> 166, but fp32 218 -> 252 causal and 16 heads x 4095 bf16 250 -> 304.
+_ALIGN_BIAS_FROM = {2: 1 << 18, 4: 1 << 19}
+_ALIGN_BIAS_BYTES = {False: 256 << 20, True: 4 << 30}
+
+
+def _aligned_bias(bias: Optional[Tensor], q: Tensor, k: Tensor, backward: bool) -> Optional[Tensor]:
+    """A bias with a row per query whose rows do not start on 16-byte boundaries, copied (once for what is broadcast over batch
+    or heads) into rows that do, which is what the kernels copy tiles from; any other bias as it is. (flash_attn's layout.)"""
+    if bias is None or bias.dim() != 4 or bias.shape[2] == 1 or q.dim() != 4 or k.dim() != 4:
+        return bias                                            # (what does not fit is refused further on)
+    if bias.dtype not in (q.dtype, torch.float32) or not bias.is_cuda or bias.device != q.device:
+        return bias
+    B, Sq, H, Sk = q.shape[0], q.shape[1], q.shape[2], k.shape[1]
+    size = bias.element_size()
+    if bias.stride(-1) != 1 or Sq * Sk < _ALIGN_BIAS_FROM[size] or tuple(bias.shape[2:]) != (Sq, Sk) or bias.stride(2) == 0:
+        return bias
+    # (the forward reads four elements at a time where rows start on a multiple of four: 12 heads x 3068 bf16 148 us, copied 192)
+    align = 16 if backward else 4 * size
+    if bias.data_ptr() % align == 0 and not any(s * size % align for s, n in zip(bias.stride()[:3], bias.shape) if n > 1):
+        return bias
+    if bias.shape[0] not in (1, B) or bias.shape[1] not in (1, H):
+        return bias
+    nb, nh = (1 if bias.stride(i) == 0 else bias.shape[i] for i in (0, 1))
+    row = -(-Sk * size // 16) * 16 // size
+    if nb * nh * Sq * row * size > _ALIGN_BIAS_BYTES[backward]:
+        return bias
+    out = torch.empty((nb, nh, Sq, row), dtype=bias.dtype, device=bias.device)
+    dev = bias.device.index
+    with torch.cuda.device(dev):
+        status = _lib.load().fo_attn_bias_rows(bias.data_ptr(), _I64x3(*bias.stride()[:3]), size, nb, nh, Sq, Sk, out.data_ptr(), row, _raw_stream(dev))
+    _lib.check(status, "fo_attn_bias_rows")
+    return out[..., :Sk]
+
+
 def _extras(bias: Optional[Tensor], dropout: Optional[Dropout]) -> _AttnExtras:
     ex = _AttnExtras()
     if bias is not None:
@@ -316,8 +354,10 @@ class _FlashAttnBSHD(Function):
     @staticmethod
     def forward(ctx, q: Tensor, k: Tensor, v: Tensor, causal: bool, softmax_scale: Optional[float], return_lse: bool,
                 dropout: Optional[Dropout], bias: Optional[Tensor] = None):
-        o, lse = attn_fwd_strided(q, k, v, (0, 2, 1, 3), causal, softmax_scale, dropout, bias)
-        ctx.save_for_backward(q, k, v, o, lse, bias)
+        rows = _aligned_bias(bias, q, k, True)
+        o, lse = attn_fwd_strided(q, k, v, (0, 2, 1, 3), causal, softmax_scale, dropout, rows)
+        # (a copy of the bias is kept for the backward beside the bias itself, whose changes in place autograd watches)
+        ctx.save_for_backward(q, k, v, o, lse, bias, rows if rows is not bias else None)
         ctx.causal = causal
         ctx.softmax_scale = softmax_scale
         ctx.dropout = dropout
@@ -328,10 +368,11 @@ class _FlashAttnBSHD(Function):
 
     @staticmethod
     def backward(ctx, dO: Tensor, *unused):
-        q, k, v, o, lse, bias = ctx.saved_tensors
+        q, k, v, o, lse, bias, rows = ctx.saved_tensors
         if bias is not None and ctx.needs_input_grad[7]:
             raise RuntimeError("FlashAttention does not support bias gradient yet")   # flash_attention_triton.py:854
-        dq, dk, dv = attn_bwd_strided(q, k, v, o, lse, dO, (0, 2, 1, 3), ctx.causal, ctx.softmax_scale, ctx.dropout, bias)
+        dq, dk, dv = attn_bwd_strided(q, k, v, o, lse, dO, (0, 2, 1, 3), ctx.causal, ctx.softmax_scale, ctx.dropout,
+                                      bias if rows is None else rows)
         return dq, dk, dv, None, None, None, None, None
 
 
@@ -381,6 +422,7 @@ def flash_attn(
     raise, as in the reference (:854)."""
     drop = None if dropout_p == 0.0 else _dropout_arg(dropout_p, dropout_state, q.shape[0] * q.shape[2] * q.shape[1] * k.shape[1])
     if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad or (bias is not None and bias.requires_grad))):
-        o, lse = attn_fwd_strided(q, k, v, (0, 2, 1, 3), causal, softmax_scale, drop, bias)
+        rows = _aligned_bias(bias, q, k, False)
+        o, lse = attn_fwd_strided(q, k, v, (0, 2, 1, 3), causal, softmax_scale, drop, rows)
         return (o, lse) if return_lse else o
     return _FlashAttnBSHD.apply(q, k, v, causal, softmax_scale, return_lse, drop, bias)

@@ -171,6 +171,15 @@ int fo_attn_bwd_dropout(const void* q, const void* k, const void* v, const void*
                         const int64_t* const* strides_host, float softmax_scale, int causal, int dtype,
                         float dropout_p, uint32_t seed, uint64_t rng_offset, void* stream);
 
+/* A bias with a query stride, copied into rows that start on 16-byte boundaries: fo_attn_fwd_ex and fo_attn_bwd_ex take such
+ * a copy (strides H*Sq*out_row, Sq*out_row, out_row elements) faster than a bias whose base or strides are not multiples of 16
+ * bytes, which they read element by element. bias: element (b, h, q, key) at b*strides[0] + h*strides[1] + q*strides[2] + key,
+ * of elt_bytes 2 or 4; out: [B, H, Sq, out_row] contiguous, 16-byte aligned, out_row >= Sk elements and a multiple of 16
+ * bytes, the elements behind the last key written as zero. (For a bias that is broadcast over batch or heads copy it once, with B
+ * or H 1, and pass strides of 0.) One launch; no counterpart in the reference. */
+int fo_attn_bias_rows(const void* bias, const int64_t* strides_host, int elt_bytes, int B, int H, int Sq, int Sk, void* out, int64_t out_row,
+                      void* stream);
+
 /* The dropout keep-mask as a tensor of its own, one byte per element of [B, H, Sq, Sk] flattened (1 = kept): what
  * fo_attn_fwd_dropout applies for the same (dropout_p, seed, rng_offset). Replaces triton_dropout_mask's kernel
  * (flash_attention_triton.py:669-717), which the reference's tests use to build the mask for attention_ref. */

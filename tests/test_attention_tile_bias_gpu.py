@@ -12,12 +12,13 @@ from test_attention_bias_gpu import DEV, _bshd, _check
 pytestmark = pytest.mark.gpu
 
 
-# (the last two: keys that are no whole number of pieces)
-@pytest.mark.parametrize("B,H,Sq,Sk", [(2, 2, 449, 456), (1, 3, 577, 584), (1, 2, 640, 640), (1, 2, 130, 8), (1, 1, 333, 1030), (2, 1, 300, 333)])
+# (the last four: keys that are no whole number of 16-byte pieces)
+@pytest.mark.parametrize("B,H,Sq,Sk", [(2, 2, 449, 456), (1, 3, 577, 584), (1, 2, 640, 640), (1, 2, 130, 8), (1, 1, 333, 1030), (2, 1, 300, 333), (1, 2, 515, 1021), (2, 1, 1021, 771)])
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("bias_f32", [False, True])
+@pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("causal,dtype", [(False, torch.float16), (True, torch.bfloat16), (False, torch.bfloat16)])
-def test_tile_bias(B, H, Sq, Sk, D, bias_f32, causal, dtype):
+def test_tile_bias(B, H, Sq, Sk, D, bias_f32, packed, causal, dtype):
     g = torch.Generator().manual_seed(Sq + Sk + D)
     q, k, v, go = (torch.randn(B, H, n, D, generator=g).to(dtype) for n in (Sq, Sk, Sk, Sq))
     bias = (2.0 * torch.randn(1 if B == 2 else B, H, Sq, Sk, generator=g)).to(torch.float32 if bias_f32 else dtype)
@@ -29,6 +30,8 @@ def test_tile_bias(B, H, Sq, Sk, D, bias_f32, causal, dtype):
     pad = -Sk % 8 + 8
     wide = torch.full(bias.shape[:-1] + (Sk + pad,), float("nan"), dtype=bias.dtype, device=DEV)
     wide[..., :Sk] = bias.to(DEV)
+    if packed:                                                # rows without a gap: copied first where they are off 16-byte boundaries
+        wide = bias.to(DEV)
     t = [_bshd(x.to(DEV)).requires_grad_(True) for x in (q, k, v)]
     o, lse = flash_attn(*t, bias=wide[..., :Sk], causal=causal, return_lse=True)
     got = torch.autograd.grad(o, t, _bshd(go.to(DEV)))
