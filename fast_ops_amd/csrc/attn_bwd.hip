@@ -268,6 +268,8 @@ __device__ __forceinline__ void store_rows_via_lds(const f32x16 (&acc)[D / 32], 
   }
 }
 constexpr int stage_bytes(int D) { return 32 * (D * 2 + 16); }   // per wave and matrix
+template <int TBIAS, int D>
+constexpr int tile_bias_bytes() { return TBIAS == 4 && D == 128 ? 3 * 32 * 32 * 4 : 2 * kBwdTile * 32 * TBIAS; }   // per wave of the dK/dV kernel: its tiles of a bias
 
 // ---------------------------------------------------------------------------------------------------------------------
 // KBIAS (without BIAS): a bias that is the same for every query (query stride 0), at no cost per score. Its 64
@@ -889,10 +891,11 @@ static_assert(softmax_grad_jobs_fit(16) && softmax_grad_jobs_fit(12) && softmax_
 // 631 -> 391 us (no dropout 387), x 8192 1957 -> 1290 (1209), x 2048 causal 187 -> 119 (105); head_dim 64, 8 x 12 heads x
 // 1024 causal 139 -> 74 (71).
 // PAD, LIVE: a head_dim below D, as in the dQ kernel (96 columns: the phases are 12 groups long, with one or two slots each).
-// TBIAS: a bias with a query stride, of so many bytes per element (2, or 4 at head_dim 64, where two fp32 tiles per wave fit
-// into LDS beside the rings). The wave's 64 queries x 32 keys of tile j+2 are copied into LDS with that tile, two buffers; a
-// block's values, read transposed (a lane owns a key), are added to the start of its S accumulators in groups that carry
-// little else: S + (b - LSE) / scale then comes out of the MFMAs.
+// TBIAS: a bias with a query stride, of so many bytes per element (2 or 4). The wave's 64 queries x 32 keys of tile j+2 are
+// copied into LDS with that tile, two buffers; a block's values, read transposed (a lane owns a key), are added to the start
+// of its S accumulators in groups that carry little else: S + (b - LSE) / scale then comes out of the MFMAs. Two fp32 tiles per
+// wave do not fit beside the rings of head_dim 128 (by 1.5 KiB of 160): there it is three buffers of half a tile (32 queries),
+// of which tile j+2's second half takes the one that held the first half of tile j+1, half a phase after that was read.
 template <typename T, int D, bool CAUSAL, bool KBIAS = false, bool DROP = false, bool PAD = false, int LIVE = D, int TBIAS = 0>
 __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(const AttnBwdParams prm) {
   static_assert(TBIAS == 0 || !(KBIAS || DROP || PAD), "not combined");
@@ -930,7 +933,12 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   if constexpr (PAD) live.init(prm.d, wave_s, lane);
   // TBIAS: the wave's tile of the bias, 64 rows x 32 keys, as it lies in memory; needs what BiasRows needs
   constexpr int BELT = TBIAS == 4 ? 4 : 2, BROW = 32 * BELT, BTILE = kBwdTile * BROW, BPIECES = BTILE / 1024, BROWS = 1024 / BROW, BLANES = BROW / 16;
-  FO_LDS char* bias_lds = (FO_LDS char*)(rowvals + 2 * NBUF * kBwdTile) + wave_s * 2 * BTILE;
+  constexpr bool HALVES = TBIAS == 4 && D == 128;
+  FO_LDS char* bias_lds = (FO_LDS char*)(rowvals + 2 * NBUF * kBwdTile) + wave_s * tile_bias_bytes<TBIAS, D>();
+  // where the 32 queries qb of tile qt lie
+  auto bias_half = [&](int qt, int qb) -> FO_LDS char* {
+    return bias_lds + (HALVES ? (uint32_t)(2 * qt + qb) % 3u * (BTILE / 2) : (uint32_t)(qt & 1) * BTILE + qb * (BTILE / 2));
+  };
   const char* bias_lane_ptr = nullptr;       // the lane's piece of row lane / BLANES
   int64_t bias_row_bytes = 0;
   if constexpr (TBIAS != 0) {
@@ -938,18 +946,22 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
     const int col = min(k0w + (lane % BLANES) * (16 / BELT), (Sk - 1) / (16 / BELT) * (16 / BELT));
     bias_lane_ptr = (const char*)prm.bias.ptr + (b * prm.bias.strides[0] + h * prm.bias.strides[1] + col) * BELT + (lane / BLANES) * bias_row_bytes;
   }
-  auto issue_bias = [&](int qt) {
-    if (qt < ja) return;                     // (causal: this wave's keys start later)
-    FO_LDS char* dst = bias_lds + (qt & 1) * BTILE;
+  auto issue_bias_half = [&](int qt, int qb) {
+    FO_LDS char* dst = bias_half(qt, qb);
     if (qt * kBwdTile + kBwdTile <= Sq) {
 #pragma unroll
-      for (int i = 0; i < BPIECES; ++i) dma16_lane_ptr(bias_lane_ptr + (int64_t)(qt * kBwdTile + i * BROWS) * bias_row_bytes, dst + i * 1024);
+      for (int i = 0; i < BPIECES / 2; ++i) dma16_lane_ptr(bias_lane_ptr + (int64_t)(qt * kBwdTile + 32 * qb + i * BROWS) * bias_row_bytes, dst + i * 1024);
     } else {
       // (queries past the end re-read the last one; masked)
 #pragma unroll
-      for (int i = 0; i < BPIECES; ++i)
-        dma16_lane_ptr(bias_lane_ptr + (int64_t)(min(qt * kBwdTile + i * BROWS + lane / BLANES, Sq - 1) - lane / BLANES) * bias_row_bytes, dst + i * 1024);
+      for (int i = 0; i < BPIECES / 2; ++i)
+        dma16_lane_ptr(bias_lane_ptr + (int64_t)(min(qt * kBwdTile + 32 * qb + i * BROWS + lane / BLANES, Sq - 1) - lane / BLANES) * bias_row_bytes, dst + i * 1024);
     }
+  };
+  auto issue_bias = [&](int qt) {
+    if (qt < ja) return;                     // (causal: this wave's keys start later)
+    issue_bias_half(qt, 0);
+    if (!HALVES || qt == ja) issue_bias_half(qt, 1);      // HALVES: see where the first half of the tile before is read
   };
   auto issue = [&](int qt, int buf) {
     if constexpr (TBIAS != 0) issue_bias(qt);
@@ -1097,7 +1109,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   s16x4 bias16[4];
   f32x16 bias32;
   auto bias_read = [&](int jt, int qb) {
-    FO_LDS const char* src = bias_lds + (jt & 1) * BTILE + qb * 32 * BROW;
+    FO_LDS const char* src = bias_half(jt, qb);
 #pragma unroll
     for (int jv = 0; jv < 4; ++jv) {
       if constexpr (BELT == 2) {
@@ -1281,6 +1293,13 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
         constexpr int N1 = NMF - 4, N0 = HALF - 1;
         if (g == 1) bias_read(j, 1);
         if (g == 3 * NMF + 1) bias_read(j + 1, 0);
+        if constexpr (HALVES) {
+          // (the values of tile j+1's first half are in registers from here on: its buffer is free)
+          if (g == 3 * NMF + HALF) {
+            asm volatile("" ::"v"(bias32) : "memory");
+            if constexpr (!SPREAD) { if (j + 2 < n_qt) issue_bias_half(j + 2, 1); }
+          }
+        }
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           if (g == 2 + e * N1 / 16) bias_add(sacc[1], e);
@@ -1317,8 +1336,10 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
             // (two buffers: tile j's values have been read in the first groups)
             constexpr int EVERY = BPIECES == NMF ? 1 : 2;
             static_assert(BPIECES * EVERY <= NMF, "at most one piece per micro-group");
+            static_assert(!HALVES || (BPIECES / 2) * EVERY >= HALF, "the second half's pieces go out once its buffer is free");
             if (i % EVERY == 0 && i / EVERY < BPIECES)
-              dma16_lane_ptr(next_bias + (i / EVERY) * BROWS * bias_row_bytes, bias_lds + (j & 1) * BTILE + (i / EVERY) * 1024);
+              dma16_lane_ptr(next_bias + (i / EVERY) * BROWS * bias_row_bytes,
+                             bias_half(j + 2, i / EVERY / (BPIECES / 2)) + (i / EVERY) % (BPIECES / 2) * 1024);
           }
         }
       }
@@ -1365,6 +1386,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       bias_read(ja, 0);
 #pragma unroll
       for (int e = 0; e < 16; ++e) bias_add(sacc[0], e);
+      if constexpr (HALVES) { if (ja + 1 < n_qt) issue_bias_half(ja + 1, 1); }
     }
   };
   if (j < n_qt) start_tile((j - qt0) % NBUF);
@@ -1449,19 +1471,22 @@ static int launch_bwd_pad(const AttnBwdParams& q, unsigned g_dq, unsigned g_dkdv
 }
 
 // A bias with a query stride whose tiles can be copied, without dropout: what the score accumulators start from in both
-// kernels. (An fp32 bias at head_dim 128 leaves no room for two workgroups of the dQ kernel per compute unit, nor for its tiles
-// beside the rings of the dK/dV kernel: that runs on the kernels of the general form.) General form -> this, bias [1, H, S, S]:
+// kernels. (An fp32 bias at head_dim 128 leaves no room for two workgroups of the dQ kernel per compute unit: that one is of the
+// general form, in front of the dK/dV kernel of this one.) General form -> this, bias [1, H, S, S]:
 // 12 heads x 3072 causal at head_dim 128 bf16 bias: dQ 156 -> 111 us, dK/dV 147 -> 90; whole backward not causal 540 -> 320;
 // at head_dim 64 235 -> 131 causal, 347 -> 209 not, with an fp32 bias 258 -> 151 and 384 -> 270.
+// fp32 bias at head_dim 128, whole backward: 12 heads x 3072 345 -> 290 causal, 585 -> 468 not; x 1024 111 -> 93; x 512 the same (87);
+// 16 x 4096 504 -> 438 and 804 -> 677.
 template <typename T, int D, bool CAUSAL, int ELT>
 static int launch_bwd_tile_bias(const AttnBwdParams& q, unsigned g_dq, unsigned g_dkdv, size_t lds_tiles, size_t lds_pipe, hipStream_t s) {
-  const size_t lds_dq = lds_tiles + kBwdWaves * BiasRows<T, ELT>::BYTES, lds_kv = lds_pipe + kBwdWaves * 2 * kBwdTile * 32 * ELT;
-  static const hipError_t a1 = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<T, D, CAUSAL, false, false, false, false, D, ELT>,
+  constexpr int DQ_ELT = D == 128 && ELT == 4 ? 0 : ELT;
+  const size_t lds_dq = lds_tiles + (DQ_ELT ? kBwdWaves * BiasRows<T, ELT>::BYTES : 512), lds_kv = lds_pipe + kBwdWaves * tile_bias_bytes<ELT, D>();
+  static const hipError_t a1 = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<T, D, CAUSAL, false, DQ_ELT == 0, false, false, D, DQ_ELT>,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dq);
   static const hipError_t a2 = hipFuncSetAttribute((const void*)attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, false, false, D, ELT>,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_kv);
   if (a1 != hipSuccess || a2 != hipSuccess) return FO_ERR_LAUNCH;
-  attn_bwd_dq_kernel<T, D, CAUSAL, false, false, false, false, D, ELT><<<g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
+  attn_bwd_dq_kernel<T, D, CAUSAL, false, DQ_ELT == 0, false, false, D, DQ_ELT><<<g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
   attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, false, false, D, ELT><<<g_dkdv, kBwdWaves * 64, lds_kv, s>>>(q);
   return launch_status();
 }
@@ -1519,7 +1544,7 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
     // (dma_ok: base and strides are multiples of 16 bytes, the query stride is not zero)
     if (p.d == D && p.bias.dma_ok && tune(g_attn_bwd_variant) != 0) {
       if (!p.bias.is_f32) return launch_bwd_tile_bias<T, D, CAUSAL, 2>(q, (unsigned)g_dq, (unsigned)g_dkdv, lds_tiles, lds_pipe, s);
-      if constexpr (D == 64) return launch_bwd_tile_bias<T, D, CAUSAL, 4>(q, (unsigned)g_dq, (unsigned)g_dkdv, lds_tiles, lds_pipe, s);
+      return launch_bwd_tile_bias<T, D, CAUSAL, 4>(q, (unsigned)g_dq, (unsigned)g_dkdv, lds_tiles, lds_pipe, s);
     }
   }
   if constexpr (!DROP && !BIAS) {

@@ -37,3 +37,12 @@ def test_tile_bias(B, H, Sq, Sk, D, bias_f32, packed, causal, dtype):
     got = torch.autograd.grad(o, t, _bshd(go.to(DEV)))
     torch.cuda.synchronize()
     _check(_bshd(o), lse, [_bshd(x) for x in got], o_ref, lse_ref, ref)
+
+
+# one to three query tiles, the last of them whole or not: where the first tiles' copies and the last ones' hand-overs meet
+@pytest.mark.parametrize("Sq,Sk", [(33, 64), (64, 128), (65, 136), (128, 260), (192, 128)])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bias_f32", [False, True])
+@pytest.mark.parametrize("causal", [False, True])
+def test_tile_bias_few_query_tiles(Sq, Sk, D, bias_f32, causal):
+    test_tile_bias(1, 2, Sq, Sk, D, bias_f32, False, causal, torch.bfloat16)
