@@ -362,8 +362,12 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
     }
   }
   typedef BiasRows<T, TBIAS == 4 ? 4 : 2> BR;
-  FO_LDS char* row_bias = smem + 4 * TILE_BYTES + wave_s * BR::BYTES;      // TBIAS: the wave's own
-  if constexpr (TBIAS != 0) BR::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, 0, row_bias, lane);
+  // (TBIAS 4 at head_dim 128: half a tile at a time, 32 keys, or two workgroups of this kernel do not fit a compute unit)
+  constexpr bool HALVES = TBIAS == 4 && D == 128;
+  typedef BiasRows<T, 4, 32> BRH;
+  FO_LDS char* row_bias = smem + 4 * TILE_BYTES + wave_s * (HALVES ? BRH::BYTES : BR::BYTES);      // TBIAS: the wave's own
+  if constexpr (HALVES) BRH::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, 0, row_bias, lane);
+  else if constexpr (TBIAS != 0) BR::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, 0, row_bias, lane);
 
   // B operands held for the whole kernel: Q^T and dO^T fragments of this lane's query row; its LSE and delta
   const int qrow = min(q0w + l32, Sq - 1);
@@ -449,7 +453,11 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
           for (int u = 0; u < 4; ++u) sacc[kb][4 * jv + u] = b4[u];
         }
     }
-    if constexpr (TBIAS != 0) {
+    if constexpr (HALVES) {
+      BRH::each(row_bias, 0, l32, hh, [&](int r, float v) { sacc[0][r] = v * per_scale; });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read: the buffer is free for the tile's other half
+      BRH::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, key0 + 32, row_bias, lane);
+    } else if constexpr (TBIAS != 0) {
       BR::each(row_bias, 0, l32, hh, [&](int r, float v) { sacc[0][r] = v * per_scale; });
       BR::each(row_bias, 1, l32, hh, [&](int r, float v) { sacc[1][r] = v * per_scale; });
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read: the buffer is free for the next tile's
@@ -462,6 +470,13 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
         sacc[kb] = Ops<T>::mfma(row_frag<T, D>(kt, kb, ks, l32, hh), qf[ks], sacc[kb]);      // S^T = K Q^T
         dpacc[kb] = Ops<T>::mfma(row_frag<T, D>(vt, kb, ks, l32, hh), gf[ks], dpacc[kb]);    // dP^T = V dO^T
       }
+    if constexpr (HALVES) {
+      // (behind the products, which cover most of the copy's way; what else is in flight was issued before it)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      BRH::each(row_bias, 0, l32, hh, [&](int r, float v) { sacc[1][r] = __builtin_fmaf(v, per_scale, sacc[1][r]); });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (tile + 1 < n_tiles) BRH::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, key0 + kBwdTile, row_bias, lane);
+    }
     // register r of block kb holds key key0 + 32*kb + 4*hh + koff(r), koff(r) = (r & 3) + 8 * (r >> 2); dead iff
     // key > q or key >= Sk
     vec8 dsf[4];
@@ -1471,22 +1486,21 @@ static int launch_bwd_pad(const AttnBwdParams& q, unsigned g_dq, unsigned g_dkdv
 }
 
 // A bias with a query stride whose tiles can be copied, without dropout: what the score accumulators start from in both
-// kernels. (An fp32 bias at head_dim 128 leaves no room for two workgroups of the dQ kernel per compute unit: that one is of the
-// general form, in front of the dK/dV kernel of this one.) General form -> this, bias [1, H, S, S]:
+// kernels. (An fp32 bias at head_dim 128 goes through half a tile's buffer in the dQ kernel, so that two of its workgroups still
+// fit a compute unit, and three in the dK/dV kernel.) General form -> this, bias [1, H, S, S]:
 // 12 heads x 3072 causal at head_dim 128 bf16 bias: dQ 156 -> 111 us, dK/dV 147 -> 90; whole backward not causal 540 -> 320;
 // at head_dim 64 235 -> 131 causal, 347 -> 209 not, with an fp32 bias 258 -> 151 and 384 -> 270.
-// fp32 bias at head_dim 128, whole backward: 12 heads x 3072 345 -> 290 causal, 585 -> 468 not; x 1024 111 -> 93; x 512 the same (87);
-// 16 x 4096 504 -> 438 and 804 -> 677.
+// fp32 bias at head_dim 128, whole backward: 12 heads x 3072 345 -> 218 causal (290 with the general dQ kernel), 585 -> 384 not (468);
+// x 1024 111 -> 88; x 512 the same (87); 16 x 4096 510 -> 371 and 803 -> 626.
 template <typename T, int D, bool CAUSAL, int ELT>
 static int launch_bwd_tile_bias(const AttnBwdParams& q, unsigned g_dq, unsigned g_dkdv, size_t lds_tiles, size_t lds_pipe, hipStream_t s) {
-  constexpr int DQ_ELT = D == 128 && ELT == 4 ? 0 : ELT;
-  const size_t lds_dq = lds_tiles + (DQ_ELT ? kBwdWaves * BiasRows<T, ELT>::BYTES : 512), lds_kv = lds_pipe + kBwdWaves * tile_bias_bytes<ELT, D>();
-  static const hipError_t a1 = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<T, D, CAUSAL, false, DQ_ELT == 0, false, false, D, DQ_ELT>,
+  const size_t lds_dq = lds_tiles + kBwdWaves * (D == 128 && ELT == 4 ? BiasRows<T, 4, 32>::BYTES : BiasRows<T, ELT>::BYTES), lds_kv = lds_pipe + kBwdWaves * tile_bias_bytes<ELT, D>();
+  static const hipError_t a1 = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<T, D, CAUSAL, false, false, false, false, D, ELT>,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dq);
   static const hipError_t a2 = hipFuncSetAttribute((const void*)attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, false, false, D, ELT>,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_kv);
   if (a1 != hipSuccess || a2 != hipSuccess) return FO_ERR_LAUNCH;
-  attn_bwd_dq_kernel<T, D, CAUSAL, false, DQ_ELT == 0, false, false, D, DQ_ELT><<<g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
+  attn_bwd_dq_kernel<T, D, CAUSAL, false, false, false, false, D, ELT><<<g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
   attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, false, false, D, ELT><<<g_dkdv, kBwdWaves * 64, lds_kv, s>>>(q);
   return launch_status();
 }

@@ -293,15 +293,15 @@ __device__ __forceinline__ void dma4_uniform_base(const void* base, uint32_t byt
 }
 
 // A bias with a query stride where a lane owns a query row (forward and dQ kernels): the wave's 32 rows x 64 keys of a key tile,
-// copied straight into LDS, ELT bytes per element, ROW bytes per row; 16-byte piece s of a row holds the row's piece
+// copied straight into LDS (or KEYS of the keys), ELT bytes per element, ROW bytes per row; 16-byte piece s of a row holds the row's piece
 // s ^ (row mod pieces), so that 32 rows' reads of the same piece are spread over the banks. One buffer per wave: once a
 // tile's values are read (they start or join its score accumulators) the next tile's copy begins. Needs the
 // 16-byte alignment of dma_ok. Pieces past the end re-read the last one that holds a key - of which the part behind the last
 // key is read too, up to the next 16-byte boundary, and may hold anything - and rows past the end the last row; the kernels
 // mask both after the bias has been applied.
-template <typename T, int ELT>
+template <typename T, int ELT, int KEYS = 64>
 struct BiasRows {
-  static constexpr int PIECE_KEYS = 16 / ELT, ROW = 64 * ELT, PIECES = ROW / 16, ROWS_PER_DMA = 64 / PIECES, BYTES = 32 * ROW;
+  static constexpr int PIECE_KEYS = 16 / ELT, ROW = KEYS * ELT, PIECES = ROW / 16, ROWS_PER_DMA = 64 / PIECES, BYTES = 32 * ROW;
   // `row0`: element (b, h, 0, 0); q0w: the wave's first row
   static __device__ __forceinline__ void copy(const BiasParams& bp, int64_t row0, int q0w, int Sq, int Sk, int key0, FO_LDS char* dst, int lane_in) {
     int lane = lane_in;
@@ -321,12 +321,12 @@ struct BiasRows {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if constexpr (ELT == 4) {
-        const f32x4 v = *(FO_LDS const f32x4*)(src + l32 * ROW + (((8 * kb + 2 * j + hh) ^ (l32 & 15)) * 16));
+        const f32x4 v = *(FO_LDS const f32x4*)(src + l32 * ROW + (((8 * kb + 2 * j + hh) ^ (l32 & (PIECES - 1))) * 16));
 #pragma unroll
         for (int u = 0; u < 4; ++u) f(4 * j + u, v[u]);
       } else {
         typedef __attribute__((ext_vector_type(4))) T vec4;
-        const vec4 v = *(FO_LDS const vec4*)(src + l32 * ROW + (((4 * kb + j) ^ (l32 & 7)) * 16) + hh * 8);
+        const vec4 v = *(FO_LDS const vec4*)(src + l32 * ROW + (((4 * kb + j) ^ (l32 & (PIECES - 1))) * 16) + hh * 8);
 #pragma unroll
         for (int u = 0; u < 4; ++u) f(4 * j + u, (float)v[u]);
       }
