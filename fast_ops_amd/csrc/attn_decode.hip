@@ -132,10 +132,12 @@ __global__ void __launch_bounds__(kDecWaves * 64) attn_decode_kernel(const Decod
     float mloc = sacc[0];
 #pragma unroll
     for (int r = 1; r < 16; ++r) mloc = fmaxf(mloc, sacc[r]);
-    mloc = fmaxf(mloc, half_swap(mloc));                                   // (finite: a tile has at least one key)
+    mloc = fmaxf(mloc, half_swap(mloc));
+    // (scores of -inf - K may hold it to take keys out - can fill all of a wave's tiles so far, whatever the other waves'
+    // keys score: its reference then stays 0 until a key counts, and its sums 0)
     if (__builtin_amdgcn_ballot_w64(mloc * c > m_run * c + kDecLazyLog2) != 0) {
       const float m_new = fmaxf(m_run, mloc);
-      const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * c);
+      const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f((m_run - m_new) * c);
       m_run = m_new;
       l_run *= alpha;
 #pragma unroll
@@ -143,7 +145,7 @@ __global__ void __launch_bounds__(kDecWaves * 64) attn_decode_kernel(const Decod
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[i][r] *= alpha;
     }
-    const float mc = m_run * c;
+    const float mc = m_run == -INFINITY ? 0.0f : m_run * c;
     vec8 pf[2];
     float psum = 0.0f;
 #pragma unroll
@@ -183,9 +185,11 @@ __global__ void __launch_bounds__(kDecWaves * 64) attn_decode_kernel(const Decod
 #pragma unroll
     for (int w = 0; w < kDecWaves; ++w) m = fmaxf(m, ml[(w * 32 + r) * 2]);
     f32x4 o4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    // (no key of this workgroup counts, those of another may: sums of 0. A row without any such key comes out as NaN.)
+    const bool none = prm.n_split > 1 && m == -INFINITY;
 #pragma unroll
     for (int w = 0; w < kDecWaves; ++w) {
-      const float f = __builtin_amdgcn_exp2f((ml[(w * 32 + r) * 2] - m) * c);      // (a wave without tiles: 0)
+      const float f = none ? 0.0f : __builtin_amdgcn_exp2f((ml[(w * 32 + r) * 2] - m) * c);      // (a wave without tiles: 0)
       l += f * ml[(w * 32 + r) * 2 + 1];
       const f32x4 part = *(FO_LDS const f32x4*)((FO_LDS float*)(smem + w * 4 * TILE_BYTES) + r * OROW + 4 * d4);
 #pragma unroll

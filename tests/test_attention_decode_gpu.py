@@ -43,3 +43,28 @@ def test_decode_against_oracle(B, H, Sq, Sk, D, dtype, multi_query, split):
     err = (o.float().cpu() - o_ref).abs()
     assert float((err - (O_ATOL + O_RTOL * o_ref.abs())).max()) <= 0, f"O: max abs err {float(err.max()):.3e}"
     assert float((lse.cpu() - lse_ref).abs().max()) <= LSE_ATOL
+
+
+# K holds -inf in the column that Q holds 1 in: those keys score -inf. They fill whole tiles of some waves, all tiles of some
+# waves, and (split 7) all tiles of some workgroups; the other keys of the row count as if they were alone.
+@pytest.mark.parametrize("split", [-1, 1, 7])
+@pytest.mark.parametrize("Sq,Sk,D,dtype,live", [(1, 2000, 128, torch.bfloat16, (0, 1000)), (8, 4096, 64, torch.float16, (0, 196)),
+                                                (32, 1000, 64, torch.bfloat16, (600, 650)), (1, 1025, 128, torch.float16, (1024, 1025))])
+def test_decode_with_keys_that_score_minus_infinity(Sq, Sk, D, dtype, live, split):
+    g = torch.Generator().manual_seed(Sk)
+    q, k, v = (torch.randn(2, 3, n, D, generator=g).to(dtype) for n in (Sq, Sk, Sk))
+    q[..., 0] = 1
+    k[..., 0] = float("-inf")
+    k[:, :, live[0]:live[1], 0] = 0
+    o_ref, lse_ref = attention_fwd_oracle(q, k, v)
+    surface._FWD_PLANS.clear()
+    _lib.tune_set("attn.decode_split", split)
+    try:
+        o, lse = multi_head_attention(q.to(DEV), k.to(DEV), v.to(DEV), return_lse=True)
+        torch.cuda.synchronize()
+    finally:
+        _lib.tune_set("attn.decode_split", -1)
+        surface._FWD_PLANS.clear()
+    err = (o.float().cpu() - o_ref).abs()
+    assert float((err - (O_ATOL + O_RTOL * o_ref.abs())).max()) <= 0, f"O: max abs err {float(err.max()):.3e}"
+    assert float((lse.cpu() - lse_ref).abs().max()) <= LSE_ATOL
