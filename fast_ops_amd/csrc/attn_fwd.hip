@@ -1803,11 +1803,8 @@ extern "C" int fo_attn_fwd_kernel(int B, int H, int Sq, int Sk, int D, const int
   for (int i = 0; i < 3; ++i) { p.ks[i] = ks[i]; p.vs[i] = vs[i]; }
   p.bias.ptr = has_bias ? (const void*)ks : nullptr;   // (only tested against NULL)
   p.bias.strides[2] = has_bias == 2 ? 0 : 1;
-  // (a call with dropout takes the form that the same call without it would, with four waves where that is the eight-wave
-  // form; this query answers for the plain kernel, which serves dropout at every size)
-  if (has_dropout) return FO_ATTN_KERNEL_ROWS128;
-  if (takes_decode(p, causal != 0, false, tune(g_attn_variant))) return FO_ATTN_KERNEL_DECODE;
-  return choose_kernel(p, D > 64 ? 128 : 64, causal != 0, false, tune(g_attn_variant));
+  if (takes_decode(p, causal != 0, has_dropout != 0, tune(g_attn_variant))) return FO_ATTN_KERNEL_DECODE;
+  return choose_kernel(p, D > 64 ? 128 : 64, causal != 0, has_dropout != 0, tune(g_attn_variant));
 }
 
 extern "C" int64_t fo_attn_fwd_workspace(int B, int H, int Sq, int Sk, int D, const int64_t* ks, const int64_t* vs, int causal) {

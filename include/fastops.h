@@ -97,12 +97,11 @@ int fo_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* 
                    const int64_t* v_strides_host, const int64_t* o_strides_host,
                    float softmax_scale, int causal, int dtype, void* ws, int64_t ws_bytes, void* stream);
 
-/* Which kernel fo_attn_fwd (or _ex, with has_bias non-zero) launches for a call of this shape
+/* Which kernel fo_attn_fwd (or _dropout / _ex, with has_dropout / has_bias non-zero) launches for a call of this shape
  * on the current device with the current "attn.variant": one of the FO_ATTN_KERNEL_* codes below, or a negative
  * fo_status where fo_attn_fwd would reject the shape. has_bias: 0 none, 1 a bias with a query stride, 2 a bias that is
- * the same for every query (query stride 0), which the pipelined kernels take as well. With has_dropout the answer is
- * always FO_ATTN_KERNEL_ROWS128, the form that serves dropout at every size; where the same call without dropout takes a
- * pipelined form, the call with it does too (with four waves where that is the eight-wave form). Launches nothing. The choice
+ * the same for every query (query stride 0), which the pipelined kernels take as well, and so does dropout (with four
+ * waves where the call without it takes the eight-wave form). Launches nothing. The choice
  * depends on the number of compute units of the current device. No reference counterpart:
  * the reference has one kernel (flash_attention_fwd.cu:164-177); tests use this to assert which code they covered. */
 enum {

@@ -42,6 +42,9 @@ def test_dropout_on_every_form(B, H, Sq, Sk, D, causal, dtype, bias, variant):
     _lib.tune_set("attn.variant", variant)
     _lib.tune_set("attn_bwd.variant", 0 if variant == 0 else -1)
     try:
+        if variant >= 0:                     # the form asked for is the form that runs
+            st = [(_lib.ctypes.c_int64 * 3)(x.stride(0), x.stride(2), x.stride(1)) for x in t[1:]]
+            assert _lib.load().fo_attn_fwd_kernel(B, H, Sq, Sk, D, *st, causal, 2 if bias else 0, 1) == variant
         o, lse = flash_attn(*t, bias=None if b is None else b.to(DEV), causal=causal, dropout_p=p, return_lse=True, dropout_state=(seed, off))
         got = torch.autograd.grad(o, t, go.to(DEV).transpose(1, 2))
         torch.cuda.synchronize()

@@ -178,10 +178,11 @@ def test_attn_kernel_query_and_stride_limit_without_device_work():
     dense = lambda S, D: I3(S * D * 4, S * D, D)
     k = lambda B, H, Sq, Sk, D, causal, bias=0, drop=0, ks=None: lib.fo_attn_fwd_kernel(
         B, H, Sq, Sk, D, ks or dense(Sk, D), ks or dense(Sk, D), causal, bias, drop)
-    # small shapes, bias and dropout always take the 128-row kernel, whatever the device
+    # small shapes and a bias with a query stride always take the 128-row kernel, whatever the device, with dropout or not
     assert k(1, 1, 128, 128, 64, 0) == _lib.FO_ATTN_KERNEL_ROWS128
     assert k(2, 16, 8192, 8192, 128, 1, bias=1) == _lib.FO_ATTN_KERNEL_ROWS128
-    assert k(2, 16, 8192, 8192, 128, 1, drop=1) == _lib.FO_ATTN_KERNEL_ROWS128
+    assert k(1, 1, 128, 128, 64, 0, drop=1) == _lib.FO_ATTN_KERNEL_ROWS128
+    assert k(2, 16, 8192, 8192, 128, 1, bias=1, drop=1) == _lib.FO_ATTN_KERNEL_ROWS128
     # forced choices are honoured where the kernel exists
     assert lib.fo_tune_set(b"attn.variant", 32) == 0
     try:
@@ -230,7 +231,19 @@ def test_attn_kernel_query_and_stride_limit_without_device_work():
         assert k(2, 16, 8192, 8192, 128, 1, bias=2) == W4 and k(2, 16, 4096, 4096, 128, 1, bias=2) == W4    # (W8 without bias)
         assert k(1, 8, 8192, 8192, 64, 0, bias=2) == W4 and k(1, 12, 4096, 4096, 64, 1, bias=2) == PIPE
         assert k(2, 16, 8192, 8256, 128, 0, bias=2) == R128 and k(2, 16, 8192, 8130, 128, 0, bias=2) == W4  # at most 8192 keys in LDS
-        assert k(2, 16, 8192, 8192, 128, 1, bias=2, drop=1) == R128
+        # dropout takes part too, in the same forms, with and without such a bias
+        assert k(2, 16, 8192, 8192, 128, 1, drop=1) == W4 and k(2, 16, 8192, 8192, 128, 1, bias=2, drop=1) == W4
+        assert k(2, 16, 4096, 4096, 128, 1, drop=1) == W4 and k(2, 16, 4096, 4096, 128, 1, bias=2, drop=1) == W4    # (W8 without)
+        assert k(1, 12, 2048, 2048, 128, 1, drop=1) == PIPE and k(8, 12, 1024, 1024, 64, 1, drop=1) == R128
+        assert k(4, 16, 1, 4000, 128, 0, drop=1) == PIPE and k(4, 16, 1, 4000, 128, 0) == _lib.FO_ATTN_KERNEL_DECODE
+    # (the eight-wave form does not exist with dropout, and neither does the exact running maximum)
+    for asked, runs in ((0, 0), (1, 0), (8, 8), (16, 32), (32, 32)):
+        assert lib.fo_tune_set(b"attn.variant", asked) == 0
+        try:
+            assert k(2, 16, 4096, 4096, 128, 1, drop=1) == runs and k(2, 16, 4096, 4096, 128, 1, bias=1, drop=1) == 0
+            assert k(2, 16, 4096, 4096, 96, 1, drop=1) == 0
+        finally:
+            lib.fo_tune_set(b"attn.variant", -1)
     # head dims other than 64 and 128 take the 128-row kernel, whatever is forced
     assert k(2, 16, 8192, 8192, 96, 1) == _lib.FO_ATTN_KERNEL_ROWS128
     assert lib.fo_attn_fwd_kernel(1, 1, 128, 128, 64, None, dense(128, 64), 0, 0, 0) == -1
