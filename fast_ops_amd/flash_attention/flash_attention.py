@@ -99,11 +99,22 @@ def _aligned_bias(bias: Optional[Tensor], q: Tensor, k: Tensor, backward: bool) 
     row = -(-Sk * size // 16) * 16 // size
     if nb * nh * Sq * row * size > _ALIGN_BIAS_BYTES[backward]:
         return bias
-    out = torch.empty((nb, nh, Sq, row), dtype=bias.dtype, device=bias.device)
+    try:
+        out = torch.empty((nb, nh, Sq, row), dtype=bias.dtype, device=bias.device)
+    except torch.OutOfMemoryError:                             # no room for a copy: the kernels read the bias as it is
+        return bias
     dev = bias.device.index
-    with torch.cuda.device(dev):
+    # (as in attn_fwd_strided: the device is made current only when it is not)
+    guard = torch.cuda.device(dev) if torch.cuda.current_device() != dev else None
+    if guard is not None:
+        guard.__enter__()
+    try:
         status = _lib.load().fo_attn_bias_rows(bias.data_ptr(), _I64x3(*bias.stride()[:3]), size, nb, nh, Sq, Sk, out.data_ptr(), row, _raw_stream(dev))
-    _lib.check(status, "fo_attn_bias_rows")
+    finally:
+        if guard is not None:
+            guard.__exit__(None, None, None)
+    if status != 0:
+        _lib.check(status, "fo_attn_bias_rows")
     return out[..., :Sk]
 
 
@@ -354,10 +365,9 @@ class _FlashAttnBSHD(Function):
     @staticmethod
     def forward(ctx, q: Tensor, k: Tensor, v: Tensor, causal: bool, softmax_scale: Optional[float], return_lse: bool,
                 dropout: Optional[Dropout], bias: Optional[Tensor] = None):
-        rows = _aligned_bias(bias, q, k, True)
-        o, lse = attn_fwd_strided(q, k, v, (0, 2, 1, 3), causal, softmax_scale, dropout, rows)
-        # (a copy of the bias is kept for the backward beside the bias itself, whose changes in place autograd watches)
-        ctx.save_for_backward(q, k, v, o, lse, bias, rows if rows is not bias else None)
+        o, lse = attn_fwd_strided(q, k, v, (0, 2, 1, 3), causal, softmax_scale, dropout, _aligned_bias(bias, q, k, False))
+        # (the bias itself, not its copy: every layer that shares a bias would hold a copy of its own until its backward)
+        ctx.save_for_backward(q, k, v, o, lse, bias)
         ctx.causal = causal
         ctx.softmax_scale = softmax_scale
         ctx.dropout = dropout
@@ -368,11 +378,11 @@ class _FlashAttnBSHD(Function):
 
     @staticmethod
     def backward(ctx, dO: Tensor, *unused):
-        q, k, v, o, lse, bias, rows = ctx.saved_tensors
+        q, k, v, o, lse, bias = ctx.saved_tensors
         if bias is not None and ctx.needs_input_grad[7]:
             raise RuntimeError("FlashAttention does not support bias gradient yet")   # flash_attention_triton.py:854
         dq, dk, dv = attn_bwd_strided(q, k, v, o, lse, dO, (0, 2, 1, 3), ctx.causal, ctx.softmax_scale, ctx.dropout,
-                                      bias if rows is None else rows)
+                                      _aligned_bias(bias, q, k, True))
         return dq, dk, dv, None, None, None, None, None
 
 

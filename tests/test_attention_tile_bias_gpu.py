@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from fast_ops.flash_attention.flash_attention import flash_attn
+from fast_ops_amd.flash_attention import flash_attention as surface
 from oracle.attention_oracle import attention_bwd_oracle, attention_fwd_oracle
 from test_attention_bias_gpu import DEV, _bshd, _check
 
@@ -46,3 +47,28 @@ def test_tile_bias(B, H, Sq, Sk, D, bias_f32, packed, causal, dtype):
 @pytest.mark.parametrize("causal", [False, True])
 def test_tile_bias_few_query_tiles(Sq, Sk, D, bias_f32, causal):
     test_tile_bias(1, 2, Sq, Sk, D, bias_f32, False, causal, torch.bfloat16)
+
+
+# (the packed rows of 1021 elements are copied into aligned ones, by the forward and by the backward)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_no_copy_of_the_bias_lives_from_forward_to_backward(dtype):
+    g = torch.Generator().manual_seed(5)
+    t = [torch.randn(1, 1021, 4, 64, generator=g).to(dtype).to(DEV).requires_grad_(True) for _ in range(3)]
+    bias = torch.randn(1, 4, 1021, 1021, generator=g).to(dtype).to(DEV)
+    assert surface._aligned_bias(bias, t[0], t[1], False) is not bias and surface._aligned_bias(bias, t[0], t[1], True) is not bias
+    before = torch.cuda.memory_allocated()
+    o = flash_attn(*t, bias=bias)
+    assert torch.cuda.memory_allocated() - before < bias.numel() * bias.element_size() // 2      # O and the LSE: an eighth of a copy
+    torch.autograd.grad(o, t, torch.ones_like(o))
+
+
+def test_bias_is_read_in_place_where_a_copy_finds_no_memory(monkeypatch):
+    empty = torch.empty
+
+    def no_room(*args, **kw):
+        if args and isinstance(args[0], tuple) and args[0][-1] == 1024:
+            raise torch.OutOfMemoryError("no room for the copy")
+        return empty(*args, **kw)
+
+    monkeypatch.setattr(torch, "empty", no_room)
+    test_tile_bias(1, 2, 515, 1021, 64, False, True, True, torch.bfloat16)
