@@ -69,25 +69,34 @@ def _expand_bias(bias: Tensor, q: Tensor, B: int, H: int, Sq: int, Sk: int) -> T
     return bias.expand(B, H, Sq, Sk)
 
 
-# When _aligned_bias copies: from so many (query, key) pairs on, by the bytes of an element - below, the copy's launch and its host
-# time cost more than it gains (12 heads, forward + backward, bf16 bias / fp32 bias: 333 keys 135 -> 153 / 135 -> 152 us, 515 keys 173 -> 149
-# / 138 -> 151, 1021 keys 465 -> 146 / 237 -> 186, 3071 keys 2418 -> 507 / 1321 -> 1000) - and up to a copy of so many bytes, without
-# and with a backward to come. The forward alone gains only while the memory-side cache (256 MiB) holds the copy: 12 heads x 3071 bf16
-# (226 MB) 332 -> 206 us and causal 210 -> 166, but fp32 218 -> 252 causal and 16 heads x 4095 bf16 250 -> 304.
-_ALIGN_BIAS_FROM = {2: 1 << 18, 4: 1 << 19}
+# When _aligned_bias copies, without and with a backward's kernels to come. From so many (query, key) pairs on, by the bytes of an
+# element: below, the launch and its host time (16 us) cost more than the copy gains (12 heads at head_dim 64, in place -> copied;
+# forward 515 keys bf16 37 -> 29 us, 725 keys 49 -> 31 and fp32 50 -> 33, 1021 keys 66 -> 36 and 64 -> 44; forward + backward with both
+# copied 515 keys bf16 155 -> 174, 725 keys 225 -> 175 and fp32 causal 145 -> 173, 1021 keys 434 -> 175 and 213 -> 174).
+# Up to so many bytes of rows (rows x bytes of an element) in the forward, whose gain grows with the keys a workgroup walks (about
+# 0.045 us per key) while the copy costs 0.45 us per MB: 12 heads x 3071 bf16 298 -> 162 us, causal 194 -> 145, 4 heads x 3071 fp32 184 ->
+# 117; beyond, 64 heads x 1021 causal bf16 69 -> 81, fp32 68 -> 140, 12 heads x 2047 fp32 125 -> 130. The backward gains at every
+# number of heads (64 heads x 1021, backward alone: bf16 412 -> 118, fp32 289 -> 245). And up to a copy of so many bytes: what
+# the memory-side cache (256 MiB) holds for the forward.
+_ALIGN_BIAS_FROM = {False: {2: 1 << 19, 4: 3 << 18}, True: {2: 1 << 18, 4: 1 << 19}}
+_ALIGN_BIAS_ROW_BYTES = 80000
 _ALIGN_BIAS_BYTES = {False: 256 << 20, True: 4 << 30}
 
 
 def _aligned_bias(bias: Optional[Tensor], q: Tensor, k: Tensor, backward: bool) -> Optional[Tensor]:
     """A bias with a row per query whose rows do not start on 16-byte boundaries, copied (once for what is broadcast over batch
     or heads) into rows that do, which is what the kernels copy tiles from; any other bias as it is. (flash_attn's layout.)"""
-    if bias is None or bias.dim() != 4 or bias.shape[2] == 1 or q.dim() != 4 or k.dim() != 4:
+    if bias is None:
+        return bias
+    shape = bias.shape
+    # (fewer pairs than are asked for in any case: the usual end of a small call, and of a bias that is the same for every query)
+    if len(shape) != 4 or shape[2] * shape[3] < 1 << 18 or shape[2] == 1 or q.dim() != 4 or k.dim() != 4:
         return bias                                            # (what does not fit is refused further on)
     if bias.dtype not in (q.dtype, torch.float32) or not bias.is_cuda or bias.device != q.device:
         return bias
     B, Sq, H, Sk = q.shape[0], q.shape[1], q.shape[2], k.shape[1]
     size = bias.element_size()
-    if bias.stride(-1) != 1 or Sq * Sk < _ALIGN_BIAS_FROM[size] or tuple(bias.shape[2:]) != (Sq, Sk) or bias.stride(2) == 0:
+    if bias.stride(-1) != 1 or Sq * Sk < _ALIGN_BIAS_FROM[backward][size] or tuple(bias.shape[2:]) != (Sq, Sk) or bias.stride(2) == 0:
         return bias
     # (the forward reads four elements at a time where rows start on a multiple of four: 12 heads x 3068 bf16 148 us, copied 192)
     align = 16 if backward else 4 * size
@@ -97,7 +106,7 @@ def _aligned_bias(bias: Optional[Tensor], q: Tensor, k: Tensor, backward: bool) 
         return bias
     nb, nh = (1 if bias.stride(i) == 0 else bias.shape[i] for i in (0, 1))
     row = -(-Sk * size // 16) * 16 // size
-    if nb * nh * Sq * row * size > _ALIGN_BIAS_BYTES[backward]:
+    if nb * nh * Sq * row * size > _ALIGN_BIAS_BYTES[backward] or (not backward and nb * nh * Sq * size > _ALIGN_BIAS_ROW_BYTES):
         return bias
     try:
         out = torch.empty((nb, nh, Sq, row), dtype=bias.dtype, device=bias.device)
@@ -432,7 +441,7 @@ def flash_attn(
     raise, as in the reference (:854)."""
     drop = None if dropout_p == 0.0 else _dropout_arg(dropout_p, dropout_state, q.shape[0] * q.shape[2] * q.shape[1] * k.shape[1])
     if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad or (bias is not None and bias.requires_grad))):
-        rows = _aligned_bias(bias, q, k, False)
+        rows = None if bias is None else _aligned_bias(bias, q, k, False)
         o, lse = attn_fwd_strided(q, k, v, (0, 2, 1, 3), causal, softmax_scale, drop, rows)
         return (o, lse) if return_lse else o
     return _FlashAttnBSHD.apply(q, k, v, causal, softmax_scale, return_lse, drop, bias)

@@ -72,3 +72,17 @@ def test_bias_is_read_in_place_where_a_copy_finds_no_memory(monkeypatch):
 
     monkeypatch.setattr(torch, "empty", no_room)
     test_tile_bias(1, 2, 515, 1021, 64, False, True, True, torch.bfloat16)
+
+
+# few rows over many keys are copied for the forward, many rows over few keys are not (the copy costs more than it gains)
+@pytest.mark.parametrize("B,H,S,bias_f32,copied", [(1, 4, 1021, True, True), (1, 64, 1021, True, False), (1, 64, 1021, False, False),
+                                                   (1, 32, 1021, False, True), (1, 4, 725, True, False), (1, 4, 515, False, False), (1, 4, 725, False, True)])
+def test_bias_rows_are_copied_where_that_gains(B, H, S, bias_f32, copied):
+    g = torch.Generator(device=DEV).manual_seed(S)
+    t = [torch.randn(B, S, H, 64, generator=g, device=DEV).to(torch.bfloat16) for _ in range(3)]
+    bias = torch.randn(B, H, S, S, generator=g, device=DEV).to(torch.float32 if bias_f32 else torch.bfloat16)
+    rows = surface._aligned_bias(bias, t[0], t[1], False)
+    assert (rows is not bias) == copied
+    assert torch.equal(rows, bias)
+    if bias_f32 == (S > 515):                                  # (where the backward's line lies)
+        assert surface._aligned_bias(bias, t[0], t[1], True) is not bias
