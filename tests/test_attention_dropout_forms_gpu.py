@@ -57,3 +57,28 @@ def test_dropout_on_every_form(B, H, Sq, Sk, D, causal, dtype, bias, variant):
     for name, a, r in zip(("dQ", "dK", "dV"), got, ref):
         e = (a.transpose(1, 2).float().cpu() - r).abs().max().item()
         assert e <= 2e-2 * max(1.0, r.abs().max().item()), f"{name}: error {e:.3e} vs magnitude {r.abs().max().item():.3e}"
+
+
+# a bias with a query stride: whole tiles of it and ragged ones, on 16-byte boundaries and off them
+@pytest.mark.parametrize("bias_dtype", ["f32", "operand"])
+@pytest.mark.parametrize("B,H,Sq,Sk,D,causal,dtype", [
+    (1, 2, 300, 1160, 128, False, torch.bfloat16), (1, 2, 700, 700, 128, True, torch.float16), (2, 1, 333, 1201, 128, False, torch.float16),
+    (1, 2, 300, 1160, 64, False, torch.float16), (1, 2, 701, 701, 64, True, torch.bfloat16)])
+def test_dropout_with_a_bias_per_query(B, H, Sq, Sk, D, causal, dtype, bias_dtype):
+    p, seed = 0.4, 987654321
+    off = _state_with_partial_rows(p, B, H, Sq, Sk, seed)
+    g = torch.Generator().manual_seed(Sq + D)
+    q, k, v, go = (torch.randn(B, H, n, D, generator=g).to(dtype) for n in (Sq, Sk, Sk, Sq))
+    b = torch.randn(1, H, Sq, Sk, generator=g).to(torch.float32 if bias_dtype == "f32" else dtype)
+    o_ref, lse_ref = attention_fwd_oracle(q, k, v, causal=causal, dropout=(p, seed, off), bias=b)
+    ref = attention_bwd_oracle(q, k, v, go, causal=causal, dropout=(p, seed, off), bias=b)
+    t = [x.to(DEV).transpose(1, 2).requires_grad_(True) for x in (q, k, v)]
+    o, lse = flash_attn(*t, bias=b.to(DEV), causal=causal, dropout_p=p, return_lse=True, dropout_state=(seed, off))
+    got = torch.autograd.grad(o, t, go.to(DEV).transpose(1, 2))
+    torch.cuda.synchronize()
+    err = (o.detach().transpose(1, 2).float().cpu() - o_ref).abs()
+    assert float((err - (O_ATOL + O_RTOL * o_ref.abs())).max()) <= 0, f"O: max abs err {float(err.max()):.3e}"
+    assert float((lse.cpu() - lse_ref).abs().max()) <= LSE_ATOL
+    for name, a, r in zip(("dQ", "dK", "dV"), got, ref):
+        e = (a.transpose(1, 2).float().cpu() - r).abs().max().item()
+        assert e <= 2e-2 * max(1.0, r.abs().max().item()), f"{name}: error {e:.3e} vs magnitude {r.abs().max().item():.3e}"
