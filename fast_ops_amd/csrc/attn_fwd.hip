@@ -1729,11 +1729,22 @@ static int check_strides(const int64_t* st, int D, bool key_or_value) {
   return FO_OK;
 }
 
-// Few query rows over many keys: the kernel of attn_decode.hip. Up to 32 rows per head, without a mask, bias or dropout.
+// Few query rows over many keys: the kernel of attn_decode.hip. Up to 32 rows per head, without a mask, bias or dropout, where
+// it was not the slower one of the two. 128-row kernels -> that kernel, one and 32 queries, at head_dim 128, 512 heads: 64 and 96
+// keys no difference (13.8 / 17.5 us), 128 keys 18.5 -> 11.2 and 20.7 -> 16.9, 256 keys 24.7 -> 17.2 and 25.8 -> 20.3; the same
+// at 1024 heads (128 keys 35 -> 23, 37 -> 31); up to 256 heads both wait for the host. At head_dim 64 the plain kernel has three
+// workgroups per compute unit and this one two, which shows with more workgroups than that and little for each to do (1024
+// heads: 128 keys 12.5 -> 11.1 and 13.0 -> 15.3, 256 keys 15.9 -> 15.5 and 17.3 -> 18.1, but 384 keys 20.8 -> 19.2 and 22.1 -> 21.6;
+// 2048 heads: 128 keys 16.5 -> 18.9 and 18.5 -> 23.3, 384 keys 35.1 -> 33.1 and 38.0 -> 35.8).
 static int decode_n_kv(const AttnParams& p) { return (p.H == 1 || (p.ks[1] == 0 && p.vs[1] == 0)) ? 1 : p.H; }
 static bool takes_decode(const AttnParams& p, bool causal, bool dropout, int forced) {
   if (forced >= 0 || causal || dropout || p.bias.ptr != nullptr || (p.d != 64 && p.d != 128)) return false;
   if (p.Sq > 32 || p.Sk < kDecodeMinKeys) return false;
+  if (p.d == 64) {
+    const int n_kv = decode_n_kv(p);
+    const int64_t blocks = (int64_t)p.B * n_kv * ((decode_rows(p.H, n_kv, p.Sq) + 31) / 32), cus = device_cus();
+    if (blocks > 2 * cus && p.Sk < 384) return false;
+  }
   return (int64_t)p.B * p.H * p.Sq < (1ll << 31);
 }
 

@@ -235,7 +235,11 @@ def test_attn_kernel_query_and_stride_limit_without_device_work():
         assert k(2, 16, 8192, 8192, 128, 1, drop=1) == W4 and k(2, 16, 8192, 8192, 128, 1, bias=2, drop=1) == W4
         assert k(2, 16, 4096, 4096, 128, 1, drop=1) == W4 and k(2, 16, 4096, 4096, 128, 1, bias=2, drop=1) == W4    # (W8 without)
         assert k(1, 12, 2048, 2048, 128, 1, drop=1) == PIPE and k(8, 12, 1024, 1024, 64, 1, drop=1) == R128
-        assert k(4, 16, 1, 4000, 128, 0, drop=1) == PIPE and k(4, 16, 1, 4000, 128, 0) == _lib.FO_ATTN_KERNEL_DECODE
+        DEC = _lib.FO_ATTN_KERNEL_DECODE
+        assert k(4, 16, 1, 4000, 128, 0, drop=1) == PIPE and k(4, 16, 1, 4000, 128, 0) == DEC
+        # few queries at head_dim 64: not with little work for more than two workgroups per compute unit
+        assert k(64, 16, 32, 383, 64, 0) != DEC and k(64, 16, 32, 384, 64, 0) == DEC and k(64, 16, 32, 128, 128, 0) == DEC
+        assert k(16, 32, 1, 128, 64, 0) == DEC and k(27, 19, 1, 128, 64, 0) != DEC      # (512 and 513 workgroups)
     # (the eight-wave form does not exist with dropout, and neither does the exact running maximum)
     for asked, runs in ((0, 0), (1, 0), (8, 8), (16, 32), (32, 32)):
         assert lib.fo_tune_set(b"attn.variant", asked) == 0
