@@ -42,7 +42,7 @@ struct AttnBwdParams {
   const void *q, *k, *v, *o, *d_o;
   const float* lse;
   float* delta;       // [B, H, Sq]: -rowsum(dO O) (1 - dropout_p), written by the dQ kernel
-  float* nlse;        // [B, H, Sq]: -LSE / softmax_scale, written by the dQ kernel beside delta (see there)
+  float* nlse;        // [B, H, Sq]: -LSE / softmax_scale (with dropout: of an LSE lower by log(1 / (1 - p))), written by the dQ kernel beside delta
   void *dq, *dk, *dv;
   int B, H, Sq, Sk;
   int d;                // true head_dim: a multiple of 8, at most the D the kernels are compiled for
@@ -381,7 +381,9 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
       gf[ks] = *(const vec8*)live_or_zero(gp + 16 * ks, 16 * ks + 8 * hh, prm.d);
     }
   }
-  const float lse2 = prm.lse[(int64_t)bh * Sq + qrow] * kLog2e;
+  // (dropout: P comes out times k = 1 / (1 - p), so that it and dS are rounded to the operand type with that factor, as the
+  // reference's are: without it fp16 gradients at p = 0.9 reach the subnormal numbers ten times earlier)
+  const float lse2 = prm.lse[(int64_t)bh * Sq + qrow] * kLog2e - (DROP ? prm.drop.keep_log2 : 0.0f);
   // delta_i = sum_d dO_id O_id (flash_attention_triton.py:273-315), negated: this lane holds half of its row's dO
   // already, so it reads the same pieces of O, and the two halves of the wave add up. Stored for the dK/dV kernel,
   // which runs after this one (a pass of its own over O and dO would be a launch more: 5 of 83 us at B=8 H=12 S=1024).
@@ -395,8 +397,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
       for (int e = 0; e < 8; ++e) delta -= (float)ov[e] * (float)gf[ks][e];
     }
     delta += half_swap(delta);
-    // dropout: with Z = 0 or 1 per element and k = 1 / (1 - p), dS = P (k Z dP - delta) = k P (Z dP - delta (1 - p)); the
-    // factor k is applied to the finished gradients
+    // dropout: with Z = 0 or 1 per element, dS = P (k Z dP - delta) = (k P) (Z dP - delta (1 - p))
     if constexpr (DROP) delta *= prm.drop.keep_prob;
     if (hh == 0 && q0w + l32 < Sq) prm.delta[(int64_t)bh * Sq + q0w + l32] = delta;
   }
@@ -411,7 +412,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
   for (int i = 0; i < DBLK; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
-  const float c = prm.scale_log2e, scale = DROP ? prm.scale * prm.drop.keep_scale : prm.scale;
+  const float c = prm.scale_log2e, scale = prm.scale;
   DropRows<1> drop;
 
   for (int tile = 0; tile < n_tiles; ++tile) {
@@ -687,7 +688,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_kernel(const Att
   for (int i = 0; i < DBLK; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) { dkacc[i][r] = 0.0f; dvacc[i][r] = 0.0f; }
-  const float c = prm.scale_log2e, scale = DROP ? prm.scale * prm.drop.keep_scale : prm.scale;
+  const float c = prm.scale_log2e, scale = prm.scale;
 
   for (int qt = qt0; qt < n_qt; ++qt) {
     const int buf = (qt - qt0) & 1;
@@ -779,7 +780,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_kernel(const Att
         for (int u = 0; u < 4; ++u) {
           const int r = 4 * j + u;
           const bool dead = decltype(masked)::value && ((u + 8 * j) < lim || (u + 8 * j) >= lim_end);
-          float shift = -l4[u] * kLog2e;
+          float shift = DROP ? __builtin_fmaf(-l4[u], kLog2e, prm.drop.keep_log2) : -l4[u] * kLog2e;      // (P times 1 / (1 - p): see the dQ kernel)
           if constexpr (BIAS && BM == 0) {
             const int qi = min(q0t + 32 * qb + 4 * hh + u + 8 * j, Sq - 1);
             shift = __builtin_fmaf(load_bias<T>(prm.bias, bias_col + (int64_t)qi * prm.bias.strides[2]), kLog2e, shift);
@@ -834,7 +835,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_kernel(const Att
     FO_LDS char* stage = smem + wave_s * stage_bytes(D);
     const int k0w_s = k0 + wave_s * 32;
     store_rows_via_lds<T, D>(dkacc, scale, stage, (T*)prm.dk + b * prm.dks[0] + h * prm.dks[1], prm.dks[2], k0w_s, Sk, prm.d, lane);
-    store_rows_via_lds<T, D>(dvacc, DROP ? prm.drop.keep_scale : 1.0f, stage, (T*)prm.dv + b * prm.dvs[0] + h * prm.dvs[1], prm.dvs[2], k0w_s, Sk, prm.d, lane);
+    store_rows_via_lds<T, D>(dvacc, 1.0f, stage, (T*)prm.dv + b * prm.dvs[0] + h * prm.dvs[1], prm.dvs[2], k0w_s, Sk, prm.d, lane);
   }
 }
 
@@ -896,8 +897,8 @@ static_assert(softmax_grad_jobs_fit(16) && softmax_grad_jobs_fit(12) && softmax_
 // lane for the whole kernel, and P = exp2(S c + b log2 e) is a fused multiply-add where the form without bias multiplies.
 // DROP (flash_attention_triton.py:524-532,551-552): dV sees the kept probabilities only, and dP reaches only them: where a
 // query's elements of the workgroup's 128 keys are all dropped, its row of the dO tile in LDS is set to zero, which is both
-// (dP = dO V^T and dV = dO^T P), and where they are all kept there is nothing to do; 1 / (1 - p) is applied to the finished
-// gradients (delta comes multiplied by 1 - p, see the dQ kernel). Each lane looks at one of the next tile's 64 rows as a
+// (dP = dO V^T and dV = dO^T P), and where they are all kept there is nothing to do; 1 / (1 - p) is part of P (-LSE / scale
+// comes with it, and delta multiplied by 1 - p: see the dQ kernel). Each lane looks at one of the next tile's 64 rows as a
 // whole (dropout_run) in the first groups of a tile, which carry no other arithmetic. A row that is neither (a few in a
 // million) counts as dropped at first. At the end the workgroup's rows of this kind, up to 64 at a time, are gathered into
 // one tile, which goes through the body once more with P of dropped elements set to zero and dP taken without delta: that
@@ -1069,7 +1070,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   for (int i = 0; i < DBLK; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) { dkacc[i][r] = 0.0f; dvacc[i][r] = 0.0f; }
-  const float c = prm.scale_log2e, scale = DROP ? prm.scale * prm.drop.keep_scale : prm.scale;
+  const float c = prm.scale_log2e, scale = prm.scale;
 
   // Per-lane byte offsets of the fragment reads inside a tile, swizzle included (what row_frag / col_frag compute; the
   // swizzle of a row does not depend on the 32-row block or 16-row step it is in). With the tile's base added once
@@ -1465,7 +1466,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
     FO_LDS char* stage = smem + wave_s * stage_bytes(D);
     const int k0w_s = k0 + wave_s * 32;
     store_rows_via_lds<T, LIVE>(dkacc, scale, stage, (T*)prm.dk + b * prm.dks[0] + h * prm.dks[1], prm.dks[2], k0w_s, Sk, prm.d, lane);
-    store_rows_via_lds<T, LIVE>(dvacc, DROP ? prm.drop.keep_scale : 1.0f, stage, (T*)prm.dv + b * prm.dvs[0] + h * prm.dvs[1], prm.dvs[2], k0w_s, Sk, prm.d, lane);
+    store_rows_via_lds<T, LIVE>(dvacc, 1.0f, stage, (T*)prm.dv + b * prm.dvs[0] + h * prm.dvs[1], prm.dvs[2], k0w_s, Sk, prm.d, lane);
   }
 }
 

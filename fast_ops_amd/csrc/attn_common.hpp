@@ -107,6 +107,7 @@ struct DropoutParams {
   uint32_t offset;        // low 32 bits of the generator offset
   float keep_scale;       // 1 / (1 - p) in fp32; 1 when dropout is off
   float keep_prob;        // 1 - p
+  float keep_log2;        // log2 of keep_scale
 };
 __host__ __device__ __forceinline__ bool dropout_keep(uint32_t index, uint32_t seed, uint32_t threshold) {
   uint32_t a = index ^ seed;
@@ -147,6 +148,7 @@ inline DropoutParams make_dropout(float p, uint32_t seed, uint64_t rng_offset) {
   d.offset = (uint32_t)rng_offset;
   d.keep_prob = 1.0f - p;
   d.keep_scale = 1.0f / d.keep_prob;
+  d.keep_log2 = log2f(d.keep_scale);
   return d;
 }
 
@@ -177,11 +179,11 @@ struct DropRows {
   template <typename P>
   __device__ __forceinline__ void look(const P& d_in, int bh, int Sq, int Sk, int row0, int tile) {
     if (__builtin_expect(tile % kDropSpanTiles == 0, 0)) {      // (laid out away from the tile loops)
-      const DropoutParams d = {d_in.seed, d_in.threshold, d_in.offset, 1.0f, 1.0f};
+      const DropoutParams d = {d_in.seed, d_in.threshold, d_in.offset, 1.0f, 1.0f, 0.0f};
       by_tile = look_at<10>(d, bh, Sq, Sk, row0, tile * 64);
     }
     if (__builtin_expect(by_tile, 0)) {
-      const DropoutParams d = {d_in.seed, d_in.threshold, d_in.offset, 1.0f, 1.0f};
+      const DropoutParams d = {d_in.seed, d_in.threshold, d_in.offset, 1.0f, 1.0f, 0.0f};
       look_at<6>(d, bh, Sq, Sk, row0, tile * 64);
     }
   }

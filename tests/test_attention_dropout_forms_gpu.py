@@ -82,3 +82,32 @@ def test_dropout_with_a_bias_per_query(B, H, Sq, Sk, D, causal, dtype, bias_dtyp
     for name, a, r in zip(("dQ", "dK", "dV"), got, ref):
         e = (a.transpose(1, 2).float().cpu() - r).abs().max().item()
         assert e <= 2e-2 * max(1.0, r.abs().max().item()), f"{name}: error {e:.3e} vs magnitude {r.abs().max().item():.3e}"
+
+
+# P and dS are rounded to the operand type with the factor 1 / (1 - p). Sizes: dS of a kept element is about 6e-7 without that
+# factor, which fp16 rounds to multiples of 2^-24 (error 2^-24 / sqrt(12) each: 1.8 % of dQ and dK, emulated in 64 bits; with the
+# factor 0.2 %), and the gradients are about 1e-5 (0.2-0.3 % from their own rounding). The general dK/dV kernel (variant 0) and the pipelined one.
+@pytest.mark.parametrize("variant", [-1, 0])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bias", [None, "key", "query"])
+def test_small_fp16_gradients_at_a_large_dropout_p(D, bias, variant):
+    p, seed, off, S = 0.9, 12345, 1 << 20, 2048      # (kept, dropped and partly dropped rows; 27 % of the elements are kept)
+    g = torch.Generator().manual_seed(D)
+    q, k, v, go = (torch.randn(1, 1, S, D, generator=g) for _ in range(4))
+    q, k, v, go = q.half(), k.half(), v.half(), (go * (1.2e-3 / D ** 0.5)).half()
+    b = None if bias is None else torch.randn(1, 1, 1 if bias == "key" else S, S, generator=g)
+    keep = torch.from_numpy(dropout_keep_mask(p, seed, off, 1, 1, S, S))
+    x = [t.double().requires_grad_(True) for t in (q, k, v)]
+    scores = x[0] @ x[1].transpose(2, 3).contiguous() / D ** 0.5 + (0 if b is None else b.double())
+    ref = torch.autograd.grad((torch.softmax(scores, -1) * keep / (1 - p)) @ x[2], x, go.double())
+    t = [y.to(DEV).transpose(1, 2).requires_grad_(True) for y in (q, k, v)]
+    _lib.tune_set("attn_bwd.variant", variant)
+    try:
+        o = flash_attn(*t, bias=None if b is None else b.to(DEV), dropout_p=p, dropout_state=(seed, off))
+        got = torch.autograd.grad(o, t, go.to(DEV).transpose(1, 2))
+        torch.cuda.synchronize()
+    finally:
+        _lib.tune_set("attn_bwd.variant", -1)
+    for name, a, r in zip(("dQ", "dK", "dV"), got, ref):
+        e = float((a.transpose(1, 2).cpu().double() - r).norm() / r.norm())
+        assert e <= 1e-2, f"{name}: relative error {e:.2e}"
