@@ -384,6 +384,12 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
   // (dropout: P comes out times k = 1 / (1 - p), so that it and dS are rounded to the operand type with that factor, as the
   // reference's are: without it fp16 gradients at p = 0.9 reach the subnormal numbers ten times earlier)
   const float lse2 = prm.lse[(int64_t)bh * Sq + qrow] * kLog2e - (DROP ? prm.drop.keep_log2 : 0.0f);
+  // TBIAS: -LSE / scale starts the scores together with the bias, its rounding error (times c) takes the LSE's place in the exponent.
+  // (The products of a row whose whole bias is large are otherwise summed at the ulp of bias / scale: at -1e5 an error of 1 % of dQ.
+  // (bias - LSE) / scale instead is an instruction more per score: 107 -> 125 us at 12 heads x 3072 causal. The dK/dV kernel has no
+  // room for a row's second value; its error there is that of -LSE / scale, rounded once: the same as of LSE * log2 e elsewhere.)
+  const float row_start = -prm.lse[(int64_t)bh * Sq + qrow] * per_scale;
+  const float row_shift = TBIAS ? __builtin_fmaf(-prm.lse[(int64_t)bh * Sq + qrow], per_scale, -row_start) * prm.scale_log2e : -lse2;
   // delta_i = sum_d dO_id O_id (flash_attention_triton.py:273-315), negated: this lane holds half of its row's dO
   // already, so it reads the same pieces of O, and the two halves of the wave add up. Stored for the dK/dV kernel,
   // which runs after this one (a pass of its own over O and dO would be a launch more: 5 of 83 us at B=8 H=12 S=1024).
@@ -405,7 +411,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
   // also wait for the tile copies in flight, which it does not see)
 #pragma unroll
   for (int ks = 0; ks < KSTEPS; ++ks) asm volatile("" ::"v"(qf[ks]), "v"(gf[ks]));
-  asm volatile("" ::"v"(lse2), "v"(delta));
+  asm volatile("" ::"v"(row_start), "v"(row_shift), "v"(delta));
 
   f32x16 acc[DBLK];
 #pragma unroll
@@ -455,12 +461,12 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
         }
     }
     if constexpr (HALVES) {
-      BRH::each(row_bias, 0, l32, hh, [&](int r, float v) { sacc[0][r] = v * per_scale; });
+      BRH::each(row_bias, 0, l32, hh, [&](int r, float v) { sacc[0][r] = __builtin_fmaf(v, per_scale, row_start); });
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read: the buffer is free for the tile's other half
       BRH::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, key0 + 32, row_bias, lane);
     } else if constexpr (TBIAS != 0) {
-      BR::each(row_bias, 0, l32, hh, [&](int r, float v) { sacc[0][r] = v * per_scale; });
-      BR::each(row_bias, 1, l32, hh, [&](int r, float v) { sacc[1][r] = v * per_scale; });
+      BR::each(row_bias, 0, l32, hh, [&](int r, float v) { sacc[0][r] = __builtin_fmaf(v, per_scale, row_start); });
+      BR::each(row_bias, 1, l32, hh, [&](int r, float v) { sacc[1][r] = __builtin_fmaf(v, per_scale, row_start); });
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read: the buffer is free for the next tile's
       if (tile + 1 < n_tiles) BR::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, key0 + kBwdTile, row_bias, lane);
     }
@@ -474,7 +480,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
     if constexpr (HALVES) {
       // (behind the products, which cover most of the copy's way; what else is in flight was issued before it)
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      BRH::each(row_bias, 0, l32, hh, [&](int r, float v) { sacc[1][r] = __builtin_fmaf(v, per_scale, sacc[1][r]); });
+      BRH::each(row_bias, 0, l32, hh, [&](int r, float v) { sacc[1][r] += __builtin_fmaf(v, per_scale, row_start); });
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (tile + 1 < n_tiles) BRH::copy(prm.bias, key_bias_row, q0 + wave_s * 32, Sq, Sk, key0 + kBwdTile, row_bias, lane);
     }
@@ -501,7 +507,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
           for (int u = 0; u < 4; ++u) {
             const int r = 4 * j + u;
             const bool dead = decltype(masked)::value && lim > -(u + 8 * j);
-            float shift = -lse2;
+            float shift = row_shift;
             if constexpr (BIAS) shift = __builtin_fmaf(b4[u], kLog2e, -lse2);
             const float p = dead ? 0.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][r], c, shift));
             dsf[kb * 2 + (r >> 3)][r & 7] = (T)(p * (dpacc[kb][r] + delta));
@@ -569,7 +575,8 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
     // -LSE / softmax_scale for the dK/dV kernel, whose score accumulators start from it: P = exp2((QK^T - LSE / scale)
     // * scale * log2 e) is then one multiplication and the exponential per element. (Stored here, from the scaled LSE
     // the loop used, and not beside delta: every register is taken while the loop runs.)
-    if (hh == 0) prm.nlse[(int64_t)bh * Sq + qi] = lse2 * prm.neg_inv_scale_log2e;
+    // (TBIAS: by the factor that kernel scales the bias with)
+    if (hh == 0) prm.nlse[(int64_t)bh * Sq + qi] = TBIAS ? row_start : lse2 * prm.neg_inv_scale_log2e;
     T* op = (T*)prm.dq + b * prm.dqs[0] + h * prm.dqs[1] + (int64_t)qi * prm.dqs[2];
 #pragma unroll
     for (int db = 0; db < DBLK; ++db)
@@ -1120,8 +1127,9 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
 #endif
   };
 
-  // TBIAS: the lane's 16 values of a block, then, times 1 / softmax_scale, added to the block's S accumulator one by one
-  const float per_scale = TBIAS ? __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, 1.0f / prm.scale))) : 0.0f;
+  // TBIAS: the lane's 16 values of a block, then, times 1 / softmax_scale, added to the block's S accumulator one by one (the same
+  // factor, to the last bit, as in the dQ kernel: -LSE / scale comes times it)
+  const float per_scale = TBIAS ? __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, kLog2e / prm.scale_log2e))) : 0.0f;
   s16x4 bias16[4];
   f32x16 bias32;
   auto bias_read = [&](int jt, int qb) {

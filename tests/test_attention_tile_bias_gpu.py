@@ -40,6 +40,34 @@ def test_tile_bias(B, H, Sq, Sk, D, bias_f32, packed, causal, dtype):
     _check(_bshd(o), lse, [_bshd(x) for x in got], o_ref, lse_ref, ref)
 
 
+# Rows whose whole bias is large: only its difference to the LSE counts, which fp32 holds exactly here. Error of P and dS in fp16
+# 2^-11 / sqrt(3) each, the same of the results: 5e-4 together. (Scores summed at the ulp of bias / scale: dQ 2e-3 to 1e-2.) dK and dV:
+# and that of LSE / scale rounded to fp32 once, up to |LSE| 2^-24 of P. The LSE is given, rounded to fp32 once.
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bias_f32", [False, True])
+@pytest.mark.parametrize("causal", [False, True])
+def test_gradients_of_rows_with_a_large_bias(D, bias_f32, causal):
+    S, scale = 456, D ** -0.5
+    g = torch.Generator().manual_seed(D)
+    q, k, v, go = (torch.randn(1, 2, S, D, generator=g).half() for _ in range(4))
+    bias = torch.randn(1, 2, S, S, generator=g) - 1e5 if bias_f32 else torch.full((1, 2, S, S), -3e4).half()
+    x = [t.double() for t in (q, k, v, go)]
+    s = x[0] @ x[1].transpose(2, 3).contiguous() * scale + bias.double()
+    if causal:
+        s = s.masked_fill(torch.ones(S, S, dtype=torch.bool).triu(1), float("-inf"))
+    lse = torch.logsumexp(s, -1).float()
+    p = torch.exp(s - lse.double()[..., None])
+    o = (p @ x[2]).half()
+    ds = p * (x[3] @ x[2].transpose(2, 3).contiguous() - (x[3] * o.double()).sum(-1, keepdim=True)) * scale
+    ref = (ds @ x[1], ds.transpose(2, 3).contiguous() @ x[0], p.transpose(2, 3).contiguous() @ x[3])
+    d = [t.to(DEV) for t in (q, k, v, o, lse, go, bias)]
+    got = surface.attn_bwd_strided(*d[:6], (0, 1, 2, 3), causal, scale, None, d[6])
+    torch.cuda.synchronize()
+    for name, a, r in zip(("dQ", "dK", "dV"), got, ref):
+        e = float((a.cpu().double() - r).norm() / r.norm())
+        assert e <= 1e-3 + (0 if name == "dQ" else float(lse.abs().max()) * 2.0 ** -24), f"{name}: relative error {e:.2e}"
+
+
 # one to three query tiles, the last of them whole or not: where the first tiles' copies and the last ones' hand-overs meet
 @pytest.mark.parametrize("Sq,Sk", [(33, 64), (64, 128), (65, 136), (128, 260), (192, 128)])
 @pytest.mark.parametrize("D", [64, 128])
