@@ -107,5 +107,12 @@ def check(status: int, what: str) -> None:
         raise RuntimeError(f"{what}: {strerror(status)} (fo_status {status})")
 
 
+# how often tune_set has been called: part of the key of whatever is worked out once from the values it sets
+tune_generation = 0
+
+
 def tune_set(key: str, value: int) -> None:
+    global tune_generation
     check(load().fo_tune_set(key.encode(), int(value)), f"fo_tune_set({key!r}, {value})")
+    with _lock:
+        tune_generation += 1

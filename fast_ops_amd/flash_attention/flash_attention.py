@@ -182,7 +182,8 @@ _FWD_PLANS: dict = {}
 
 
 def _fwd_plan(q: Tensor, k: Tensor, v: Tensor, dims: Tuple[int, int, int, int]) -> _FwdPlan:
-    key = (q.shape, q.stride(), k.shape, k.stride(), v.shape, v.stride(), q.dtype, k.dtype, v.dtype, q.device, k.device, v.device, dims)
+    # (the scratch memory of a plan depends on what _lib.tune_set has set)
+    key = (q.shape, q.stride(), k.shape, k.stride(), v.shape, v.stride(), q.dtype, k.dtype, v.dtype, q.device, k.device, v.device, dims, _lib.tune_generation)
     plan = _FWD_PLANS.get(key)
     if plan is not None:
         return plan

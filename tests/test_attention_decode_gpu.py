@@ -4,7 +4,7 @@ row block; against the oracle with the forward's tolerances."""
 import pytest
 import torch
 
-from fast_ops.flash_attention.flash_attention import multi_head_attention
+from fast_ops.flash_attention.flash_attention import flash_attn, multi_head_attention
 from fast_ops_amd import _lib
 from fast_ops_amd.flash_attention import flash_attention as surface
 from oracle.attention_oracle import attention_fwd_oracle
@@ -30,7 +30,6 @@ def test_decode_against_oracle(B, H, Sq, Sk, D, dtype, multi_query, split):
     k, v = (t[:, :, :Sk].expand(B, H, Sk, D) for t in cache)
     o_ref, lse_ref = attention_fwd_oracle(q, k, v)
     kd, vd = (t.to(DEV)[:, :, :Sk].expand(B, H, Sk, D) for t in cache)
-    surface._FWD_PLANS.clear()                       # (a plan remembers the workspace of its shape)
     assert _lib.tune_set("attn.decode_split", split) is None
     try:
         o, lse = multi_head_attention(q.to(DEV), kd, vd, return_lse=True)
@@ -39,7 +38,6 @@ def test_decode_against_oracle(B, H, Sq, Sk, D, dtype, multi_query, split):
         torch.cuda.synchronize()
     finally:
         _lib.tune_set("attn.decode_split", -1)
-        surface._FWD_PLANS.clear()
     err = (o.float().cpu() - o_ref).abs()
     assert float((err - (O_ATOL + O_RTOL * o_ref.abs())).max()) <= 0, f"O: max abs err {float(err.max()):.3e}"
     assert float((lse.cpu() - lse_ref).abs().max()) <= LSE_ATOL
@@ -57,14 +55,44 @@ def test_decode_with_keys_that_score_minus_infinity(Sq, Sk, D, dtype, live, spli
     k[..., 0] = float("-inf")
     k[:, :, live[0]:live[1], 0] = 0
     o_ref, lse_ref = attention_fwd_oracle(q, k, v)
-    surface._FWD_PLANS.clear()
     _lib.tune_set("attn.decode_split", split)
     try:
         o, lse = multi_head_attention(q.to(DEV), k.to(DEV), v.to(DEV), return_lse=True)
         torch.cuda.synchronize()
     finally:
         _lib.tune_set("attn.decode_split", -1)
-        surface._FWD_PLANS.clear()
     err = (o.float().cpu() - o_ref).abs()
+    assert float((err - (O_ATOL + O_RTOL * o_ref.abs())).max()) <= 0, f"O: max abs err {float(err.max()):.3e}"
+    assert float((lse.cpu() - lse_ref).abs().max()) <= LSE_ATOL
+
+
+# a shape's first call may fall into a time when another kernel, or fewer workgroups per row block, were asked for
+@pytest.mark.parametrize("key,value", [("attn.variant", 0), ("attn.decode_split", 1)])
+def test_workspace_follows_what_is_asked_for(key, value):
+    q, k, v = (torch.randn(1, 4, n, 128, device=DEV, dtype=torch.bfloat16) for n in (1, 4352 + len(key), 4352 + len(key)))
+    dims = (0, 1, 2, 3)
+    _lib.tune_set(key, value)
+    try:
+        assert surface._fwd_plan(q, k, v, dims).ws_bytes == 0
+    finally:
+        _lib.tune_set(key, -1)
+    assert surface._fwd_plan(q, k, v, dims).ws_bytes > 0
+
+
+# the [B, S, H, D] layout, several rows per head; keys that all heads share with values of their own (only the keys' head stride is 0)
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Sq,Sk,shared_keys", [(1, 1500, False), (7, 801, False), (1, 1500, True), (5, 801, True)])
+def test_decode_layouts(Sq, Sk, D, shared_keys):
+    g = torch.Generator().manual_seed(Sk + D)
+    q, k, v = (torch.randn(2, n, 6, D, generator=g).to(torch.bfloat16) for n in (Sq, Sk, Sk))
+    if shared_keys:
+        k = k[:, :, :1].expand(2, Sk, 6, D)
+    o_ref, lse_ref = attention_fwd_oracle(*(t.transpose(1, 2) for t in (q, k, v)))
+    kd = k[:, :, :1].contiguous().to(DEV).expand(2, Sk, 6, D) if shared_keys else k.to(DEV)
+    o, lse = flash_attn(q.to(DEV), kd, v.to(DEV), return_lse=True)
+    I3 = lambda t: (_lib.ctypes.c_int64 * 3)(t.stride(0), t.stride(2), t.stride(1))
+    assert _lib.load().fo_attn_fwd_kernel(2, 6, Sq, Sk, D, I3(kd), I3(v), 0, 0, 0) == _lib.FO_ATTN_KERNEL_DECODE
+    torch.cuda.synchronize()
+    err = (o.transpose(1, 2).float().cpu() - o_ref).abs()
     assert float((err - (O_ATOL + O_RTOL * o_ref.abs())).max()) <= 0, f"O: max abs err {float(err.max()):.3e}"
     assert float((lse.cpu() - lse_ref).abs().max()) <= LSE_ATOL
