@@ -2,6 +2,7 @@
 its outcomes: rows kept, rows dropped, and rows in which the mask changes (those are hashed element by element, in the
 dK/dV kernel in a second visit of the tile). Against the oracle with the same mask; tolerances as in
 test_attention_dropout_gpu.py."""
+import numpy as np
 import pytest
 import torch
 
@@ -111,3 +112,71 @@ def test_small_fp16_gradients_at_a_large_dropout_p(D, bias, variant):
     for name, a, r in zip(("dQ", "dK", "dV"), got, ref):
         e = float((a.transpose(1, 2).cpu().double() - r).norm() / r.norm())
         assert e <= 1e-2, f"{name}: relative error {e:.2e}"
+
+
+def _verdicts(first, seed, threshold):
+    """The kernels' look at aligned blocks of 128 indices as a whole (dropout_block<7>): 0 dropped, 1 kept, 2 neither."""
+    x = ((first ^ np.uint32(seed)) & np.uint32(0xFFFFFF80)).astype(np.uint32)
+    y = (x ^ (x >> 4)) & np.uint32(0xFFFFFF80)
+    z0 = ((y ^ np.uint32(0xDEADBEEF)) & np.uint32(0xFFFFFF80)) + (y << 5)
+    a0, a1 = z0 >> 13, (z0 + np.uint32(33 * 127)) >> 13
+    w0, w1, t = a0 ^ (a0 >> 11), a1 ^ (a1 >> 11), threshold >> 13
+    return np.where((w0 > t) & (w1 > t), 1, np.where((w0 < t) & (w1 < t), 0, 2))
+
+
+def _partly_dropped_block(p, seed):
+    """The first index of an aligned block of 128 of which 32 to 96 are kept."""
+    threshold = np.uint32(int(np.float32(p) * np.float32(4294967295)))
+    for chunk in range(0, 1 << 32, 1 << 28):
+        first = (np.arange(1 << 21, dtype=np.uint32) << np.uint32(7)) + np.uint32(chunk)
+        for x in first[_verdicts(first, seed, threshold) == 2]:
+            if 32 <= dropout_keep_mask(p, seed, int(x), 1, 1, 1, 128).sum() <= 96:
+                return int(x)
+    raise AssertionError("no such block")
+
+
+# Rows of the dropout mask that are neither kept nor dropped over a workgroup's 128 keys take part in the dK/dV kernel's tile of
+# gathered rows only: what they contribute is shown to be more than the tolerance forgives. Two keys: more than the 64 rows that fit
+# that tile, so that it is worked on several times, and taken up again in the middle of a tile of rows. (block: which 128 keys.)
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.bfloat16), (64, torch.float16), (128, torch.float16)])
+@pytest.mark.parametrize("Sq,Sk,row,block,causal", [(300, 300, 200, 0, True), (300, 300, 290, 1, True), (300, 300, 77, 0, True),
+                                                    (200, 520, 150, 3, False), (700, 2, 100, 0, False), (700, 2, 301, 0, True)])
+def test_gathered_rows_of_the_key_gradients(Sq, Sk, row, block, causal, D, dtype):
+    p, seed, B, H = 0.4, 987654321, 1, 2
+    k_, scale = 1 / (1 - p), D ** -0.5
+    off = (_partly_dropped_block(p, seed) - ((Sq + row) * Sk + 128 * block)) % (1 << 32)      # in the second head
+    keep = torch.from_numpy(dropout_keep_mask(p, seed, off, B, H, Sq, Sk))
+    seen = torch.ones(Sq, Sk, dtype=torch.bool)
+    if causal:
+        seen = seen.tril()
+    g = torch.Generator().manual_seed(Sq + D)
+    q, k, v, go = (torch.randn(B, H, n, D, generator=g) for n in (Sq, Sk, Sk, Sq))
+    if Sk == 2:                                               # (the block lies over 64 rows)
+        row += int(keep[0, 1, row:].any(-1).nonzero()[0])
+    here = torch.nonzero(keep[0, 1, row] & seen[row])[:, 0]
+    here = here[(here >= 128 * block) & (here < 128 * block + 128)]
+    q[0, 1, row] = k[0, 1, here[len(here) // 2]] * (5.7 / D ** 0.5)       # about half of the row's probability on one of these keys
+    q, k, v, go = (t.to(dtype) for t in (q, k, v, go))
+    ref = attention_bwd_oracle(q, k, v, go, causal=causal, dropout=(p, seed, off))
+    tol = [2e-2 * max(1.0, r.abs().max().item()) for r in ref]
+
+    # what the gathered rows contribute
+    threshold = np.uint32(int(np.float32(p) * np.float32(4294967295)))
+    first = ((off + np.arange(H * Sq, dtype=np.int64)[:, None] * Sk + np.arange(0, Sk, 128)[None]) % (1 << 32)).astype(np.uint32)
+    a, b = (_verdicts(f, seed, threshold) for f in (first, first + np.uint32(127)))
+    mixed = torch.from_numpy((a != b) | (a == 2)).reshape(H, Sq, -1)
+    assert mixed[1, row, block] and (Sk > 2 or mixed[1].sum() > 64)
+    of_rows = (mixed.repeat_interleave(128, -1)[..., :Sk] & keep[0] & seen).float()
+    scores = (q.float() @ k.float().transpose(2, 3).contiguous() * scale).masked_fill(~seen, float("-inf"))
+    pz = torch.softmax(scores, -1) * of_rows * k_
+    missing_v = pz.transpose(2, 3).contiguous() @ go.float()
+    missing_k = (pz * (go.float() @ v.float().transpose(2, 3).contiguous())).transpose(2, 3).contiguous() @ q.float() * scale
+    assert missing_k.abs().max() > 4 * tol[1] and missing_v.abs().max() > 4 * tol[2]
+
+    t = [x.to(DEV).transpose(1, 2).requires_grad_(True) for x in (q, k, v)]
+    o = flash_attn(*t, causal=causal, dropout_p=p, dropout_state=(seed, off))
+    got = torch.autograd.grad(o, t, go.to(DEV).transpose(1, 2))
+    torch.cuda.synchronize()
+    for name, x, r, lim in zip(("dQ", "dK", "dV"), got, ref, tol):
+        e = (x.transpose(1, 2).float().cpu() - r).abs().max().item()
+        assert e <= lim, f"{name}: error {e:.3e} vs {lim:.3e}"

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from fast_ops.flash_attention.flash_attention import flash_attn
+from fast_ops_amd import _lib
 from fast_ops_amd.flash_attention import flash_attention as surface
 from oracle.attention_oracle import attention_bwd_oracle, attention_fwd_oracle
 from test_attention_bias_gpu import DEV, _bshd, _check
@@ -114,3 +115,53 @@ def test_bias_rows_are_copied_where_that_gains(B, H, S, bias_f32, copied):
     assert torch.equal(rows, bias)
     if bias_f32 == (S > 515):                                  # (where the backward's line lies)
         assert surface._aligned_bias(bias, t[0], t[1], True) is not bias
+
+
+def _unaligned_bias(form, B, H, S, dtype, g):
+    if form == "heads":                                        # one bias for all heads, expanded
+        return torch.randn(B, 1, S, S, generator=g).to(dtype).to(DEV).expand(B, H, S, S)
+    if form == "batch":
+        return torch.randn(1, H, S, S, generator=g).to(dtype).to(DEV)
+    if form == "transposed":                                   # heads outside of the batch
+        return torch.randn(H, B, S, S, generator=g).to(dtype).to(DEV).transpose(0, 1)
+    return torch.randn(B, H, S, S + 15, generator=g).to(dtype).to(DEV)[..., 1:S + 1]      # rows and their base off 16 bytes
+
+
+# the layouts a bias can come in before it is copied, and the calls whose other kernels read the copy: dropout, narrow head dims
+@pytest.mark.parametrize("form", ["heads", "batch", "transposed", "sliced"])
+@pytest.mark.parametrize("D,drop,bias_f32,causal", [(64, 0.0, False, True), (128, 0.0, True, False), (128, 0.3, False, False), (64, 0.3, True, True), (80, 0.0, False, False)])
+def test_copied_bias_in_every_layout(form, D, drop, bias_f32, causal):
+    B, H, S, dtype, state = 2, 2, 901, torch.bfloat16, (987654321, 4 << 20)
+    g = torch.Generator().manual_seed(D + len(form))
+    q, k, v, go = (torch.randn(B, H, S, D, generator=g).to(dtype) for _ in range(4))
+    bias = _unaligned_bias(form, B, H, S, torch.float32 if bias_f32 else dtype, g)
+    t = [_bshd(x.to(DEV)).requires_grad_(True) for x in (q, k, v)]
+    for backward in (False, True):
+        rows = surface._aligned_bias(bias, t[0], t[1], backward)
+        assert rows is not bias and torch.equal(rows.expand(bias.shape), bias)
+        assert rows.data_ptr() % 16 == 0 and all(s * rows.element_size() % 16 == 0 for s in rows.stride()[:3])
+        assert rows.numel() * (H if form == "heads" else 1) == bias.numel()
+    opts = dict(causal=causal, dropout=(drop, *state)) if drop else dict(causal=causal)
+    o_ref, lse_ref = attention_fwd_oracle(q, k, v, bias=bias.cpu(), **opts)
+    ref = attention_bwd_oracle(q, k, v, go, bias=bias.cpu(), **opts)
+    call = lambda: flash_attn(*t, bias=bias, causal=causal, return_lse=True, dropout_p=drop, dropout_state=state if drop else None)
+    with torch.no_grad():
+        o_eval, _ = call()
+    o, lse = call()
+    got = torch.autograd.grad(o, t, _bshd(go.to(DEV)))
+    torch.cuda.synchronize()
+    assert torch.equal(o, o_eval)
+    _check(_bshd(o), lse, [_bshd(x) for x in got], o_ref, lse_ref, ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,Sq,Sk", [(1, 1, 1, 1), (2, 3, 5, 7), (1, 2, 33, 257), (2, 1, 3, 16)])
+def test_rows_of_the_copy(B, H, Sq, Sk, dtype):
+    bias = torch.randn(B, H, Sq, Sk + 3, device=DEV).to(dtype)[..., 2:Sk + 2]
+    size, n = bias.element_size(), 16 // bias.element_size()
+    row = -(-Sk // n) * n
+    out = torch.full((B * H * Sq + 1, row), float("nan"), dtype=dtype, device=DEV)       # (a row behind the last that stays as it is)
+    st = (_lib.ctypes.c_int64 * 3)(*bias.stride()[:3])
+    assert _lib.load().fo_attn_bias_rows(bias.data_ptr(), st, size, B, H, Sq, Sk, out.data_ptr(), row, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out[:-1, :Sk], bias.reshape(-1, Sk)) and bool((out[:-1, Sk:] == 0).all()) and bool(out[-1].isnan().all())
