@@ -1531,7 +1531,7 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
   static const hipError_t a3 = hipFuncSetAttribute((const void*)attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, DROP>,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_pipe);
   if (a1 != hipSuccess || a2 != hipSuccess || a3 != hipSuccess) return FO_ERR_LAUNCH;
-  // a bias without a query stride: the forms of the dQ kernel and (without dropout) of the pipelined dK/dV kernel that
+  // a bias without a query stride: the forms of the dQ kernel and of the pipelined dK/dV kernel that
   // take it at no cost per score (attn_bwd.variant 0 keeps the general bias kernels, which tests compare them with)
   const bool key_bias = BIAS && p.bias.strides[2] == 0 && tune(g_attn_bwd_variant) != 0;
   if constexpr (BIAS) {

@@ -1609,7 +1609,7 @@ int launch(const AttnParams& p, bool causal, bool dropout, hipStream_t stream) {
   // tests compare the two)
   const bool key_bias = p.bias.ptr != nullptr && p.bias.strides[2] == 0 && asked != FO_ATTN_KERNEL_ROWS128_EXACT;
   if (p.bias.ptr != nullptr && !key_bias) {
-    // tiles that can be copied (dma_ok: base and strides are multiples of 16 bytes) and start the score accumulators
+    // tiles that can be copied (dma_ok: base and strides are multiples of 16 bytes), whose values join the finished scores
     if (!dropout && p.d == D && p.bias.dma_ok && asked != FO_ATTN_KERNEL_ROWS128_EXACT) {
       if (p.bias.is_f32) return causal ? launch_one<T, D, true, true, 0, false, false, false, false, D, 4>(p, stream)
                                        : launch_one<T, D, false, true, 0, false, false, false, false, D, 4>(p, stream);

@@ -189,6 +189,10 @@ int fo_dropout_mask(uint8_t* keep, int64_t n_elements, float dropout_p, uint32_t
  * "matrix" bias [.,.,Sq,Sk], broadcast over batch and heads, are all expressed by strides: element (b, h, q, key) is
  * read at bias + b*bias_strides[0] + h*bias_strides[1] + q*bias_strides[2] + key, a stride of 0 broadcasting that
  * dimension. bias_dtype is FO_DTYPE_F32 or the dtype of q. No gradient is computed for the bias (nor does the reference).
+ * Where a bias with a query stride has its base and its three strides on multiples of 16 bytes, rows are read in pieces of 16
+ * bytes: up to the next such boundary behind the last key (at most 14 bytes, inside the piece that holds that key; what stands
+ * there does not matter, NaN included). Memory that ends with the last key of the last row is safe to pass, since no piece
+ * leaves the 16 bytes its key lies in; another stream may write to what follows in that piece at any time.
  * extras == NULL, or bias == NULL and dropout_p == 0, is exactly fo_attn_fwd / fo_attn_bwd. */
 typedef struct fo_attn_extras {
   const void* bias;          /* NULL = no bias */
