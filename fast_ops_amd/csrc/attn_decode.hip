@@ -11,9 +11,10 @@
 //     the loop, 64 KiB of copies in flight per compute unit at head_dim 128;
 //   * row maxima, row sums and O of the waves are merged in LDS at the end, those of several workgroups by a second kernel
 //     from fp32 partial results in the caller's workspace.
-// One query per head, bf16, K/V not in the caches, 128-row kernels -> this, us per call: B=4 H=32, 4001 keys at head_dim
-// 128 73 -> 53 (the kernel alone 41.5 us = 6.3 TB/s, the merge 4.8), B=1 H=32, 4096 keys 64 -> 20, 16384 keys 239 -> 54,
-// B=16 H=32, 2048 keys 140 -> 96, B=1 H=12, 8192 keys at head_dim 64 81 -> 15; 16 queries, B=16 H=32, 9000 keys at 64
+// One query per head, bf16, the better one of the 128-row kernels -> this, us per call, keys that no cache holds (a GiB of K/V taken
+// in turn; in brackets the same K/V again and again): B=4 H=32, 4001 keys at head_dim 128 69 -> 53 (62 -> 44; the kernel alone
+// 41 us = 6.4 TB/s, the merge 4.6), B=1 H=32, 4096 keys 64 -> 20 (54 -> 17), 16384 keys 239 -> 57 (195 -> 51), B=16 H=32, 2048 keys 98 -> 96
+// (98 -> 96), B=1 H=12, 8192 keys at head_dim 64 81 -> 15 (81 -> 14). The same K/V: 16 queries, B=16 H=32, 9000 keys at 64
 // 348 -> 201; multi-query B=14 H=32, 1697 keys at 128 96 -> 15.
 #include <type_traits>
 
