@@ -54,6 +54,7 @@ SOURCES = {
     "attn_bwd_bf16_d128.hip": ["-mllvm", "-pragma-unroll-threshold=400000"],
     "attn_bwd_f16_d64.hip": ["-mllvm", "-pragma-unroll-threshold=400000"],
     "attn_bwd_f16_d128.hip": ["-mllvm", "-pragma-unroll-threshold=400000"],
+    "attn_bwd_dq_of_ds.hip": [],
     "attn_decode.hip": [],
     "dropout_mask.hip": [],
     "bias_rows.hip": [],

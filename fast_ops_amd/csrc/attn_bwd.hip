@@ -8,7 +8,8 @@
 // fp32 scores and accumulators; P and dS are rounded to the operand type before the second GEMMs, as the reference
 // does (:515,:562-563).
 //
-// Two launches, no atomics, no scratch beyond the caller's [2, B, H, Sq] fp32 workspace (delta and -LSE / scale):
+// Two launches, no atomics, no scratch beyond the caller's [2, B, H, Sq] fp32 workspace (delta and -LSE / scale), or, where the caller
+// gives memory for it, dS kept by the dK/dV kernel and dQ computed from that (attn_bwd.hpp, attn_bwd_dq_of_ds.hip). The two:
 //   1. attn_bwd_dq_kernel: one workgroup per 128 query rows (4 waves x 32), walks the key tiles like the forward
 //      kernel. Scores are computed transposed, S^T = K Q^T and dP^T = V dO^T (A operands = K / V rows from LDS, B
 //      operands = Q^T / dO^T held in registers), so a lane owns one query: LSE and delta are per-lane scalars and
@@ -30,43 +31,9 @@
 
 #include <mutex>
 
-#include "attn_common.hpp"
+#include "attn_bwd.hpp"
 
 namespace fo {
-
-constexpr int kBwdWaves = 4;
-constexpr int kBwdRows = 32 * kBwdWaves;   // rows (queries or keys) owned by a workgroup
-constexpr int kBwdTile = 64;               // rows of a streamed tile
-
-struct AttnBwdParams {
-  const void *q, *k, *v, *o, *d_o;
-  const float* lse;
-  float* delta;       // [B, H, Sq]: -rowsum(dO O) (1 - dropout_p), written by the dQ kernel
-  float* nlse;        // [B, H, Sq]: -LSE / softmax_scale (with dropout: of an LSE lower by log(1 / (1 - p))), written by the dQ kernel beside delta
-  void *dq, *dk, *dv;
-  int B, H, Sq, Sk;
-  int d;                // true head_dim: a multiple of 8, at most the D the kernels are compiled for
-  int64_t qs[3], ks[3], vs[3], os[3], dos[3], dqs[3], dks[3], dvs[3];   // element strides: batch, head, sequence
-  float scale, scale_log2e, neg_inv_scale_log2e;   // softmax scale, scale * log2 e, -1 / (scale * log2 e)
-  int head_group;       // heads per group in the order of the workgroups (see bwd_item)
-  DropoutParams drop;   // used by the kernels instantiated with dropout only
-  BiasParams bias;      // used by the kernels instantiated with bias only
-};
-
-// Which (head, block) a workgroup of the dQ or dK/dV kernel owns. Blocks are numbered in the order they should start:
-// when causal, the heaviest first (the last query blocks, the first key blocks), so that the light ones fill the gaps
-// at the end. Taking every head's block 0, then every head's block 1, ... walks through the operands of all heads
-// once per block index; with many heads they no longer stay in the caches between two visits (512 heads of 2 MiB:
-// the kernels become HBM-bound), so the heads are taken in groups of head_group, group after group.
-__device__ inline void bwd_item(const AttnBwdParams& prm, int n_blk, int& bh, int& blk) {
-  const int n_bh = prm.B * prm.H, per_group = prm.head_group * n_blk;
-  const int grp = blockIdx.x / per_group, r = blockIdx.x - grp * per_group;
-  const int heads = min(prm.head_group, n_bh - grp * prm.head_group);
-  bh = grp * prm.head_group + r % heads;
-  blk = r / heads;
-}
-
-constexpr float kLog2e = 1.4426950408889634f;
 
 // acc += A B with the accumulator pinned in AGPRs. Left to the compiler, the 128 accumulator registers of dK and dV are
 // kept elsewhere between uses and copied in and out around every MFMA (eight extra VALU instructions per MFMA). Inside
@@ -846,6 +813,15 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_kernel(const Att
   }
 }
 
+// 16 bytes per lane to a wave-uniform address + byte_off + IMM. (Inline assembly: nothing waits for it. A VALU instruction that
+// writes the data registers may not follow a store of more than 8 bytes at once, which the compiler does not see here: hence the wait states.)
+template <int IMM, typename V>
+__device__ __forceinline__ void store16_uniform_base(char* base, uint32_t byte_off, V data) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("global_store_dwordx4 %0, %1, %2 offset:%3 nt\n\ts_nop 1" ::"v"(byte_off), "v"(data), "s"(base), "n"(IMM) : "memory");
+#endif
+}
+
 // ---------------------------------------------------------------------------------------------------------------------
 // The softmax-gradient jobs of one tile of the pipelined dK/dV kernel (see its tile_body): 48 slots, slot s = eight per
 // half-phase from the second half of phase 1 on. stage 0 = A of element r (P = exp2(S c)), stage 1 = B of elements r and
@@ -919,7 +895,12 @@ static_assert(softmax_grad_jobs_fit(16) && softmax_grad_jobs_fit(12) && softmax_
 // of its S accumulators in groups that carry little else: S + (b - LSE) / scale then comes out of the MFMAs. Two fp32 tiles per
 // wave do not fit beside the rings of head_dim 128 (by 1.5 KiB of 160): there it is three buffers of half a tile (32 queries),
 // of which tile j+2's second half takes the one that held the first half of tile j+1, half a phase after that was read.
-template <typename T, int D, bool CAUSAL, bool KBIAS = false, bool DROP = false, bool PAD = false, int LIVE = D, int TBIAS = 0>
+// DS: dS is kept for attn_bwd_dq_of_ds_kernel (ds_chunk). A tile's four pieces per wave are stored in the first groups of the next
+// tile, which carry no other arithmetic and come behind every copy that the next hand-over waits for: that one then waits
+// for all but the last four of the wave's memory operations, which complete in order. The stores carry nt: nothing of this kernel
+// reads them, and they would push Q and dO out of the cache (12 heads x 4096 not causal: 204 us without DS, 230 with plain stores, 217
+// with nt; 64 heads x 2048 causal 143, 166, 155).
+template <typename T, int D, bool CAUSAL, bool KBIAS = false, bool DROP = false, bool PAD = false, int LIVE = D, int TBIAS = 0, bool DS = false>
 __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(const AttnBwdParams prm) {
   static_assert(TBIAS == 0 || !(KBIAS || DROP || PAD), "not combined");
   static_assert(!(PAD && (DROP || KBIAS)), "the second visit of dropout's rows copies whole rows");
@@ -1036,8 +1017,8 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
   };
-  auto hand_over = [&](int j) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  auto hand_over = [&](int j, auto behind) {      // `behind`: memory operations of this wave that nobody waits for yet
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(behind)::value) : "memory");
     if constexpr (DROP) drop_rows(j, (j + 1 - qt0) % NBUF);
     __builtin_amdgcn_s_barrier();
     if (j + 2 < n_qt) issue(j + 2, (j + 2 - qt0) % NBUF);
@@ -1118,6 +1099,19 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   typedef __attribute__((ext_vector_type(4))) int i32x4;
   typedef __attribute__((ext_vector_type(2))) T vec2;
   i32x4 pf[2][2], dsf[2][2];
+  // DS: this wave's chunks (of tile 0 on), and the lane's place in the two kinds of pieces of one (see ds_chunk)
+  char* ds_wave = nullptr;
+  uint32_t ds_off[2] = {0, 0};
+  [[maybe_unused]] const int64_t ds_tile_bytes = ds_key_blocks(Sk) * kDsChunk;
+  if constexpr (DS) {
+    ds_wave = prm.ds + ds_chunk(prm, bh, k0w / 32, 0);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) ds_off[t] = (uint32_t)(1024 * t + ((l32 ^ (4 * t)) * 32) + 16 * hh);
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) dsf[qb][t] = i32x4{0, 0, 0, 0};
+  }
 
   [[maybe_unused]] auto zero_acc = [](f32x16& acc) {
 #pragma unroll
@@ -1260,6 +1254,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
     const char* next_g = nullptr;
     const char* next_rows = nullptr;
     const char* next_bias = nullptr;
+    [[maybe_unused]] char* ds_prev = nullptr;
     uint32_t next_q_dst = 0;
     FO_LDS char* next_rows_dst = nullptr;
     __builtin_amdgcn_sched_barrier(0);
@@ -1269,7 +1264,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       if (g == 3 * NMF) {
         // the hand-over, between phases 3 and 4 (see hand_over)
         if constexpr (SPREAD) {
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DS ? 4 : 0) : "memory");
           if constexpr (DROP) drop_rows(j, nbuf);
           __builtin_amdgcn_s_barrier();
           const int b2 = buf == 0 ? NBUF - 1 : buf - 1, which = wave_s & 1;   // (waves 2 and 3 repeat the row values of waves 0 and 1)
@@ -1280,7 +1275,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
           next_rows_dst = (FO_LDS char*)(rowvals + (NBUF * which + b2) * kBwdTile);
           if constexpr (TBIAS != 0) next_bias = bias_lane_ptr + (int64_t)(j + 2) * kBwdTile * bias_row_bytes;
         } else if constexpr (!AGAIN) {
-          if (j + 1 < n_qt) hand_over(j);
+          if (j + 1 < n_qt) hand_over(j, std::integral_constant<int, DS ? 4 : 0>{});
         }
       }
       // (two wait states where an MFMA may follow the VALU instruction that wrote its B operand: behind the hand-over,
@@ -1295,6 +1290,12 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
         else mfma_acc_agpr<T>(dvacc[db], fr[g % kFragAhead], __builtin_bit_cast(vec8, pf[ph - 2][t]));
       }
       refill(g);
+      if constexpr (DS && !AGAIN) {
+        // dS of the tile before. (The wave's first tile has none: what it stores, in its own place, it stores anew after it.)
+        if (g == 0) ds_prev = ds_wave + (int64_t)max(j - 1, ja) * ds_tile_bytes;
+        if (g < 2) store16_uniform_base<0>(ds_prev, ds_off[g], dsf[0][g]);
+        else if (g < 4) store16_uniform_base<2048>(ds_prev, ds_off[g - 2], dsf[1][g - 2]);
+      }
       if constexpr (DROP && !AGAIN) {
         // (pieces of drop_look(j + 1), pinned to their groups)
         if (g == 1) { drop_first = drop_index(j + 1); asm volatile("" : "+v"(drop_first)); }
@@ -1382,7 +1383,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   int j = qt0 - 1;
   for (; j <= min(ja, n_qt) - 1 && j <= n_qt - 2; ++j) {
     if constexpr (DROP) drop_look(j + 1);
-    hand_over(j);
+    hand_over(j, std::integral_constant<int, 0>{});
   }
   // Tiles that need the mask are a prefix (the causal diagonal) and possibly the last tile (queries past the end).
   // One loop per kind, each with a single body: with alternatives inside one loop the compiler moves the 128
@@ -1425,6 +1426,16 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   for (; j < n_qt && !needs_mask(j); ++j, next_buf()) tile_body(j, buf, std::false_type{}, std::false_type{}, std::false_type{});
   for (; j < n_qt; ++j, next_buf()) tile_body(j, buf, std::true_type{}, std::false_type{}, std::false_type{});
 
+  if constexpr (DS) {
+    if (ja < n_qt) {                         // the last tile's
+      char* last = ds_wave + (int64_t)(n_qt - 1) * ds_tile_bytes;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        store16_uniform_base<0>(last, ds_off[t], dsf[0][t]);
+        store16_uniform_base<2048>(last, ds_off[t], dsf[1][t]);
+      }
+    }
+  }
   if constexpr (DROP) {
     // rows that are partly dropped (`again` and what follows from it is the same for every wave)
     int slot_row = 0, n_slots = 0;           // lane i holds the row of slot i
@@ -1447,6 +1458,30 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       start_tile(0);
       zero_acc(dpacc[0]);
       tile_body(n_slots, 0, std::false_type{}, std::false_type{}, std::true_type{});
+      if constexpr (DS) {
+        // what the tile adds to the dS stored for its rows (by this wave, and complete: see the wait above)
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            typedef typename Ops<T>::vec8 vec8_t;
+            const vec8_t more = __builtin_bit_cast(vec8_t, dsf[qb][t]);
+            T* at[8];
+            T old[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+              const int slot_at = 32 * qb + 16 * t + 4 * hh + (u & 3) + 8 * (u >> 2), row = slot_at < n_slots ? gathered[slot_at] : 0;
+              const int x = row & 15, t2 = (row >> 4) & 1;
+              at[u] = (T*)(ds_wave + (int64_t)(row / kBwdTile) * ds_tile_bytes + ((row >> 5) & 1) * 2048 + t2 * 1024 + ((l32 ^ (4 * t2)) * 32) +
+                           ((x >> 2) & 1) * 16 + ((x & 3) + 4 * (x >> 3)) * 2);
+              if (slot_at >= n_slots || (CAUSAL && key > row)) at[u] = nullptr;
+              old[u] = at[u] != nullptr ? *at[u] : (T)0.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+              if (at[u] != nullptr) *at[u] = (T)((float)old[u] + (float)more[u]);
+          }
+      }
       n_slots = 0;
     };
     int jt = qt0 - 1;
@@ -1478,6 +1513,18 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   }
 }
 
+// rows, dK/dV with dS kept, dQ of dS
+template <typename T, bool CAUSAL, bool KBIAS, bool DROP, bool PAD, int LIVE, int TBIAS>
+static int launch_bwd_ds(const AttnBwdParams& q, unsigned g_dkdv, size_t lds_kv, hipStream_t s) {
+  static const hipError_t a = hipFuncSetAttribute((const void*)attn_bwd_dkdv_pipe_kernel<T, 128, CAUSAL, KBIAS, DROP, PAD, LIVE, TBIAS, true>,
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_kv);
+  if (a != hipSuccess) return FO_ERR_LAUNCH;
+  const int st = launch_bwd_rows<T>(q, DROP, TBIAS != 0, s);
+  if (st != FO_OK) return st;
+  attn_bwd_dkdv_pipe_kernel<T, 128, CAUSAL, KBIAS, DROP, PAD, LIVE, TBIAS, true><<<g_dkdv, kBwdWaves * 64, lds_kv, s>>>(q);
+  return launch_dq_of_ds<T>(q, CAUSAL, TBIAS != 0, s);
+}
+
 // A head_dim below the D columns the kernels are laid out for, without bias and dropout: the pipelined dK/dV kernel, and
 // products over the next multiple of 32 columns. B=4 H=16, 777 x 1250, head_dim 80, bf16: dQ 67.5 -> 55.4 us, dK/dV 137 ->
 // 72.6 us (plain kernel over 128 columns, every tile copied with lane addresses -> this).
@@ -1489,6 +1536,9 @@ static int launch_bwd_pad(const AttnBwdParams& q, unsigned g_dq, unsigned g_dkdv
   static const hipError_t a2 = hipFuncSetAttribute((const void*)attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, false, true, LIVE_KV>,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_pipe);
   if (a1 != hipSuccess || a2 != hipSuccess) return FO_ERR_LAUNCH;
+  if constexpr (D == 128) {
+    if (q.ds != nullptr) return launch_bwd_ds<T, CAUSAL, false, false, true, LIVE, 0>(q, g_dkdv, lds_pipe, s);
+  }
   attn_bwd_dq_kernel<T, D, CAUSAL, false, false, false, true, LIVE><<<g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
   attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, false, true, LIVE_KV><<<g_dkdv, kBwdWaves * 64, lds_pipe, s>>>(q);
   return launch_status();
@@ -1509,6 +1559,9 @@ static int launch_bwd_tile_bias(const AttnBwdParams& q, unsigned g_dq, unsigned 
   static const hipError_t a2 = hipFuncSetAttribute((const void*)attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, false, false, D, ELT>,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_kv);
   if (a1 != hipSuccess || a2 != hipSuccess) return FO_ERR_LAUNCH;
+  if constexpr (D == 128) {
+    if (q.ds != nullptr) return launch_bwd_ds<T, CAUSAL, false, false, false, D, ELT>(q, g_dkdv, lds_kv, s);
+  }
   attn_bwd_dq_kernel<T, D, CAUSAL, false, false, false, false, D, ELT><<<g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
   attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, false, false, false, D, ELT><<<g_dkdv, kBwdWaves * 64, lds_kv, s>>>(q);
   return launch_status();
@@ -1557,6 +1610,9 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
   // (delta is computed by the dQ kernel, which the dK/dV kernel follows)
   if constexpr (BIAS) {
     if (key_bias) {
+      if constexpr (D == 128) {
+        if (q.ds != nullptr && p.d == D) return launch_bwd_ds<T, CAUSAL, true, DROP, false, D, 0>(q, (unsigned)g_dkdv, lds_pipe, s);
+      }
       attn_bwd_dq_kernel<T, D, CAUSAL, DROP, false, true><<<(unsigned)g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
       if (p.d == D) attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, true, DROP><<<(unsigned)g_dkdv, kBwdWaves * 64, lds_pipe, s>>>(q);
       else attn_bwd_dkdv_kernel<T, D, CAUSAL, DROP, BIAS><<<(unsigned)g_dkdv, kBwdWaves * 64, lds_dkdv, s>>>(q);
@@ -1576,6 +1632,10 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
       return p.d <= NARROW ? launch_bwd_pad<T, D, CAUSAL, NARROW>(q, (unsigned)g_dq, (unsigned)g_dkdv, lds_dq, lds_pipe, s)
                            : launch_bwd_pad<T, D, CAUSAL, D>(q, (unsigned)g_dq, (unsigned)g_dkdv, lds_dq, lds_pipe, s);
     }
+  }
+  if constexpr (!BIAS && D == 128) {
+    if (q.ds != nullptr && p.d == D && tune(g_attn_bwd_variant) != 0)
+      return launch_bwd_ds<T, CAUSAL, false, DROP, false, D, 0>(q, (unsigned)g_dkdv, lds_pipe, s);
   }
   attn_bwd_dq_kernel<T, D, CAUSAL, DROP, BIAS><<<(unsigned)g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
   // attn_bwd.variant 0 selects the plain dK/dV kernel everywhere (tests compare the two)
@@ -1654,11 +1714,34 @@ static int scratch_of_current_device(float** out) {
   return FO_OK;
 }
 
+// The workspace of fo_attn_bwd_ws: the two values per query row, then dS where it is kept.
+static int64_t rows_ws_bytes(int B, int H, int Sq) { return ((int64_t)B * H * Sq * 2 * (int64_t)sizeof(float) + 255) & ~255ll; }
+static int64_t ds_bytes_of(int B, int H, int Sq, int Sk) { return (int64_t)B * H * ds_key_blocks(Sk) * ds_query_tiles(Sq) * kDsChunk; }
+// When dS is kept. Not at head_dim 64 and below, where computing the scores again costs half as much and reading dS the same: 8 x 12
+// heads x 1024 causal 77 us -> 82, 16 x 16 x 1024 157 -> 223. At head_dim 128, whole backward, scores again -> dS kept:
+//   12 heads x 4096, per-key bias, dropout 440 -> 347 us; x 3072 causal, bf16 bias with a query stride 200 -> 144; x 6144 853 -> 713
+//   4 heads x 2048 .. 8192 causal: the dQ kernel's workgroups walk their keys 2.2 us per 64 alone on their CU, reading dS 0.8 us:
+//   2 x 4 x 4096 217 -> 159; so from 1536 keys whatever the size
+//   fewer keys: with the rows' kernel and a third launch it takes 96 MiB of dS to gain: 192 heads x 512 125 -> 115, 64 x 1024 125 -> 114,
+//   64 x 768 not causal 90 -> 89, 16 x 1024 72 -> 76, 4 heads x 128 70 -> 73 (these wait for their host);
+//   twice that up to head_dim 96, whose scores cost 3/4: 64 heads x 777 x 1250 at 80 (128 MiB), forward and backward 148.8 -> 147.7
+//   up to 2 GiB, what a caller's memory is asked for; beyond, the gain shrinks with the traffic that no cache holds: 12 x 8192
+//   causal (1.6 GiB) 639 -> 594, 64 x 4096 causal (2 GiB) 877 -> 846, 512 x 2048 (4 GiB) 3402 -> 3392.
+constexpr int64_t kDsFromBytes = 96ll << 20, kDsMaxBytes = 2ll << 30;
+constexpr int kDsFromKeys = 1536;
+static bool bwd_keeps_ds(int B, int H, int Sq, int Sk, int D) {
+  const int asked = tune(g_attn_bwd_keep_ds);
+  if (asked == 0 || D <= 64 || (int64_t)B * H > (1 << 20) || ds_key_blocks(Sk) * ds_query_tiles(Sq) > kDsMaxBytes / kDsChunk) return false;
+  const int64_t bytes = ds_bytes_of(B, H, Sq, Sk);
+  return bytes <= kDsMaxBytes && (asked == 1 || Sk >= kDsFromKeys || bytes >= (D > 96 ? kDsFromBytes : 2 * kDsFromBytes));
+}
+
 static int attn_bwd_impl(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
                          float* delta_ws, void* dq, void* dk, void* dv, int B, int H, int Sq, int Sk, int D,
                          const int64_t* const* strides_host, float softmax_scale, int causal, int dtype, float dropout_p,
                          uint32_t seed, uint64_t rng_offset, const void* bias, const int64_t* bias_strides, int bias_dtype,
-                         void* stream, bool static_ws = false) {
+                         void* stream, bool static_ws = false, int64_t ws_bytes = 0) {
+  // ws_bytes: how much memory delta_ws points to where the caller says so (fo_attn_bwd_ws); dS is kept behind its two rows of values
   // static_ws: delta_ws is ignored and the library's own per-device array takes its place (fo_attn_bwd_static_ws)
   if (!q || !k || !v || !o || !d_o || !lse || (!delta_ws && !static_ws) || !dq || !dk || !dv || !strides_host) return FO_ERR_NULL_POINTER;
   for (int t = 0; t < 8; ++t)
@@ -1695,6 +1778,9 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   AttnBwdParams p;
   p.q = q; p.k = k; p.v = v; p.o = o; p.d_o = d_o; p.lse = lse; p.delta = delta_ws; p.nlse = delta_ws + (int64_t)B * H * Sq; p.dq = dq; p.dk = dk; p.dv = dv;
   p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.d = D;
+  p.ds = nullptr;
+  if (bwd_keeps_ds(B, H, Sq, Sk, D) && ws_bytes >= rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk) && !((uintptr_t)delta_ws & 15u))
+    p.ds = (char*)delta_ws + rows_ws_bytes(B, H, Sq);
   int64_t* dst[8] = {p.qs, p.ks, p.vs, p.os, p.dos, p.dqs, p.dks, p.dvs};
   for (int t = 0; t < 8; ++t)
     for (int i = 0; i < 3; ++i) dst[t][i] = strides_host[t][i];
@@ -1754,5 +1840,20 @@ extern "C" int fo_attn_bwd_ex(const void* q, const void* k, const void* v, const
   return attn_bwd_impl(q, k, v, o, d_o, lse, delta_ws, dq, dk, dv, B, H, Sq, Sk, D, strides_host, softmax_scale, causal, dtype,
                        extras->dropout_p, extras->dropout_seed, extras->dropout_offset, extras->bias, extras->bias_strides,
                        extras->bias_dtype, stream);
+}
+extern "C" int64_t fo_attn_bwd_workspace(int B, int H, int Sq, int Sk, int D) {
+  if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || D < 8 || D > 128 || D % 8 != 0 || (int64_t)B * H * Sq > (1ll << 40)) return 0;
+  return rows_ws_bytes(B, H, Sq) + (bwd_keeps_ds(B, H, Sq, Sk, D) ? ds_bytes_of(B, H, Sq, Sk) : 0);
+}
+
+extern "C" int fo_attn_bwd_ws(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
+                              void* dq, void* dk, void* dv, int B, int H, int Sq, int Sk, int D,
+                              const int64_t* const* strides_host, float softmax_scale, int causal, int dtype,
+                              const fo_attn_extras* extras, void* ws, int64_t ws_bytes, void* stream) {
+  if (ws_bytes < (int64_t)B * H * Sq * 2 * (int64_t)sizeof(float)) return FO_ERR_BAD_SHAPE;
+  const fo_attn_extras none = {};
+  const fo_attn_extras& x = extras ? *extras : none;
+  return attn_bwd_impl(q, k, v, o, d_o, lse, (float*)ws, dq, dk, dv, B, H, Sq, Sk, D, strides_host, softmax_scale, causal, dtype,
+                       x.dropout_p, x.dropout_seed, x.dropout_offset, x.bias, x.bias_strides, x.bias_dtype, stream, false, ws_bytes);
 }
 #endif  // FO_ATTN_UNIT == 0

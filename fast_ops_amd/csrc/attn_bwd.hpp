@@ -1,0 +1,62 @@
+// What the translation units of the attention backward share: attn_bwd.hip (dK/dV and the dQ kernel that computes the scores
+// again) and attn_bwd_dq_of_ds.hip (dQ from stored dS).
+#pragma once
+#include "attn_common.hpp"
+
+namespace fo {
+
+constexpr int kBwdWaves = 4;
+constexpr int kBwdRows = 32 * kBwdWaves;   // rows (queries or keys) owned by a workgroup
+constexpr int kBwdTile = 64;               // rows of a streamed tile
+
+struct AttnBwdParams {
+  const void *q, *k, *v, *o, *d_o;
+  const float* lse;
+  float* delta;       // [B, H, Sq]: -rowsum(dO O) (1 - dropout_p), written by the dQ kernel
+  char* ds;           // not null: where the dK/dV kernel leaves dS for the dQ kernel (see ds_chunk)
+  float* nlse;        // [B, H, Sq]: -LSE / softmax_scale (with dropout: of an LSE lower by log(1 / (1 - p))), written by the dQ kernel beside delta
+  void *dq, *dk, *dv;
+  int B, H, Sq, Sk;
+  int d;                // true head_dim: a multiple of 8, at most the D the kernels are compiled for
+  int64_t qs[3], ks[3], vs[3], os[3], dos[3], dqs[3], dks[3], dvs[3];   // element strides: batch, head, sequence
+  float scale, scale_log2e, neg_inv_scale_log2e;   // softmax scale, scale * log2 e, -1 / (scale * log2 e)
+  int head_group;       // heads per group in the order of the workgroups (see bwd_item)
+  DropoutParams drop;   // used by the kernels instantiated with dropout only
+  BiasParams bias;      // used by the kernels instantiated with bias only
+};
+
+// Which (head, block) a workgroup of the dQ or dK/dV kernel owns. Blocks are numbered in the order they should start:
+// when causal, the heaviest first (the last query blocks, the first key blocks), so that the light ones fill the gaps
+// at the end. Taking every head's block 0, then every head's block 1, ... walks through the operands of all heads
+// once per block index; with many heads they no longer stay in the caches between two visits (512 heads of 2 MiB:
+// the kernels become HBM-bound), so the heads are taken in groups of head_group, group after group.
+__device__ inline void bwd_item(const AttnBwdParams& prm, int n_blk, int& bh, int& blk) {
+  const int n_bh = prm.B * prm.H, per_group = prm.head_group * n_blk;
+  const int grp = blockIdx.x / per_group, r = blockIdx.x - grp * per_group;
+  const int heads = min(prm.head_group, n_bh - grp * prm.head_group);
+  bh = grp * prm.head_group + r % heads;
+  blk = r / heads;
+}
+
+constexpr float kLog2e = 1.4426950408889634f;
+
+// ---------------------------------------------------------------------------------------------------------------------
+// dQ from stored dS, where that has room (ds_bytes_of): the dK/dV kernel runs first and leaves dS, rounded to the operand
+// type for its own dK = dS^T Q, in memory, and dQ is one product of it with K. That saves computing S, dP and the exponential a second
+// time - two of the backward's seven products - for 2 bytes written and read per (query, key) pair, which the memory-side cache
+// holds for most of the sizes this is chosen at. -LSE / scale and -delta then come from a kernel of their own.
+//
+// dS lies in chunks of 64 queries x 32 keys (4 KiB): block qb of 32 queries x group t of 16 queries, 1 KiB each; inside one, a key's 16
+// queries are 32 bytes, in the order in which the dK/dV kernel's lanes hold them: position 8 hh + u is query (u & 3) + 8 (u >> 2) + 4 hh
+// of the 16. The chunks of a query tile follow one another, as the dQ kernel reads them. Key k of group t stands at place k ^ 4 t: two groups' keys that one transposing LDS read takes lie in different banks.
+constexpr int kDsChunk = 4096;
+__host__ __device__ inline int64_t ds_key_blocks(int Sk) { return ((int64_t)Sk + kBwdRows - 1) / kBwdRows * (kBwdRows / 32); }
+__host__ __device__ inline int64_t ds_query_tiles(int Sq) { return ((int64_t)Sq + kBwdTile - 1) / kBwdTile; }
+// byte offset of the chunk of 32-key block kb and 64-query tile qt
+__device__ inline int64_t ds_chunk(const AttnBwdParams& prm, int bh, int kb, int qt) {
+  return (((int64_t)bh * ds_query_tiles(prm.Sq) + qt) * ds_key_blocks(prm.Sk) + kb) * kDsChunk;
+}
+template <typename T> int launch_bwd_rows(const AttnBwdParams& p, bool drop, bool tile_bias, hipStream_t s);
+template <typename T> int launch_dq_of_ds(const AttnBwdParams& p, bool causal, bool tile_bias, hipStream_t s);
+
+}  // namespace fo

@@ -1,0 +1,230 @@
+// dQ of the attention backward from stored dS (see attn_bwd.hpp), and the two values per query row that the dK/dV kernel needs first.
+#include <type_traits>
+
+#include "attn_bwd.hpp"
+
+namespace fo {
+
+// (read once: kept out of the way of K, which the workgroups of a head share in the cache)
+__device__ __forceinline__ void dma16_uniform_base_nt(const void* base, uint32_t byte_off, FO_LDS void* dst) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)dst)), "v"(byte_off), "s"(base) : "memory", "m0");
+#endif
+}
+
+constexpr int kD = 128;      // columns the kernels are laid out for
+
+// -delta and -LSE / scale of every query row, for the dK/dV kernel where the dQ kernel runs after it (which otherwise computes
+// both): delta_i = sum_d dO_id O_id (flash_attention_triton.py:273-315). 16 lanes per row, 16 bytes each of O and dO.
+constexpr int kRowsPerWg = 64;
+template <typename T, bool DROP, bool TBIAS>
+__global__ void __launch_bounds__(256) attn_bwd_rows_kernel(const AttnBwdParams prm) {
+  typedef typename Ops<T>::vec8 vec8;
+  constexpr int N = kRowsPerWg / 16;
+  const int n_blk = (prm.Sq + kRowsPerWg - 1) / kRowsPerWg, bh = blockIdx.x / n_blk, q0 = (blockIdx.x - bh * n_blk) * kRowsPerWg;
+  const int b = bh / prm.H, h = bh - b * prm.H, col = 8 * (threadIdx.x & 15), row = q0 + (threadIdx.x >> 4);
+  const T* o = (const T*)prm.o + b * prm.os[0] + h * prm.os[1] + col;
+  const T* g = (const T*)prm.d_o + b * prm.dos[0] + h * prm.dos[1] + col;
+  vec8 ov[N], gv[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int64_t qi = min(row + 16 * i, prm.Sq - 1);
+    ov[i] = *(const vec8*)live_or_zero(o + qi * prm.os[2], col, prm.d);
+    gv[i] = *(const vec8*)live_or_zero(g + qi * prm.dos[2], col, prm.d);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    float delta = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) delta -= (float)ov[i][e] * (float)gv[i][e];
+#pragma unroll
+    for (int s = 1; s < 16; s <<= 1) delta += __shfl_xor(delta, s);
+    if (col != 0 || row + 16 * i >= prm.Sq) continue;
+    const int64_t at = (int64_t)bh * prm.Sq + row + 16 * i;
+    const float lse = prm.lse[at];
+    prm.delta[at] = DROP ? delta * prm.drop.keep_prob : delta;      // (the factors: see the dQ kernel of attn_bwd.hip)
+    prm.nlse[at] = TBIAS ? -lse * (kLog2e / prm.scale_log2e) : (lse * kLog2e - (DROP ? prm.drop.keep_log2 : 0.0f)) * prm.neg_inv_scale_log2e;
+  }
+}
+
+// dQ^T = K^T dS^T: a wave owns 32 query rows and walks 32-key tiles of K (shared by the workgroup's four waves) and dS
+// (its own) through a ring of four LDS buffers, one barrier per tile; both operands by transposing reads. Bound by reading dS where there
+// are workgroups enough, else by a workgroup's chain per tile (0.4 us: 12 heads x 3072 causal 40 us; with reads, conditions and products in
+// the order they come to mind 48). 12 heads x 4096 (0.4 GB of dS) 98 us = 4.1 TB/s of dS: the dQ kernel that computes the scores again takes
+// 172; copied without nt, dS pushes K out of the cache: 131. Five or eight buffers, or 64 rows per wave, gain nothing (131, 131 / 108-170).
+// TBIAS: P of a row whose bias is large as a whole is off by the rounding of -LSE / scale, one factor per row, made good here.
+template <typename T, bool CAUSAL, int LIVE, bool PAD, bool TBIAS, int SLOTS>
+__global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_of_ds_kernel(const AttnBwdParams prm) {
+  typedef typename Ops<T>::vec8 vec8;
+  constexpr int D = kD, TILE = 32, ROW_BYTES = D * 2, CHUNKS = ROW_BYTES / 16, ROWS_PER_DMA = 1024 / ROW_BYTES;
+  constexpr int K_BYTES = TILE * ROW_BYTES, DS_BYTES = 2048, SLOT = K_BYTES + kBwdWaves * DS_BYTES;
+  constexpr int NK = K_BYTES / 1024 / kBwdWaves, ND = DS_BYTES / 1024, NI = NK + ND;
+  constexpr int DBLK = LIVE / 32;
+  extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
+  FO_LDS char* smem = (FO_LDS char*)smem_raw;      // slots: K tile | dS of each wave
+  const int wave_s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5, L16 = lane & 15, g16 = (lane >> 4) & 1;
+  const int Sq = prm.Sq, Sk = prm.Sk, n_qblk = (Sq + kBwdRows - 1) / kBwdRows, n_qt = (int)ds_query_tiles(Sq);
+  int bh, qblk;
+  bwd_item(prm, n_qblk, bh, qblk);
+  qblk = n_qblk - 1 - qblk;                        // heaviest causal blocks first
+  const int b = bh / prm.H, h = bh % prm.H;
+  const T* kbase = (const T*)prm.k + b * prm.ks[0] + h * prm.ks[1];
+  const int block32 = qblk * kBwdWaves + wave_s;                      // the wave's block of 32 queries
+  const int qt = min(block32 >> 1, n_qt - 1);                         // (rows past the end: the chunk exists, nothing is stored)
+  const char* ds = prm.ds + ds_chunk(prm, bh, 0, qt) + (wave_s & 1) * 2048;
+  const int all_tiles = (Sk + TILE - 1) / TILE;
+  // (causal: key blocks past a 64-query tile's last query left no dS for it)
+  const int n_tiles = CAUSAL ? min(all_tiles, 4 * (qblk + 1)) : all_tiles, my_tiles = CAUSAL ? min(n_tiles, 2 * qt + 2) : n_tiles;
+
+  uint32_t k_off[NK];
+#pragma unroll
+  for (int i = 0; i < NK; ++i) {
+    const int row = (wave_s * NK + i) * ROWS_PER_DMA + lane / CHUNKS;
+    k_off[i] = (uint32_t)(row * (int)prm.ks[2] + ((lane % CHUNKS) ^ swz<D>(row)) * 8) * 2u;
+  }
+  const bool k_off_ok = prm.ks[2] < (1 << 23);
+  const uint32_t lane16 = (uint32_t)lane * 16u;
+  auto issue = [&](int tile, int slot_i, auto inside) {
+    FO_LDS char* slot = smem + slot_i * SLOT;
+    if (decltype(inside)::value || (!PAD && k_off_ok && tile * TILE + TILE <= Sk)) {
+      const char* src = (const char*)(kbase + (int64_t)(tile * TILE) * prm.ks[2]);
+#pragma unroll
+      for (int i = 0; i < NK; ++i) dma16_uniform_base(src, k_off[i], slot + (wave_s * NK + i) * 1024);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NK; ++i) {
+        const int row = (wave_s * NK + i) * ROWS_PER_DMA + lane / CHUNKS, col = ((lane % CHUNKS) ^ swz<D>(row)) * 8;
+        // (keys past the end re-read the last one; their dS counts as zero below)
+        dma16_lane_ptr(live_or_zero(kbase + (int64_t)min(tile * TILE + row, Sk - 1) * prm.ks[2] + col, col, prm.d), slot + (wave_s * NK + i) * 1024);
+      }
+    }
+    const char* src = ds + (int64_t)tile * kDsChunk;
+#pragma unroll
+    for (int t = 0; t < ND; ++t) dma16_uniform_base_nt(src + 1024 * t, lane16, slot + K_BYTES + wave_s * DS_BYTES + 1024 * t);
+  };
+  f32x16 acc[DBLK];
+#pragma unroll
+  for (int i = 0; i < DBLK; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
+#pragma unroll
+  for (int i = 0; i < SLOTS - 1; ++i)
+    if (i < n_tiles) issue(i, i, std::false_type{});
+
+  // Byte offsets of the fragment reads inside a slot (K as col_frag computes them; dS: keys r and r + 8 of a 16-key step, four
+  // queries' worth of 8 bytes). A 16-key step further is an immediate.
+  const int r0 = 4 * hh + (L16 >> 2), sub = (L16 & 1) * 8;
+  uint32_t k_at[DBLK][2], ds_at[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int r = r0 + 8 * u;
+#pragma unroll
+    for (int db = 0; db < DBLK; ++db) k_at[db][u] = (uint32_t)(r * ROW_BYTES + ((4 * db + 2 * g16 + ((L16 & 3) >> 1)) ^ swz<D>(r)) * 16 + sub);
+    ds_at[u] = (uint32_t)(K_BYTES + wave_s * DS_BYTES + g16 * 1024 + ((r ^ (4 * g16)) * 32) + (L16 & 3) * 8);
+  }
+  auto tr_read = [&](uint32_t at, int imm) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16((FO_LDS s16x4*)(smem + at + imm)); };
+  auto joined = [](s16x4 lo, s16x4 hi) { return __builtin_bit_cast(vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)); };
+  // every fragment of a tile is asked for before its first product
+  auto products = [&](int tile, int slot_i, auto ragged) {
+    const uint32_t slot = (uint32_t)(slot_i * SLOT);
+    vec8 kv[2][DBLK], dsv[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      s16x4 lo = tr_read(ds_at[0] + slot, 512 * t), hi = tr_read(ds_at[1] + slot, 512 * t);
+      if constexpr (decltype(ragged)::value) {
+        const int left = Sk - (tile * TILE + 16 * t + 4 * hh);      // element e of lo (hi) is key e (8 + e) from there
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { lo[e] = e < left ? lo[e] : (short)0; hi[e] = 8 + e < left ? hi[e] : (short)0; }
+      }
+      dsv[t] = joined(lo, hi);
+#pragma unroll
+      for (int db = 0; db < DBLK; ++db) kv[t][db] = joined(tr_read(k_at[db][0] + slot, 16 * t * ROW_BYTES), tr_read(k_at[db][1] + slot, 16 * t * ROW_BYTES));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int db = 0; db < DBLK; ++db) acc[db] = Ops<T>::mfma(kv[t][db], dsv[t], acc[db]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (every read is back before the next barrier)
+  };
+  int slot_i = 0, tile = 0;
+  // Tile `tile` has landed when all but the copies of the SLOTS - 2 tiles after it have; behind the barrier that holds for everyone,
+  // and nobody reads the tile before it any more, whose slot takes tile + SLOTS - 1.
+  // (one straight loop for the tiles that copy a whole one ahead; causal: they count for every wave, whose last tiles differ by two)
+  static_assert(SLOTS > 2, "");
+  if (!PAD && k_off_ok)
+    for (const int end = min(n_tiles, Sk / TILE) - (SLOTS - 1); tile < end; ++tile, slot_i = slot_i == SLOTS - 1 ? 0 : slot_i + 1) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SLOTS - 2) * NI) : "memory");
+      __builtin_amdgcn_s_barrier();
+      issue(tile + SLOTS - 1, slot_i == 0 ? SLOTS - 1 : slot_i - 1, std::true_type{});
+      products(tile, slot_i, std::false_type{});
+    }
+  for (; tile < n_tiles; ++tile, slot_i = slot_i == SLOTS - 1 ? 0 : slot_i + 1) {
+    if (tile + SLOTS - 2 < n_tiles) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SLOTS - 2) * NI) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    if (tile + SLOTS - 1 < n_tiles) issue(tile + SLOTS - 1, slot_i == 0 ? SLOTS - 1 : slot_i - 1, std::false_type{});
+    if (CAUSAL && tile >= my_tiles) continue;
+    if (tile * TILE + TILE > Sk) products(tile, slot_i, std::true_type{});
+    else products(tile, slot_i, std::false_type{});
+  }
+  // column l32 of the result is position l32 of the block (see attn_bwd.hpp)
+  const int qi = block32 * 32 + 16 * (l32 >> 4) + (l32 & 3) + 8 * ((l32 >> 2) & 1) + 4 * ((l32 >> 3) & 1);
+  if (qi >= Sq) return;
+  float mul = prm.scale;
+  if constexpr (TBIAS) {
+    const float per_scale = kLog2e / prm.scale_log2e, lse = prm.lse[(int64_t)bh * Sq + qi];
+    mul *= __builtin_amdgcn_exp2f(__builtin_fmaf(-lse, per_scale, lse * per_scale) * prm.scale_log2e);
+  }
+  T* op = (T*)prm.dq + b * prm.dqs[0] + h * prm.dqs[1] + (int64_t)qi * prm.dqs[2];
+#pragma unroll
+  for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg) {
+      typedef __attribute__((ext_vector_type(4))) T vec4;
+      vec4 o4;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) o4[u] = (T)(acc[db][rg * 4 + u] * mul);
+      if (32 * db + 8 * rg + 4 * hh < prm.d) *(vec4*)(op + 32 * db + 8 * rg + 4 * hh) = o4;
+    }
+}
+
+template <typename T>
+int launch_bwd_rows(const AttnBwdParams& p, bool drop, bool tile_bias, hipStream_t s) {
+  const unsigned grid = (unsigned)((int64_t)p.B * p.H * ((p.Sq + kRowsPerWg - 1) / kRowsPerWg));
+  if (drop) attn_bwd_rows_kernel<T, true, false><<<grid, 256, 0, s>>>(p);
+  else if (tile_bias) attn_bwd_rows_kernel<T, false, true><<<grid, 256, 0, s>>>(p);
+  else attn_bwd_rows_kernel<T, false, false><<<grid, 256, 0, s>>>(p);
+  return launch_status();
+}
+
+template <typename T, bool CAUSAL, int LIVE, bool PAD, bool TBIAS, int SLOTS>
+static int launch_one(const AttnBwdParams& p, hipStream_t s) {
+  constexpr int lds = SLOTS * (32 * kD * 2 + kBwdWaves * 2048);
+  static const hipError_t a = hipFuncSetAttribute((const void*)attn_bwd_dq_of_ds_kernel<T, CAUSAL, LIVE, PAD, TBIAS, SLOTS>,
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (a != hipSuccess) return FO_ERR_LAUNCH;
+  const unsigned grid = (unsigned)((int64_t)p.B * p.H * ((p.Sq + kBwdRows - 1) / kBwdRows));
+  attn_bwd_dq_of_ds_kernel<T, CAUSAL, LIVE, PAD, TBIAS, SLOTS><<<grid, kBwdWaves * 64, lds, s>>>(p);
+  return launch_status();
+}
+template <typename T, bool CAUSAL, int LIVE, bool PAD, bool TBIAS>
+static int launch_form(const AttnBwdParams& p, hipStream_t s) {
+  return launch_one<T, CAUSAL, LIVE, PAD, TBIAS, 4>(p, s);
+}
+template <typename T>
+int launch_dq_of_ds(const AttnBwdParams& p, bool causal, bool tile_bias, hipStream_t s) {
+  if (p.d == kD) {
+    if (tile_bias) return causal ? launch_form<T, true, 128, false, true>(p, s) : launch_form<T, false, 128, false, true>(p, s);
+    return causal ? launch_form<T, true, 128, false, false>(p, s) : launch_form<T, false, 128, false, false>(p, s);
+  }
+  if (p.d <= 96) return causal ? launch_form<T, true, 96, true, false>(p, s) : launch_form<T, false, 96, true, false>(p, s);
+  return causal ? launch_form<T, true, 128, true, false>(p, s) : launch_form<T, false, 128, true, false>(p, s);
+}
+template int launch_bwd_rows<__bf16>(const AttnBwdParams&, bool, bool, hipStream_t);
+template int launch_bwd_rows<_Float16>(const AttnBwdParams&, bool, bool, hipStream_t);
+template int launch_dq_of_ds<__bf16>(const AttnBwdParams&, bool, bool, hipStream_t);
+template int launch_dq_of_ds<_Float16>(const AttnBwdParams&, bool, bool, hipStream_t);
+
+}  // namespace fo

@@ -13,6 +13,7 @@ std::atomic<int> g_attn_decode_split{-1};
 std::atomic<int> g_attn_tail{-1};
 std::atomic<int> g_attn_balance{-1};
 std::atomic<int> g_attn_bwd_order{-1};
+std::atomic<int> g_attn_bwd_keep_ds{-1};
 }  // namespace fo
 
 extern "C" const char* fo_strerror(int status) {
@@ -73,6 +74,10 @@ extern "C" int fo_tune_set(const char* key, int value) {
     fo::g_attn_balance = value; return FO_OK;
   }
   if (strcmp(key, "attn_bwd.order") == 0) { fo::g_attn_bwd_order = value; return FO_OK; }
+  if (strcmp(key, "attn_bwd.keep_ds") == 0) {
+    if (value > 1) return FO_ERR_UNSUPPORTED;
+    fo::g_attn_bwd_keep_ds = value; return FO_OK;
+  }
   return FO_ERR_UNSUPPORTED;
 }
 
@@ -87,6 +92,7 @@ extern "C" int fo_tune_get(const char* key) {
   if (strcmp(key, "attn.tail") == 0) return fo::tune(fo::g_attn_tail);
   if (strcmp(key, "attn.balance") == 0) return fo::tune(fo::g_attn_balance);
   if (strcmp(key, "attn_bwd.order") == 0) return fo::tune(fo::g_attn_bwd_order);
+  if (strcmp(key, "attn_bwd.keep_ds") == 0) return fo::tune(fo::g_attn_bwd_keep_ds);
   if (strcmp(key, "build.ablations") == 0) {
 #if defined(FO_ABLATIONS)
     return 1;

@@ -263,7 +263,7 @@ class _BwdPlan:
     """What a backward call of one (shapes, strides, dtypes, devices, layout) needs besides the data pointers, as _FwdPlan.
     (Checks, stride arrays and the switch of the device took 12 of the 31 us such a call cost the host, and a training step of a
     small model waits for its host: B=8 H=12 S=1024 D=64 causal with dropout 132 -> 117 us per step.)"""
-    __slots__ = ("B", "H", "Sq", "Sk", "D", "strides", "arrays", "dtype_code", "device_index", "delta_shape")
+    __slots__ = ("B", "H", "Sq", "Sk", "D", "strides", "arrays", "dtype_code", "device_index", "ws_bytes")
 
 
 _BWD_PLANS: dict = {}
@@ -271,7 +271,7 @@ _BWD_PLANS: dict = {}
 
 def _bwd_plan(q: Tensor, k: Tensor, v: Tensor, o: Tensor, d_o: Tensor, dims: Tuple[int, int, int, int]) -> _BwdPlan:
     key = (q.shape, q.stride(), k.shape, k.stride(), v.shape, v.stride(), o.stride(), d_o.stride(), q.dtype, k.dtype, v.dtype,
-           q.device, k.device, v.device, dims)
+           q.device, k.device, v.device, dims, _lib.tune_generation)      # (the workspace depends on what _lib.tune_set has set)
     plan = _BWD_PLANS.get(key)
     if plan is not None:
         return plan
@@ -285,7 +285,7 @@ def _bwd_plan(q: Tensor, k: Tensor, v: Tensor, o: Tensor, d_o: Tensor, dims: Tup
     plan.strides = (ctypes.POINTER(ctypes.c_int64) * 8)(*[ctypes.cast(a, ctypes.POINTER(ctypes.c_int64)) for a in plan.arrays])
     plan.dtype_code = _DTYPE_CODE[q.dtype]
     plan.device_index = q.device.index if q.device.index is not None else torch.cuda.current_device()
-    plan.delta_shape = (2, plan.B, plan.H, plan.Sq)
+    plan.ws_bytes = _lib.load().fo_attn_bwd_workspace(plan.B, plan.H, plan.Sq, plan.Sk, plan.D)
     if len(_BWD_PLANS) > 4096:
         _BWD_PLANS.clear()
     _BWD_PLANS[key] = plan
@@ -312,7 +312,11 @@ def attn_bwd_strided(
     dq = torch.empty(q.shape, dtype=q.dtype, device=device)
     dk = torch.empty(k.shape, dtype=k.dtype, device=device)
     dv = torch.empty(v.shape, dtype=v.dtype, device=device)
-    delta = torch.empty(plan.delta_shape, dtype=torch.float32, device=device)   # workspace: -delta and -LSE / scale per row
+    # workspace: -delta and -LSE / scale per row, and dS where it is kept; without memory for that, the rows' values alone
+    try:
+        ws = torch.empty(plan.ws_bytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        ws = torch.empty(8 * plan.B * plan.H * plan.Sq, dtype=torch.uint8, device=device)
     if bias is not None:
         bias = _expand_bias(bias, q, plan.B, plan.H, plan.Sq, plan.Sk)
     lib = _lib.load()
@@ -323,20 +327,15 @@ def attn_bwd_strided(
         guard.__enter__()
     try:
         stream = _raw_stream(dev)
-        args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr(), delta.data_ptr(),
-                dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), plan.B, plan.H, plan.Sq, plan.Sk, plan.D, plan.strides, scale,
-                1 if causal else 0, plan.dtype_code)
-        if bias is not None:
-            status = lib.fo_attn_bwd_ex(*args, ctypes.byref(_extras(bias, dropout)), stream)
-        elif dropout is None or dropout[0] == 0.0:
-            status = lib.fo_attn_bwd(*args, stream)
-        else:
-            status = lib.fo_attn_bwd_dropout(*args, float(dropout[0]), dropout[1] & 0xFFFFFFFF, dropout[2] % (1 << 64), stream)
+        extras = None if bias is None and (dropout is None or dropout[0] == 0.0) else ctypes.byref(_extras(bias, dropout))
+        status = lib.fo_attn_bwd_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr(),
+                                    dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), plan.B, plan.H, plan.Sq, plan.Sk, plan.D, plan.strides, scale,
+                                    1 if causal else 0, plan.dtype_code, extras, ws.data_ptr(), ws.numel(), stream)
     finally:
         if guard is not None:
             guard.__exit__(None, None, None)
     if status != 0:
-        _lib.check(status, "fo_attn_bwd")
+        _lib.check(status, "fo_attn_bwd_ws")
     return dq, dk, dv
 
 
