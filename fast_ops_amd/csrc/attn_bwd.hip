@@ -206,35 +206,6 @@ __device__ __forceinline__ void copy_two_tiles64_inside(const T* base_a, int64_t
   }
 }
 
-// A wave's 32 finished gradient rows (accumulator layout: lane = row l32, registers 4*rg + u = columns
-// 32*db + 8*rg + 4*hh + u) written to memory. Straight from the registers that is 8 bytes per lane to 32 different
-// rows per instruction (4.3 us per workgroup for dK and dV, during which the workgroup's LDS and registers keep the
-// next one waiting); instead the rows are rounded into LDS (`stage`, 32 rows padded by 16 bytes each, this wave's
-// own) and leave as whole 16-byte pieces, 64 lanes covering consecutive rows. Rows from n_rows on and columns from the true head_dim `d` on are not written.
-template <typename T, int D>
-__device__ __forceinline__ void store_rows_via_lds(const f32x16 (&acc)[D / 32], float mul, FO_LDS char* stage, T* base, int64_t stride,
-                                                   int row0, int n_rows, int d, int lane) {
-  constexpr int ROW_BYTES = D * 2, OROW = ROW_BYTES + 16, CH = ROW_BYTES / 16;
-  typedef __attribute__((ext_vector_type(4))) T vec4;
-  typedef __attribute__((ext_vector_type(4))) int i32x4;
-  const int l32 = lane & 31, hh = lane >> 5;
-#pragma unroll
-  for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-    for (int rg = 0; rg < 4; ++rg) {
-      vec4 o4;
-#pragma unroll
-      for (int u = 0; u < 4; ++u) o4[u] = (T)(acc[db][rg * 4 + u] * mul);
-      *(FO_LDS vec4*)(stage + l32 * OROW + (32 * db + 8 * rg + 4 * hh) * 2) = o4;
-    }
-#pragma unroll
-  for (int it = 0; it < 32 * CH / 64; ++it) {
-    const int idx = it * 64 + lane, row = idx / CH, ch = idx % CH;
-    const i32x4 piece = *(FO_LDS const i32x4*)(stage + row * OROW + ch * 16);
-    if (row0 + row < n_rows && ch * 8 < d) *(i32x4*)(base + (int64_t)(row0 + row) * stride + ch * 8) = piece;
-  }
-}
-constexpr int stage_bytes(int D) { return 32 * (D * 2 + 16); }   // per wave and matrix
 template <int TBIAS, int D>
 constexpr int tile_bias_bytes() { return TBIAS == 4 && D == 128 ? 3 * 32 * 32 * 4 : 2 * kBwdTile * 32 * TBIAS; }   // per wave of the dK/dV kernel: its tiles of a bias
 
@@ -895,7 +866,7 @@ static_assert(softmax_grad_jobs_fit(16) && softmax_grad_jobs_fit(12) && softmax_
 // of its S accumulators in groups that carry little else: S + (b - LSE) / scale then comes out of the MFMAs. Two fp32 tiles per
 // wave do not fit beside the rings of head_dim 128 (by 1.5 KiB of 160): there it is three buffers of half a tile (32 queries),
 // of which tile j+2's second half takes the one that held the first half of tile j+1, half a phase after that was read.
-// DS: dS is kept for attn_bwd_dq_of_ds_kernel (ds_chunk). A tile's four pieces per wave are stored in the first groups of the next
+// DS: dS is kept for attn_bwd_dq_of_ds_kernel (ds_chunk), and several workgroups may share a block's query tiles (prm.items). A tile's four pieces per wave are stored in the first groups of the next
 // tile, which carry no other arithmetic and come behind every copy that the next hand-over waits for: that one then waits
 // for all but the last four of the wave's memory operations, which complete in order. The stores carry nt: nothing of this kernel
 // reads them, and they would push Q and dO out of the cache (12 heads x 4096 not causal: 204 us without DS, 230 with plain stores, 217
@@ -919,15 +890,28 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   const int wave_s = __builtin_amdgcn_readfirstlane(wave);
   const int lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   int bh, kblk;                                       // key block 0 has the most queries when causal: heaviest first
-  bwd_item(prm, (prm.Sk + kBwdRows - 1) / kBwdRows, bh, kblk);
+  [[maybe_unused]] uint32_t item = kWholeBlock;       // DS: the piece of the block's query tiles this workgroup takes
+  if (DS && prm.n_items > 0) {
+    const int n_bh = prm.B * prm.H, e = blockIdx.x / n_bh;
+    bh = blockIdx.x - e * n_bh;
+    item = prm.items[e];
+    kblk = item & 255u;
+  } else {
+    bwd_item(prm, (prm.Sk + kBwdRows - 1) / kBwdRows, bh, kblk);
+  }
   const int b = bh / prm.H, h = bh % prm.H;
   const int k0 = kblk * kBwdRows, k0w = k0 + wave_s * 32;
   const int Sq = prm.Sq, Sk = prm.Sk;
   const T* qbase = (const T*)prm.q + b * prm.qs[0] + h * prm.qs[1];
   const T* gbase = (const T*)prm.d_o + b * prm.dos[0] + h * prm.dos[1];
-  const int n_qt = (Sq + kBwdTile - 1) / kBwdTile;
-  const int qt0 = CAUSAL ? min(k0 / kBwdTile, n_qt) : 0;     // queries before the block's first key never attend it
-  const int ja = CAUSAL ? min(k0w / kBwdTile, n_qt) : 0;     // ... and this wave's keys start later still
+  int n_qt = (Sq + kBwdTile - 1) / kBwdTile;                 // the workgroup's query tiles are [qt0, n_qt)
+  int qt0 = CAUSAL ? min(k0 / kBwdTile, n_qt) : 0;           // queries before the block's first key never attend it
+  if constexpr (DS) {
+    const int pieces = (item >> 12) & 15, piece = (item >> 8) & 15, len = n_qt - qt0;
+    n_qt = qt0 + len * (piece + 1) / pieces;
+    qt0 += len * piece / pieces;
+  }
+  const int ja = CAUSAL ? min(max(k0w / kBwdTile, qt0), n_qt) : qt0;     // ... and this wave's keys start later still
 
   TileLaneOffsets<T, D> qlo, glo;
   qlo.init(prm.qs[2], PAD ? D : prm.d, wave_s, lane);
@@ -1421,7 +1405,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
 #if FO_BWD_SPREAD
   // (from here on only a last tile that crosses the end of Q needs the mask; tiles j with tile j+2 wholly inside Q)
   if (qlo.ok && glo.ok)
-    for (const int end = Sq / kBwdTile - 2; j < end; ++j, next_buf()) tile_body(j, buf, std::false_type{}, std::true_type{}, std::false_type{});
+    for (const int end = (DS ? min(Sq / kBwdTile, n_qt) : Sq / kBwdTile) - 2; j < end; ++j, next_buf()) tile_body(j, buf, std::false_type{}, std::true_type{}, std::false_type{});
 #endif
   for (; j < n_qt && !needs_mask(j); ++j, next_buf()) tile_body(j, buf, std::false_type{}, std::false_type{}, std::false_type{});
   for (; j < n_qt; ++j, next_buf()) tile_body(j, buf, std::true_type{}, std::false_type{}, std::false_type{});
@@ -1503,6 +1487,23 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
 
   acc_fence(dkacc);
   acc_fence(dvacc);
+  if constexpr (DS) {
+    if ((item >> 16) != kWholeBlock >> 16) {
+      // a piece of a block: the accumulators as they stand, for the dQ kernel's last workgroups (merge_dkdv) to add
+      char* part = dkdv_part(prm, item >> 16, bh, wave_s) + lane * 16;
+#pragma unroll
+      for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          f32x4 dk4, dv4;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) { dk4[u] = dkacc[db][4 * rg + u]; dv4[u] = dvacc[db][4 * rg + u]; }
+          *(f32x4*)(part + (4 * db + rg) * 1024) = dk4;
+          *(f32x4*)(part + kPartBytes / 8 + (4 * db + rg) * 1024) = dv4;
+        }
+      return;
+    }
+  }
   // (the tile buffers are free once every wave is past its last tile; dK, then dV, through the wave's own piece of them)
   __syncthreads();
   {
@@ -1521,7 +1522,8 @@ static int launch_bwd_ds(const AttnBwdParams& q, unsigned g_dkdv, size_t lds_kv,
   if (a != hipSuccess) return FO_ERR_LAUNCH;
   const int st = launch_bwd_rows<T>(q, DROP, TBIAS != 0, s);
   if (st != FO_OK) return st;
-  attn_bwd_dkdv_pipe_kernel<T, 128, CAUSAL, KBIAS, DROP, PAD, LIVE, TBIAS, true><<<g_dkdv, kBwdWaves * 64, lds_kv, s>>>(q);
+  const unsigned grid = q.n_items > 0 ? (unsigned)(q.n_items * q.B * q.H) : g_dkdv;
+  attn_bwd_dkdv_pipe_kernel<T, 128, CAUSAL, KBIAS, DROP, PAD, LIVE, TBIAS, true><<<grid, kBwdWaves * 64, lds_kv, s>>>(q);
   return launch_dq_of_ds<T>(q, CAUSAL, TBIAS != 0, s);
 }
 
@@ -1736,6 +1738,118 @@ static bool bwd_keeps_ds(int B, int H, int Sq, int Sk, int D) {
   return bytes <= kDsMaxBytes && (asked == 1 || Sk >= kDsFromKeys || bytes >= (D > 96 ? kDsFromBytes : 2 * kDsFromBytes));
 }
 
+// Which key blocks' query tiles several workgroups share (attn_bwd.hpp). A workgroup of the dK/dV kernel has a compute unit to itself,
+// so a launch takes as long as the unit that ends last: 12 heads x 3072 are 288 workgroups for 256 units, two rounds of which the
+// second is an eighth full; causal they are 288 of 48, 46, ... 2 tiles; 4 heads x 2048 are 64. Every candidate (the blocks of the
+// last round, or all, in 2 to 4 pieces; causal: those above a share of a unit's mean) is laid out as the hardware would, longest first,
+// with two tiles' time to start a piece, one to leave its sums and 128 KiB of them to add; the best is taken if it ends before 0.82
+// (causal 0.90) of the time of whole blocks: units that are idle let the others run at a higher clock, so that less than what is
+// laid out is gained. Whole backward, whole blocks -> shared, us, in brackets the share laid out:
+//   4 heads x 4096 causal, key bias, dropout 158 -> 109 (0.52); 6 x 3000 the same 131 -> 96 (0.60); 6 x 2500, dropout 120 -> 95 (0.68)
+//   12 x 3072 237 -> 201, with a bf16 bias with a query stride 298 -> 253 (0.69); 8 x 3072 causal with one 121 -> 111 (0.73); 8 x 4096
+//   causal 147 -> 138 (0.77); 12 x 6144 709 -> 661 (0.80); 12 x 3072 causal 134 -> 125, with a bias 152 -> 150 (0.89)
+//   not taken: 12 x 4096 335 -> 348, with key bias and dropout 360 -> 352 (0.84); 6 x 4096 165 -> 158 in 4 pieces (1.1)
+constexpr int kCus = 256, kMaxPieces = 4;
+struct DkdvPlan {
+  int n_items = 0, n_merges = 0, n_parts = 0;
+  uint32_t items[kMaxItems], merges[kMaxMerges];
+};
+// when the last of n_bh workgroups for each of n entries (cost[], longest first) ends, each on the unit that is free first
+static int makespan(const int* cost, int n, int n_bh) {
+  struct { int at, units; } grp[2 * kMaxItems + 2];      // units free from a time on, ascending
+  int n_grp = 1, last = 0;
+  grp[0] = {0, kCus};
+  for (int e = 0; e < n; ++e)
+    for (int left = n_bh; left > 0;) {
+      const int take = left < grp[0].units ? left : grp[0].units, end = grp[0].at + cost[e];
+      left -= take;
+      last = end > last ? end : last;
+      if ((grp[0].units -= take) == 0) {
+        for (int i = 1; i < n_grp; ++i) grp[i - 1] = grp[i];
+        --n_grp;
+      }
+      int at = n_grp;
+      while (at > 0 && grp[at - 1].at > end) --at;
+      if (at > 0 && grp[at - 1].at == end) { grp[at - 1].units += take; continue; }
+      for (int i = n_grp; i > at; --i) grp[i] = grp[i - 1];
+      grp[at] = {end, take};
+      ++n_grp;
+    }
+  return last;
+}
+static DkdvPlan make_dkdv_plan(int n_bh, int Sq, int Sk, bool causal, int asked) {
+  DkdvPlan best;
+  const int n_blk = (Sk + kBwdRows - 1) / kBwdRows, n_qt = (Sq + kBwdTile - 1) / kBwdTile;
+  if (asked == 0 || n_blk > kMaxItems || n_bh > kCus || (asked < 0 && (int64_t)n_bh * n_blk > 4 * kCus)) return best;
+  // (the heads in one group, see launch_bwd)
+  if (2 * ((int64_t)Sq + Sk) * 128 * 2 * n_bh > (256ll << 20)) return best;
+  auto tiles = [&](int blk) { const int first = kBwdRows / kBwdTile * blk; return causal ? (first < n_qt ? n_qt - first : 0) : n_qt; };
+  int64_t sum = 0;
+  for (int blk = 0; blk < n_blk; ++blk) sum += tiles(blk);
+  const int mean = (int)((sum * n_bh + kCus - 1) / kCus);
+  int cost[kMaxItems], best_time = 0;
+  // pieces_of(blk) for every block -> entries, longest first; false if there are too many
+  auto lay_out = [&](auto pieces_of, DkdvPlan& plan) -> bool {
+    for (int blk = 0; blk < n_blk; ++blk) {
+      const int s = pieces_of(blk);
+      if (plan.n_items + s > kMaxItems || (s > 1 && plan.n_merges == kMaxMerges)) return false;
+      if (s > 1) plan.merges[plan.n_merges++] = (uint32_t)blk | (uint32_t)s << 12 | (uint32_t)plan.n_parts << 16;
+      for (int i = 0; i < s; ++i) {
+        const uint32_t item = (uint32_t)blk | (uint32_t)i << 8 | (uint32_t)s << 12 | (s > 1 ? (uint32_t)plan.n_parts++ << 16 : kWholeBlock >> 16 << 16);
+        const int c = 2 * (tiles(blk) * (i + 1) / s - tiles(blk) * i / s) + 4 + (s > 1 ? 2 : 0);    // half tiles
+        int at = plan.n_items++;
+        for (; at > 0 && cost[at - 1] < c; --at) { cost[at] = cost[at - 1]; plan.items[at] = plan.items[at - 1]; }
+        cost[at] = c;
+        plan.items[at] = item;
+      }
+    }
+    return true;
+  };
+  auto consider = [&](auto pieces_of, bool forced) {
+    DkdvPlan plan;
+    if (!lay_out(pieces_of, plan) || plan.n_merges == 0) return;
+    const int time = makespan(cost, plan.n_items, n_bh) + plan.n_parts * n_bh / 32 + 4;
+    if (forced || time < best_time) { best_time = time; best = plan; }
+  };
+  if (asked > 1) {
+    consider([&](int blk) { const int t = tiles(blk); return t < 1 ? 1 : t < asked ? t : asked; }, true);
+    return best;
+  }
+  DkdvPlan whole;
+  if (!lay_out([](int) { return 1; }, whole)) return best;
+  best_time = makespan(cost, whole.n_items, n_bh) * (causal ? 90 : 82) / 100;
+  constexpr int kMinTiles = 4;
+  auto fits = [&](int blk, int s) { const int most = tiles(blk) / kMinTiles; return s < most ? s : most > 1 ? most : 1; };
+  if (causal) {
+    for (int f = 4; f >= 2; --f) {
+      const int most = mean * f / 4 > kMinTiles ? mean * f / 4 : kMinTiles;
+      consider([&](int blk) { const int s = (tiles(blk) + most - 1) / most; return fits(blk, s > kMaxPieces ? kMaxPieces : s); }, false);
+    }
+  } else {
+    const int rest = ((n_bh * n_blk) % kCus + n_bh - 1) / n_bh;
+    for (int s = 2; s <= kMaxPieces; ++s) {
+      consider([&](int blk) { return blk >= n_blk - rest ? fits(blk, s) : 1; }, false);
+      consider([&](int blk) { return fits(blk, s); }, false);
+    }
+  }
+  return best;
+}
+// (a step of a model asks for the same one over and over: kept per thread)
+static const DkdvPlan& dkdv_plan(int B, int H, int Sq, int Sk, bool causal) {
+  struct Key { int n_bh, Sq, Sk, causal, asked; };
+  static thread_local Key key = {0, 0, 0, 0, 0};
+  static thread_local DkdvPlan plan;
+  const int asked = tune(g_attn_bwd_order) >= 0 ? 0 : tune(g_attn_bwd_split);
+  if (key.n_bh != B * H || key.Sq != Sq || key.Sk != Sk || key.causal != (int)causal || key.asked != asked) {
+    plan = make_dkdv_plan(B * H, Sq, Sk, causal, asked);
+    key = {B * H, Sq, Sk, (int)causal, asked};
+  }
+  return plan;
+}
+static int64_t part_bytes_of(int B, int H, int Sq, int Sk, bool causal) {
+  return dkdv_plan(B, H, Sq, Sk, causal).n_parts * (int64_t)B * H * kPartBytes;
+}
+
 static int attn_bwd_impl(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
                          float* delta_ws, void* dq, void* dk, void* dv, int B, int H, int Sq, int Sk, int D,
                          const int64_t* const* strides_host, float softmax_scale, int causal, int dtype, float dropout_p,
@@ -1781,6 +1895,18 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   p.ds = nullptr;
   if (bwd_keeps_ds(B, H, Sq, Sk, D) && ws_bytes >= rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk) && !((uintptr_t)delta_ws & 15u))
     p.ds = (char*)delta_ws + rows_ws_bytes(B, H, Sq);
+  p.n_items = p.n_merges = 0;
+  p.part = nullptr;
+  if (p.ds != nullptr) {
+    const int64_t before = rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk);
+    const DkdvPlan& plan = dkdv_plan(B, H, Sq, Sk, causal != 0);
+    if (plan.n_items > 0 && ws_bytes >= before + plan.n_parts * (int64_t)B * H * kPartBytes) {
+      p.part = (char*)delta_ws + before;
+      p.n_items = plan.n_items; p.n_merges = plan.n_merges;
+      for (int i = 0; i < plan.n_items; ++i) p.items[i] = plan.items[i];
+      for (int i = 0; i < plan.n_merges; ++i) p.merges[i] = plan.merges[i];
+    }
+  }
   int64_t* dst[8] = {p.qs, p.ks, p.vs, p.os, p.dos, p.dqs, p.dks, p.dvs};
   for (int t = 0; t < 8; ++t)
     for (int i = 0; i < 3; ++i) dst[t][i] = strides_host[t][i];
@@ -1843,7 +1969,9 @@ extern "C" int fo_attn_bwd_ex(const void* q, const void* k, const void* v, const
 }
 extern "C" int64_t fo_attn_bwd_workspace(int B, int H, int Sq, int Sk, int D) {
   if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || D < 8 || D > 128 || D % 8 != 0 || (int64_t)B * H * Sq > (1ll << 40)) return 0;
-  return rows_ws_bytes(B, H, Sq) + (bwd_keeps_ds(B, H, Sq, Sk, D) ? ds_bytes_of(B, H, Sq, Sk) : 0);
+  if (!bwd_keeps_ds(B, H, Sq, Sk, D)) return rows_ws_bytes(B, H, Sq);
+  const int64_t causal = part_bytes_of(B, H, Sq, Sk, true), full = part_bytes_of(B, H, Sq, Sk, false);
+  return rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk) + (causal > full ? causal : full);
 }
 
 extern "C" int fo_attn_bwd_ws(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,

@@ -9,6 +9,13 @@ constexpr int kBwdWaves = 4;
 constexpr int kBwdRows = 32 * kBwdWaves;   // rows (queries or keys) owned by a workgroup
 constexpr int kBwdTile = 64;               // rows of a streamed tile
 
+// An item of the dK/dV kernel that keeps dS: key block | piece << 8 | pieces << 12 | part << 16; the block's query tiles are shared by
+// `pieces` workgroups, each of which leaves its sums in part `part` (of every head: see dkdv_part). A merge: key block | pieces << 12 |
+// first part << 16.
+constexpr int kMaxItems = 96, kMaxMerges = 48;
+constexpr uint32_t kWholeBlock = 0xFFFF1000u;
+constexpr int kPartBytes = 2 * kBwdRows * 128 * 4;     // dK and dV of a block in fp32: each wave's accumulators, 1 KiB per four registers
+
 struct AttnBwdParams {
   const void *q, *k, *v, *o, *d_o;
   const float* lse;
@@ -23,6 +30,10 @@ struct AttnBwdParams {
   int head_group;       // heads per group in the order of the workgroups (see bwd_item)
   DropoutParams drop;   // used by the kernels instantiated with dropout only
   BiasParams bias;      // used by the kernels instantiated with bias only
+  // dS kept: how the query tiles of key blocks are shared (see kWholeBlock); n_items 0 = a workgroup per block, as bwd_item has it
+  char* part;
+  int n_items, n_merges;
+  uint32_t items[kMaxItems], merges[kMaxMerges];
 };
 
 // Which (head, block) a workgroup of the dQ or dK/dV kernel owns. Blocks are numbered in the order they should start:
@@ -36,6 +47,10 @@ __device__ inline void bwd_item(const AttnBwdParams& prm, int n_blk, int& bh, in
   const int heads = min(prm.head_group, n_bh - grp * prm.head_group);
   bh = grp * prm.head_group + r % heads;
   blk = r / heads;
+}
+
+__device__ inline char* dkdv_part(const AttnBwdParams& prm, uint32_t part, int bh, int wave) {
+  return prm.part + ((int64_t)part * prm.B * prm.H + bh) * kPartBytes + wave * (kPartBytes / kBwdWaves);
 }
 
 constexpr float kLog2e = 1.4426950408889634f;
@@ -58,5 +73,35 @@ __device__ inline int64_t ds_chunk(const AttnBwdParams& prm, int bh, int kb, int
 }
 template <typename T> int launch_bwd_rows(const AttnBwdParams& p, bool drop, bool tile_bias, hipStream_t s);
 template <typename T> int launch_dq_of_ds(const AttnBwdParams& p, bool causal, bool tile_bias, hipStream_t s);
+
+// A wave's 32 finished gradient rows (accumulator layout: lane = row l32, registers 4*rg + u = columns
+// 32*db + 8*rg + 4*hh + u) written to memory. Straight from the registers that is 8 bytes per lane to 32 different
+// rows per instruction (4.3 us per workgroup for dK and dV, during which the workgroup's LDS and registers keep the
+// next one waiting); instead the rows are rounded into LDS (`stage`, 32 rows padded by 16 bytes each, this wave's
+// own) and leave as whole 16-byte pieces, 64 lanes covering consecutive rows. Rows from n_rows on and columns from the true head_dim `d` on are not written.
+template <typename T, int D>
+__device__ __forceinline__ void store_rows_via_lds(const f32x16 (&acc)[D / 32], float mul, FO_LDS char* stage, T* base, int64_t stride,
+                                                   int row0, int n_rows, int d, int lane) {
+  constexpr int ROW_BYTES = D * 2, OROW = ROW_BYTES + 16, CH = ROW_BYTES / 16;
+  typedef __attribute__((ext_vector_type(4))) T vec4;
+  typedef __attribute__((ext_vector_type(4))) int i32x4;
+  const int l32 = lane & 31, hh = lane >> 5;
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg) {
+      vec4 o4;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) o4[u] = (T)(acc[db][rg * 4 + u] * mul);
+      *(FO_LDS vec4*)(stage + l32 * OROW + (32 * db + 8 * rg + 4 * hh) * 2) = o4;
+    }
+#pragma unroll
+  for (int it = 0; it < 32 * CH / 64; ++it) {
+    const int idx = it * 64 + lane, row = idx / CH, ch = idx % CH;
+    const i32x4 piece = *(FO_LDS const i32x4*)(stage + row * OROW + ch * 16);
+    if (row0 + row < n_rows && ch * 8 < d) *(i32x4*)(base + (int64_t)(row0 + row) * stride + ch * 8) = piece;
+  }
+}
+constexpr int stage_bytes(int D) { return 32 * (D * 2 + 16); }   // per wave and matrix
 
 }  // namespace fo

@@ -47,6 +47,35 @@ __global__ void __launch_bounds__(256) attn_bwd_rows_kernel(const AttnBwdParams 
   }
 }
 
+// dK and dV of a key block whose query tiles several workgroups of the dK/dV kernel shared: their sums added, in order, in the lanes that
+// held them. By the last workgroups of the dQ launch, beside its others (they have what the launch before left, as those do).
+template <typename T, int LIVE>
+__device__ __forceinline__ void merge_dkdv(const AttnBwdParams& prm, int at, FO_LDS char* smem) {
+  const int n_bh = prm.B * prm.H, m = at / n_bh, bh = at - m * n_bh, b = bh / prm.H, h = bh - b * prm.H;
+  const int wave_s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const uint32_t w = prm.merges[m];
+  const int k0w = (int)(w & 255u) * kBwdRows + wave_s * 32, pieces = (w >> 12) & 15;
+#pragma unroll 1
+  for (int mat = 0; mat < 2; ++mat) {
+    f32x16 acc[LIVE / 32];
+#pragma unroll
+    for (int i = 0; i < LIVE / 32; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
+    for (int i = 0; i < pieces; ++i) {
+      const char* part = dkdv_part(prm, (w >> 16) + i, bh, wave_s) + mat * (kPartBytes / 8) + lane * 16;
+#pragma unroll
+      for (int g = 0; g < LIVE / 8; ++g) {
+        const f32x4 v = *(const f32x4*)(part + g * 1024);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[g >> 2][4 * (g & 3) + u] += v[u];
+      }
+    }
+    if (mat == 0) store_rows_via_lds<T, LIVE>(acc, prm.scale, smem + wave_s * stage_bytes(kD), (T*)prm.dk + b * prm.dks[0] + h * prm.dks[1], prm.dks[2], k0w, prm.Sk, prm.d, lane);
+    else store_rows_via_lds<T, LIVE>(acc, 1.0f, smem + wave_s * stage_bytes(kD), (T*)prm.dv + b * prm.dvs[0] + h * prm.dvs[1], prm.dvs[2], k0w, prm.Sk, prm.d, lane);
+  }
+}
+
 // dQ^T = K^T dS^T: a wave owns 32 query rows and walks 32-key tiles of K (shared by the workgroup's four waves) and dS
 // (its own) through a ring of four LDS buffers, one barrier per tile; both operands by transposing reads. Bound by reading dS where there
 // are workgroups enough, else by a workgroup's chain per tile (0.4 us: 12 heads x 3072 causal 40 us; with reads, conditions and products in
@@ -65,6 +94,8 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_of_ds_kernel(co
   const int wave_s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5, L16 = lane & 15, g16 = (lane >> 4) & 1;
   const int Sq = prm.Sq, Sk = prm.Sk, n_qblk = (Sq + kBwdRows - 1) / kBwdRows, n_qt = (int)ds_query_tiles(Sq);
+  const int n_dq = prm.B * prm.H * n_qblk;
+  if ((int)blockIdx.x >= n_dq) return merge_dkdv<T, LIVE>(prm, (int)blockIdx.x - n_dq, smem);
   int bh, qblk;
   bwd_item(prm, n_qblk, bh, qblk);
   qblk = n_qblk - 1 - qblk;                        // heaviest causal blocks first
@@ -205,7 +236,7 @@ static int launch_one(const AttnBwdParams& p, hipStream_t s) {
   static const hipError_t a = hipFuncSetAttribute((const void*)attn_bwd_dq_of_ds_kernel<T, CAUSAL, LIVE, PAD, TBIAS, SLOTS>,
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (a != hipSuccess) return FO_ERR_LAUNCH;
-  const unsigned grid = (unsigned)((int64_t)p.B * p.H * ((p.Sq + kBwdRows - 1) / kBwdRows));
+  const unsigned grid = (unsigned)((int64_t)p.B * p.H * ((p.Sq + kBwdRows - 1) / kBwdRows + p.n_merges));
   attn_bwd_dq_of_ds_kernel<T, CAUSAL, LIVE, PAD, TBIAS, SLOTS><<<grid, kBwdWaves * 64, lds, s>>>(p);
   return launch_status();
 }

@@ -46,7 +46,7 @@ const char* fo_strerror(int status);
 int fo_version(void);
 
 /* Tuning hook for benchmarks, profiling and tests: selects a kernel variant or a workgroup order by name
- * ("lion.variant", "attn.variant", "attn_bwd.variant", "attn.order", "attn.balance", "attn.keep_on", "attn.tail", "attn.decode_split", "attn_bwd.order", "attn_bwd.keep_ds"). Every value it accepts selects
+ * ("lion.variant", "attn.variant", "attn_bwd.variant", "attn.order", "attn.balance", "attn.keep_on", "attn.tail", "attn.decode_split", "attn_bwd.order", "attn_bwd.keep_ds", "attn_bwd.split"). Every value it accepts selects
  * code that computes the same function as the default; value -1 restores the default (the measured best). Returns
  * FO_OK, or FO_ERR_UNSUPPORTED for an unknown key or a value that selects nothing. The settings are process-global
  * atomics: a call reads each one once, a call already issued is not affected. fo_tune_get additionally answers
@@ -216,7 +216,8 @@ int fo_attn_bwd_ex(const void* q, const void* k, const void* v, const void* o, c
  * fo_attn_bwd (FO_ERR_BAD_SHAPE below), used by this call only until the stream has passed it and never needing to be cleared.
  * fo_attn_bwd_workspace answers how many bytes a call of a shape can use (0 where the shape itself is not taken): where
  * that is more than the rows' values (head_dim above 64, up to 2 GiB), with so many, 16-byte aligned, the call keeps dS (2 bytes per query and key, rounded up to 64 queries x 128 keys) and dQ is computed from it
- * instead of from the scores once more, where the shape and the bias allow (three launches, still no atomics, deterministic);
+ * instead of from the scores once more, where the shape and the bias allow (three launches, still no atomics, deterministic; where
+ * few workgroups would fill the chip badly several share the queries of a block of keys, their fp32 sums of dK and dV behind dS);
  * with less it computes what fo_attn_bwd_ex computes. extras may be NULL. No reference counterpart. */
 int64_t fo_attn_bwd_workspace(int B, int H, int Sq, int Sk, int D);
 int fo_attn_bwd_ws(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,

@@ -1,0 +1,60 @@
+"""Key blocks of the backward whose query tiles several workgroups share (attn_bwd.split, where dS is kept): the sums of a
+block's pieces added by the dQ launch. Every block in 2 to 4 pieces, down to pieces of one 64-query tile and blocks of fewer tiles than pieces,
+against the same call with a workgroup per block: dQ, from the same dS, to the bit; dK and dV to the rounding of their fp32 sums in another
+order, and of dS where rows that are partly dropped are added a second time."""
+import pytest
+import torch
+
+from fast_ops.flash_attention.flash_attention import flash_attn
+from fast_ops_amd import _lib
+from test_attention_dropout_forms_gpu import _state_with_partial_rows
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+CASES = [
+    # B, H, Sq, Sk, D, causal, bias, dropout
+    (1, 2, 64, 200, 128, False, None, 0.0), (1, 3, 129, 65, 128, False, None, 0.0), (2, 2, 321, 129, 128, False, None, 0.0),
+    (1, 2, 700, 1250, 80, False, None, 0.0), (1, 2, 257, 300, 104, True, None, 0.0), (1, 3, 515, 515, 128, True, None, 0.0),
+    (1, 2, 320, 900, 128, True, None, 0.0), (1, 2, 900, 320, 128, True, None, 0.0), (2, 2, 640, 384, 128, False, "key", 0.0),
+    (1, 2, 577, 577, 128, True, "rows", 0.0), (1, 2, 450, 260, 128, False, "rows", 0.0), (1, 2, 385, 400, 128, True, "rows32", 0.0),
+    (1, 2, 450, 128, 128, False, "rows32", 0.0), (1, 2, 1100, 1100, 128, True, None, 0.4), (1, 2, 2200, 700, 128, False, "key", 0.4),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"B{c[0]}H{c[1]}q{c[2]}k{c[3]}d{c[4]}{'c' if c[5] else 'f'}{c[6] or ''}{c[7] or ''}")
+def test_split_blocks(case, dtype):
+    B, H, Sq, Sk, D, causal, bias_kind, p = case
+    g = torch.Generator().manual_seed(Sq * 7 + Sk + D)
+    q, k, v, go = (torch.randn(B, n, H, D, generator=g).to(dtype).to(DEV) for n in (Sq, Sk, Sk, Sq))
+    bias = None
+    if bias_kind == "key":
+        bias = torch.randn(1, 1, 1, Sk, generator=g).to(DEV)
+    elif bias_kind is not None:
+        wide = torch.randn(1, H, Sq, (Sk + 15) // 16 * 16, generator=g).to(torch.float32 if bias_kind == "rows32" else dtype)
+        bias = wide.to(DEV)[..., :Sk]
+    state = _state_with_partial_rows(p, B, H, Sq, Sk, 987654321) if p else None
+    t = [x.requires_grad_(True) for x in (q, k, v)]
+
+    def backward(split):
+        _lib.tune_set("attn_bwd.split", split)
+        o = flash_attn(*t, bias=bias, causal=causal, dropout_p=p, dropout_state=(987654321, state) if p else None)
+        return torch.autograd.grad(o, t, go)
+
+    _lib.tune_set("attn_bwd.keep_ds", 1)       # (also where it does not pay)
+    try:
+        whole = backward(0)
+        runs = {n: backward(n) for n in (2, 3, 4)}
+    finally:
+        _lib.tune_set("attn_bwd.keep_ds", -1)
+        _lib.tune_set("attn_bwd.split", -1)
+    for n, grads in runs.items():
+        for name, a, b in zip(("dQ", "dK", "dV"), grads, whole):
+            assert bool(torch.isfinite(a).all()), (n, name)
+            if name == "dQ" and not p:
+                assert torch.equal(a, b), (n, name)
+                continue
+            # sums that differ by fp32 rounding, each rounded to the operand type: now and then to its neighbour
+            a, b = a.double(), b.double()
+            assert (a - b).norm().item() <= (1e-3 if dtype == torch.bfloat16 else 1.5e-4) * b.norm().item(), (n, name)
