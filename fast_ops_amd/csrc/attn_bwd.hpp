@@ -19,7 +19,7 @@ constexpr int kPartBytes = 2 * kBwdRows * 128 * 4;     // dK and dV of a block i
 struct AttnBwdParams {
   const void *q, *k, *v, *o, *d_o;
   const float* lse;
-  float* delta;       // [B, H, Sq]: -rowsum(dO O) (1 - dropout_p), written by the dQ kernel
+  float* delta;       // [B, H, Sq]: -rowsum(dO O) (1 - dropout_p), written by the dQ kernel (dS kept: by attn_bwd_rows_kernel)
   char* ds;           // not null: where the dK/dV kernel leaves dS for the dQ kernel (see ds_chunk)
   float* nlse;        // [B, H, Sq]: -LSE / softmax_scale (with dropout: of an LSE lower by log(1 / (1 - p))), written by the dQ kernel beside delta
   void *dq, *dk, *dv;

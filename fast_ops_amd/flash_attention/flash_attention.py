@@ -296,7 +296,7 @@ def attn_bwd_strided(
     q: Tensor, k: Tensor, v: Tensor, o: Tensor, lse: Tensor, d_o: Tensor, dims: Tuple[int, int, int, int], causal: bool,
     softmax_scale: Optional[float], dropout: Optional[Dropout] = None, bias: Optional[Tensor] = None,
 ) -> Tuple[Tensor, Tensor, Tensor]:
-    """Launches fo_attn_bwd. Returns (dQ, dK, dV) with the shapes and dtypes of q, k, v (dense; a K/V whose heads are
+    """Launches fo_attn_bwd_ws. Returns (dQ, dK, dV) with the shapes and dtypes of q, k, v (dense; a K/V whose heads are
     an expanded view gets a full-size gradient, which autograd then reduces)."""
     if d_o.dtype != q.dtype or d_o.shape != q.shape:
         _check_inputs(q, k, v)
