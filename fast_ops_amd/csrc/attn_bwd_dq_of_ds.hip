@@ -49,14 +49,15 @@ __global__ void __launch_bounds__(256) attn_bwd_rows_kernel(const AttnBwdParams 
 
 // dK and dV of a key block whose query tiles several workgroups of the dK/dV kernel shared: their sums added, in order, in the lanes that
 // held them. By the last workgroups of the dQ launch, beside its others (they have what the launch before left, as those do).
-template <typename T, int LIVE>
+template <typename T, int LIVE, int TEAMS>
 __device__ __forceinline__ void merge_dkdv(const AttnBwdParams& prm, int at, FO_LDS char* smem) {
   const int n_bh = prm.B * prm.H, m = at / n_bh, bh = at - m * n_bh, b = bh / prm.H, h = bh - b * prm.H;
-  const int wave_s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave_s = wave_all % kBwdWaves, lane = threadIdx.x & 63;
+  FO_LDS char* stage = smem + wave_all * stage_bytes(kD);
   const uint32_t w = prm.merges[m];
   const int k0w = (int)(w & 255u) * kBwdRows + wave_s * 32, pieces = (w >> 12) & 15;
 #pragma unroll 1
-  for (int mat = 0; mat < 2; ++mat) {
+  for (int mat = wave_all / kBwdWaves; mat < 2; mat += TEAMS) {
     f32x16 acc[LIVE / 32];
 #pragma unroll
     for (int i = 0; i < LIVE / 32; ++i)
@@ -71,31 +72,32 @@ __device__ __forceinline__ void merge_dkdv(const AttnBwdParams& prm, int at, FO_
         for (int u = 0; u < 4; ++u) acc[g >> 2][4 * (g & 3) + u] += v[u];
       }
     }
-    if (mat == 0) store_rows_via_lds<T, LIVE>(acc, prm.scale, smem + wave_s * stage_bytes(kD), (T*)prm.dk + b * prm.dks[0] + h * prm.dks[1], prm.dks[2], k0w, prm.Sk, prm.d, lane);
-    else store_rows_via_lds<T, LIVE>(acc, 1.0f, smem + wave_s * stage_bytes(kD), (T*)prm.dv + b * prm.dvs[0] + h * prm.dvs[1], prm.dvs[2], k0w, prm.Sk, prm.d, lane);
+    if (mat == 0) store_rows_via_lds<T, LIVE>(acc, prm.scale, stage, (T*)prm.dk + b * prm.dks[0] + h * prm.dks[1], prm.dks[2], k0w, prm.Sk, prm.d, lane);
+    else store_rows_via_lds<T, LIVE>(acc, 1.0f, stage, (T*)prm.dv + b * prm.dvs[0] + h * prm.dvs[1], prm.dvs[2], k0w, prm.Sk, prm.d, lane);
   }
 }
 
 // dQ^T = K^T dS^T: a wave owns 32 query rows and walks 32-key tiles of K (shared by the workgroup's four waves) and dS
 // (its own) through a ring of four LDS buffers, one barrier per tile; both operands by transposing reads. Bound by reading dS where there
-// are workgroups enough, else by a workgroup's chain per tile (0.4 us: 12 heads x 3072 causal 40 us; with reads, conditions and products in
+// are workgroups enough, else by a workgroup's chain per tile (0.4 us, the unit's LDS: 12 heads x 3072 causal 40 us; with reads, conditions and products in
 // the order they come to mind 48). 12 heads x 4096 (0.4 GB of dS) 98 us = 4.1 TB/s of dS: the dQ kernel that computes the scores again takes
 // 172; copied without nt, dS pushes K out of the cache: 131. Five or eight buffers, or 64 rows per wave, gain nothing (131, 131 / 108-170).
+// TEAMS 2: eight waves, the second four with the odd tiles and a ring of their own; the two teams' sums are added at the end (see launch_form).
 // TBIAS: P of a row whose bias is large as a whole is off by the rounding of -LSE / scale, one factor per row, made good here.
-template <typename T, bool CAUSAL, int LIVE, bool PAD, bool TBIAS, int SLOTS>
-__global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_of_ds_kernel(const AttnBwdParams prm) {
+template <typename T, bool CAUSAL, int LIVE, bool PAD, bool TBIAS, int SLOTS, int TEAMS>
+__global__ void __launch_bounds__(TEAMS * kBwdWaves * 64, 2) attn_bwd_dq_of_ds_kernel(const AttnBwdParams prm) {
   typedef typename Ops<T>::vec8 vec8;
   constexpr int D = kD, TILE = 32, ROW_BYTES = D * 2, CHUNKS = ROW_BYTES / 16, ROWS_PER_DMA = 1024 / ROW_BYTES;
   constexpr int K_BYTES = TILE * ROW_BYTES, DS_BYTES = 2048, SLOT = K_BYTES + kBwdWaves * DS_BYTES;
   constexpr int NK = K_BYTES / 1024 / kBwdWaves, ND = DS_BYTES / 1024, NI = NK + ND;
   constexpr int DBLK = LIVE / 32;
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
-  FO_LDS char* smem = (FO_LDS char*)smem_raw;      // slots: K tile | dS of each wave
-  const int wave_s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), team = wave_all / kBwdWaves, wave_s = wave_all % kBwdWaves;
+  FO_LDS char* smem = (FO_LDS char*)smem_raw + team * SLOTS * SLOT;      // the team's slots: K tile | dS of each wave
   const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5, L16 = lane & 15, g16 = (lane >> 4) & 1;
   const int Sq = prm.Sq, Sk = prm.Sk, n_qblk = (Sq + kBwdRows - 1) / kBwdRows, n_qt = (int)ds_query_tiles(Sq);
   const int n_dq = prm.B * prm.H * n_qblk;
-  if ((int)blockIdx.x >= n_dq) return merge_dkdv<T, LIVE>(prm, (int)blockIdx.x - n_dq, smem);
+  if ((int)blockIdx.x >= n_dq) return merge_dkdv<T, LIVE, TEAMS>(prm, (int)blockIdx.x - n_dq, (FO_LDS char*)smem_raw);
   int bh, qblk;
   bwd_item(prm, n_qblk, bh, qblk);
   qblk = n_qblk - 1 - qblk;                        // heaviest causal blocks first
@@ -141,7 +143,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_of_ds_kernel(co
     for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
 #pragma unroll
   for (int i = 0; i < SLOTS - 1; ++i)
-    if (i < n_tiles) issue(i, i, std::false_type{});
+    if (TEAMS * i + team < n_tiles) issue(TEAMS * i + team, i, std::false_type{});
 
   // Byte offsets of the fragment reads inside a slot (K as col_frag computes them; dS: keys r and r + 8 of a 16-key step, four
   // queries' worth of 8 bytes). A 16-key step further is an immediate.
@@ -179,26 +181,51 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_of_ds_kernel(co
       for (int db = 0; db < DBLK; ++db) acc[db] = Ops<T>::mfma(kv[t][db], dsv[t], acc[db]);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (every read is back before the next barrier)
   };
-  int slot_i = 0, tile = 0;
-  // Tile `tile` has landed when all but the copies of the SLOTS - 2 tiles after it have; behind the barrier that holds for everyone,
-  // and nobody reads the tile before it any more, whose slot takes tile + SLOTS - 1.
+  int slot_i = 0, it = 0;                               // the team's tiles are TEAMS it + team; every wave meets the same barriers
+  const int n_it = (n_tiles + TEAMS - 1) / TEAMS;
+  // Its tile `it` has landed when all but the copies of the SLOTS - 2 tiles after it have; behind the barrier that holds for everyone,
+  // and nobody reads the tile before it any more, whose slot takes the tile SLOTS - 1 further on.
   // (one straight loop for the tiles that copy a whole one ahead; causal: they count for every wave, whose last tiles differ by two)
   static_assert(SLOTS > 2, "");
   if (!PAD && k_off_ok)
-    for (const int end = min(n_tiles, Sk / TILE) - (SLOTS - 1); tile < end; ++tile, slot_i = slot_i == SLOTS - 1 ? 0 : slot_i + 1) {
+    for (const int end = min(n_tiles, Sk / TILE) / TEAMS - (SLOTS - 1); it < end; ++it, slot_i = slot_i == SLOTS - 1 ? 0 : slot_i + 1) {
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SLOTS - 2) * NI) : "memory");
       __builtin_amdgcn_s_barrier();
-      issue(tile + SLOTS - 1, slot_i == 0 ? SLOTS - 1 : slot_i - 1, std::true_type{});
-      products(tile, slot_i, std::false_type{});
+      issue(TEAMS * (it + SLOTS - 1) + team, slot_i == 0 ? SLOTS - 1 : slot_i - 1, std::true_type{});
+      products(TEAMS * it + team, slot_i, std::false_type{});
     }
-  for (; tile < n_tiles; ++tile, slot_i = slot_i == SLOTS - 1 ? 0 : slot_i + 1) {
-    if (tile + SLOTS - 2 < n_tiles) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SLOTS - 2) * NI) : "memory");
+  for (; it < n_it; ++it, slot_i = slot_i == SLOTS - 1 ? 0 : slot_i + 1) {
+    const int tile = TEAMS * it + team;
+    if (tile + TEAMS * (SLOTS - 2) < n_tiles) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SLOTS - 2) * NI) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
-    if (tile + SLOTS - 1 < n_tiles) issue(tile + SLOTS - 1, slot_i == 0 ? SLOTS - 1 : slot_i - 1, std::false_type{});
-    if (CAUSAL && tile >= my_tiles) continue;
+    if (tile + TEAMS * (SLOTS - 1) < n_tiles) issue(tile + TEAMS * (SLOTS - 1), slot_i == 0 ? SLOTS - 1 : slot_i - 1, std::false_type{});
+    if ((CAUSAL || TEAMS > 1) && tile >= my_tiles) continue;
     if (tile * TILE + TILE > Sk) products(tile, slot_i, std::true_type{});
     else products(tile, slot_i, std::false_type{});
+  }
+  if constexpr (TEAMS > 1) {
+    // the second team's sums, through its slots (which its waves are past), added by the first
+    static_assert(TEAMS == 2 && kBwdWaves * DBLK * 4096 <= SLOTS * SLOT, "");
+    FO_LDS char* sums = (FO_LDS char*)smem_raw + SLOTS * SLOT + wave_s * (DBLK * 4096) + lane * 16;
+    __syncthreads();
+    if (team == 1) {
+#pragma unroll
+      for (int g = 0; g < 4 * DBLK; ++g) {
+        f32x4 v;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = acc[g >> 2][4 * (g & 3) + u];
+        *(FO_LDS f32x4*)(sums + g * 1024) = v;
+      }
+    }
+    __syncthreads();
+    if (team == 1) return;
+#pragma unroll
+    for (int g = 0; g < 4 * DBLK; ++g) {
+      const f32x4 v = *(FO_LDS const f32x4*)(sums + g * 1024);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[g >> 2][4 * (g & 3) + u] += v[u];
+    }
   }
   // column l32 of the result is position l32 of the block (see attn_bwd.hpp)
   const int qi = block32 * 32 + 16 * (l32 >> 4) + (l32 & 3) + 8 * ((l32 >> 2) & 1) + 4 * ((l32 >> 3) & 1);
@@ -230,19 +257,31 @@ int launch_bwd_rows(const AttnBwdParams& p, bool drop, bool tile_bias, hipStream
   return launch_status();
 }
 
-template <typename T, bool CAUSAL, int LIVE, bool PAD, bool TBIAS, int SLOTS>
+template <typename T, bool CAUSAL, int LIVE, bool PAD, bool TBIAS, int SLOTS, int TEAMS>
 static int launch_one(const AttnBwdParams& p, hipStream_t s) {
-  constexpr int lds = SLOTS * (32 * kD * 2 + kBwdWaves * 2048);
-  static const hipError_t a = hipFuncSetAttribute((const void*)attn_bwd_dq_of_ds_kernel<T, CAUSAL, LIVE, PAD, TBIAS, SLOTS>,
+  constexpr int lds = TEAMS * SLOTS * (32 * kD * 2 + kBwdWaves * 2048);
+  static const hipError_t a = hipFuncSetAttribute((const void*)attn_bwd_dq_of_ds_kernel<T, CAUSAL, LIVE, PAD, TBIAS, SLOTS, TEAMS>,
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (a != hipSuccess) return FO_ERR_LAUNCH;
   const unsigned grid = (unsigned)((int64_t)p.B * p.H * ((p.Sq + kBwdRows - 1) / kBwdRows + p.n_merges));
-  attn_bwd_dq_of_ds_kernel<T, CAUSAL, LIVE, PAD, TBIAS, SLOTS><<<grid, kBwdWaves * 64, lds, s>>>(p);
+  attn_bwd_dq_of_ds_kernel<T, CAUSAL, LIVE, PAD, TBIAS, SLOTS, TEAMS><<<grid, TEAMS * kBwdWaves * 64, lds, s>>>(p);
   return launch_status();
 }
+// Two teams: the chain of tiles is half as long and a workgroup has its unit to itself, as two of one team would have it together. It
+// gains where units would hold two and others one, or causal ones of unequal length, for a good while: this kernel, one team -> two, us,
+//   causal: 12 x 3072 with a bias 47.1 -> 41.6, 12 x 4096 61.3 -> 50.8, 16 x 4096 74.0 -> 58.5, 4 x 8192 94.0 -> 83.8, 32 x 1800 36.1 -> 31.9,
+//     12 x 6144 105 -> 98, 12 x 8192 (768 blocks) 171 -> 166; not: 32 x 4096 (1024) 122 -> 131, 64 x 1024 24.8 -> 26.1, 16 x 2048 (256) 25.1 -> 25.8
+//   not causal: 12 x 3072 (288 blocks) 76.4 -> 68.7; not: 12 x 4096 (384) 90.4 -> 91.6, 24 x 2304 (432) 57.5 -> 60.1, 64 x 2048 110 -> 126
+// At other head dims a lone workgroup is slowed by the addresses of its lanes, not by the unit's LDS: 8 x 500 x 1600 at 104 31.1 -> 20.8,
+// 32 x 777 x 2000 at 80 (224 blocks) 34.6 -> 25.2; not: 64 x 777 x 1250 (448) 30.3 -> 34.4.
 template <typename T, bool CAUSAL, int LIVE, bool PAD, bool TBIAS>
 static int launch_form(const AttnBwdParams& p, hipStream_t s) {
-  return launch_one<T, CAUSAL, LIVE, PAD, TBIAS, 4>(p, s);
+  constexpr int kUnits = 256, kTwoTeamsFromKeys = 1536;
+  const int64_t n_bh = (int64_t)p.B * p.H, blocks = n_bh * ((p.Sq + kBwdRows - 1) / kBwdRows);
+  bool two = PAD && blocks <= kUnits;
+  if (!PAD && p.Sk >= kTwoTeamsFromKeys)
+    two = CAUSAL ? blocks + n_bh * p.n_merges > kUnits && blocks <= 3 * kUnits : blocks > kUnits && blocks <= kUnits + kUnits / 4;
+  return two ? launch_one<T, CAUSAL, LIVE, PAD, TBIAS, 4, 2>(p, s) : launch_one<T, CAUSAL, LIVE, PAD, TBIAS, 4, 1>(p, s);
 }
 template <typename T>
 int launch_dq_of_ds(const AttnBwdParams& p, bool causal, bool tile_bias, hipStream_t s) {
