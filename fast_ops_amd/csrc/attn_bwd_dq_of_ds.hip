@@ -114,13 +114,16 @@ __global__ void __launch_bounds__(TEAMS * kBwdWaves * 64, 2) attn_bwd_dq_of_ds_k
 #pragma unroll
   for (int i = 0; i < NK; ++i) {
     const int row = (wave_s * NK + i) * ROWS_PER_DMA + lane / CHUNKS;
-    k_off[i] = (uint32_t)(row * (int)prm.ks[2] + ((lane % CHUNKS) ^ swz<D>(row)) * 8) * 2u;
+    // (a column past the head_dim re-reads the last 8: a column of K makes that column of dQ alone, which is not stored. So other head dims take
+    // the straight loop too: 8 x 500 x 1600 at 104 30.1 -> 17.7 us, 64 x 1500 x 3000 at 96 129 -> 112)
+    const int col = ((lane % CHUNKS) ^ swz<D>(row)) * 8;
+    k_off[i] = (uint32_t)(row * (int)prm.ks[2] + (PAD ? min(col, prm.d - 8) : col)) * 2u;
   }
   const bool k_off_ok = prm.ks[2] < (1 << 23);
   const uint32_t lane16 = (uint32_t)lane * 16u;
   auto issue = [&](int tile, int slot_i, auto inside) {
     FO_LDS char* slot = smem + slot_i * SLOT;
-    if (decltype(inside)::value || (!PAD && k_off_ok && tile * TILE + TILE <= Sk)) {
+    if (decltype(inside)::value || (k_off_ok && tile * TILE + TILE <= Sk)) {
       const char* src = (const char*)(kbase + (int64_t)(tile * TILE) * prm.ks[2]);
 #pragma unroll
       for (int i = 0; i < NK; ++i) dma16_uniform_base(src, k_off[i], slot + (wave_s * NK + i) * 1024);
@@ -187,7 +190,7 @@ __global__ void __launch_bounds__(TEAMS * kBwdWaves * 64, 2) attn_bwd_dq_of_ds_k
   // and nobody reads the tile before it any more, whose slot takes the tile SLOTS - 1 further on.
   // (one straight loop for the tiles that copy a whole one ahead; causal: they count for every wave, whose last tiles differ by two)
   static_assert(SLOTS > 2, "");
-  if (!PAD && k_off_ok)
+  if (k_off_ok)
     for (const int end = min(n_tiles, Sk / TILE) / TEAMS - (SLOTS - 1); it < end; ++it, slot_i = slot_i == SLOTS - 1 ? 0 : slot_i + 1) {
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SLOTS - 2) * NI) : "memory");
       __builtin_amdgcn_s_barrier();
@@ -272,15 +275,13 @@ static int launch_one(const AttnBwdParams& p, hipStream_t s) {
 //   causal: 12 x 3072 with a bias 47.1 -> 41.6, 12 x 4096 61.3 -> 50.8, 16 x 4096 74.0 -> 58.5, 4 x 8192 94.0 -> 83.8, 32 x 1800 36.1 -> 31.9,
 //     12 x 6144 105 -> 98, 12 x 8192 (768 blocks) 171 -> 166; not: 32 x 4096 (1024) 122 -> 131, 64 x 1024 24.8 -> 26.1, 16 x 2048 (256) 25.1 -> 25.8
 //   not causal: 12 x 3072 (288 blocks) 76.4 -> 68.7; not: 12 x 4096 (384) 90.4 -> 91.6, 24 x 2304 (432) 57.5 -> 60.1, 64 x 2048 110 -> 126
-// At other head dims a lone workgroup is slowed by the addresses of its lanes, not by the unit's LDS: 8 x 500 x 1600 at 104 31.1 -> 20.8,
-// 32 x 777 x 2000 at 80 (224 blocks) 34.6 -> 25.2; not: 64 x 777 x 1250 (448) 30.3 -> 34.4.
+// and at other head dims the same: 24 x 2000 causal at 112 34.0 -> 26.8, 12 x 3000 causal 41.1 -> 37.8; not: 64 x 777 x 1250 at 80 (448) 30.5 -> 35.0,
+// 24 x 1500 at 112 (288) 40.2 -> 40.7, 16 x 2000 at 96 (256) 25.2 -> 26.0.
 template <typename T, bool CAUSAL, int LIVE, bool PAD, bool TBIAS>
 static int launch_form(const AttnBwdParams& p, hipStream_t s) {
   constexpr int kUnits = 256, kTwoTeamsFromKeys = 1536;
   const int64_t n_bh = (int64_t)p.B * p.H, blocks = n_bh * ((p.Sq + kBwdRows - 1) / kBwdRows);
-  bool two = PAD && blocks <= kUnits;
-  if (!PAD && p.Sk >= kTwoTeamsFromKeys)
-    two = CAUSAL ? blocks + n_bh * p.n_merges > kUnits && blocks <= 3 * kUnits : blocks > kUnits && blocks <= kUnits + kUnits / 4;
+  const bool two = p.Sk >= kTwoTeamsFromKeys && (CAUSAL ? blocks + n_bh * p.n_merges > kUnits && blocks <= 3 * kUnits : blocks > kUnits && blocks <= kUnits + kUnits / 4);
   return two ? launch_one<T, CAUSAL, LIVE, PAD, TBIAS, 4, 2>(p, s) : launch_one<T, CAUSAL, LIVE, PAD, TBIAS, 4, 1>(p, s);
 }
 template <typename T>

@@ -1,6 +1,6 @@
 """dQ from stored dS where two teams of waves share a workgroup's keys (even and odd 32-key tiles, sums added at the end): launches of the
-sizes that form is chosen at (head_dim 128: 257 to 320 blocks, causal up to 768, from 1536 keys; other head dims: up to 256 blocks), odd and even
-numbers of tiles, ragged last tiles, fewer tiles than the rings hold. Against the path that computes the scores once more."""
+sizes that form is chosen at (257 to 320 blocks, causal up to 768, from 1536 keys), odd and even numbers of tiles, ragged last tiles, fewer
+tiles than the rings hold (causal, the first blocks), and head dims off 128 in either form. Against the path that computes the scores once more."""
 import pytest
 import torch
 
@@ -15,6 +15,7 @@ CASES = [
     (144, 129, 1536, 128, False, False), (144, 256, 1537, 128, False, False), (260, 1, 1567, 128, False, False), (144, 200, 1600, 128, False, True),
     (144, 200, 1537, 128, True, False), (260, 64, 1569, 128, True, False), (24, 1700, 1536, 128, True, False), (20, 1665, 1665, 128, True, True),
     (2, 150, 20, 72, False, False), (3, 150, 33, 80, False, False), (2, 300, 95, 104, True, False), (2, 130, 1249, 112, False, False), (4, 513, 257, 96, True, False),
+    (144, 200, 1569, 72, False, False), (24, 1700, 1537, 104, True, False), (144, 256, 1600, 96, False, False), (20, 1665, 1665, 80, True, False),
 ]
 
 
