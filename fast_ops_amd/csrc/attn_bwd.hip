@@ -1726,7 +1726,8 @@ static int64_t ds_bytes_of(int B, int H, int Sq, int Sk) { return (int64_t)B * H
 //   2 x 4 x 4096 217 -> 159; so from 1536 keys whatever the size
 //   fewer keys: with the rows' kernel and a third launch it takes 96 MiB of dS to gain: 192 heads x 512 125 -> 115, 64 x 1024 125 -> 114,
 //   64 x 768 not causal 90 -> 89, 16 x 1024 72 -> 76, 4 heads x 128 70 -> 73 (these wait for their host);
-//   twice that up to head_dim 96, whose scores cost 3/4: 64 heads x 777 x 1250 at 80 (128 MiB), forward and backward 148.8 -> 147.7
+//   half as much again up to head_dim 96, whose scores cost 3/4, forward and backward: 96 heads x 700 x 1100 at 72 (149 MiB) 146 -> 139, 48 x 1450 x
+//   1100 at 96 (155) 144 -> 133, 128 x 600 x 900 at 80 (160) 137 -> 132; 64 x 777 x 1250 at 80 (130) 113.2 -> 113.3, 64 x 1024 at 96 causal (128) 86 -> 88
 //   up to 2 GiB, what a caller's memory is asked for; beyond, the gain shrinks with the traffic that no cache holds: 12 x 8192
 //   causal (1.6 GiB) 639 -> 594, 64 x 4096 causal (2 GiB) 877 -> 846, 512 x 2048 (4 GiB) 3402 -> 3392.
 constexpr int64_t kDsFromBytes = 96ll << 20, kDsMaxBytes = 2ll << 30;
@@ -1735,7 +1736,7 @@ static bool bwd_keeps_ds(int B, int H, int Sq, int Sk, int D) {
   const int asked = tune(g_attn_bwd_keep_ds);
   if (asked == 0 || D <= 64 || (int64_t)B * H > (1 << 20) || ds_key_blocks(Sk) * ds_query_tiles(Sq) > kDsMaxBytes / kDsChunk) return false;
   const int64_t bytes = ds_bytes_of(B, H, Sq, Sk);
-  return bytes <= kDsMaxBytes && (asked == 1 || Sk >= kDsFromKeys || bytes >= (D > 96 ? kDsFromBytes : 2 * kDsFromBytes));
+  return bytes <= kDsMaxBytes && (asked == 1 || Sk >= kDsFromKeys || bytes >= (D > 96 ? kDsFromBytes : kDsFromBytes + kDsFromBytes / 2));
 }
 
 // Which key blocks' query tiles several workgroups share (attn_bwd.hpp). A workgroup of the dK/dV kernel has a compute unit to itself,
