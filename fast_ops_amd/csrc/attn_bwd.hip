@@ -72,6 +72,28 @@ __device__ __forceinline__ void mfma_scores_vgpr(f32x16& acc, typename Ops<T>::v
   acc = Ops<T>::mfma(a, b, acc);
 #endif
 }
+// the first of a chain, started from zero or from registers that stay as they are
+template <typename T>
+__device__ __forceinline__ void mfma_scores_vgpr_first(f32x16& acc, typename Ops<T>::vec8 a, typename Ops<T>::vec8 b, const f32x16& start) {
+#if defined(__HIP_DEVICE_COMPILE__) && !FO_MFMA_NOPS
+  if constexpr (std::is_same<T, __bf16>::value) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "v"(b), "v"(start));
+  else asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "v"(b), "v"(start));
+#else
+  acc = Ops<T>::mfma(a, b, start);
+#endif
+}
+template <typename T>
+__device__ __forceinline__ void mfma_scores_vgpr_first(f32x16& acc, typename Ops<T>::vec8 a, typename Ops<T>::vec8 b) {
+#if defined(__HIP_DEVICE_COMPILE__) && !FO_MFMA_NOPS
+  if constexpr (std::is_same<T, __bf16>::value) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
+  else asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
+#else
+  f32x16 zero;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) zero[r] = 0.0f;
+  acc = Ops<T>::mfma(a, b, zero);
+#endif
+}
 template <int N>
 __device__ __forceinline__ void acc_fence(f32x16 (&acc)[N]) {
 #if defined(__HIP_DEVICE_COMPILE__) && !FO_MFMA_NOPS
@@ -871,10 +893,16 @@ static_assert(softmax_grad_jobs_fit(16) && softmax_grad_jobs_fit(12) && softmax_
 // for all but the last four of the wave's memory operations, which complete in order. The stores carry nt: nothing of this kernel
 // reads them, and they would push Q and dO out of the cache (12 heads x 4096 not causal: 204 us without DS, 230 with plain stores, 217
 // with nt; 64 heads x 2048 causal 143, 166, 155).
+// SHIFT (DS without TBIAS): dQ is made of this kernel's P then, and P has to be as exact as the dQ kernel's own. So S starts from zero (KBIAS: from
+// bias / scale, sixteen registers that stay as they are), and -LSE log2 e, read from LDS where -LSE / scale is otherwise, joins in the exponent:
+// P = exp2(S c + shift), a fused multiply-add in the place of the multiplication. Started from -LSE / scale, S is summed at the ulp of the LSE: fp32
+// error of P at 4096 unit normal keys 7.4e-7 rms instead of 3.0e-7. (This kernel alone, start values -> shift: 12 heads x 4096 with key bias and
+// dropout 287 -> 280 us, without 235 -> 234, 12 x 3072 causal 73 -> 74, 48 x 1450 x 1100 at head_dim 96 83 -> 84.)
 template <typename T, int D, bool CAUSAL, bool KBIAS = false, bool DROP = false, bool PAD = false, int LIVE = D, int TBIAS = 0, bool DS = false>
 __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(const AttnBwdParams prm) {
   static_assert(TBIAS == 0 || !(KBIAS || DROP || PAD), "not combined");
   static_assert(!(PAD && (DROP || KBIAS)), "the second visit of dropout's rows copies whole rows");
+  constexpr bool SHIFT = DS && TBIAS == 0;
   typedef typename Ops<T>::vec8 vec8;
   constexpr int TILE_BYTES = kBwdTile * D * 2;
   constexpr int KSTEPS = LIVE / 16;
@@ -1034,7 +1062,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   const int key = k0w + l32;
   float bias_lane = 0.0f;
   if constexpr (KBIAS) {
-    bias_lane = load_bias<T>(prm.bias, b * prm.bias.strides[0] + h * prm.bias.strides[1] + min(key, Sk - 1)) * kLog2e;
+    bias_lane = load_bias<T>(prm.bias, b * prm.bias.strides[0] + h * prm.bias.strides[1] + min(key, Sk - 1)) * (SHIFT ? kLog2e / prm.scale_log2e : kLog2e);
     asm volatile("" : "+v"(bias_lane));      // (waited for here, not inside the loops, where copies are in flight)
   }
   f32x16 dkacc[DBLK], dvacc[DBLK];
@@ -1079,6 +1107,15 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
   static_assert((4 * NMF) % kFragAhead == 0, "the fragment ring runs on across tiles");
   vec8 fr[kFragAhead];         // A operands, fetched kFragAhead micro-groups ahead of their MFMA
   f32x16 sacc[2], dpacc[2];
+  [[maybe_unused]] f32x16 shift[2];       // SHIFT: what the exponent of the rows of a block starts from
+  [[maybe_unused]] f32x16 bias_start;     // ... and the key's bias / softmax_scale, from which S does, in every register (as in the dQ kernel)
+  if constexpr (SHIFT && KBIAS) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) bias_start[r] = bias_lane;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(bias_start));   // (sixteen registers, not one)
+#endif
+  }
   // P and dS as B operands: pairs of 16-bit values, kept as 32-bit words so that a finished pair can be pinned
   typedef __attribute__((ext_vector_type(4))) int i32x4;
   typedef __attribute__((ext_vector_type(2))) T vec2;
@@ -1218,7 +1255,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
 #if defined(__HIP_DEVICE_COMPILE__)
       if constexpr (AGAIN) asm volatile("" : "+v"(sv));      // (read here, not earlier: see the wait states at the end of tile_body)
 #endif
-      pv[qb][r] = dead ? 0.0f : __builtin_amdgcn_exp2f(KBIAS ? __builtin_fmaf(sv, c, bias_lane) : sv * c);
+      pv[qb][r] = dead ? 0.0f : __builtin_amdgcn_exp2f(SHIFT ? __builtin_fmaf(sv, c, shift[qb][r]) : KBIAS ? __builtin_fmaf(sv, c, bias_lane) : sv * c);
     };
     auto stage_b = [&](int qb, int r) {          // elements r and r + 1
       const float ds0 = pv[qb][r] * dpacc[qb][r], ds1 = pv[qb][r + 1] * dpacc[qb][r + 1];
@@ -1266,7 +1303,9 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       // whose paths join here, and where the last B job of the tile ends right before its first reader)
       if (AGAIN || g == 3 * NMF || g == 3 * NMF + HALF) asm volatile("s_nop 1");
       if (ph < 2) {
-        if (i < KSTEPS) mfma_scores_vgpr<T>(sacc[ph], fr[g % kFragAhead], kf[i]);
+        if (SHIFT && KBIAS && i == 0) mfma_scores_vgpr_first<T>(sacc[ph], fr[g % kFragAhead], kf[i], bias_start);
+        else if (SHIFT && i == 0) mfma_scores_vgpr_first<T>(sacc[ph], fr[g % kFragAhead], kf[i]);
+        else if (i < KSTEPS) mfma_scores_vgpr<T>(sacc[ph], fr[g % kFragAhead], kf[i]);
         else mfma_scores_vgpr<T>(dpacc[ph], fr[g % kFragAhead], vf[i - KSTEPS]);
       } else {
         const int t = i / (2 * DBLK), db = (i >> 1) % DBLK;
@@ -1293,9 +1332,9 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
         if constexpr (AGAIN) zero_acc(dpacc[1]);
         else start_acc(dpacc[1], rowvals + (NBUF + buf) * kBwdTile, 1);
       }
-      if (g == 1) start_acc(sacc[1], rowvals + buf * kBwdTile, 1);
+      if (g == 1) start_acc(SHIFT ? shift[1] : sacc[1], rowvals + buf * kBwdTile, 1);
       if (g == 3 * NMF) start_acc(dpacc[0], rowvals + (NBUF + nbuf) * kBwdTile, 0);
-      if (g == 3 * NMF + 1) start_acc(sacc[0], rowvals + nbuf * kBwdTile, 0);
+      if (g == 3 * NMF + 1) start_acc(SHIFT ? shift[0] : sacc[0], rowvals + nbuf * kBwdTile, 0);
       if constexpr (TBIAS != 0) {
         // (block 1: from group 2 to two groups before its first MFMA; block 0 of the next tile: in the last half-phase but
         // for its last group - the groups without, or with the least, softmax-gradient arithmetic)
@@ -1389,7 +1428,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       for (int u = 0; u < 4; ++u) dpacc[0][4 * jv + u] = d4[u];
       const f32x4 n4 = *(FO_LDS const f32x4*)(rowvals + buf * kBwdTile + 8 * jv + 4 * hh);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) sacc[0][4 * jv + u] = n4[u];
+      for (int u = 0; u < 4; ++u) (SHIFT ? shift[0] : sacc[0])[4 * jv + u] = n4[u];
     }
     if constexpr (TBIAS != 0) {
       bias_read(ja, 0);

@@ -21,7 +21,8 @@ struct AttnBwdParams {
   const float* lse;
   float* delta;       // [B, H, Sq]: -rowsum(dO O) (1 - dropout_p), written by the dQ kernel (dS kept: by attn_bwd_rows_kernel)
   char* ds;           // not null: where the dK/dV kernel leaves dS for the dQ kernel (see ds_chunk)
-  float* nlse;        // [B, H, Sq]: -LSE / softmax_scale (with dropout: of an LSE lower by log(1 / (1 - p))), written by the dQ kernel beside delta
+  float* nlse;        // [B, H, Sq], written with delta: -LSE / softmax_scale (with dropout: of an LSE lower by log(1 / (1 - p))); dS kept, but for a bias
+                      // with a query stride: -LSE log2 e of the same LSE
   void *dq, *dk, *dv;
   int B, H, Sq, Sk;
   int d;                // true head_dim: a multiple of 8, at most the D the kernels are compiled for
@@ -59,7 +60,7 @@ constexpr float kLog2e = 1.4426950408889634f;
 // dQ from stored dS, where that has room (ds_bytes_of): the dK/dV kernel runs first and leaves dS, rounded to the operand
 // type for its own dK = dS^T Q, in memory, and dQ is one product of it with K. That saves computing S, dP and the exponential a second
 // time - two of the backward's seven products - for 2 bytes written and read per (query, key) pair, which the memory-side cache
-// holds for most of the sizes this is chosen at. -LSE / scale and -delta then come from a kernel of their own.
+// holds for most of the sizes this is chosen at. The rows' LSE and delta then come from a kernel of their own.
 //
 // dS lies in chunks of 64 queries x 32 keys (4 KiB): block qb of 32 queries x group t of 16 queries, 1 KiB each; inside one, a key's 16
 // queries are 32 bytes, in the order in which the dK/dV kernel's lanes hold them: position 8 hh + u is query (u & 3) + 8 (u >> 2) + 4 hh

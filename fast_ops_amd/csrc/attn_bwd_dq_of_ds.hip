@@ -14,8 +14,8 @@ __device__ __forceinline__ void dma16_uniform_base_nt(const void* base, uint32_t
 
 constexpr int kD = 128;      // columns the kernels are laid out for
 
-// -delta and -LSE / scale of every query row, for the dK/dV kernel where the dQ kernel runs after it (which otherwise computes
-// both): delta_i = sum_d dO_id O_id (flash_attention_triton.py:273-315). 16 lanes per row, 16 bytes each of O and dO.
+// -delta and the value of the LSE (AttnBwdParams::nlse) of every query row, for the dK/dV kernel where the dQ kernel runs after it (which
+// otherwise computes both): delta_i = sum_d dO_id O_id (flash_attention_triton.py:273-315). 16 lanes per row, 16 bytes each of O and dO.
 constexpr int kRowsPerWg = 64;
 template <typename T, bool DROP, bool TBIAS>
 __global__ void __launch_bounds__(256) attn_bwd_rows_kernel(const AttnBwdParams prm) {
@@ -43,7 +43,7 @@ __global__ void __launch_bounds__(256) attn_bwd_rows_kernel(const AttnBwdParams 
     const int64_t at = (int64_t)bh * prm.Sq + row + 16 * i;
     const float lse = prm.lse[at];
     prm.delta[at] = DROP ? delta * prm.drop.keep_prob : delta;      // (the factors: see the dQ kernel of attn_bwd.hip)
-    prm.nlse[at] = TBIAS ? -lse * (kLog2e / prm.scale_log2e) : (lse * kLog2e - (DROP ? prm.drop.keep_log2 : 0.0f)) * prm.neg_inv_scale_log2e;
+    prm.nlse[at] = TBIAS ? -lse * (kLog2e / prm.scale_log2e) : -(lse * kLog2e - (DROP ? prm.drop.keep_log2 : 0.0f));
   }
 }
 
