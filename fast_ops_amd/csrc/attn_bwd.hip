@@ -878,7 +878,7 @@ static_assert(softmax_grad_jobs_fit(16) && softmax_grad_jobs_fit(12) && softmax_
 // whole (dropout_run) in the first groups of a tile, which carry no other arithmetic. A row that is neither (a few in a
 // million) counts as dropped at first. At the end the workgroup's rows of this kind, up to 64 at a time, are gathered into
 // one tile, which goes through the body once more with P of dropped elements set to zero and dP taken without delta: that
-// adds just what is missing. (A tile for each of them: 232 us at 12 heads x 4096 keys, of which 30 us were waited for.)
+// adds just what is missing. (DS: dS of those elements is written anew, whole and rounded once, for dQ.) (A tile for each of them: 232 us at 12 heads x 4096 keys, of which 30 us were waited for.)
 // Whole backward at p = 0.1, with every element hashed in the plain kernel -> this: 12 heads x 4096 keys at head_dim 128
 // 631 -> 391 us (no dropout 387), x 8192 1957 -> 1290 (1209), x 2048 causal 187 -> 119 (105); head_dim 64, 8 x 12 heads x
 // 1024 causal 139 -> 74 (71).
@@ -1242,6 +1242,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       }
     }
     float pv[2][16];            // P of a block between its two stages
+    [[maybe_unused]] int full[2][8];      // AGAIN, DS: pairs of dS with delta
     auto stage_a = [&](int qb, int r) {
       const int koff = (r & 3) + 8 * (r >> 2);
       bool dead = false;
@@ -1266,6 +1267,11 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       asm volatile("" : "+v"(pw), "+v"(dsw));
       pf[qb][r >> 3][(r & 7) >> 1] = pw;
       dsf[qb][r >> 3][(r & 7) >> 1] = dsw;
+      if constexpr (AGAIN && DS) {
+        FO_LDS const float* d2 = rowvals + NBUF * kBwdTile + 32 * qb + 4 * hh + (r & 3) + 8 * (r >> 2);
+        const vec2 full2 = {(T)(pv[qb][r] * (dpacc[qb][r] + d2[0])), (T)(pv[qb][r + 1] * (dpacc[qb][r + 1] + d2[1]))};
+        full[qb][r >> 1] = __builtin_bit_cast(int, full2);
+      }
     };
     auto slot = [&](int s) {
       const SoftmaxGradJob job = softmax_grad_job(s);      // (s is a constant once the loop is unrolled)
@@ -1401,6 +1407,17 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       }
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (AGAIN && DS) {
+      // dS of the kept elements of the gathered rows, whole, in the place of what the tiles left (by this wave, and complete: see
+      // the wait in add_slots), which holds -P delta for them as for the dropped ones
+#pragma unroll
+      for (int e = 0; e < 32; ++e) {
+        const int row = gathered[32 * (e >> 4) + 4 * hh + (e & 3) + 8 * ((e & 15) >> 2)], x = row & 15, t2 = (row >> 4) & 1;
+        if ((alive >> e) & 1u)
+          *(T*)(ds_wave + (int64_t)(row / kBwdTile) * ds_tile_bytes + ((row >> 5) & 1) * 2048 + t2 * 1024 + ((l32 ^ (4 * t2)) * 32) + ((x >> 2) & 1) * 16 +
+                ((x & 3) + 4 * (x >> 3)) * 2) = __builtin_bit_cast(vec2, full[e >> 4][(e & 15) >> 1])[e & 1];
+      }
+    }
   };
 
   int j = qt0 - 1;
@@ -1474,6 +1491,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       }
       if (wave_s == 0) {
         dma4_lane_ptr((const float*)prm.nlse + (int64_t)bh * Sq + slot_row, rowvals);
+        if constexpr (DS) dma4_lane_ptr((const float*)prm.delta + (int64_t)bh * Sq + slot_row, rowvals + NBUF * kBwdTile);
         gathered[lane] = slot_row;
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1481,30 +1499,6 @@ __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(cons
       start_tile(0);
       zero_acc(dpacc[0]);
       tile_body(n_slots, 0, std::false_type{}, std::false_type{}, std::true_type{});
-      if constexpr (DS) {
-        // what the tile adds to the dS stored for its rows (by this wave, and complete: see the wait above)
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            typedef typename Ops<T>::vec8 vec8_t;
-            const vec8_t more = __builtin_bit_cast(vec8_t, dsf[qb][t]);
-            T* at[8];
-            T old[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-              const int slot_at = 32 * qb + 16 * t + 4 * hh + (u & 3) + 8 * (u >> 2), row = slot_at < n_slots ? gathered[slot_at] : 0;
-              const int x = row & 15, t2 = (row >> 4) & 1;
-              at[u] = (T*)(ds_wave + (int64_t)(row / kBwdTile) * ds_tile_bytes + ((row >> 5) & 1) * 2048 + t2 * 1024 + ((l32 ^ (4 * t2)) * 32) +
-                           ((x >> 2) & 1) * 16 + ((x & 3) + 4 * (x >> 3)) * 2);
-              if (slot_at >= n_slots || (CAUSAL && key > row)) at[u] = nullptr;
-              old[u] = at[u] != nullptr ? *at[u] : (T)0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-              if (at[u] != nullptr) *at[u] = (T)((float)old[u] + (float)more[u]);
-          }
-      }
       n_slots = 0;
     };
     int jt = qt0 - 1;
