@@ -1646,7 +1646,7 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
   if constexpr (BIAS) {
     if (key_bias) {
       if constexpr (D == 128) {
-        if (q.ds != nullptr && p.d == D) return launch_bwd_ds<T, CAUSAL, true, DROP, false, D, 0>(q, (unsigned)g_dkdv, lds_pipe, s);
+        if (q.ds != nullptr) return launch_bwd_ds<T, CAUSAL, true, DROP, false, D, 0>(q, (unsigned)g_dkdv, lds_pipe, s);
       }
       attn_bwd_dq_kernel<T, D, CAUSAL, DROP, false, true><<<(unsigned)g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
       if (p.d == D) attn_bwd_dkdv_pipe_kernel<T, D, CAUSAL, true, DROP><<<(unsigned)g_dkdv, kBwdWaves * 64, lds_pipe, s>>>(q);
@@ -1669,7 +1669,7 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
     }
   }
   if constexpr (!BIAS && D == 128) {
-    if (q.ds != nullptr && p.d == D && tune(g_attn_bwd_variant) != 0)
+    if (q.ds != nullptr && p.d == D)
       return launch_bwd_ds<T, CAUSAL, false, DROP, false, D, 0>(q, (unsigned)g_dkdv, lds_pipe, s);
   }
   attn_bwd_dq_kernel<T, D, CAUSAL, DROP, BIAS><<<(unsigned)g_dq, kBwdWaves * 64, lds_dq, s>>>(q);
@@ -1767,9 +1767,28 @@ constexpr int64_t kDsFromBytes = 96ll << 20, kDsMaxBytes = 2ll << 30;
 constexpr int kDsFromKeys = 1536;
 static bool bwd_keeps_ds(int B, int H, int Sq, int Sk, int D) {
   const int asked = tune(g_attn_bwd_keep_ds);
-  if (asked == 0 || D <= 64 || (int64_t)B * H > (1 << 20) || ds_key_blocks(Sk) * ds_query_tiles(Sq) > kDsMaxBytes / kDsChunk) return false;
+  if (asked == 0 || D <= 64 || tune(g_attn_bwd_variant) == 0 || (int64_t)B * H > (1 << 20) || ds_key_blocks(Sk) * ds_query_tiles(Sq) > kDsMaxBytes / kDsChunk) return false;
   const int64_t bytes = ds_bytes_of(B, H, Sq, Sk);
   return bytes <= kDsMaxBytes && (asked == 1 || Sk >= kDsFromKeys || bytes >= (D > 96 ? kDsFromBytes : kDsFromBytes + kDsFromBytes / 2));
+}
+
+// ... and for which calls: those that launch_bwd gives to the pipelined dK/dV kernel. The others (a bias with a query stride whose tiles cannot be
+// copied, or together with dropout; head dims off 128 with any bias or dropout) have no use for the memory.
+static bool bwd_form_keeps_ds(int D, bool drop, const BiasParams& bias) {
+  if (bias.ptr == nullptr) return D == 128 || !drop;
+  return D == 128 && (bias.strides[2] == 0 || (bias.dma_ok && !drop));
+}
+static BiasParams make_bias(const void* bias, const int64_t* strides, bool is_f32) {
+  BiasParams b;
+  b.ptr = bias;
+  for (int i = 0; i < 3; ++i) b.strides[i] = bias ? strides[i] : 0;
+  b.is_f32 = is_f32;
+  const uintptr_t elt = is_f32 ? 4 : 2;
+  // (dK/dV kernel: tiles of the bias are copied into LDS in 16-byte pieces)
+  b.dma_ok = bias && b.strides[2] != 0 && ((uintptr_t)bias % 16) == 0 && (b.strides[0] * elt) % 16 == 0 && (b.strides[1] * elt) % 16 == 0 &&
+             (b.strides[2] * elt) % 16 == 0;
+  b.vec_ok = bias && ((uintptr_t)bias % (4 * elt)) == 0 && b.strides[0] % 4 == 0 && b.strides[1] % 4 == 0 && b.strides[2] % 4 == 0;
+  return b;
 }
 
 // Which key blocks' query tiles several workgroups share (attn_bwd.hpp). A workgroup of the dK/dV kernel has a compute unit to itself,
@@ -1926,8 +1945,9 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   AttnBwdParams p;
   p.q = q; p.k = k; p.v = v; p.o = o; p.d_o = d_o; p.lse = lse; p.delta = delta_ws; p.nlse = delta_ws + (int64_t)B * H * Sq; p.dq = dq; p.dk = dk; p.dv = dv;
   p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.d = D;
+  p.bias = make_bias(bias, bias_strides, bias_dtype == FO_DTYPE_F32);
   p.ds = nullptr;
-  if (bwd_keeps_ds(B, H, Sq, Sk, D) && ws_bytes >= rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk) && !((uintptr_t)delta_ws & 15u))
+  if (ws_bytes > 0 && bwd_keeps_ds(B, H, Sq, Sk, D) && bwd_form_keeps_ds(D, dropout_p > 0.0f, p.bias) && ws_bytes >= rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk) && !((uintptr_t)delta_ws & 15u))
     p.ds = (char*)delta_ws + rows_ws_bytes(B, H, Sq);
   p.n_items = p.n_merges = 0;
   p.part = nullptr;
@@ -1950,16 +1970,6 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool c = causal != 0, drop = dropout_p > 0.0f;
   p.drop = make_dropout(dropout_p, seed, rng_offset);
-  p.bias.ptr = bias;
-  for (int i = 0; i < 3; ++i) p.bias.strides[i] = bias ? bias_strides[i] : 0;
-  p.bias.is_f32 = bias_dtype == FO_DTYPE_F32;
-  {
-    const uintptr_t elt = p.bias.is_f32 ? 4 : 2;
-    // (dK/dV kernel: tiles of the bias are copied into LDS in 16-byte pieces)
-    p.bias.dma_ok = bias && p.bias.strides[2] != 0 && ((uintptr_t)bias % 16) == 0 && (p.bias.strides[0] * elt) % 16 == 0 &&
-                    (p.bias.strides[1] * elt) % 16 == 0 && (p.bias.strides[2] * elt) % 16 == 0;
-    p.bias.vec_ok = bias && ((uintptr_t)bias % (4 * elt)) == 0 && p.bias.strides[0] % 4 == 0 && p.bias.strides[1] % 4 == 0 && p.bias.strides[2] % 4 == 0;
-  }
   // kernels are compiled for 64 and 128 columns; a head_dim in between runs on the next one with zero columns
   const bool has_bias = bias != nullptr;
   if (dtype == FO_DTYPE_BF16) return D > 64 ? launch_bwd_of<__bf16, 128>(p, c, drop, has_bias, s) : launch_bwd_of<__bf16, 64>(p, c, drop, has_bias, s);
@@ -2001,8 +2011,19 @@ extern "C" int fo_attn_bwd_ex(const void* q, const void* k, const void* v, const
                        extras->dropout_p, extras->dropout_seed, extras->dropout_offset, extras->bias, extras->bias_strides,
                        extras->bias_dtype, stream);
 }
+static bool bwd_ws_shape_ok(int B, int H, int Sq, int Sk, int D) {
+  return B > 0 && H > 0 && Sq > 0 && Sk > 0 && D >= 8 && D <= 128 && D % 8 == 0 && (int64_t)B * H <= (1ll << 40) / Sq;
+}
+extern "C" int64_t fo_attn_bwd_workspace_ex(int B, int H, int Sq, int Sk, int D, int causal, const fo_attn_extras* extras) {
+  if (!bwd_ws_shape_ok(B, H, Sq, Sk, D)) return 0;
+  const fo_attn_extras none = {};
+  const fo_attn_extras& x = extras ? *extras : none;
+  if (!bwd_keeps_ds(B, H, Sq, Sk, D) || !bwd_form_keeps_ds(D, x.dropout_p > 0.0f, make_bias(x.bias, x.bias_strides, x.bias_dtype == FO_DTYPE_F32)))
+    return rows_ws_bytes(B, H, Sq);
+  return rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk) + part_bytes_of(B, H, Sq, Sk, causal != 0);
+}
 extern "C" int64_t fo_attn_bwd_workspace(int B, int H, int Sq, int Sk, int D) {
-  if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || D < 8 || D > 128 || D % 8 != 0 || (int64_t)B * H * Sq > (1ll << 40)) return 0;
+  if (!bwd_ws_shape_ok(B, H, Sq, Sk, D)) return 0;
   if (!bwd_keeps_ds(B, H, Sq, Sk, D)) return rows_ws_bytes(B, H, Sq);
   const int64_t causal = part_bytes_of(B, H, Sq, Sk, true), full = part_bytes_of(B, H, Sq, Sk, false);
   return rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk) + (causal > full ? causal : full);

@@ -263,7 +263,7 @@ class _BwdPlan:
     """What a backward call of one (shapes, strides, dtypes, devices, layout) needs besides the data pointers, as _FwdPlan.
     (Checks, stride arrays and the switch of the device took 12 of the 31 us such a call cost the host, and a training step of a
     small model waits for its host: B=8 H=12 S=1024 D=64 causal with dropout 132 -> 117 us per step.)"""
-    __slots__ = ("B", "H", "Sq", "Sk", "D", "strides", "arrays", "dtype_code", "device_index", "ws_bytes")
+    __slots__ = ("B", "H", "Sq", "Sk", "D", "strides", "arrays", "dtype_code", "device_index", "ws_bytes")   # ws_bytes: see _bwd_ws_bytes
 
 
 _BWD_PLANS: dict = {}
@@ -285,11 +285,24 @@ def _bwd_plan(q: Tensor, k: Tensor, v: Tensor, o: Tensor, d_o: Tensor, dims: Tup
     plan.strides = (ctypes.POINTER(ctypes.c_int64) * 8)(*[ctypes.cast(a, ctypes.POINTER(ctypes.c_int64)) for a in plan.arrays])
     plan.dtype_code = _DTYPE_CODE[q.dtype]
     plan.device_index = q.device.index if q.device.index is not None else torch.cuda.current_device()
-    plan.ws_bytes = _lib.load().fo_attn_bwd_workspace(plan.B, plan.H, plan.Sq, plan.Sk, plan.D)
+    plan.ws_bytes = {}
     if len(_BWD_PLANS) > 4096:
         _BWD_PLANS.clear()
     _BWD_PLANS[key] = plan
     return plan
+
+
+def _bwd_ws_bytes(plan: _BwdPlan, causal: bool, bias: Optional[Tensor], dropout: Optional[Dropout], extras) -> int:
+    """The workspace a call can use, asked once per plan and form of the call (mask, dropout or none, layout of the bias): only some keep dS."""
+    form = (causal, extras is not None and dropout is not None and dropout[0] > 0.0,
+            None if bias is None else (bias.stride(), bias.data_ptr() % 16, bias.dtype))
+    n = plan.ws_bytes.get(form)
+    if n is None:
+        n = _lib.load().fo_attn_bwd_workspace_ex(plan.B, plan.H, plan.Sq, plan.Sk, plan.D, 1 if causal else 0, extras)
+        if len(plan.ws_bytes) > 64:
+            plan.ws_bytes.clear()
+        plan.ws_bytes[form] = n
+    return n
 
 
 def attn_bwd_strided(
@@ -312,13 +325,14 @@ def attn_bwd_strided(
     dq = torch.empty(q.shape, dtype=q.dtype, device=device)
     dk = torch.empty(k.shape, dtype=k.dtype, device=device)
     dv = torch.empty(v.shape, dtype=v.dtype, device=device)
-    # workspace: -delta and -LSE / scale per row, and dS where it is kept; without memory for that, the rows' values alone
-    try:
-        ws = torch.empty(plan.ws_bytes, dtype=torch.uint8, device=device)
-    except torch.OutOfMemoryError:
-        ws = torch.empty(8 * plan.B * plan.H * plan.Sq, dtype=torch.uint8, device=device)
     if bias is not None:
         bias = _expand_bias(bias, q, plan.B, plan.H, plan.Sq, plan.Sk)
+    extras = None if bias is None and (dropout is None or dropout[0] == 0.0) else ctypes.byref(_extras(bias, dropout))
+    # workspace: two values per row, and dS where it is kept; without memory for that, the rows' values alone
+    try:
+        ws = torch.empty(_bwd_ws_bytes(plan, causal, bias, dropout, extras), dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        ws = torch.empty(8 * plan.B * plan.H * plan.Sq, dtype=torch.uint8, device=device)
     lib = _lib.load()
     dev = plan.device_index
     # (as in the forward: the device is made current only when it is not)
@@ -327,7 +341,6 @@ def attn_bwd_strided(
         guard.__enter__()
     try:
         stream = _raw_stream(dev)
-        extras = None if bias is None and (dropout is None or dropout[0] == 0.0) else ctypes.byref(_extras(bias, dropout))
         status = lib.fo_attn_bwd_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr(),
                                     dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), plan.B, plan.H, plan.Sq, plan.Sk, plan.D, plan.strides, scale,
                                     1 if causal else 0, plan.dtype_code, extras, ws.data_ptr(), ws.numel(), stream)

@@ -214,12 +214,17 @@ int fo_attn_bwd_ex(const void* q, const void* k, const void* v, const void* o, c
 
 /* fo_attn_bwd_ex with a workspace of the caller's choice: ws_bytes bytes on the device, at least the [2, B, H, Sq] fp32 of
  * fo_attn_bwd (FO_ERR_BAD_SHAPE below), used by this call only until the stream has passed it and never needing to be cleared.
- * fo_attn_bwd_workspace answers how many bytes a call of a shape can use (0 where the shape itself is not taken): where
- * that is more than the rows' values (head_dim above 64, up to 2 GiB), with so many, 16-byte aligned, the call keeps dS (2 bytes per query and key, rounded up to 64 queries x 128 keys) and dQ is computed from it
- * instead of from the scores once more, where the shape and the bias allow (three launches, still no atomics, deterministic; where
- * few workgroups would fill the chip badly several share the queries of a block of keys, their fp32 sums of dK and dV behind dS);
- * with less it computes what fo_attn_bwd_ex computes. extras may be NULL. No reference counterpart. */
+ * fo_attn_bwd_workspace_ex answers how many bytes the call with this shape, mask, bias and dropout can use (0 where the shape itself is
+ * not taken; of extras, which may be NULL, it looks at the bias's strides, type and alignment and at whether there is dropout):
+ * where that is more than the rows' values, with so many, 16-byte aligned, the call keeps dS (2 bytes per query and key, rounded up to
+ * 64 queries x 128 keys, at most 2 GiB) and dQ is computed from it instead of from the scores once more (three launches, still no atomics, deterministic).
+ * Where few workgroups would fill the chip badly several share the queries of a block of keys, and leave 128 KiB each of
+ * fp32 sums of dK and dV behind dS (part of the answer; with room for dS alone each block stays whole).
+ * Kept at head_dim above 64: without a bias (off 128 also without dropout), and at 128 with a bias that has no query stride, or
+ * one on 16-byte boundaries without dropout. With less memory the call computes what fo_attn_bwd_ex computes.
+ * fo_attn_bwd_workspace: the most that any call of the shape can use. No reference counterpart. */
 int64_t fo_attn_bwd_workspace(int B, int H, int Sq, int Sk, int D);
+int64_t fo_attn_bwd_workspace_ex(int B, int H, int Sq, int Sk, int D, int causal, const fo_attn_extras* extras_host);
 int fo_attn_bwd_ws(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
                    void* dq, void* dk, void* dv, int B, int H, int Sq, int Sk, int D,
                    const int64_t* const* strides_host, float softmax_scale, int causal, int dtype,

@@ -1,0 +1,84 @@
+"""How much workspace the attention backward asks for (fo_attn_bwd_workspace_ex): dS only for the calls that keep it."""
+import ctypes
+
+import pytest
+import torch
+
+from fast_ops.flash_attention.flash_attention import flash_attn
+from fast_ops_amd import _lib
+from fast_ops_amd.flash_attention.flash_attention import _AttnExtras
+
+DEV = "cuda:0"
+B, H, S = 1, 8, 2048
+ROWS = 8 * B * H * S
+DS = 2 * B * H * S * S
+PART = 2 * 128 * 128 * 4                # one block's fp32 sums of dK and dV
+
+
+def _asked(D, causal=False, bias=None, p=0.0):
+    """bias: (address, strides, dtype)"""
+    ex = _AttnExtras()
+    if bias is not None:
+        ex.bias, ex.bias_strides, ex.bias_dtype = bias[0], (ctypes.c_int64 * 3)(*bias[1]), bias[2]
+    ex.dropout_p = p
+    return _lib.load().fo_attn_bwd_workspace_ex(B, H, S, S, D, int(causal), ctypes.byref(ex))
+
+
+KEY = (0x1000, (S, 0, 0), _lib.FO_DTYPE_F32)
+TILES = (0x1000, (0, S * S, S), _lib.FO_DTYPE_BF16)
+TILES32 = (0x1000, (0, S * S, S), _lib.FO_DTYPE_F32)
+ODD_ROWS = (0x1000, (0, S * (S + 1), S + 1), _lib.FO_DTYPE_BF16)
+ODD_BASE = (0x1002, (0, S * S, S), _lib.FO_DTYPE_BF16)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_calls_that_keep_ds(causal):
+    for D, bias, p in [(128, None, 0.0), (128, None, 0.3), (72, None, 0.0), (96, None, 0.0), (120, None, 0.0), (128, KEY, 0.0), (128, KEY, 0.3),
+                       (128, TILES, 0.0), (128, TILES32, 0.0)]:
+        n = _asked(D, causal, bias, p)
+        assert n >= ROWS + DS and (n - ROWS - DS) % (B * H * PART) == 0, (D, bias, p)
+        assert n <= _lib.load().fo_attn_bwd_workspace(B, H, S, S, D)
+    assert _lib.load().fo_attn_bwd_workspace_ex(B, H, S, S, 128, int(causal), None) == _asked(128, causal)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_calls_that_do_not(causal):
+    for D, bias, p in [(96, None, 0.3), (72, KEY, 0.0), (104, TILES, 0.0), (128, TILES, 0.3), (128, ODD_ROWS, 0.0), (128, ODD_BASE, 0.0), (64, None, 0.0),
+                       (32, KEY, 0.3)]:
+        assert _asked(D, causal, bias, p) == ROWS, (D, bias, p)
+    _lib.tune_set("attn_bwd.variant", 0)
+    try:
+        assert _asked(128, causal) == ROWS
+    finally:
+        _lib.tune_set("attn_bwd.variant", -1)
+
+
+def test_shapes_that_are_not_taken():
+    ask = lambda *a: (_lib.load().fo_attn_bwd_workspace_ex(*a, 0, None), _lib.load().fo_attn_bwd_workspace(*a))
+    big = 2 ** 31 - 1
+    for shape in [(0, 1, 1, 1, 64), (1, -1, 1, 1, 64), (1, 1, 0, 1, 64), (1, 1, 1, 0, 64), (1, 1, 1, 1, 12), (1, 1, 1, 1, 136), (big, big, big, 1, 128)]:
+        assert ask(*shape) == (0, 0), shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,bias,p", [(96, None, 0.3), (96, "key", 0.0), (128, "rows", 0.3), (128, None, 0.0)])
+def test_memory_of_a_backward(D, bias, p):
+    g = torch.Generator(device=DEV).manual_seed(D)
+    q, k, v, go = (torch.randn(B, S, H, D, generator=g, device=DEV).to(torch.bfloat16) for _ in range(4))
+    if bias == "key":
+        bias = torch.randn(B, 1, 1, S, generator=g, device=DEV)
+    elif bias is not None:
+        bias = torch.randn(1, 1, S, S, generator=g, device=DEV).to(torch.bfloat16)
+    t = [x.requires_grad_(True) for x in (q, k, v)]
+    o = flash_attn(*t, bias=bias, dropout_p=p, dropout_state=(1, 4) if p else None)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    torch.autograd.grad(o, t, go)
+    torch.cuda.synchronize()
+    used = torch.cuda.max_memory_allocated() - before
+    grads = 3 * q.numel() * 2
+    kept = D == 128 and bias is None
+    assert (used >= grads + ROWS + DS) == kept, used
+    if not kept:
+        assert used <= grads + ROWS + (1 << 20), used
