@@ -263,7 +263,7 @@ class _BwdPlan:
     """What a backward call of one (shapes, strides, dtypes, devices, layout) needs besides the data pointers, as _FwdPlan.
     (Checks, stride arrays and the switch of the device took 12 of the 31 us such a call cost the host, and a training step of a
     small model waits for its host: B=8 H=12 S=1024 D=64 causal with dropout 132 -> 117 us per step.)"""
-    __slots__ = ("B", "H", "Sq", "Sk", "D", "strides", "arrays", "dtype_code", "device_index", "ws_bytes")   # ws_bytes: see _bwd_ws_bytes
+    __slots__ = ("B", "H", "Sq", "Sk", "D", "strides", "arrays", "dtype_code", "device_index", "ws_bytes")   # ws_bytes: see _bwd_workspace
 
 
 _BWD_PLANS: dict = {}
@@ -292,17 +292,36 @@ def _bwd_plan(q: Tensor, k: Tensor, v: Tensor, o: Tensor, d_o: Tensor, dims: Tup
     return plan
 
 
-def _bwd_ws_bytes(plan: _BwdPlan, causal: bool, bias: Optional[Tensor], dropout: Optional[Dropout], extras) -> int:
-    """The workspace a call can use, asked once per plan and form of the call (mask, dropout or none, layout of the bias): only some keep dS."""
-    form = (causal, extras is not None and dropout is not None and dropout[0] > 0.0,
-            None if bias is None else (bias.stride(), bias.data_ptr() % 16, bias.dtype))
-    n = plan.ws_bytes.get(form)
-    if n is None:
+# after a workspace did not fit: how many calls go without asking for so much again (asking makes the caching allocator give its
+# cached blocks back, and the calls after it allocate anew)
+_BWD_WS_RETRY = 256
+
+
+def _bwd_workspace(plan: _BwdPlan, causal: bool, bias: Optional[Tensor], dropout: Optional[Dropout], extras, device) -> Tensor:
+    """The workspace of a call: two values per row, and, in the forms of a call that keep it, dS, and behind that the partial sums
+    of key blocks that several workgroups share. Without memory for all of that dS alone, or the rows' values. What is asked for
+    is worked out once per plan and form (mask, dropout or none, layout of the bias)."""
+    form = (causal, dropout is not None and dropout[0] > 0.0, None if bias is None else (bias.stride(), bias.data_ptr() % 16, bias.dtype))
+    entry = plan.ws_bytes.get(form)
+    if entry is None:
         n = _lib.load().fo_attn_bwd_workspace_ex(plan.B, plan.H, plan.Sq, plan.Sk, plan.D, 1 if causal else 0, extras)
+        rows = (8 * plan.B * plan.H * plan.Sq + 255) // 256 * 256
+        ds = rows + 2 * plan.B * plan.H * (-(-plan.Sq // 64) * 64) * (-(-plan.Sk // 128) * 128)
         if len(plan.ws_bytes) > 64:
             plan.ws_bytes.clear()
-        plan.ws_bytes[form] = n
-    return n
+        entry = plan.ws_bytes[form] = [0, 0, [n] + [s for s in (ds, rows) if s < n]]      # first size to ask for, calls it is kept for, sizes
+    sizes = entry[2]
+    if entry[0]:
+        entry[1] -= 1
+        if entry[1] < 0:
+            entry[0] = 0
+    for i in range(entry[0], len(sizes)):
+        try:
+            return torch.empty(sizes[i], dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            if i + 1 == len(sizes):
+                raise
+            entry[0], entry[1] = i + 1, _BWD_WS_RETRY
 
 
 def attn_bwd_strided(
@@ -328,11 +347,7 @@ def attn_bwd_strided(
     if bias is not None:
         bias = _expand_bias(bias, q, plan.B, plan.H, plan.Sq, plan.Sk)
     extras = None if bias is None and (dropout is None or dropout[0] == 0.0) else ctypes.byref(_extras(bias, dropout))
-    # workspace: two values per row, and dS where it is kept; without memory for that, the rows' values alone
-    try:
-        ws = torch.empty(_bwd_ws_bytes(plan, causal, bias, dropout, extras), dtype=torch.uint8, device=device)
-    except torch.OutOfMemoryError:
-        ws = torch.empty(8 * plan.B * plan.H * plan.Sq, dtype=torch.uint8, device=device)
+    ws = _bwd_workspace(plan, causal, bias, dropout, extras, device)
     lib = _lib.load()
     dev = plan.device_index
     # (as in the forward: the device is made current only when it is not)

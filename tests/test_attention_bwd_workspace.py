@@ -6,6 +6,7 @@ import torch
 
 from fast_ops.flash_attention.flash_attention import flash_attn
 from fast_ops_amd import _lib
+from fast_ops_amd.flash_attention import flash_attention as fa
 from fast_ops_amd.flash_attention.flash_attention import _AttnExtras
 
 DEV = "cuda:0"
@@ -58,6 +59,78 @@ def test_shapes_that_are_not_taken():
     big = 2 ** 31 - 1
     for shape in [(0, 1, 1, 1, 64), (1, -1, 1, 1, 64), (1, 1, 0, 1, 64), (1, 1, 1, 0, 64), (1, 1, 1, 1, 12), (1, 1, 1, 1, 136), (big, big, big, 1, 128)]:
         assert ask(*shape) == (0, 0), shape
+
+
+def test_a_workspace_that_does_not_fit_is_not_asked_for_again(monkeypatch):
+    plan = fa._BwdPlan()
+    plan.B, plan.H, plan.Sq, plan.Sk, plan.D, plan.ws_bytes = 1, 4, S, S, 128, {}
+    full = _lib.load().fo_attn_bwd_workspace_ex(1, 4, S, S, 128, 1, None)
+    rows = 8 * 4 * S
+    ds = rows + 2 * 4 * S * S
+    assert full > ds
+    asked, fits = [], [rows]
+
+    def empty(n, **kw):
+        asked.append(n)
+        if n > fits[0]:
+            raise torch.OutOfMemoryError("no room")
+        return n
+
+    monkeypatch.setattr(fa.torch, "empty", empty)
+    call = lambda: fa._bwd_workspace(plan, True, None, None, None, "cpu")
+    assert call() == rows and asked == [full, ds, rows]
+    asked.clear()
+    for _ in range(fa._BWD_WS_RETRY):
+        assert call() == rows
+    assert set(asked) == {rows}
+    asked.clear()
+    fits[0] = ds
+    assert call() == ds and asked == [full, ds]
+    assert call() == ds and asked == [full, ds, ds]
+    fits[0] = rows                       # less than before
+    assert call() == rows and asked == [full, ds, ds, ds, rows]
+    fits[0] = 0
+    with pytest.raises(torch.OutOfMemoryError):
+        call()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("room", ["dS", "rows"])
+def test_backward_without_room(monkeypatch, room):
+    """The gradients of a call whose workspace does not fit: with room for dS alone dQ is the same to the bit (and every block of
+    keys whole), with room for the rows' values alone the call is the one that computes the scores again."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    t = [torch.randn(1, S, 4, 128, generator=g, device=DEV).to(torch.bfloat16).requires_grad_(True) for _ in range(3)]
+    go = torch.randn(1, S, 4, 128, generator=g, device=DEV).to(torch.bfloat16)
+    backward = lambda: torch.autograd.grad(flash_attn(*t, causal=True), t, go)
+    full = _lib.load().fo_attn_bwd_workspace_ex(1, 4, S, S, 128, 1, None)
+    ds = 8 * 4 * S + 2 * 4 * S * S
+    assert full > ds
+    free = backward()
+    _lib.tune_set("attn_bwd.keep_ds" if room == "rows" else "attn_bwd.split", 0)
+    try:
+        expected = backward()
+    finally:
+        _lib.tune_set("attn_bwd.keep_ds", -1)
+        _lib.tune_set("attn_bwd.split", -1)
+    real, refused = torch.empty, []
+
+    def empty(*a, **kw):
+        if kw.get("dtype") == torch.uint8 and a[0] > (ds if room == "dS" else ds - 1):
+            refused.append(a[0])
+            raise torch.OutOfMemoryError("no room")
+        return real(*a, **kw)
+
+    monkeypatch.setattr(fa.torch, "empty", empty)
+    got = [backward() for _ in range(3)]
+    monkeypatch.undo()
+    assert refused == ([full] if room == "dS" else [full, ds])       # by the first call alone
+    for grads in got:
+        for a, b in zip(grads, expected):
+            assert torch.equal(a, b)
+    if room == "dS":
+        assert torch.equal(got[0][0], free[0]) and not torch.equal(got[0][1], free[1])
+    _lib.tune_set("attn_bwd.split", -1)      # (a new plan for whoever comes next)
 
 
 @pytest.mark.gpu
