@@ -1887,17 +1887,21 @@ static DkdvPlan make_dkdv_plan(int n_bh, int Sq, int Sk, bool causal, int asked)
   }
   return best;
 }
-// (a step of a model asks for the same one over and over: kept per thread)
+// (A step of a model asks for the same few over and over, and a plan takes 2 to 40 us: the last ones are kept per thread. With one place,
+// layers of two shapes in turn worked theirs out at every call.)
 static const DkdvPlan& dkdv_plan(int B, int H, int Sq, int Sk, bool causal) {
-  struct Key { int n_bh, Sq, Sk, causal, asked; };
-  static thread_local Key key = {0, 0, 0, 0, 0};
-  static thread_local DkdvPlan plan;
+  struct Place { int n_bh, Sq, Sk, causal, asked; DkdvPlan plan; };
+  constexpr int kPlaces = 8;
+  static thread_local Place places[kPlaces];      // (n_bh 0: empty)
+  static thread_local int oldest = 0;
   const int asked = tune(g_attn_bwd_order) >= 0 ? 0 : tune(g_attn_bwd_split);
-  if (key.n_bh != B * H || key.Sq != Sq || key.Sk != Sk || key.causal != (int)causal || key.asked != asked) {
-    plan = make_dkdv_plan(B * H, Sq, Sk, causal, asked);
-    key = {B * H, Sq, Sk, (int)causal, asked};
-  }
-  return plan;
+  for (const Place& p : places)
+    if (p.n_bh == B * H && p.Sq == Sq && p.Sk == Sk && p.causal == (int)causal && p.asked == asked) return p.plan;
+  Place& p = places[oldest];
+  oldest = (oldest + 1) % kPlaces;
+  p.n_bh = B * H; p.Sq = Sq; p.Sk = Sk; p.causal = (int)causal; p.asked = asked;
+  p.plan = make_dkdv_plan(B * H, Sq, Sk, causal, asked);
+  return p.plan;
 }
 static int64_t part_bytes_of(int B, int H, int Sq, int Sk, bool causal) {
   return dkdv_plan(B, H, Sq, Sk, causal).n_parts * (int64_t)B * H * kPartBytes;

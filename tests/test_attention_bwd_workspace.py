@@ -1,5 +1,7 @@
 """How much workspace the attention backward asks for (fo_attn_bwd_workspace_ex): dS only for the calls that keep it."""
 import ctypes
+import math
+import time
 
 import pytest
 import torch
@@ -59,6 +61,24 @@ def test_shapes_that_are_not_taken():
     big = 2 ** 31 - 1
     for shape in [(0, 1, 1, 1, 64), (1, -1, 1, 1, 64), (1, 1, 0, 1, 64), (1, 1, 1, 0, 64), (1, 1, 1, 1, 12), (1, 1, 1, 1, 136), (big, big, big, 1, 128)]:
         assert ask(*shape) == (0, 0), shape
+
+
+def test_shapes_in_turn_do_not_plan_anew():
+    """Layers of several shapes ask in turn: how the key blocks are shared is worked out once for each, not at every call (2 to 40 us)."""
+    ask = _lib.load().fo_attn_bwd_workspace_ex
+
+    def per_call(lengths):
+        best = math.inf
+        for _ in range(7):
+            t0 = time.perf_counter()
+            for _ in range(100):
+                for n in lengths:
+                    ask(1, 4, n, n, 128, 1, None)
+            best = min(best, (time.perf_counter() - t0) / (100 * len(lengths)))
+        return best
+
+    one = per_call([8192] * 4)
+    assert per_call([8192, 7168, 6144, 5120]) < 3.0 * one
 
 
 def test_a_workspace_that_does_not_fit_is_not_asked_for_again(monkeypatch):
