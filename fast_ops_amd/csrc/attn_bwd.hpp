@@ -1,19 +1,11 @@
 // What the translation units of the attention backward share: attn_bwd.hip (dK/dV and the dQ kernel that computes the scores
 // again) and attn_bwd_dq_of_ds.hip (dQ from stored dS).
 #pragma once
+#include "attn_bwd_plan.hpp"
 #include "attn_common.hpp"
 
 namespace fo {
 
-constexpr int kBwdWaves = 4;
-constexpr int kBwdRows = 32 * kBwdWaves;   // rows (queries or keys) owned by a workgroup
-constexpr int kBwdTile = 64;               // rows of a streamed tile
-
-// An item of the dK/dV kernel that keeps dS: key block | piece << 8 | pieces << 12 | part << 16; the block's query tiles are shared by
-// `pieces` workgroups, each of which leaves its sums in part `part` (of every head: see dkdv_part). A merge: key block | pieces << 12 |
-// first part << 16.
-constexpr int kMaxItems = 96, kMaxMerges = 48;
-constexpr uint32_t kWholeBlock = 0xFFFF1000u;
 constexpr int kPartBytes = 2 * kBwdRows * 128 * 4;     // dK and dV of a block in fp32: each wave's accumulators, 1 KiB per four registers
 
 struct AttnBwdParams {

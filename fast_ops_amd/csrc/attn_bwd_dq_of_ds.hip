@@ -279,9 +279,10 @@ static int launch_one(const AttnBwdParams& p, hipStream_t s) {
 // 24 x 1500 at 112 (288) 40.2 -> 40.7, 16 x 2000 at 96 (256) 25.2 -> 26.0.
 template <typename T, bool CAUSAL, int LIVE, bool PAD, bool TBIAS>
 static int launch_form(const AttnBwdParams& p, hipStream_t s) {
-  constexpr int kUnits = 256, kTwoTeamsFromKeys = 1536;
+  constexpr int kTwoTeamsFromKeys = 1536;
+  const int64_t units = device_cus();
   const int64_t n_bh = (int64_t)p.B * p.H, blocks = n_bh * ((p.Sq + kBwdRows - 1) / kBwdRows);
-  const bool two = p.Sk >= kTwoTeamsFromKeys && (CAUSAL ? blocks + n_bh * p.n_merges > kUnits && blocks <= 3 * kUnits : blocks > kUnits && blocks <= kUnits + kUnits / 4);
+  const bool two = p.Sk >= kTwoTeamsFromKeys && (CAUSAL ? blocks + n_bh * p.n_merges > units && blocks <= 3 * units : blocks > units && blocks <= units + units / 4);
   return two ? launch_one<T, CAUSAL, LIVE, PAD, TBIAS, 4, 2>(p, s) : launch_one<T, CAUSAL, LIVE, PAD, TBIAS, 4, 1>(p, s);
 }
 template <typename T>

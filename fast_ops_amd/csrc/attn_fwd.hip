@@ -1381,20 +1381,6 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   return (int)group;
 }
 
-// compute units of the current device (asked once per device; 256 where no device answers)
-static int device_cus() {
-  constexpr int kMaxDev = 64;
-  static std::atomic<int> cached[kMaxDev];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return 256;
-  int n = cached[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cached[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
 template <typename T, int D, bool CAUSAL, int QB, int DBG = 0, int BM = kWideBM, bool VBIAS = false, bool DROP = false>
 static int launch_wide(AttnParams p, hipStream_t stream) {
   constexpr bool KEEP_ON = BM == kWideBM && !VBIAS;      // (as in the kernel)

@@ -347,7 +347,6 @@ def attn_bwd_strided(
     if bias is not None:
         bias = _expand_bias(bias, q, plan.B, plan.H, plan.Sq, plan.Sk)
     extras = None if bias is None and (dropout is None or dropout[0] == 0.0) else ctypes.byref(_extras(bias, dropout))
-    ws = _bwd_workspace(plan, causal, bias, dropout, extras, device)
     lib = _lib.load()
     dev = plan.device_index
     # (as in the forward: the device is made current only when it is not)
@@ -356,6 +355,7 @@ def attn_bwd_strided(
         guard.__enter__()
     try:
         stream = _raw_stream(dev)
+        ws = _bwd_workspace(plan, causal, bias, dropout, extras, device)      # (asked with the device current: it depends on its compute units)
         status = lib.fo_attn_bwd_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr(),
                                     dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), plan.B, plan.H, plan.Sq, plan.Sk, plan.D, plan.strides, scale,
                                     1 if causal else 0, plan.dtype_code, extras, ws.data_ptr(), ws.numel(), stream)
