@@ -1815,15 +1815,16 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
                          float* delta_ws, void* dq, void* dk, void* dv, int B, int H, int Sq, int Sk, int D,
                          const int64_t* const* strides_host, float softmax_scale, int causal, int dtype, float dropout_p,
                          uint32_t seed, uint64_t rng_offset, const void* bias, const int64_t* bias_strides, int bias_dtype,
-                         void* stream, bool static_ws = false, int64_t ws_bytes = 0) {
-  // ws_bytes: how much memory delta_ws points to where the caller says so (fo_attn_bwd_ws); dS is kept behind its two rows of values
+                         void* stream, bool static_ws = false, int64_t ws_bytes = -1) {
+  // ws_bytes: how much memory delta_ws points to where the caller says so (fo_attn_bwd_ws; else -1); dS is kept behind its two rows of values
   // static_ws: delta_ws is ignored and the library's own per-device array takes its place (fo_attn_bwd_static_ws)
   if (!q || !k || !v || !o || !d_o || !lse || (!delta_ws && !static_ws) || !dq || !dk || !dv || !strides_host) return FO_ERR_NULL_POINTER;
   for (int t = 0; t < 8; ++t)
     if (!strides_host[t]) return FO_ERR_NULL_POINTER;
   if (dtype != FO_DTYPE_F16 && dtype != FO_DTYPE_BF16) return FO_ERR_BAD_DTYPE;
   if (D < 8 || D > 128 || D % 8 != 0) return FO_ERR_BAD_HEAD_DIM;
-  if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || (int64_t)B * H * Sq > (1ll << 40)) return FO_ERR_BAD_SHAPE;
+  if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || (int64_t)B * H > (1ll << 40) / Sq) return FO_ERR_BAD_SHAPE;
+  if (ws_bytes != -1 && ws_bytes < (int64_t)B * H * Sq * 2 * (int64_t)sizeof(float)) return FO_ERR_BAD_SHAPE;
   for (int t = 0; t < 8; ++t) {
     // rows start on 16-byte boundaries (8 elements); only the inputs K and V may repeat a head (stride 0 = multi-query)
     for (int i = 0; i < 3; ++i)
@@ -1941,7 +1942,7 @@ extern "C" int fo_attn_bwd_ws(const void* q, const void* k, const void* v, const
                               void* dq, void* dk, void* dv, int B, int H, int Sq, int Sk, int D,
                               const int64_t* const* strides_host, float softmax_scale, int causal, int dtype,
                               const fo_attn_extras* extras, void* ws, int64_t ws_bytes, void* stream) {
-  if (ws_bytes < (int64_t)B * H * Sq * 2 * (int64_t)sizeof(float)) return FO_ERR_BAD_SHAPE;
+  if (ws_bytes < 0) return FO_ERR_BAD_SHAPE;
   const fo_attn_extras none = {};
   const fo_attn_extras& x = extras ? *extras : none;
   return attn_bwd_impl(q, k, v, o, d_o, lse, (float*)ws, dq, dk, dv, B, H, Sq, Sk, D, strides_host, softmax_scale, causal, dtype,

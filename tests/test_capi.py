@@ -106,6 +106,22 @@ def test_attn_backward_bias_dropout_argument_validation_without_device():
     assert lib.fo_dropout_mask(ok, 0, 0.5, 1, 0, None) == 0                            # nothing to do, nothing launched
 
 
+def test_attn_backward_workspace_argument_validation_without_device():
+    lib = _lib.load()
+    s = (ctypes.c_int64 * 3)(128 * 64, 64 * 128 * 4, 64)
+    strides = (ctypes.POINTER(ctypes.c_int64) * 8)(*[ctypes.cast(s, ctypes.POINTER(ctypes.c_int64))] * 8)
+    ok = 0x1000
+    bwd = lambda **kw: lib.fo_attn_bwd_ws(
+        kw.get("q", ok), ok, ok, ok, ok, ok, ok, ok, kw.get("dv", ok), kw.get("B", 1), kw.get("H", 1), kw.get("Sq", 128), 128, kw.get("D", 64),
+        kw.get("strides", strides), kw.get("scale", 0.125), 0, kw.get("dtype", 1), None, kw.get("ws", ok), kw.get("bytes", 8 * 128), None)
+    assert bwd(q=None) == -1 and bwd(dv=None) == -1 and bwd(ws=None) == -1 and bwd(strides=None) == -1
+    assert bwd(dtype=2) == -2 and bwd(D=100) == -3 and bwd(scale=0.0) == -4
+    assert bwd(bytes=8 * 128 - 1) == -4 and bwd(bytes=0) == -4 and bwd(bytes=-1) == -4
+    assert bwd(Sq=0) == -4 and bwd(B=-1) == -4
+    assert bwd(B=1 << 30, H=1 << 30, Sq=16, bytes=16) == -4           # (B H Sq is 0 modulo 2^64)
+    assert bwd(ws=0x1002) == -6
+
+
 def test_lion_argument_validation_without_device():
     lib = _lib.load()
     c = _lib.FoLionConsts()
