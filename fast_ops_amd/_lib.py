@@ -49,6 +49,7 @@ SIGNATURES = {
     "fo_attn_bwd_ex": (ctypes.c_int, [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.POINTER(_I64P), ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]),
     "fo_attn_bwd_workspace": (ctypes.c_int64, [ctypes.c_int] * 5),
     "fo_attn_bwd_workspace_ex": (ctypes.c_int64, [ctypes.c_int] * 6 + [ctypes.c_void_p]),
+    "fo_attn_bwd_kernels": (ctypes.c_int, [ctypes.c_int] * 6 + [ctypes.c_void_p, ctypes.c_int64]),
     "fo_attn_bwd_ws": (ctypes.c_int, [ctypes.c_void_p] * 9 + [ctypes.c_int] * 5 + [ctypes.POINTER(_I64P), ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]),
     "fo_attn_bwd_dropout": (ctypes.c_int, [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.POINTER(_I64P), ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_float, ctypes.c_uint32, ctypes.c_uint64, ctypes.c_void_p]),
     "fo_lion_make_consts": (ctypes.c_int, [ctypes.c_double] * 4 + [ctypes.POINTER(FoLionConsts)]),

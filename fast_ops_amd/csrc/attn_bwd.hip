@@ -1811,6 +1811,19 @@ static int64_t part_bytes_of(int B, int H, int Sq, int Sk, bool causal) {
   return dkdv_plan(B, H, Sq, Sk, causal).n_parts * (int64_t)B * H * kPartBytes;
 }
 
+// What a call does with its workspace: where dS lies in it (0: not kept), and the sums of shared key blocks (plan null: none are shared).
+struct BwdForm { int64_t ds_at, part_at; const DkdvPlan* plan; };
+static BwdForm bwd_form(int B, int H, int Sq, int Sk, int D, bool causal, bool drop, const BiasParams& bias, const void* ws, int64_t ws_bytes) {
+  BwdForm f = {0, 0, nullptr};
+  if (ws_bytes <= 0 || ((uintptr_t)ws & 15u) || !bwd_keeps_ds(B, H, Sq, Sk, D) || !bwd_form_keeps_ds(D, drop, bias)) return f;
+  const int64_t rows = rows_ws_bytes(B, H, Sq), end = rows + ds_bytes_of(B, H, Sq, Sk);
+  if (ws_bytes < end) return f;
+  f.ds_at = rows;
+  const DkdvPlan& plan = dkdv_plan(B, H, Sq, Sk, causal);
+  if (plan.n_items > 0 && ws_bytes >= end + plan.n_parts * (int64_t)B * H * kPartBytes) { f.part_at = end; f.plan = &plan; }
+  return f;
+}
+
 static int attn_bwd_impl(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
                          float* delta_ws, void* dq, void* dk, void* dv, int B, int H, int Sq, int Sk, int D,
                          const int64_t* const* strides_host, float softmax_scale, int causal, int dtype, float dropout_p,
@@ -1855,20 +1868,16 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   p.q = q; p.k = k; p.v = v; p.o = o; p.d_o = d_o; p.lse = lse; p.delta = delta_ws; p.nlse = delta_ws + (int64_t)B * H * Sq; p.dq = dq; p.dk = dk; p.dv = dv;
   p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.d = D;
   p.bias = make_bias(bias, bias_strides, bias_dtype == FO_DTYPE_F32);
-  p.ds = nullptr;
-  if (ws_bytes > 0 && bwd_keeps_ds(B, H, Sq, Sk, D) && bwd_form_keeps_ds(D, dropout_p > 0.0f, p.bias) && ws_bytes >= rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk) && !((uintptr_t)delta_ws & 15u))
-    p.ds = (char*)delta_ws + rows_ws_bytes(B, H, Sq);
+  const BwdForm form = bwd_form(B, H, Sq, Sk, D, causal != 0, dropout_p > 0.0f, p.bias, delta_ws, ws_bytes);
+  p.ds = form.ds_at > 0 ? (char*)delta_ws + form.ds_at : nullptr;
   p.n_items = p.n_merges = 0;
   p.part = nullptr;
-  if (p.ds != nullptr) {
-    const int64_t before = rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk);
-    const DkdvPlan& plan = dkdv_plan(B, H, Sq, Sk, causal != 0);
-    if (plan.n_items > 0 && ws_bytes >= before + plan.n_parts * (int64_t)B * H * kPartBytes) {
-      p.part = (char*)delta_ws + before;
-      p.n_items = plan.n_items; p.n_merges = plan.n_merges;
-      for (int i = 0; i < plan.n_items; ++i) p.items[i] = plan.items[i];
-      for (int i = 0; i < plan.n_merges; ++i) p.merges[i] = plan.merges[i];
-    }
+  if (form.plan != nullptr) {
+    const DkdvPlan& plan = *form.plan;
+    p.part = (char*)delta_ws + form.part_at;
+    p.n_items = plan.n_items; p.n_merges = plan.n_merges;
+    for (int i = 0; i < plan.n_items; ++i) p.items[i] = plan.items[i];
+    for (int i = 0; i < plan.n_merges; ++i) p.merges[i] = plan.merges[i];
   }
   int64_t* dst[8] = {p.qs, p.ks, p.vs, p.os, p.dos, p.dqs, p.dks, p.dvs};
   for (int t = 0; t < 8; ++t)
@@ -1930,6 +1939,15 @@ extern "C" int64_t fo_attn_bwd_workspace_ex(int B, int H, int Sq, int Sk, int D,
   if (!bwd_keeps_ds(B, H, Sq, Sk, D) || !bwd_form_keeps_ds(D, x.dropout_p > 0.0f, make_bias(x.bias, x.bias_strides, x.bias_dtype == FO_DTYPE_F32)))
     return rows_ws_bytes(B, H, Sq);
   return rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk) + part_bytes_of(B, H, Sq, Sk, causal != 0);
+}
+extern "C" int fo_attn_bwd_kernels(int B, int H, int Sq, int Sk, int D, int causal, const fo_attn_extras* extras, int64_t ws_bytes) {
+  if (!bwd_ws_shape_ok(B, H, Sq, Sk, D)) return FO_ERR_BAD_SHAPE;
+  const fo_attn_extras none = {};
+  const fo_attn_extras& x = extras ? *extras : none;
+  const BwdForm f = bwd_form(B, H, Sq, Sk, D, causal != 0, x.dropout_p > 0.0f, make_bias(x.bias, x.bias_strides, x.bias_dtype == FO_DTYPE_F32), nullptr, ws_bytes);
+  if (f.ds_at == 0) return 0;
+  return FO_ATTN_BWD_KEEPS_DS | (f.plan != nullptr ? FO_ATTN_BWD_SHARES_BLOCKS : 0) |
+         (dq_two_teams((int64_t)B * H, Sq, Sk, causal != 0, f.plan != nullptr ? f.plan->n_merges : 0) ? FO_ATTN_BWD_DQ_TWO_TEAMS : 0);
 }
 extern "C" int64_t fo_attn_bwd_workspace(int B, int H, int Sq, int Sk, int D) {
   if (!bwd_ws_shape_ok(B, H, Sq, Sk, D)) return 0;

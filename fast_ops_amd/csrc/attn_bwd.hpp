@@ -64,6 +64,20 @@ __host__ __device__ inline int64_t ds_query_tiles(int Sq) { return ((int64_t)Sq 
 __device__ inline int64_t ds_chunk(const AttnBwdParams& prm, int bh, int kb, int qt) {
   return (((int64_t)bh * ds_query_tiles(prm.Sq) + qt) * ds_key_blocks(prm.Sk) + kb) * kDsChunk;
 }
+// Two teams of waves in a workgroup of that kernel: the chain of tiles is half as long and a workgroup has its unit to itself, as two of one team would have it together. It
+// gains where units would hold two and others one, or causal ones of unequal length, for a good while: this kernel, one team -> two, us,
+//   causal: 12 x 3072 with a bias 47.1 -> 41.6, 12 x 4096 61.3 -> 50.8, 16 x 4096 74.0 -> 58.5, 4 x 8192 94.0 -> 83.8, 32 x 1800 36.1 -> 31.9,
+//     12 x 6144 105 -> 98, 12 x 8192 (768 blocks) 171 -> 166; not: 32 x 4096 (1024) 122 -> 131, 64 x 1024 24.8 -> 26.1, 16 x 2048 (256) 25.1 -> 25.8
+//   not causal: 12 x 3072 (288 blocks) 76.4 -> 68.7; not: 12 x 4096 (384) 90.4 -> 91.6, 24 x 2304 (432) 57.5 -> 60.1, 64 x 2048 110 -> 126
+// and at other head dims the same: 24 x 2000 causal at 112 34.0 -> 26.8, 12 x 3000 causal 41.1 -> 37.8; not: 64 x 777 x 1250 at 80 (448) 30.5 -> 35.0,
+// 24 x 1500 at 112 (288) 40.2 -> 40.7, 16 x 2000 at 96 (256) 25.2 -> 26.0.
+inline bool dq_two_teams(int64_t n_bh, int Sq, int Sk, bool causal, int n_merges) {
+  constexpr int kTwoTeamsFromKeys = 1536;
+  const int asked = tune(g_attn_bwd_dq_teams);
+  if (asked > 0) return asked == 2;
+  const int64_t units = device_cus(), blocks = n_bh * ((Sq + kBwdRows - 1) / kBwdRows);
+  return Sk >= kTwoTeamsFromKeys && (causal ? blocks + n_bh * n_merges > units && blocks <= 3 * units : blocks > units && blocks <= units + units / 4);
+}
 template <typename T> int launch_bwd_rows(const AttnBwdParams& p, bool drop, bool tile_bias, hipStream_t s);
 template <typename T> int launch_dq_of_ds(const AttnBwdParams& p, bool causal, bool tile_bias, hipStream_t s);
 

@@ -82,7 +82,7 @@ __device__ __forceinline__ void merge_dkdv(const AttnBwdParams& prm, int at, FO_
 // are workgroups enough, else by a workgroup's chain per tile (0.4 us, the unit's LDS: 12 heads x 3072 causal 40 us; with reads, conditions and products in
 // the order they come to mind 48). 12 heads x 4096 (0.4 GB of dS) 98 us = 4.1 TB/s of dS: the dQ kernel that computes the scores again takes
 // 172; copied without nt, dS pushes K out of the cache: 131. Five or eight buffers, or 64 rows per wave, gain nothing (131, 131 / 108-170).
-// TEAMS 2: eight waves, the second four with the odd tiles and a ring of their own; the two teams' sums are added at the end (see launch_form).
+// TEAMS 2: eight waves, the second four with the odd tiles and a ring of their own; the two teams' sums are added at the end (see dq_two_teams).
 // TBIAS: P of a row whose bias is large as a whole is off by the rounding of -LSE / scale, one factor per row, made good here.
 template <typename T, bool CAUSAL, int LIVE, bool PAD, bool TBIAS, int SLOTS, int TEAMS>
 __global__ void __launch_bounds__(TEAMS * kBwdWaves * 64, 2) attn_bwd_dq_of_ds_kernel(const AttnBwdParams prm) {
@@ -270,19 +270,9 @@ static int launch_one(const AttnBwdParams& p, hipStream_t s) {
   attn_bwd_dq_of_ds_kernel<T, CAUSAL, LIVE, PAD, TBIAS, SLOTS, TEAMS><<<grid, TEAMS * kBwdWaves * 64, lds, s>>>(p);
   return launch_status();
 }
-// Two teams: the chain of tiles is half as long and a workgroup has its unit to itself, as two of one team would have it together. It
-// gains where units would hold two and others one, or causal ones of unequal length, for a good while: this kernel, one team -> two, us,
-//   causal: 12 x 3072 with a bias 47.1 -> 41.6, 12 x 4096 61.3 -> 50.8, 16 x 4096 74.0 -> 58.5, 4 x 8192 94.0 -> 83.8, 32 x 1800 36.1 -> 31.9,
-//     12 x 6144 105 -> 98, 12 x 8192 (768 blocks) 171 -> 166; not: 32 x 4096 (1024) 122 -> 131, 64 x 1024 24.8 -> 26.1, 16 x 2048 (256) 25.1 -> 25.8
-//   not causal: 12 x 3072 (288 blocks) 76.4 -> 68.7; not: 12 x 4096 (384) 90.4 -> 91.6, 24 x 2304 (432) 57.5 -> 60.1, 64 x 2048 110 -> 126
-// and at other head dims the same: 24 x 2000 causal at 112 34.0 -> 26.8, 12 x 3000 causal 41.1 -> 37.8; not: 64 x 777 x 1250 at 80 (448) 30.5 -> 35.0,
-// 24 x 1500 at 112 (288) 40.2 -> 40.7, 16 x 2000 at 96 (256) 25.2 -> 26.0.
 template <typename T, bool CAUSAL, int LIVE, bool PAD, bool TBIAS>
 static int launch_form(const AttnBwdParams& p, hipStream_t s) {
-  constexpr int kTwoTeamsFromKeys = 1536;
-  const int64_t units = device_cus();
-  const int64_t n_bh = (int64_t)p.B * p.H, blocks = n_bh * ((p.Sq + kBwdRows - 1) / kBwdRows);
-  const bool two = p.Sk >= kTwoTeamsFromKeys && (CAUSAL ? blocks + n_bh * p.n_merges > units && blocks <= 3 * units : blocks > units && blocks <= units + units / 4);
+  const bool two = dq_two_teams((int64_t)p.B * p.H, p.Sq, p.Sk, CAUSAL, p.n_merges);
   return two ? launch_one<T, CAUSAL, LIVE, PAD, TBIAS, 4, 2>(p, s) : launch_one<T, CAUSAL, LIVE, PAD, TBIAS, 4, 1>(p, s);
 }
 template <typename T>

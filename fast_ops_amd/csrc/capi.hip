@@ -15,6 +15,7 @@ std::atomic<int> g_attn_balance{-1};
 std::atomic<int> g_attn_bwd_order{-1};
 std::atomic<int> g_attn_bwd_keep_ds{-1};
 std::atomic<int> g_attn_bwd_split{-1};
+std::atomic<int> g_attn_bwd_dq_teams{-1};
 }  // namespace fo
 
 extern "C" const char* fo_strerror(int status) {
@@ -83,6 +84,10 @@ extern "C" int fo_tune_set(const char* key, int value) {
     if (value == 1 || value > 4) return FO_ERR_UNSUPPORTED;      // 0 = never, 2 to 4 = every block in so many pieces
     fo::g_attn_bwd_split = value; return FO_OK;
   }
+  if (strcmp(key, "attn_bwd.dq_teams") == 0) {
+    if (value == 0 || value > 2) return FO_ERR_UNSUPPORTED;
+    fo::g_attn_bwd_dq_teams = value; return FO_OK;
+  }
   return FO_ERR_UNSUPPORTED;
 }
 
@@ -99,6 +104,7 @@ extern "C" int fo_tune_get(const char* key) {
   if (strcmp(key, "attn_bwd.order") == 0) return fo::tune(fo::g_attn_bwd_order);
   if (strcmp(key, "attn_bwd.keep_ds") == 0) return fo::tune(fo::g_attn_bwd_keep_ds);
   if (strcmp(key, "attn_bwd.split") == 0) return fo::tune(fo::g_attn_bwd_split);
+  if (strcmp(key, "attn_bwd.dq_teams") == 0) return fo::tune(fo::g_attn_bwd_dq_teams);
   if (strcmp(key, "build.ablations") == 0) {
 #if defined(FO_ABLATIONS)
     return 1;

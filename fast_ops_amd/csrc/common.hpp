@@ -28,6 +28,7 @@ extern std::atomic<int> g_attn_bwd_variant;
 extern std::atomic<int> g_attn_bwd_order;   // attention backward: -1 automatic, 0 all heads in one group, n > 0 groups of n heads
 extern std::atomic<int> g_attn_bwd_keep_ds;   // attention backward: -1 automatic, 0 never keeps dS, 1 wherever it can be kept
 extern std::atomic<int> g_attn_bwd_split;   // attention backward, dS kept: -1 automatic, 0 a workgroup per key block, 2 to 4 every block's queries in so many pieces
+extern std::atomic<int> g_attn_bwd_dq_teams;   // attention backward, dQ of kept dS: -1 automatic, 1 or 2 teams of waves per workgroup
 extern std::atomic<int> g_attn_balance;   // 128-row attention kernel, causal: 0 plain heaviest-first order also where a launch fits the chip at once, otherwise (default) balanced
 extern std::atomic<int> g_attn_tail;      // 256-row attention kernel, non-causal: 0 = never hand the last round to the 128-row form (see launch_rows256_w4_noncausal)
 extern std::atomic<int> g_attn_decode_split;   // attn_decode.hip: -1 automatic, n >= 1 workgroups that share the keys of a row block

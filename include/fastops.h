@@ -46,7 +46,7 @@ const char* fo_strerror(int status);
 int fo_version(void);
 
 /* Tuning hook for benchmarks, profiling and tests: selects a kernel variant or a workgroup order by name
- * ("lion.variant", "attn.variant", "attn_bwd.variant", "attn.order", "attn.balance", "attn.keep_on", "attn.tail", "attn.decode_split", "attn_bwd.order", "attn_bwd.keep_ds", "attn_bwd.split"). Every value it accepts selects
+ * ("lion.variant", "attn.variant", "attn_bwd.variant", "attn.order", "attn.balance", "attn.keep_on", "attn.tail", "attn.decode_split", "attn_bwd.order", "attn_bwd.keep_ds", "attn_bwd.split", "attn_bwd.dq_teams"). Every value it accepts selects
  * code that computes the same function as the default; value -1 restores the default (the measured best). Returns
  * FO_OK, or FO_ERR_UNSUPPORTED for an unknown key or a value that selects nothing. The settings are process-global
  * atomics: a call reads each one once, a call already issued is not affected. fo_tune_get additionally answers
@@ -226,6 +226,10 @@ int fo_attn_bwd_ex(const void* q, const void* k, const void* v, const void* o, c
  * fo_attn_bwd_workspace: the most that any call of the shape can use. No reference counterpart. */
 int64_t fo_attn_bwd_workspace(int B, int H, int Sq, int Sk, int D);
 int64_t fo_attn_bwd_workspace_ex(int B, int H, int Sq, int Sk, int D, int causal, const fo_attn_extras* extras_host);
+/* Which kernels fo_attn_bwd_ws chooses for such a call with so much (aligned) workspace: 0 = the scores are computed again for dQ, else the sum
+ * of what follows; FO_ERR_BAD_SHAPE where the shape is not taken. Launches nothing. */
+enum { FO_ATTN_BWD_KEEPS_DS = 1, FO_ATTN_BWD_SHARES_BLOCKS = 2, FO_ATTN_BWD_DQ_TWO_TEAMS = 4 };
+int fo_attn_bwd_kernels(int B, int H, int Sq, int Sk, int D, int causal, const fo_attn_extras* extras_host, int64_t ws_bytes);
 int fo_attn_bwd_ws(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
                    void* dq, void* dk, void* dv, int B, int H, int Sq, int Sk, int D,
                    const int64_t* const* strides_host, float softmax_scale, int causal, int dtype,

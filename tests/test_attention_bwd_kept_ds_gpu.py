@@ -73,6 +73,7 @@ def test_kept_ds(case, dtype):
     try:
         full = lib.fo_attn_bwd_workspace(B, H, Sq, Sk, D)
         assert full >= small + 2 * B * H * Sq * Sk
+        assert [lib.fo_attn_bwd_kernels(B, H, Sq, Sk, D, int(causal), ex, n) & 1 for n in (full, small)] == [1, 0]      # the forms that run below
         kept, again = backward(full), backward(small)
     finally:
         _lib.tune_set("attn_bwd.keep_ds", -1)

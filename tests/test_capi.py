@@ -167,7 +167,8 @@ def test_tune_hook():
     assert lib.fo_tune_set(b"lion.variant", -1) == 0
     assert lib.fo_tune_set(b"no.such.key", 1) == -8
     # every key the kernels read: default -1 (the library's choice), settable, readable
-    for key, value in ((b"attn.variant", 16), (b"attn_bwd.variant", 0), (b"attn.order", 2), (b"attn.balance", 0), (b"attn.keep_on", 1), (b"attn.tail", 0), (b"attn_bwd.order", 2)):
+    for key, value in ((b"attn.variant", 16), (b"attn_bwd.variant", 0), (b"attn.order", 2), (b"attn.balance", 0), (b"attn.keep_on", 1), (b"attn.tail", 0), (b"attn_bwd.order", 2),
+                       (b"attn_bwd.keep_ds", 0), (b"attn_bwd.keep_ds", 1), (b"attn_bwd.split", 0), (b"attn_bwd.split", 4), (b"attn_bwd.dq_teams", 1), (b"attn_bwd.dq_teams", 2)):
         assert lib.fo_tune_get(key) == -1
         assert lib.fo_tune_set(key, value) == 0 and lib.fo_tune_get(key) == value
         assert lib.fo_tune_set(key, -1) == 0 and lib.fo_tune_get(key) == -1
@@ -186,6 +187,9 @@ def test_tune_hook_accepts_only_kernels_that_compute_the_function():
     assert lib.fo_tune_set(b"attn_bwd.variant", 2) == -8
     assert lib.fo_tune_set(b"attn.keep_on", 3) == -8
     assert lib.fo_tune_set(b"lion.variant", 32) == -8
+    assert lib.fo_tune_set(b"attn_bwd.keep_ds", 2) == -8
+    assert lib.fo_tune_set(b"attn_bwd.split", 1) == -8 and lib.fo_tune_set(b"attn_bwd.split", 5) == -8
+    assert lib.fo_tune_set(b"attn_bwd.dq_teams", 0) == -8 and lib.fo_tune_set(b"attn_bwd.dq_teams", 3) == -8
 
 
 def test_attn_kernel_query_and_stride_limit_without_device_work():
