@@ -68,6 +68,8 @@ _PIPE = r"attn_bwd_dkdv_pipe_kernel"
 _WIDE = r"attn_fwd_wide_kernel.*ELi0ELi\d+ELb[01]ELb[01]EEEvNS_10AttnParamsE"
 ASM_LINTED = {"attn_fwd_bf16_d64.hip": _WIDE, "attn_fwd_bf16_d128.hip": _WIDE, "attn_fwd_f16_d64.hip": _WIDE, "attn_fwd_f16_d128.hip": _WIDE,
               "attn_bwd_bf16_d64.hip": _PIPE, "attn_bwd_bf16_d128.hip": _PIPE, "attn_bwd_f16_d64.hip": _PIPE, "attn_bwd_f16_d128.hip": _PIPE}
+# sources without inline-assembly MFMAs whose direct-to-LDS copies are checked (asm_lint.lint_m0_file; in those above they are as well)
+M0_LINTED = ["attn_bwd_dq_of_ds.hip", "attn_decode.hip"]
 
 
 def _hipcc() -> str:
@@ -103,7 +105,7 @@ def _compile_one(hipcc: str, src: str, extra: list, force: bool, verbose: bool) 
     stale = force or not os.path.exists(obj) or os.path.getmtime(obj) < max(os.path.getmtime(src_path), _newest_header_mtime())
     if not stale:
         return obj
-    if src not in ASM_LINTED:
+    if src not in ASM_LINTED and src not in M0_LINTED:
         _run_hipcc([hipcc] + COMMON_FLAGS + extra + ["-c", src_path, "-o", obj], src, verbose)
         return obj
     # Kernels with inline-assembly MFMAs: first without wait states in front of the MFMAs of the inner loops, keeping
@@ -111,12 +113,12 @@ def _compile_one(hipcc: str, src: str, extra: list, force: bool, verbose: bool) 
     # check finds one, compile again with the wait states.
     from .asm_lint import lint_file, lint_m0_file
 
-    def compile_and_lint(nops: int):
-        _run_hipcc([hipcc] + COMMON_FLAGS + extra + [f"-DFO_MFMA_NOPS={nops}", "-save-temps=obj", "-c", src_path, "-o", obj], src, verbose)
+    def compile_and_lint(defines: list):
+        _run_hipcc([hipcc] + COMMON_FLAGS + extra + defines + ["-save-temps=obj", "-c", src_path, "-o", obj], src, verbose)
         asm = os.path.join(OBJ_DIR, f"{stem}-hip-amdgcn-amd-amdhsa-{ARCH}.s")
         if not os.path.exists(asm):
             raise RuntimeError(f"{src}: {asm} was not produced, the generated assembly cannot be checked")
-        problems = lint_file(asm, ASM_LINTED[src])
+        problems = lint_file(asm, ASM_LINTED[src]) if src in ASM_LINTED else []
         # the direct-to-LDS copies are inline assembly too: M0 written and read back to back has no fallback build, it is
         # an error in the source
         m0_problems = lint_m0_file(asm)
@@ -129,13 +131,16 @@ def _compile_one(hipcc: str, src: str, extra: list, force: bool, verbose: bool) 
             raise RuntimeError(f"{src}: the assembly check found no kernel to look at ({ASM_LINTED[src]!r} is out of date)")
         return problems
 
-    problems = compile_and_lint(0)
+    if src in M0_LINTED:
+        compile_and_lint([])
+        return obj
+    problems = compile_and_lint(["-DFO_MFMA_NOPS=0"])
     if problems:
         if verbose:
             print(f"{src}: {len(problems)} MFMA hazard(s) without wait states, e.g. {problems[0]}\n  -> compiling with wait states", flush=True)
         # the object that is linked is the one that was checked: the build with wait states goes through the same check
         # (a hazard that remains there is an error in the source)
-        problems = compile_and_lint(1)
+        problems = compile_and_lint(["-DFO_MFMA_NOPS=1"])
         if problems:
             raise RuntimeError(f"{src}: {len(problems)} MFMA hazard(s) remain with wait states in front of every MFMA, e.g. {problems[0]}")
     elif verbose:

@@ -52,3 +52,21 @@ def test_lds_dma_right_after_an_m0_write_is_flagged():
     assert not lint(f"s_mov_b32 s4, s5\n{dma}")                          # not M0
     assert not lint("s_mov_b32 m0, s5\nbuffer_load_dword v1, s[8:11], 0 offen")   # not an LDS-DMA
     assert not lint("s_mov_b32 m0, s5\nds_read_b128 v[0:3], v30")
+
+
+def test_every_source_with_lds_copies_is_checked():
+    """... by the build: a source that issues such copies (itself, or through the file it includes) and is in neither list would go unchecked."""
+    import os
+    import re
+
+    from fast_ops_amd import build
+
+    copies = re.compile(r"\bdma(16|4)_\w+\s*\(|_load_lds_|BiasRows<")
+    found = []
+    for src in build.SOURCES:
+        text = open(os.path.join(build.CSRC, src)).read()
+        for inc in re.findall(r'#include "(\w+\.hip)"', text):
+            text += open(os.path.join(build.CSRC, inc)).read()
+        if copies.search(text) and src not in build.INCLUDED_SOURCES:      # (as they stand those hold no kernel)
+            found.append(src)
+    assert len(found) >= 10 and sorted(found) == sorted([*build.ASM_LINTED, *build.M0_LINTED])
