@@ -1763,20 +1763,35 @@ static int64_t ds_bytes_of(int B, int H, int Sq, int Sk) { return (int64_t)B * H
 //   1100 at 96 (155) 144 -> 133, 128 x 600 x 900 at 80 (160) 137 -> 132; 64 x 777 x 1250 at 80 (130) 113.2 -> 113.3, 64 x 1024 at 96 causal (128) 86 -> 88
 //   up to 2 GiB, what a caller's memory is asked for; beyond, the gain shrinks with the traffic that no cache holds: 12 x 8192
 //   causal (1.6 GiB) 639 -> 594, 64 x 4096 causal (2 GiB) 877 -> 846, 512 x 2048 (4 GiB) 3402 -> 3392.
+// With many heads (B H) the launches fill the chip without it, the operands come from memory as well, and dS pays only while the caches hold it:
+//   head_dim above 96: to 96 heads at any size (96 x 3072 x 2048 978 -> 925, x 2048 x 4096, 1.5 GiB, 1285 -> 1291); to 192 not causal to 2048 keys (192 x
+//   1024 x 2048 715 -> 702, x 2048 x 2048 1351 -> 1325), else to 384 MiB (192 x 1024 causal 252 -> 249, 128 x 384 x 4096 456 -> 454; not 192 x 384 x 4096,
+//   576 MiB, 678 -> 688, 160 x 256 x 8192, 640, 911 -> 938, 192 x 1536 x 2048 causal, 1152, 504 -> 518); more heads to 512 keys (384 x 512 248 -> 238,
+//   768 x 2048 x 512 1634 -> 1544), not beyond: 256 x 128 x 4096 476 -> 516, 256 x 256 x 2048 337 -> 350, 384 x 384 x 2048 658 -> 682, 512 x 128 x
+//   1024 256 -> 261, 768 x 1024 causal 993 -> 1025; between lie gains as well (320 x 320 x 1024 292 -> 280)
+//   with dropout, or a bias with a query stride, which the other dQ kernel pays for a second time, with any number of heads: 384 x 1536, dropout
+//   1615 -> 1564, causal 991 -> 987; 384 x 1536 with a bf16 bias 1706 -> 1644, causal 1096 -> 1034; 384 x 128 x 2048 404 -> 404
+//   up to 96: to 64 heads at any size (48 x 3072 x 4096 801 -> 785, 24 x 4096 281 -> 266), to 128 to 192 MiB (128 x 128 x 4096 248 -> 237, 96 x 1024 163 -> 160;
+//   not 128 x 384 x 4096, 384 MiB, 392 -> 407, 96 x 2048 x 4096 1061 -> 1157), not with more: 160 x 256 x 2048 208 -> 217, 256 x 128 x 2048 211 ->
+//   230, 192 x 2048 x 1024 594 -> 636, 384 x 1024 633 -> 687, 768 x 1024 causal 845 -> 933
 constexpr int64_t kDsFromBytes = 96ll << 20, kDsMaxBytes = 2ll << 30;
 constexpr int kDsFromKeys = 1536;
-static bool bwd_keeps_ds(int B, int H, int Sq, int Sk, int D) {
+struct BwdCall { bool causal, drop; BiasParams bias; };
+static int64_t ds_bytes_that_pay(int64_t heads, int Sk, int D, const BwdCall& c) {
+  if (D <= 96) return heads <= 64 ? kDsMaxBytes : heads <= 128 ? 192ll << 20 : 0;
+  if (heads <= 96 || Sk <= 512 || c.drop || (c.bias.ptr != nullptr && c.bias.strides[2] != 0)) return kDsMaxBytes;
+  return heads > 192 ? 0 : !c.causal && Sk <= 2048 ? kDsMaxBytes : 384ll << 20;
+}
+// The calls that can keep it are those that launch_bwd gives to the pipelined dK/dV kernel. The others (a bias with a query stride whose tiles
+// cannot be copied, or together with dropout; head dims off 128 with any bias or dropout) have no use for the memory.
+static bool bwd_keeps_ds(int B, int H, int Sq, int Sk, int D, const BwdCall& c) {
   const int asked = tune(g_attn_bwd_keep_ds);
   if (asked == 0 || D <= 64 || tune(g_attn_bwd_variant) == 0 || (int64_t)B * H > (1 << 20) || ds_key_blocks(Sk) * ds_query_tiles(Sq) > kDsMaxBytes / kDsChunk) return false;
+  if (D != 128 && (c.drop || c.bias.ptr != nullptr)) return false;
+  if (c.bias.ptr != nullptr && c.bias.strides[2] != 0 && (!c.bias.dma_ok || c.drop)) return false;
   const int64_t bytes = ds_bytes_of(B, H, Sq, Sk);
-  return bytes <= kDsMaxBytes && (asked == 1 || Sk >= kDsFromKeys || bytes >= (D > 96 ? kDsFromBytes : kDsFromBytes + kDsFromBytes / 2));
-}
-
-// ... and for which calls: those that launch_bwd gives to the pipelined dK/dV kernel. The others (a bias with a query stride whose tiles cannot be
-// copied, or together with dropout; head dims off 128 with any bias or dropout) have no use for the memory.
-static bool bwd_form_keeps_ds(int D, bool drop, const BiasParams& bias) {
-  if (bias.ptr == nullptr) return D == 128 || !drop;
-  return D == 128 && (bias.strides[2] == 0 || (bias.dma_ok && !drop));
+  if (asked == 1) return bytes <= kDsMaxBytes;
+  return bytes <= ds_bytes_that_pay((int64_t)B * H, Sk, D, c) && (Sk >= kDsFromKeys || bytes >= (D > 96 ? kDsFromBytes : kDsFromBytes + kDsFromBytes / 2));
 }
 static BiasParams make_bias(const void* bias, const int64_t* strides, bool is_f32) {
   BiasParams b;
@@ -1813,13 +1828,13 @@ static int64_t part_bytes_of(int B, int H, int Sq, int Sk, bool causal) {
 
 // What a call does with its workspace: where dS lies in it (0: not kept), and the sums of shared key blocks (plan null: none are shared).
 struct BwdForm { int64_t ds_at, part_at; const DkdvPlan* plan; };
-static BwdForm bwd_form(int B, int H, int Sq, int Sk, int D, bool causal, bool drop, const BiasParams& bias, const void* ws, int64_t ws_bytes) {
+static BwdForm bwd_form(int B, int H, int Sq, int Sk, int D, const BwdCall& c, const void* ws, int64_t ws_bytes) {
   BwdForm f = {0, 0, nullptr};
-  if (ws_bytes <= 0 || ((uintptr_t)ws & 15u) || !bwd_keeps_ds(B, H, Sq, Sk, D) || !bwd_form_keeps_ds(D, drop, bias)) return f;
+  if (ws_bytes <= 0 || ((uintptr_t)ws & 15u) || !bwd_keeps_ds(B, H, Sq, Sk, D, c)) return f;
   const int64_t rows = rows_ws_bytes(B, H, Sq), end = rows + ds_bytes_of(B, H, Sq, Sk);
   if (ws_bytes < end) return f;
   f.ds_at = rows;
-  const DkdvPlan& plan = dkdv_plan(B, H, Sq, Sk, causal);
+  const DkdvPlan& plan = dkdv_plan(B, H, Sq, Sk, c.causal);
   if (plan.n_items > 0 && ws_bytes >= end + plan.n_parts * (int64_t)B * H * kPartBytes) { f.part_at = end; f.plan = &plan; }
   return f;
 }
@@ -1868,7 +1883,7 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   p.q = q; p.k = k; p.v = v; p.o = o; p.d_o = d_o; p.lse = lse; p.delta = delta_ws; p.nlse = delta_ws + (int64_t)B * H * Sq; p.dq = dq; p.dk = dk; p.dv = dv;
   p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.d = D;
   p.bias = make_bias(bias, bias_strides, bias_dtype == FO_DTYPE_F32);
-  const BwdForm form = bwd_form(B, H, Sq, Sk, D, causal != 0, dropout_p > 0.0f, p.bias, delta_ws, ws_bytes);
+  const BwdForm form = bwd_form(B, H, Sq, Sk, D, BwdCall{causal != 0, dropout_p > 0.0f, p.bias}, delta_ws, ws_bytes);
   p.ds = form.ds_at > 0 ? (char*)delta_ws + form.ds_at : nullptr;
   p.n_items = p.n_merges = 0;
   p.part = nullptr;
@@ -1932,28 +1947,32 @@ extern "C" int fo_attn_bwd_ex(const void* q, const void* k, const void* v, const
 static bool bwd_ws_shape_ok(int B, int H, int Sq, int Sk, int D) {
   return B > 0 && H > 0 && Sq > 0 && Sk > 0 && D >= 8 && D <= 128 && D % 8 == 0 && (int64_t)B * H <= (1ll << 40) / Sq;
 }
-extern "C" int64_t fo_attn_bwd_workspace_ex(int B, int H, int Sq, int Sk, int D, int causal, const fo_attn_extras* extras) {
+static BwdCall bwd_call(int causal, const fo_attn_extras* x) {
+  if (!x) return BwdCall{causal != 0, false, make_bias(nullptr, nullptr, false)};
+  return BwdCall{causal != 0, x->dropout_p > 0.0f, make_bias(x->bias, x->bias_strides, x->bias_dtype == FO_DTYPE_F32)};
+}
+static int64_t bwd_ws_bytes(int B, int H, int Sq, int Sk, int D, const BwdCall& c) {
   if (!bwd_ws_shape_ok(B, H, Sq, Sk, D)) return 0;
-  const fo_attn_extras none = {};
-  const fo_attn_extras& x = extras ? *extras : none;
-  if (!bwd_keeps_ds(B, H, Sq, Sk, D) || !bwd_form_keeps_ds(D, x.dropout_p > 0.0f, make_bias(x.bias, x.bias_strides, x.bias_dtype == FO_DTYPE_F32)))
-    return rows_ws_bytes(B, H, Sq);
-  return rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk) + part_bytes_of(B, H, Sq, Sk, causal != 0);
+  if (!bwd_keeps_ds(B, H, Sq, Sk, D, c)) return rows_ws_bytes(B, H, Sq);
+  return rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk) + part_bytes_of(B, H, Sq, Sk, c.causal);
+}
+extern "C" int64_t fo_attn_bwd_workspace_ex(int B, int H, int Sq, int Sk, int D, int causal, const fo_attn_extras* extras) {
+  return bwd_ws_bytes(B, H, Sq, Sk, D, bwd_call(causal, extras));
+}
+extern "C" int64_t fo_attn_bwd_workspace(int B, int H, int Sq, int Sk, int D) {
+  int64_t most = 0;
+  for (int i = 0; i < 4; ++i) {        // (whatever keeps dS at a shape: one of these does, and a bias asks for no more)
+    const int64_t n = bwd_ws_bytes(B, H, Sq, Sk, D, BwdCall{(i & 1) != 0, (i & 2) != 0, make_bias(nullptr, nullptr, false)});
+    most = n > most ? n : most;
+  }
+  return most;
 }
 extern "C" int fo_attn_bwd_kernels(int B, int H, int Sq, int Sk, int D, int causal, const fo_attn_extras* extras, int64_t ws_bytes) {
   if (!bwd_ws_shape_ok(B, H, Sq, Sk, D)) return FO_ERR_BAD_SHAPE;
-  const fo_attn_extras none = {};
-  const fo_attn_extras& x = extras ? *extras : none;
-  const BwdForm f = bwd_form(B, H, Sq, Sk, D, causal != 0, x.dropout_p > 0.0f, make_bias(x.bias, x.bias_strides, x.bias_dtype == FO_DTYPE_F32), nullptr, ws_bytes);
+  const BwdForm f = bwd_form(B, H, Sq, Sk, D, bwd_call(causal, extras), nullptr, ws_bytes);
   if (f.ds_at == 0) return 0;
   return FO_ATTN_BWD_KEEPS_DS | (f.plan != nullptr ? FO_ATTN_BWD_SHARES_BLOCKS : 0) |
          (dq_two_teams((int64_t)B * H, Sq, Sk, causal != 0, f.plan != nullptr ? f.plan->n_merges : 0) ? FO_ATTN_BWD_DQ_TWO_TEAMS : 0);
-}
-extern "C" int64_t fo_attn_bwd_workspace(int B, int H, int Sq, int Sk, int D) {
-  if (!bwd_ws_shape_ok(B, H, Sq, Sk, D)) return 0;
-  if (!bwd_keeps_ds(B, H, Sq, Sk, D)) return rows_ws_bytes(B, H, Sq);
-  const int64_t causal = part_bytes_of(B, H, Sq, Sk, true), full = part_bytes_of(B, H, Sq, Sk, false);
-  return rows_ws_bytes(B, H, Sq) + ds_bytes_of(B, H, Sq, Sk) + (causal > full ? causal : full);
 }
 
 extern "C" int fo_attn_bwd_ws(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,

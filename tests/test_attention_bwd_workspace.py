@@ -56,6 +56,33 @@ def test_calls_that_do_not(causal):
         _lib.tune_set("attn_bwd.variant", -1)
 
 
+def test_sizes_at_which_ds_is_kept():
+    """... are those where that is faster: with many heads only while the caches hold dS, with very many not beyond 512 keys."""
+    lib = _lib.load()
+    def kept(heads, Sq, Sk, D, causal=0, bias=None, p=0.0):
+        ex = _AttnExtras()
+        if bias is not None:
+            ex.bias, ex.bias_strides, ex.bias_dtype = bias[0], (ctypes.c_int64 * 3)(*bias[1]), bias[2]
+        ex.dropout_p = p
+        room = lib.fo_attn_bwd_workspace(1, heads, Sq, Sk, D)
+        got = lib.fo_attn_bwd_kernels(1, heads, Sq, Sk, D, causal, ctypes.byref(ex), room)
+        assert got == lib.fo_attn_bwd_kernels(1, heads, Sq, Sk, D, causal, ctypes.byref(ex), 4 << 30)      # no call can use more
+        return got & 1
+
+    for shape in [(96, 2048, 4096, 128), (4, 1, 1536, 128), (160, 384, 2048, 128), (192, 1024, 1024, 104), (192, 2048, 2048, 128), (192, 1024, 1024, 128, 1),
+                  (384, 512, 512, 128), (48, 3072, 4096, 96), (128, 128, 4096, 72), (384, 1024, 1024, 128, 0, None, 0.1), (384, 1024, 1024, 128, 1, TILES)]:
+        assert kept(*shape) == 1, shape
+    for shape in [(192, 384, 4096, 128), (192, 2048, 2048, 128, 1), (256, 128, 4096, 128), (384, 384, 2048, 104), (512, 256, 1024, 128),
+                  (384, 1024, 1024, 128, 0, KEY), (16, 1024, 1024, 128), (2, 4096, 1535, 96),
+                  (128, 384, 4096, 96), (160, 256, 2048, 96), (384, 1024, 1024, 72), (129, 1024, 1024, 96)]:
+        assert kept(*shape) == 0, shape
+    _lib.tune_set("attn_bwd.keep_ds", 1)
+    try:
+        assert kept(384, 1024, 1024, 72) == 1
+    finally:
+        _lib.tune_set("attn_bwd.keep_ds", -1)
+
+
 def test_shapes_that_are_not_taken():
     ask = lambda *a: (_lib.load().fo_attn_bwd_workspace_ex(*a, 0, None), _lib.load().fo_attn_bwd_workspace(*a))
     big = 2 ** 31 - 1
