@@ -866,7 +866,7 @@ static_assert(softmax_grad_jobs_fit(16) && softmax_grad_jobs_fit(12) && softmax_
 //   1: S, then dP of block 0 | 2: S, then dP of block 1 | 3: dV, dK of block 0 | 4: dV, dK of block 1
 // as micro-groups of one MFMA, the LDS read of the A operand needed kFragAhead groups later and a share of the tile's
 // softmax-gradient arithmetic (see tile_body), fenced so that the compiler keeps the groups apart. The accumulators of
-// S and dP do not start from zero but from -LSE / scale and -delta of their rows (written by the dQ kernel, read from
+// S and dP do not start from zero but from -LSE / scale and -delta of their rows (written by the launch before, read from
 // LDS straight into the registers while they are idle), so that P = exp2((QK^T - LSE / scale) c) and dS = P (dP - delta)
 // are two multiplications and the exponential.
 // KBIAS: with a bias that is the same for every query (query stride 0): a lane owns a key, so the bias is one value per
@@ -1642,7 +1642,7 @@ static int launch_bwd(const AttnBwdParams& p, hipStream_t s) {
     if (group <= 0 || group > n_bh) group = n_bh;
     q.head_group = (int)group;
   }
-  // (delta is computed by the dQ kernel, which the dK/dV kernel follows)
+  // (delta is computed by the dQ kernel, which the dK/dV kernel follows; where dS is kept, by the rows' kernel before both)
   if constexpr (BIAS) {
     if (key_bias) {
       if constexpr (D == 128) {

@@ -222,6 +222,7 @@ int fo_attn_bwd_ex(const void* q, const void* k, const void* v, const void* o, c
  * fp32 sums of dK and dV behind dS (part of the answer; with room for dS alone each block stays whole).
  * Kept at head_dim above 64: without a bias (off 128 also without dropout), and at 128 with a bias that has no query stride, or
  * one on 16-byte boundaries without dropout. With less memory the call computes what fo_attn_bwd_ex computes.
+ * (A causal call is answered with the whole rectangle of queries and keys, of which it uses the half below the diagonal.)
  * (Of the current device, as the call: how the blocks are shared depends on the number of its compute units.)
  * fo_attn_bwd_workspace: the most that any call of the shape can use. No reference counterpart. */
 int64_t fo_attn_bwd_workspace(int B, int H, int Sq, int Sk, int D);
