@@ -11,6 +11,7 @@ import torch
 
 from fast_ops.flash_attention.flash_attention import flash_attn
 from fast_ops_amd import _lib
+from fast_ops_amd.flash_attention.flash_attention import attn_bwd_strided, attn_fwd_strided
 from oracle.attention_oracle import attention_bwd_oracle
 from test_attention_dropout_forms_gpu import _state_with_partial_rows
 
@@ -87,3 +88,48 @@ def test_kept_ds(case, dtype):
     for name, a, b in zip(("dQ", "dK", "dV"), kept, again):
         a, b = a.float(), b.float()
         assert (a - b).norm().item() <= (2e-3 if dtype == torch.bfloat16 else 3e-4) * b.norm().item() + 4e-4, name
+
+
+def _operand(kind, n, H, D, g, dtype):
+    """[1, n, H, D] in memory as a program may have it: dense; one of three in a packed projection; heads first; one head seen by all;
+    rows as far apart as 32-bit offsets do not reach."""
+    new = lambda *shape: torch.randn(*shape, generator=g, device=DEV).to(dtype)
+    if kind == "packed":
+        return new(1, n, 3, H, D)[:, :, 1]
+    if kind == "heads_first":
+        return new(1, H, n, D).transpose(1, 2)
+    if kind == "one_head":
+        return new(1, n, 1, D).expand(1, n, H, D)
+    if kind == "far_rows":
+        far = torch.empty(((n - 1) << 23) + H * D, dtype=dtype, device=DEV).as_strided((1, n, H, D), (8, 1 << 23, D, 1))
+        return far.copy_(new(1, n, H, D))
+    return new(1, n, H, D)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("q_kind,kv_kind,go_kind,Sq,Sk,D,causal,p", [
+    ("packed", "packed", "dense", 300, 300, 128, True, 0.0), ("heads_first", "heads_first", "heads_first", 129, 391, 80, False, 0.0),
+    ("dense", "one_head", "packed", 257, 450, 128, False, 0.0), ("packed", "one_head", "heads_first", 333, 97, 104, True, 0.0),
+    ("dense", "far_rows", "dense", 200, 70, 128, False, 0.0), ("far_rows", "dense", "far_rows", 70, 333, 96, False, 0.0),
+    ("far_rows", "far_rows", "packed", 75, 75, 128, True, 0.4), ("packed", "heads_first", "heads_first", 700, 1300, 128, False, 0.4)])
+def test_layouts(q_kind, kv_kind, go_kind, Sq, Sk, D, causal, p, dtype):
+    H = 3
+    g = torch.Generator(device=DEV).manual_seed(Sq + Sk + D)
+    q, k, v = (_operand(kind, n, H, D, g, dtype) for kind, n in ((q_kind, Sq), (kv_kind, Sk), (kv_kind, Sk)))
+    go = _operand(go_kind, Sq, H, D, g, dtype)
+    drop = (p, 987654321, 4004 * 17) if p else None
+    o, lse = attn_fwd_strided(q, k, v, (0, 2, 1, 3), causal, None, drop)
+    grads = {}
+    try:
+        for keep, split in ((0, 0), (1, 0), (1, 3)):
+            _lib.tune_set("attn_bwd.keep_ds", keep)
+            _lib.tune_set("attn_bwd.split", split)
+            grads[keep, split] = attn_bwd_strided(q, k, v, o, lse, go, (0, 2, 1, 3), causal, None, drop)
+    finally:
+        _lib.tune_set("attn_bwd.keep_ds", -1)
+        _lib.tune_set("attn_bwd.split", -1)
+    for form in ((1, 0), (1, 3)):
+        for name, a, b in zip(("dQ", "dK", "dV"), grads[form], grads[0, 0]):
+            a, b = a.double(), b.double()
+            assert bool(torch.isfinite(a).all()), (form, name)
+            assert (a - b).norm().item() <= (2e-3 if dtype == torch.bfloat16 else 3e-4) * b.norm().item() + 4e-4, (form, name)      # (as above)

@@ -22,7 +22,9 @@ def _step(params, opt, go, causal):
     opt.step()
 
 
-@pytest.mark.parametrize("shape,causal", [((2, 4, 512, 64), True), ((1, 8, 1024, 128), False)])
+@pytest.mark.parametrize("shape,causal", [((2, 4, 512, 64), True), ((1, 8, 1024, 128), False),
+                                          # the backward that keeps dS in a workspace of the graph's own: key blocks shared, dQ in two teams
+                                          ((1, 12, 3072, 128), True), ((1, 4, 2048, 128), False)])
 def test_training_step_replayed_from_a_graph_equals_eager_steps(shape, causal):
     B, H, S, D = shape
     gen = torch.Generator().manual_seed(S + D)

@@ -14,6 +14,7 @@ import torch
 
 from fast_ops.flash_attention.flash_attention import multi_head_attention
 from fast_ops.lion.lion_optimizer import Lion
+from fast_ops_amd import _lib
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -25,6 +26,9 @@ WORKLOADS = [
     (3, 5, 700, 64, torch.float16, False),
     (4, 32, 2048, 128, torch.bfloat16, True),
     (2, 3, 515, 40, torch.bfloat16, True),
+    # and two whose backward keeps dS in a workspace of its own, with key blocks that workgroups share
+    (1, 4, 2048, 128, torch.bfloat16, True),
+    (1, 6, 1700, 96, torch.float16, False),
 ]
 PARAM_SIZES = [(257, 129), (8192,), (40000,), (3,)]
 
@@ -97,6 +101,39 @@ def test_four_host_threads_on_their_own_streams():
         assert len(results[w]) == len(alone[w])
         for i, (a, b) in enumerate(zip(results[w], alone[w])):
             assert _same(a, b), f"worker {w}, tensor {i}: differs from the single-threaded run"
+
+
+def test_two_host_threads_that_keep_ds():
+    lib = _lib.load()
+    for w in (4, 5):
+        B, H, S, D, _, causal = WORKLOADS[w]
+        assert lib.fo_attn_bwd_kernels(B, H, S, S, D, int(causal), None, lib.fo_attn_bwd_workspace_ex(B, H, S, S, D, int(causal), None)) & 1
+    iters = 50
+    alone = [_loop(w, iters) for w in (4, 5)]
+    torch.cuda.synchronize()
+    results, errors = [None, None], []
+    start = threading.Barrier(2)
+
+    def work(i):
+        try:
+            s = torch.cuda.Stream(device=DEV)
+            with torch.cuda.stream(s):
+                start.wait()
+                results[i] = _loop(4 + i, iters)
+            s.synchronize()
+        except BaseException as e:                      # noqa: BLE001 - reported by the main thread
+            errors.append((i, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=300)
+    assert not errors, errors
+    torch.cuda.synchronize()
+    for i in range(2):
+        for j, (a, b) in enumerate(zip(results[i], alone[i])):
+            assert _same(a, b), f"worker {4 + i}, tensor {j}: differs from the single-threaded run"
 
 
 def test_two_streams_from_one_thread():
