@@ -896,8 +896,8 @@ static_assert(softmax_grad_jobs_fit(16) && softmax_grad_jobs_fit(12) && softmax_
 // SHIFT (DS without TBIAS): dQ is made of this kernel's P then, and P has to be as exact as the dQ kernel's own. So S starts from zero (KBIAS: from
 // bias / scale, sixteen registers that stay as they are), and -LSE log2 e, read from LDS where -LSE / scale is otherwise, joins in the exponent:
 // P = exp2(S c + shift), a fused multiply-add in the place of the multiplication. Started from -LSE / scale, S is summed at the ulp of the LSE: fp32
-// error of P at 4096 unit normal keys 7.4e-7 rms instead of 3.0e-7. (This kernel alone, start values -> shift: 12 heads x 4096 with key bias and
-// dropout 287 -> 280 us, without 235 -> 234, 12 x 3072 causal 73 -> 74, 48 x 1450 x 1100 at head_dim 96 83 -> 84.)
+// error of P at 4096 unit normal keys 7.4e-7 rms instead of 3.0e-7. (This kernel alone, start values -> shift, over several runs in turn: 12 heads x
+// 4096 with key bias and dropout 269-291 -> 272-283 us, without 224-237 -> 227-234, 12 x 3072 causal 70-73 -> 72-74, 48 x 1450 x 1100 at head_dim 96 83 -> 84.)
 template <typename T, int D, bool CAUSAL, bool KBIAS = false, bool DROP = false, bool PAD = false, int LIVE = D, int TBIAS = 0, bool DS = false>
 __global__ void __launch_bounds__(kBwdWaves * 64) attn_bwd_dkdv_pipe_kernel(const AttnBwdParams prm) {
   static_assert(TBIAS == 0 || !(KBIAS || DROP || PAD), "not combined");
