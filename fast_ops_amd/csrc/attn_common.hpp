@@ -162,8 +162,11 @@ inline DropoutParams make_dropout(float p, uint32_t seed, uint64_t rng_offset) {
 // element per lane. (Hashing such spans whole, or such tiles whole, is little work in total, but all of it falls on a few
 // workgroups that the launch then waits for: 193 and 159 us at 12 heads x 4096 keys, where no dropout takes 124 us.)
 // Forward at p = 0.1, head_dim 128, hashing every element -> this: 12 heads x 4096 keys 181 -> 133 us (no dropout 124), x 8192
-// 562 -> 435 (364), x 2048 causal 62 -> 38 (32); head_dim 64, 8 x 12 heads x 1024 causal 44 -> 24 (25). What is left is the
-// workgroups whose rows the mask's bands begin or end in, and one branch per step for the others.
+// 562 -> 435 (364), x 2048 causal 62 -> 38 (32); head_dim 64, 8 x 12 heads x 1024 causal 44 -> 24 (25). What was left is the
+// workgroups whose rows the mask's bands begin or end in, for which a launch of one workgroup per unit waits: the pipelined forward
+// kernel reads the mask as words that are always there (Words) instead of asking every step whether it applies one, and the verdicts
+// of a span's tiles are worked out together (look_at_span), over the tests per tile: 12 heads x 4096 132 -> 129 -> 124 us (no dropout
+// 105), x 8192 437 -> 427 -> 410 (357), 6 x 3000 64 -> 59 -> 57 (44).
 constexpr int kDropSpanTiles = 1024 / 64;
 template <int QB>
 struct DropRows {
@@ -172,6 +175,7 @@ struct DropRows {
   bool by_tile = false;
   uint32_t bits[QB][2];                 // all ones / all zeros: the lane's row of block b is kept / dropped; kMasked: the lane's row of block b: bit (r & 3) + 8 (r >> 2) of word kb = the element in register r of
                                         // the 32-key block kb is kept
+  uint32_t tiles[QB];                   // by_tile: bit t = the lane's row of block b is kept over tile t of the span, bit 16 + t = dropped
   static __device__ __forceinline__ uint32_t index(const DropoutParams& d, int bh, int Sq, int Sk, int row, int key) {
     return d.offset + ((uint32_t)bh * (uint32_t)Sq + (uint32_t)row) * (uint32_t)Sk + (uint32_t)key;
   }
@@ -180,37 +184,103 @@ struct DropRows {
   __device__ __forceinline__ void look(const P& d_in, int bh, int Sq, int Sk, int row0, int tile) {
     if (__builtin_expect(tile % kDropSpanTiles == 0, 0)) {      // (laid out away from the tile loops)
       const DropoutParams d = {d_in.seed, d_in.threshold, d_in.offset, 1.0f, 1.0f, 0.0f};
-      by_tile = look_at<10>(d, bh, Sq, Sk, row0, tile * 64);
+      look_at_span(d, bh, Sq, Sk, row0, tile * 64);
     }
     if (__builtin_expect(by_tile, 0)) {
       const DropoutParams d = {d_in.seed, d_in.threshold, d_in.offset, 1.0f, 1.0f, 0.0f};
-      look_at<6>(d, bh, Sq, Sk, row0, tile * 64);
+      look_at_tile(d, bh, Sq, Sk, row0, tile);
     }
   }
-  // 2^L keys from key0 on; true if some row is neither kept nor dropped as a whole (L = 6: its bits are then hashed)
-  template <int L>
-  __device__ __forceinline__ bool look_at(const DropoutParams& d, int bh, int Sq, int Sk, int row0, int key0) {
+  // The next kDropSpanTiles tiles from key0 on as a whole; where some row is neither kept nor dropped over all of them, every row's
+  // verdict for each of the tiles. A tile's 64 elements lie in two of the 64-element blocks of dropout_block, neighbours share one: 17
+  // blocks for the 16 tiles, nine by each half of the wave (which hold the same rows).
+  __device__ __forceinline__ void look_at_span(const DropoutParams& d, int bh, int Sq, int Sk, int row0, int key0) {
     const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
     bool any_mixed = false, any_keep = false, any_drop = false;
 #pragma unroll
     for (int b = 0; b < QB; ++b) {
-      const int v = dropout_run<L>(index(d, bh, Sq, Sk, row0 + 32 * b + l32, key0), 1u << L, d.seed, d.threshold);
+      const int v = dropout_run<10>(index(d, bh, Sq, Sk, row0 + 32 * b + l32, key0), 64 * kDropSpanTiles, d.seed, d.threshold);
       bits[b][0] = bits[b][1] = v == kKeepAll ? 0xFFFFFFFFu : 0u;
       any_keep |= __builtin_amdgcn_ballot_w64(v == kKeepAll) != 0;
       any_drop |= __builtin_amdgcn_ballot_w64(v == kDropAll) != 0;
-      uint32_t mixed = (uint32_t)__builtin_amdgcn_ballot_w64(v == kDropMixed);      // (both halves of the wave hold the same rows)
-      any_mixed |= mixed != 0;
-      if constexpr (L == 6) {
-        while (mixed != 0) {
-          const int i = __builtin_ctz(mixed);
-          mixed &= mixed - 1;
-          const uint64_t k = __builtin_amdgcn_ballot_w64(dropout_keep(index(d, bh, Sq, Sk, row0 + 32 * b + i, key0 + lane), d.seed, d.threshold));
-          if (l32 == i) { bits[b][0] = (uint32_t)k >> (4 * hh); bits[b][1] = (uint32_t)(k >> 32) >> (4 * hh); }
-        }
+      any_mixed |= __builtin_amdgcn_ballot_w64(v == kDropMixed) != 0;
+    }
+    state = any_keep && any_drop ? kRows : any_keep ? kKeepAll : kDropAll;
+    by_tile = any_mixed;
+    if (!any_mixed) return;
+    constexpr int kHalf = kDropSpanTiles / 2;
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      uint32_t at = index(d, bh, Sq, Sk, row0 + 32 * b + l32, key0 + 64 * kHalf * hh), keep = 0u, drop = 0u;
+#pragma unroll 1
+      for (int i = 0; i <= kHalf; ++i, at += 64u) {
+        const int v = dropout_block<6>(at, d.seed, d.threshold);
+        keep |= (v == kKeepAll ? 1u : 0u) << i;
+        drop |= (v == kDropAll ? 1u : 0u) << i;
+      }
+      keep &= keep >> 1;
+      drop &= drop >> 1;
+      const uint32_t mine = (keep & ((1u << kHalf) - 1u)) | (drop & ((1u << kHalf) - 1u)) << kDropSpanTiles;
+      const uint32_t other = __builtin_bit_cast(uint32_t, half_swap(__builtin_bit_cast(float, mine)));
+      tiles[b] = hh ? other | mine << kHalf : mine | other << kHalf;
+    }
+  }
+  // one of those tiles; its rows that are neither are hashed
+  __device__ __forceinline__ void look_at_tile(const DropoutParams& d, int bh, int Sq, int Sk, int row0, int tile) {
+    const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5, t = tile % kDropSpanTiles;
+    uint64_t mixed_rows = 0, keep_rows = 0, drop_rows = 0;
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      const bool keep = (tiles[b] >> t) & 1u, drop_it = (tiles[b] >> (t + kDropSpanTiles)) & 1u;
+      bits[b][0] = bits[b][1] = keep ? 0xFFFFFFFFu : 0u;
+      keep_rows |= __builtin_amdgcn_ballot_w64(keep);
+      drop_rows |= __builtin_amdgcn_ballot_w64(drop_it);
+      const uint64_t neither = __builtin_amdgcn_ballot_w64(!keep && !drop_it);
+      mixed_rows |= neither;
+      uint32_t mixed = (uint32_t)neither;                       // (both halves of the wave hold the same rows)
+      while (mixed != 0) {
+        const int i = __builtin_ctz(mixed);
+        mixed &= mixed - 1;
+        const uint64_t k = __builtin_amdgcn_ballot_w64(dropout_keep(index(d, bh, Sq, Sk, row0 + 32 * b + i, tile * 64 + lane), d.seed, d.threshold));
+        if (l32 == i) { bits[b][0] = (uint32_t)k >> (4 * hh); bits[b][1] = (uint32_t)(k >> 32) >> (4 * hh); }
       }
     }
-    state = any_mixed ? kMasked : any_keep && any_drop ? kRows : any_keep ? kKeepAll : kDropAll;
-    return any_mixed;
+    state = mixed_rows != 0 ? kMasked : keep_rows != 0 && drop_rows != 0 ? kRows : keep_rows != 0 ? kKeepAll : kDropAll;
+  }
+  // What the pipelined forward kernel keeps of the state: an AND mask per pair of P values, word [kb][b][r / 2] for registers r and r + 1 of
+  // 32-key block kb. Set where a span begins and at the tiles of a span that is looked at tile by tile; nothing else of a tile asks
+  // what the state is.
+  typedef uint32_t Words[2][QB][8];
+  template <typename P>
+  __device__ __forceinline__ void look(const P& d_in, int bh, int Sq, int Sk, int row0, int tile, Words& words) {
+    if (__builtin_expect(tile % kDropSpanTiles != 0 && !by_tile, 1)) return;
+    look(d_in, bh, Sq, Sk, row0, tile);
+    if (state == kMasked) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int b = 0; b < QB; ++b)
+#pragma unroll
+          for (int w = 0; w < 8; ++w) {
+            const int at = 2 * (w & 1) + 8 * (w >> 1);
+            const uint32_t lo = (uint32_t)((int)(bits[b][kb] << (31 - at)) >> 31), hi = (uint32_t)((int)(bits[b][kb] << (30 - at)) >> 31);
+            words[kb][b][w] = (lo & 0xFFFFu) | (hi & 0xFFFF0000u);
+          }
+    } else {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int b = 0; b < QB; ++b)
+#pragma unroll
+          for (int w = 0; w < 8; ++w) words[kb][b][w] = bits[b][0];
+    }
+    // (opaque: the words stay in registers as they are)
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int b = 0; b < QB; ++b)
+#pragma unroll
+        for (int w = 0; w < 8; ++w) asm volatile("" : "+v"(words[kb][b][w]));
   }
   // P of the 32-key block kb as two B operands (registers 0..7 and 8..15) per block of rows. (One branch, straight code where
   // whole rows are dropped: every taken branch holds up a wave that is alone on its SIMD, and with one per case and block a

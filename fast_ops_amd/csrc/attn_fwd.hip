@@ -960,6 +960,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   static_assert(KSTEPS % RD == 0, "fragment ring");
   i32x4 KF[RD], VF[RD];        // LDS fragment rings, refilled RD fragments ahead of use
   DropRows<QB> drop;
+  typename DropRows<QB>::Words drop_words;
   float m_run[QB], l_run[QB];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) { m_run[qb] = -INFINITY; l_run[qb] = 0.0f; }
@@ -1105,6 +1106,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
           if (e & 1) {
             const vec2 pk = {(T)ex[e - 1], (T)ex[e]};
             int pki = __builtin_bit_cast(int, pk);
+            if constexpr (DROP) pki &= (int)drop_words[P][b2][r >> 1];  // (after the row sum: flash_attention_triton.py:216-219)
             asm volatile("" : "+v"(pki));
             PF[P][b2][r >> 3][(r & 7) >> 1] = pki;
           }
@@ -1153,7 +1155,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
           ps += p0;
           ps += p1;
           const vec2 pk = {(T)p0, (T)p1};
-          PF[P][b2][r >> 3][(r & 7) >> 1] = __builtin_bit_cast(int, pk);
+          PF[P][b2][r >> 3][(r & 7) >> 1] = DROP ? __builtin_bit_cast(int, pk) & (int)drop_words[P][b2][r >> 1] : __builtin_bit_cast(int, pk);
         }
         psum[b2] = ps;
         m_run[b2] = m_new;
@@ -1165,19 +1167,9 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     }
 #pragma unroll
     for (int b2 = 0; b2 < QB; ++b2) l_run[b2] += psum[b2];
-    if constexpr (DROP) {
-      if (__builtin_expect(drop.state != kKeepAll, 0)) {
-        drop.apply(P, PF[P]);
-        // (pinned here, with the wait states the next MFMAs need between a VALU write and their read)
-#pragma unroll
-        for (int b2 = 0; b2 < QB; ++b2) asm volatile("" : "+v"(PF[P][b2][0]), "+v"(PF[P][b2][1]));
-      }
-      asm volatile("s_nop 1");
-      __builtin_amdgcn_sched_barrier(0);
-    }
   };
   auto drop_look = [&](int j) {
-    if constexpr (DROP) drop.look(prm.drop, bh, Sq, Sk, q0w, j);
+    if constexpr (DROP) drop.look(prm.drop, bh, Sq, Sk, q0w, j, drop_words);
   };
   using std::integral_constant;
   typedef integral_constant<int, 0> P0;
