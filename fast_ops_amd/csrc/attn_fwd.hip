@@ -670,9 +670,24 @@ __host__ __device__ inline int wide_items(int n_qblk, bool causal) { return caus
 constexpr int kVBiasKeys = 8192;
 constexpr float kNoKeyYet = -1.0e30f;   // reference of a row all of whose keys so far a bias of -inf has removed
 
-template <typename T, int D, bool CAUSAL, int QB, int DBG, int BM = kWideBM, bool VBIAS = false, bool DROP = false>
-__global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 128 || VBIAS) ? 1 : 2) attn_fwd_wide_kernel(const AttnParams prm_arg) {
+// A bias with a query stride in the pipelined kernel: each wave copies the 32 rows x 32 keys of a step into a ring of its own, in
+// LDS behind the rings of K and V, four steps ahead, and a lane holds the 16 values of a step in registers a step before it. Rows of a half
+// tile are 32 ELT bytes = PIECES pieces of 16; piece s of row r lies at place s ^ (r / ROWS_PER_BANKS) of the row, so that the reads of one
+// piece by 32 rows are spread over all banks. (Not copied with nt: the two halves of a cache line are asked for a step apart, 60 -> 86 us at
+// 12 heads x 3072 causal. A fifth wave that touches the lines four tiles ahead gains nothing from memory either, 72 -> 77: it is not
+// latency that a bias from memory costs, but short pieces of many rows.)
+template <int ELT>
+struct BiasRing {
+  static constexpr int SLOTS = 4, ROW = 32 * ELT, PIECES = ROW / 16, PIECE_KEYS = 16 / ELT, SLOT = 32 * ROW, DMAS = SLOT / 1024, ROWS_PER_DMA = 64 / PIECES;
+  static constexpr int ROWS_PER_BANKS = 256 / ROW, WAVE_BYTES = SLOTS * SLOT;
+  static __device__ __forceinline__ int place(int row, int piece) { return piece ^ ((row / ROWS_PER_BANKS) & (PIECES - 1)); }
+};
+
+// TBIAS: bytes per element of a bias with a query stride (128 rows, no dropout; 0: none)
+template <typename T, int D, bool CAUSAL, int QB, int DBG, int BM = kWideBM, bool VBIAS = false, bool DROP = false, int TBIAS = 0>
+__global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 128 || VBIAS || TBIAS != 0) ? 1 : 2) attn_fwd_wide_kernel(const AttnParams prm_arg) {
   const AttnParams& prm = prm_arg;
+  static_assert(TBIAS == 0 || (BM == kBM && QB == 1 && !VBIAS && !DROP), "form with a bias per query");
   // VBIAS: an additive bias that is the same for every query of a head (query stride 0: the reference's "vector" bias,
   // flash_attention_triton.py:176-186, e.g. a key padding mask). The head's row of it, at most kVBiasKeys keys, is put
   // into LDS once per workgroup as fp32 divided by softmax_scale, so that (S + b / scale) * scale * log2 e is the biased
@@ -683,6 +698,8 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   // 369, causal 210 instead of 204; x 4096 causal 71.2 instead of 69.2, x 2048 37.2 instead of 35.9.) A bias of -inf removes a key; a row whose keys so far are all removed has the reference
   // kNoKeyYet, a large negative number, against which removed keys give 0 and the first key that counts overflows the
   // row sum once (recovery path), which multiplies the row's empty O and l by 0 (left padding: one step per row).
+  // TBIAS: the bias joins a score where that is scaled: exp2(S c + (b log2 e - m)), two instructions per score more, with m, the reference,
+  // in the base-2 domain (so that a row whose bias is large as a whole loses nothing to it).
   // BM = 256: the form described above. BM = 128 (QB = 1): the same pipeline with four waves x 32 rows, one query block
   // per workgroup in the 128-row kernel's order (heaviest causal blocks first), for shapes that give the chip too few
   // 256-row workgroups: a workgroup's time per key tile is what bounds those, and this pipeline's is less than half the
@@ -932,6 +949,54 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     last_batch = issue_batch(-1);
   }
 
+  // TBIAS: half tiles of 32 keys; the copies of a half tile past the last key re-read the last piece (masked)
+  typedef BiasRing<TBIAS == 4 ? 4 : 2> BR;
+  typedef typename std::conditional<TBIAS == 4, float, T>::type BE;
+  typedef __attribute__((ext_vector_type(4))) BE be4;
+  FO_LDS char* const bias_ring = smem + 2 * kRing * TILE_BYTES + wave_s * BR::WAVE_BYTES;
+  const BE* bias_row[TBIAS ? BR::DMAS : 1];
+  be4 bias_of[2][4];                     // of steps s and s + 1, by parity: registers 4 j .. 4 j + 3 (keys 8 j + 4 hh ..)
+  if constexpr (TBIAS != 0) {
+#pragma unroll
+    for (int i = 0; i < BR::DMAS; ++i) {
+      const int row = i * BR::ROWS_PER_DMA + lane / BR::PIECES;
+      bias_row[i] = (const BE*)prm.bias.ptr + b * prm.bias.strides[0] + h * prm.bias.strides[1] + (int64_t)min(q0w + row, Sq - 1) * prm.bias.strides[2];
+    }
+  }
+  auto issue_bias = [&](int sub, int i) {            // copy i of a half tile, anywhere
+    if constexpr (TBIAS != 0) {
+      int lane_here = lane;
+      asm volatile("" : "+v"(lane_here));            // (worked out where it is needed: no registers held for it)
+      const int row = i * BR::ROWS_PER_DMA + lane_here / BR::PIECES;
+      const int key = min(sub * 32 + BR::place(row, lane_here % BR::PIECES) * BR::PIECE_KEYS, (Sk - 1) / BR::PIECE_KEYS * BR::PIECE_KEYS);
+      dma16_lane_ptr(bias_row[i] + key, bias_ring + (sub & (BR::SLOTS - 1)) * BR::SLOT + i * 1024);
+    }
+  };
+  auto load_bias_of = [&](int sub, int j4) -> be4 {
+    // (fp32: 16 bytes of a lane are a piece; operand type: half of one)
+    const int at = l32 * BR::ROW + (TBIAS == 4 ? BR::place(l32, 2 * j4 + hh) * 16 : BR::place(l32, j4) * 16 + 8 * hh);
+    return *(FO_LDS const be4*)(bias_ring + (sub & (BR::SLOTS - 1)) * BR::SLOT + at);
+  };
+  // In the loop whose steps issue the copies of K and V between their products those of the bias take pointers that move on by a half
+  // tile per step.
+  const BE* bias_at[TBIAS ? BR::DMAS : 1];
+  // Before step s the half tile s + 1, which it reads into registers, has to have landed. It was asked for in step s - 3; what was asked for
+  // after that step may be in flight: the half tiles of steps s - 2 and s - 1, and the copies of K and V of those two steps (spread), or,
+  // where they go out at the top of a tile, the batch of the tile before (at the top) or of this one (in the middle).
+  auto bias_wait = [&](int batch) {
+    if constexpr (TBIAS != 0) {
+      if (batch == 2 * NBLK) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NBLK + 2 * BR::DMAS) : "memory");
+      else if (batch == NBLK) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NBLK + 2 * BR::DMAS) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * BR::DMAS) : "memory");
+    }
+  };
+  if constexpr (TBIAS != 0) {
+#pragma unroll
+    for (int sub = 0; sub < BR::SLOTS; ++sub)
+#pragma unroll
+      for (int i = 0; i < BR::DMAS; ++i) issue_bias(sub, i);
+  }
+
   if (first_block) load_q(bh, qblk);
   if constexpr (VBIAS) {
     // the keys this workgroup sees (a causal pair's first block is the longer one), while its first tiles and its Q are on their way
@@ -1015,6 +1080,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     typedef AsmMfma<T, !(decltype(in_loop)::value && !FO_MFMA_NOPS)> Mfma;
     constexpr int P = decltype(parity)::value;
     constexpr bool HAS_QK = decltype(has_qk)::value, HAS_PV = decltype(has_pv)::value, MASK = decltype(masked)::value;
+    constexpr bool SPREAD_HERE = decltype(spread)::value && HAS_QK && HAS_PV;
     constexpr int NM = QB * KSTEPS;                                     // MFMAs of one kind
     constexpr int NMF = (HAS_QK ? NM : 0) + (HAS_PV ? NM : 0);          // micro-groups with an MFMA
     constexpr int NEL = 16 * QB;                                        // scores per lane
@@ -1036,10 +1102,9 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     const uint32_t vb0 = v_lane + sub_base(s - 1), vb1 = v_lane + sub_base(s);
     float mc[QB], psum[QB];
 #pragma unroll
-    for (int b2 = 0; b2 < QB; ++b2) { mc[b2] = m_run[b2] * c; psum[b2] = 0.0f; }
+    for (int b2 = 0; b2 < QB; ++b2) { mc[b2] = TBIAS ? m_run[b2] : m_run[b2] * c; psum[b2] = 0.0f; }
     // copies this step issues between its MFMAs (spread): the K blocks of tile dma_tile in the step of an even sub-tile,
     // the V blocks in that of an odd one
-    constexpr bool SPREAD_HERE = decltype(spread)::value && HAS_QK && HAS_PV;
     uint32_t dma_off = 0;
     FO_LDS char* dma_dst = smem;
     if constexpr (SPREAD_HERE) {
@@ -1099,6 +1164,24 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
           for (int r = 0; r < 16; ++r) S[P][b2][r] = (lim > -((r & 3) + 8 * (r >> 2))) ? -INFINITY : S[P][b2][r];
         }
       }
+      if constexpr (TBIAS != 0) {
+        // the next step's values, and the copies of half tile s + 4 into the slot that this step's came from: from the group on in which
+        // the last of them have been used (score 8 of a lane in group GE(8) - 2), i.e. have arrived
+        constexpr int GB0 = GE0 + (8 * NE) / NEL;
+#pragma unroll
+        for (int j4 = 0; j4 < 4; ++j4)
+          if (g == 2 + j4 / 2) bias_of[P ^ 1][j4] = load_bias_of(s + 1, j4);
+#pragma unroll
+        for (int i = 0; i < BR::DMAS; ++i)
+          if (g == (GB0 + i * 4 / BR::DMAS < G ? GB0 + i * 4 / BR::DMAS : G - 1)) {
+            if constexpr (SPREAD_HERE) {
+              dma16_lane_ptr(bias_at[i], bias_ring + (s & (BR::SLOTS - 1)) * BR::SLOT + i * 1024);
+              bias_at[i] += 32;
+            } else {
+              issue_bias(s + 4, i);
+            }
+          }
+      }
       // Three stages, one micro-group apart, so that no instruction of a group waits for another one of the same
       // group: scale-and-shift of score e in group GE(e) - 1, its exponential in GE(e), the row sum and (for a finished
       // pair) the rounding to the operand type for P.V (flash_attention_triton.py:237) in GE(e) + 1.
@@ -1106,8 +1189,18 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
       for (int e = 0; e < NEL; ++e) {
         const int ge = GE0 + 1 + (e * NE) / NEL;
         const int b2 = el_qb(e), r = el_reg(e);
+        if constexpr (TBIAS != 0) {
+          if (ge - 2 == g) {
+            float bv = (float)bias_of[P][r >> 2][r & 3];
+            // (what is read for keys past the end may be anything; their scores are -inf)
+            if (MASK) bv = (s * 32 + 4 * hh + (r & 3) + 8 * (r >> 2) < Sk) ? bv : 0.0f;
+            ex[e] = __builtin_fmaf(bv, 1.4426950408889634f, -mc[b2]);
+            asm volatile("" : "+v"(ex[e]));
+          }
+        }
         if (ge - 1 == g) {
-          ex[e] = (DBG & 2) ? S[P][b2][r] : __builtin_fmaf(S[P][b2][r], c, -mc[b2]);
+          if constexpr (TBIAS != 0) ex[e] = __builtin_fmaf(S[P][b2][r], c, ex[e]);
+          else ex[e] = (DBG & 2) ? S[P][b2][r] : __builtin_fmaf(S[P][b2][r], c, -mc[b2]);
           asm volatile("" : "+v"(ex[e]));                              // pins the instruction to this micro-group
         }
         if (ge == g) {
@@ -1141,6 +1234,17 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
       // rare: true row maxima of this sub-tile, new references, P and row sums again, O and l rescaled
 #pragma unroll
       for (int d = 0; d < DBLK; ++d) mfma_result_fence_a(oacc[d]);
+      const float cr = TBIAS ? 1.0f : c;
+      if constexpr (TBIAS != 0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const float x = S[P][0][4 * j + u], biased = __builtin_fmaf(x, c, (float)bias_of[P][j][u] * 1.4426950408889634f);
+            S[P][0][4 * j + u] = (MASK && x == -INFINITY) ? x : biased;
+          }
+        }
+      }
 #pragma unroll
       for (int b2 = 0; b2 < QB; ++b2) {
         float mloc = S[P][b2][0];
@@ -1148,13 +1252,13 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
         for (int r = 1; r < 16; ++r) mloc = fmaxf(mloc, S[P][b2][r]);
         mloc = fmaxf(mloc, half_swap(mloc));
         const float m_new = fmaxf(m_run[b2], mloc);                    // finite: key 0 is never masked (a bias: see kNoKeyYet)
-        const float alpha = __builtin_amdgcn_exp2f((m_run[b2] - m_new) * c);
-        const float mcn = m_new * c;
+        const float alpha = __builtin_amdgcn_exp2f((m_run[b2] - m_new) * cr);
+        const float mcn = m_new * cr;
         float ps = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {
-          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[P][b2][r], c, -mcn));
-          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[P][b2][r + 1], c, -mcn));
+          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[P][b2][r], cr, -mcn));
+          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[P][b2][r + 1], cr, -mcn));
           ps += p0;
           ps += p1;
           const vec2 pk = {(T)p0, (T)p1};
@@ -1183,8 +1287,10 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   // ---- tile loop. Tile j runs the steps of sub-tiles 2j and 2j+1; they read K(j), K(j+1), V(j-1), V(j).
   // At its top, copy batches up to (j-2) must have landed - K(j+1) and V(j) are among them - while batch (j-1) may still
   // be in flight; after the barrier every wave is done with tile j-1, so batch j may overwrite K(j-1) and V(j-2).
-  auto tile_top = [&](int j, bool spread_this = false) -> bool {
-    if (!(DBG & 32)) {
+  auto tile_top = [&](int j, bool spread_this = false, bool idle = false) -> bool {
+    // (the copies of the bias that a wave at work issued since are a constant number: bias_wait. It covers those of K and V.)
+    if (TBIAS != 0 && !idle) bias_wait(last_batch);
+    else if (!(DBG & 32)) {
       // (as many copies may stay in flight as this wave issued in the batch before: 0, one matrix's or both)
       if (__builtin_expect(last_batch == 2 * NBLK, 1)) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NBLK) : "memory");
       else if (last_batch >= NBLK) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NBLK) : "memory");
@@ -1245,6 +1351,10 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
 #pragma unroll
     for (int j4 = 0; j4 < 4; ++j4) load_key_bias(1, j4);
   }
+  if constexpr (TBIAS != 0) {
+#pragma unroll
+    for (int j4 = 0; j4 < 4; ++j4) bias_of[0][j4] = load_bias_of(0, j4);
+  }
   // The reference of the exponentials starts as the row maximum of the first sub-tile (dead keys left out as the step
   // will mask them: lim as there, sub-tile 0; key 0 is never dead, so the maximum is finite). Started from -inf, the
   // first step takes the recovery path - maxima, every exponential a second time, 64 accumulator registers rescaled -
@@ -1256,13 +1366,15 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     float mloc = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      mloc = fmaxf(mloc, (lim > -((r & 3) + 8 * (r >> 2))) ? -INFINITY : S[0][b2][r]);
+      float sv = S[0][b2][r];
+      if constexpr (TBIAS != 0) sv = __builtin_fmaf(sv, c, (float)bias_of[0][r >> 2][r & 3] * 1.4426950408889634f);
+      mloc = fmaxf(mloc, (lim > -((r & 3) + 8 * (r >> 2))) ? -INFINITY : sv);
     }
     m_run[b2] = fmaxf(mloc, half_swap(mloc));
     // (a bias may have removed every key of the sub-tile: the reference then starts from a large negative number
     // instead of -inf, so that a removed key gives exp2(-inf) = 0 and not exp2(-inf + inf); the first key that counts
     // overflows the row sum and the recovery path moves the reference to it, with O and l multiplied by exp2(-huge) = 0)
-    if constexpr (VBIAS) m_run[b2] = fmaxf(m_run[b2], kNoKeyYet);
+    if constexpr (VBIAS || TBIAS != 0) m_run[b2] = fmaxf(m_run[b2], kNoKeyYet);
   }
   drop_look(0);
   step(0, P0{}, Y{}, N{}, Y{}, N{}, N{}, -1, N{});   // (its reference is its own row maximum: every P <= 1, no recovery)
@@ -1270,15 +1382,25 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   // Should the steps above have parked registers in scratch memory (they do not at present), wait here, visibly to
   // the compiler, for any reload still in flight: otherwise it guards the first use inside the loops with a vmcnt(0)
   // wait that executes on every iteration and also drains the copies in flight, which it does not see.
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), nothing else
+  // (TBIAS has none: its copies stay in flight)
+  if constexpr (TBIAS == 0) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), nothing else
   last_batch = (DBG & 1) ? 0 : issue_batch(0);
   int j = 1;
   if constexpr (SPREAD_DMA) {
     // unmasked tiles whose copies (K three tiles, V two tiles ahead) are whole tiles: the steps issue them
+    if constexpr (TBIAS != 0) {
+#pragma unroll
+      for (int i = 0; i < BR::DMAS; ++i) {
+        const int row = i * BR::ROWS_PER_DMA + lane / BR::PIECES;
+        bias_at[i] = bias_row[i] + (2 * j + 4) * 32 + BR::place(row, lane % BR::PIECES) * BR::PIECE_KEYS;
+        asm volatile("" : "+v"(bias_at[i]));
+      }
+    }
     for (; j < min(min(j_mask, n_w - 1), n_full - 3); ++j) {
       tile_top(j, true);
       drop_look(j);
       step(2 * j, P0{}, Y{}, Y{}, N{}, Y{}, Y{}, j + 3);
+      bias_wait(2 * NBLK);
       step(2 * j + 1, P1{}, Y{}, Y{}, N{}, Y{}, Y{}, j + 2);
     }
   }
@@ -1286,18 +1408,21 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     tile_top(j);
     drop_look(j);
     step(2 * j, P0{}, Y{}, Y{}, N{}, Y{}, N{}, -1);
+    bias_wait(last_batch);
     step(2 * j + 1, P1{}, Y{}, Y{}, N{}, Y{}, N{}, -1);
   }
   for (; j < n_w - 1; ++j) {
     tile_top(j);
     drop_look(j);
     step(2 * j, P0{}, Y{}, Y{}, Y{}, Y{}, N{}, -1);
+    bias_wait(last_batch);
     step(2 * j + 1, P1{}, Y{}, Y{}, Y{}, Y{}, N{}, -1);
   }
   if (j < n_w) {
     tile_top(j);
     drop_look(j);
     step(2 * j, P0{}, Y{}, Y{}, Y{}, N{}, N{}, -1);
+    bias_wait(last_batch);
     step(2 * j + 1, P1{}, N{}, Y{}, Y{}, N{}, N{}, -1);
     ++j;
   }
@@ -1313,7 +1438,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     }
   }
   // tiles in which this wave has nothing to do (causal): keep feeding the workgroup's rings
-  for (; j < n_tiles; ++j) tile_top(j);
+  for (; j < n_tiles; ++j) tile_top(j, false, true);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if (has_next) load_q(next_bh, next_qblk);   // (they arrive while this block's O is written)
 
@@ -1366,7 +1491,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
       __builtin_amdgcn_sched_barrier(0);
     }
     if (qi < Sq && prm.lse != nullptr && hh == 0)
-      prm.lse[(int64_t)bh * Sq + qi] = (m_run[qb] * c + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f;
+      prm.lse[(int64_t)bh * Sq + qi] = (TBIAS ? m_run[qb] + __builtin_amdgcn_logf(l_tot) : m_run[qb] * c + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f;
     if constexpr (KEEP_ON) write_rows(32 * qb, 32);
   }
   if constexpr (!KEEP_ON) write_rows(0, 32 * QB);
@@ -1392,14 +1517,14 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   return (int)group;
 }
 
-template <typename T, int D, bool CAUSAL, int QB, int DBG = 0, int BM = kWideBM, bool VBIAS = false, bool DROP = false>
+template <typename T, int D, bool CAUSAL, int QB, int DBG = 0, int BM = kWideBM, bool VBIAS = false, bool DROP = false, int TBIAS = 0>
 static int launch_wide(AttnParams p, hipStream_t stream) {
   constexpr bool KEEP_ON = BM == kWideBM && !VBIAS;      // (as in the kernel)
   // rings; bias row; or the rows of O staged behind the first six slots of the rings, 32 rows of D + 8 elements per wave
   // (eight waves at head_dim 128: seven of them there, see the kernel)
   constexpr int kWavesHere = BM / (32 * QB);
   constexpr size_t kStageAll = (size_t)(kRing + 2) * kBN * D * 2 + kWavesHere * 32 * (D * 2 + 16);
-  const size_t lds = KEEP_ON ? (kStageAll > 160 * 1024 ? kStageAll - 32 * (D * 2 + 16) : kStageAll) : 2 * (size_t)kRing * kBN * D * 2 + (VBIAS ? kVBiasKeys * 4 : 0);
+  const size_t lds = KEEP_ON ? (kStageAll > 160 * 1024 ? kStageAll - 32 * (D * 2 + 16) : kStageAll) : 2 * (size_t)kRing * kBN * D * 2 + (VBIAS ? kVBiasKeys * 4 : 0) + (TBIAS ? kWaves * BiasRing<TBIAS == 4 ? 4 : 2>::WAVE_BYTES : 0);
   if (VBIAS && (p.Sk + kBN - 1) / kBN * kBN > kVBiasKeys) return FO_ERR_UNSUPPORTED;
   p.n_qblk = (p.Sq + BM - 1) / BM;
   unsigned grid = (unsigned)((BM == kWideBM ? wide_items(p.n_qblk, CAUSAL) : p.n_qblk) * p.B * p.H);
@@ -1419,10 +1544,10 @@ static int launch_wide(AttnParams p, hipStream_t stream) {
   }
   p.heavy_first = (CAUSAL && BM != kWideBM) ? heavy_first_group(p, D) : 0;
   p.order_n = 0;
-  static const hipError_t attr = hipFuncSetAttribute((const void*)attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS, DROP>,
+  static const hipError_t attr = hipFuncSetAttribute((const void*)attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS, DROP, TBIAS>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return FO_ERR_LAUNCH;
-  attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS, DROP><<<grid, BM / (32 * QB) * 64, lds, stream>>>(p);
+  attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS, DROP, TBIAS><<<grid, BM / (32 * QB) * 64, lds, stream>>>(p);
   return launch_status();
 }
 
@@ -1512,12 +1637,28 @@ static int launch_one(const AttnParams& p, hipStream_t stream) {
 // `forced` is the value of attn.variant (-1: the library's choice). Values from 256 on are timing ablations and exist
 // only in a build with FO_ABLATIONS.
 static int choose_kernel(const AttnParams& p, int D, bool causal, bool dropout, int forced) {
-  // a bias with a query stride and head dims other than 64 and 128 run on the 128-row kernel; a bias that is the same for
+  // head dims other than 64 and 128 run on the 128-row kernel, and most calls with a bias with a query stride; a bias that is the same for
   // every query (and short enough for the pipelined kernel to keep it in LDS) takes part in the choice, and so does dropout
   const bool key_bias = p.bias.ptr != nullptr && p.bias.strides[2] == 0 && ((int64_t)p.Sk + kBN - 1) / kBN * kBN <= kVBiasKeys;
-  if ((p.bias.ptr != nullptr && !key_bias) || p.d != D) return FO_ATTN_KERNEL_ROWS128;
   // The 256-row kernel addresses a head's keys with 32-bit byte offsets ...
   const bool wide_ok = (int64_t)p.Sk * (p.ks[2] > p.vs[2] ? p.ks[2] : p.vs[2]) * 2 < (1ll << 31);
+  if (p.bias.ptr != nullptr && p.bias.strides[2] != 0) {
+    // A bias with a query stride whose tiles can be copied, without dropout: the 128-row pipelined form as well (at head_dim 128 not an
+    // fp32 one: the rings leave 32 KiB of LDS, two of the four half tiles a wave's ring needs), where there are few workgroups for the
+    // chip, as below; its two instructions per score more are why the line lies nearer. Plain -> pipelined, us, bf16 bias that the
+    // memory-side cache holds (in brackets one read from memory): head_dim 128 12 heads x 1024 32.0 -> 26.4, x 2048 56 -> 43 (57 -> 51),
+    // 8 x 1536 42 -> 32, causal 12 x 1024 30.6 -> 26.1, x 2048 56 -> 43 (56 -> 45), x 3072 83 -> 60 (84 -> 72), x 4096 (384 workgroups)
+    // 114 -> 91 (114 -> 103); not: 12 x 3072 (288) 111 -> 122, 64 x 1024 causal (512) 37.0 -> 39.4; head_dim 64 12 x 2048 44 -> 36 (fp32
+    // 48 -> 45), causal 12 x 3072 63 -> 47 (fp32 74 -> 62), x 4096 84 -> 63 (fp32 128 -> 119); not: 12 x 3072 86 -> 90, 64 x 1024 causal
+    // 26.8 -> 29.5. (From so many (query, key) pairs on: 12 x 512 gains 18.7 -> 17.3 us, and up to there a bias whose rows lie off
+    // 16-byte boundaries is read in place, by the plain kernel, so that both give the same bits.)
+    constexpr int64_t kRowBiasPipePairs = 3 << 18;
+    if (p.d != D || dropout || !p.bias.dma_ok || !wide_ok || (D == 128 && p.bias.is_f32)) return FO_ATTN_KERNEL_ROWS128;
+    if (forced >= 0) return forced == FO_ATTN_KERNEL_ROWS128_PIPE ? FO_ATTN_KERNEL_ROWS128_PIPE : FO_ATTN_KERNEL_ROWS128;
+    const int64_t wgs128 = ((int64_t)p.Sq + kBM - 1) / kBM * p.B * p.H, cus = device_cus();
+    return (int64_t)p.Sq * p.Sk >= kRowBiasPipePairs && wgs128 <= (causal ? cus + cus / 2 : cus) ? FO_ATTN_KERNEL_ROWS128_PIPE : FO_ATTN_KERNEL_ROWS128;
+  }
+  if ((p.bias.ptr != nullptr && !key_bias) || p.d != D) return FO_ATTN_KERNEL_ROWS128;
   // ... and needs one 256-row workgroup (two query blocks each when causal) per CU to be worth it: below that the
   // 128-row kernel, with four times as many workgroups, fills the chip better
   const int n_cu = device_cus();
@@ -1608,6 +1749,10 @@ int launch(const AttnParams& p, bool causal, bool dropout, hipStream_t stream) {
   if (p.bias.ptr != nullptr && !key_bias) {
     // tiles that can be copied (dma_ok: base and strides are multiples of 16 bytes), whose values join the finished scores
     if (!dropout && p.d == D && p.bias.dma_ok && asked != FO_ATTN_KERNEL_ROWS128_EXACT) {
+      if (choose_kernel(p, D, causal, false, asked) == FO_ATTN_KERNEL_ROWS128_PIPE) {
+        if (!p.bias.is_f32) return causal ? launch_wide<T, D, true, 1, 0, kBM, false, false, 2>(p, stream) : launch_wide<T, D, false, 1, 0, kBM, false, false, 2>(p, stream);
+        if constexpr (D == 64) return causal ? launch_wide<T, D, true, 1, 0, kBM, false, false, 4>(p, stream) : launch_wide<T, D, false, 1, 0, kBM, false, false, 4>(p, stream);
+      }
       if (p.bias.is_f32) return causal ? launch_one<T, D, true, true, 0, false, false, false, false, D, 4>(p, stream)
                                        : launch_one<T, D, false, true, 0, false, false, false, false, D, 4>(p, stream);
       return causal ? launch_one<T, D, true, true, 0, false, false, false, false, D, 2>(p, stream)
@@ -1820,6 +1965,8 @@ extern "C" int fo_attn_fwd_kernel(int B, int H, int Sq, int Sk, int D, const int
   for (int i = 0; i < 3; ++i) { p.ks[i] = ks[i]; p.vs[i] = vs[i]; }
   p.bias.ptr = has_bias ? (const void*)ks : nullptr;   // (only tested against NULL)
   p.bias.strides[2] = has_bias == 2 ? 0 : 1;
+  p.bias.dma_ok = has_bias >= 3;
+  p.bias.is_f32 = has_bias == 4;
   if (takes_decode(p, causal != 0, has_dropout != 0, tune(g_attn_variant))) return FO_ATTN_KERNEL_DECODE;
   return choose_kernel(p, D > 64 ? 128 : 64, causal != 0, has_dropout != 0, tune(g_attn_variant));
 }

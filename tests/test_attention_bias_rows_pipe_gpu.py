@@ -1,0 +1,64 @@
+"""A bias with a query stride in the pipelined 128-row forward kernel, whose waves copy half tiles of 32 keys of it into a ring: key
+counts around the half tile, the tile and the length of the rings, rows longer than the keys with NaN behind them, masked keys, a bias
+that is large for whole rows, one that grows along the keys (the reference of the exponentials moves at every step), broadcasting.
+Against the oracle; tolerances as in test_attention_bias_gpu.py."""
+import pytest
+import torch
+
+from fast_ops.flash_attention.flash_attention import flash_attn
+from fast_ops_amd import _lib
+from oracle.attention_oracle import attention_fwd_oracle
+from test_attention_bias_gpu import DEV, _bshd, _check
+
+pytestmark = pytest.mark.gpu
+
+
+def _kernel(B, H, Sq, Sk, D, causal, bias_f32):
+    dense = (_lib.ctypes.c_int64 * 3)(H * Sk * D, Sk * D, D)
+    return _lib.load().fo_attn_fwd_kernel(B, H, Sq, Sk, D, dense, dense, int(causal), 4 if bias_f32 else 3, 0)
+
+
+@pytest.mark.parametrize("kind", ["noise", "masked", "large rows", "growing"])
+@pytest.mark.parametrize("D,bias_f32", [(128, False), (64, False), (64, True)])
+@pytest.mark.parametrize("B,H,Sq,Sk,causal,dtype", [
+    (1, 2, 40, 8, False, torch.bfloat16), (1, 1, 130, 33, False, torch.float16), (2, 1, 97, 64, False, torch.bfloat16), (1, 2, 128, 72, True, torch.float16),
+    (1, 1, 300, 200, False, torch.bfloat16), (2, 2, 256, 256, True, torch.bfloat16), (1, 1, 257, 321, False, torch.float16),
+    (1, 2, 333, 333, True, torch.bfloat16), (1, 1, 129, 1030, False, torch.bfloat16), (1, 1, 1100, 700, True, torch.float16)])
+def test_rows_of_bias_in_the_pipelined_kernel(B, H, Sq, Sk, causal, dtype, D, bias_f32, kind):
+    g = torch.Generator().manual_seed(Sq + Sk + D)
+    q, k, v = (torch.randn(B, H, n, D, generator=g).to(dtype) for n in (Sq, Sk, Sk))
+    bias = 2.0 * torch.randn(1, H, Sq, Sk, generator=g)              # (broadcast over the batch)
+    if kind == "masked":
+        if not causal:
+            bias[:, :, Sq // 2:, :Sk // 3] = float("-inf")           # whole half tiles and parts of one, left ...
+        bias[:, :, ::3, Sk - Sk // 4:] = float("-inf")               # ... and right
+    elif kind == "large rows":
+        bias[:, :, ::2] += 512.0 if not bias_f32 and dtype is torch.bfloat16 else 1000.0
+    elif kind == "growing":
+        bias += torch.arange(Sk) * 0.5
+    bias = bias.to(torch.float32 if bias_f32 else dtype)
+    o_ref, lse_ref = attention_fwd_oracle(q, k, v, causal=causal, bias=bias)
+    wide = torch.full(bias.shape[:-1] + (Sk + 16 - Sk % 8,), float("nan"), dtype=bias.dtype, device=DEV)
+    wide[..., :Sk] = bias.to(DEV)
+    _lib.tune_set("attn.variant", _lib.FO_ATTN_KERNEL_ROWS128_PIPE)
+    try:
+        assert _kernel(B, H, Sq, Sk, D, causal, bias_f32) == _lib.FO_ATTN_KERNEL_ROWS128_PIPE
+        o, lse = flash_attn(*(_bshd(x.to(DEV)) for x in (q, k, v)), bias=wide[..., :Sk], causal=causal, return_lse=True)
+        torch.cuda.synchronize()
+    finally:
+        _lib.tune_set("attn.variant", -1)
+    # (an LSE of about 1000 in fp32: its own rounding is 6e-5, a product with log2 e and one with ln 2 add as much each)
+    _check(_bshd(o), lse, [], o_ref, lse_ref, [])
+
+
+def test_the_rule():
+    pipe, plain = _lib.FO_ATTN_KERNEL_ROWS128_PIPE, _lib.FO_ATTN_KERNEL_ROWS128
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for D, f32 in [(128, False), (64, False), (64, True)]:
+        assert _kernel(1, cus // 16, 2048, 2048, D, False, f32) == pipe           # one workgroup per unit
+        assert _kernel(1, cus // 16 + 1, 2048, 2048, D, False, f32) == plain
+        assert _kernel(1, cus * 3 // 2 // 16, 2048, 2048, D, True, f32) == pipe   # one and a half when causal
+        assert _kernel(1, cus * 3 // 2 // 16 + 1, 2048, 2048, D, True, f32) == plain
+        assert _kernel(1, 4, 1024, 768, D, True, f32) == pipe and _kernel(1, 4, 1024, 767, D, True, f32) == plain
+    assert _kernel(1, 4, 2048, 2048, 128, True, True) == plain                    # fp32 at head_dim 128
+    assert _kernel(1, 4, 2048, 2048, 96, True, False) == plain                    # a head_dim off 64 and 128
