@@ -46,6 +46,8 @@ SIGNATURES = {
     "fo_attn_bias_rows": (ctypes.c_int, [ctypes.c_void_p, _I64P] + [ctypes.c_int] * 5 + [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]),
     "fo_dropout_mask": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int64, ctypes.c_float, ctypes.c_uint32, ctypes.c_uint64, ctypes.c_void_p]),
     "fo_attn_fwd_ex": (ctypes.c_int, [ctypes.c_void_p] * 5 + [ctypes.c_int] * 5 + [_I64P] * 4 + [ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]),
+    "fo_attn_fwd_workspace_ex": (ctypes.c_int64, [ctypes.c_int] * 5 + [_I64P] * 2 + [ctypes.c_int, ctypes.c_void_p]),
+    "fo_attn_fwd_ex_ws": (ctypes.c_int, [ctypes.c_void_p] * 5 + [ctypes.c_int] * 5 + [_I64P] * 4 + [ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]),
     "fo_attn_bwd_ex": (ctypes.c_int, [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.POINTER(_I64P), ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]),
     "fo_attn_bwd_workspace": (ctypes.c_int64, [ctypes.c_int] * 5),
     "fo_attn_bwd_workspace_ex": (ctypes.c_int64, [ctypes.c_int] * 6 + [ctypes.c_void_p]),

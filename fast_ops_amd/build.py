@@ -63,9 +63,9 @@ SOURCES = {
 INCLUDED_SOURCES = ["attn_fwd.hip", "attn_bwd.hip"]
 # sources whose generated assembly is checked by asm_lint: source -> regular expression of the kernel symbols to check
 # (the instantiations with a non-zero last template argument are timing experiments with wrong results by design)
-# (attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS, DROP, TBIAS>: DBG is followed by BM, two truth values and the bytes of a bias)
+# (attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS, DROP, TBIAS, PARTS>: DBG is followed by BM, two truth values, the bytes of a bias and one)
 _PIPE = r"attn_bwd_dkdv_pipe_kernel"
-_WIDE = r"attn_fwd_wide_kernel.*ELi0ELi\d+ELb[01]ELb[01]ELi[024]EEEvNS_10AttnParamsE"
+_WIDE = r"attn_fwd_wide_kernel.*ELi0ELi\d+ELb[01]ELb[01]ELi[024]ELb[01]EEEvNS_10AttnParamsE"
 ASM_LINTED = {"attn_fwd_bf16_d64.hip": _WIDE, "attn_fwd_bf16_d128.hip": _WIDE, "attn_fwd_f16_d64.hip": _WIDE, "attn_fwd_f16_d128.hip": _WIDE,
               "attn_bwd_bf16_d64.hip": _PIPE, "attn_bwd_bf16_d128.hip": _PIPE, "attn_bwd_f16_d64.hip": _PIPE, "attn_bwd_f16_d128.hip": _PIPE}
 # sources without inline-assembly MFMAs whose direct-to-LDS copies are checked (asm_lint.lint_m0_file; in those above they are as well)

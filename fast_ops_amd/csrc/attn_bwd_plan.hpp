@@ -53,13 +53,13 @@ inline int makespan(const int* cost, int n, int n_bh, int cus) {
     }
   return last;
 }
-inline DkdvPlan make_dkdv_plan(int n_bh, int Sq, int Sk, bool causal, int asked, int cus) {
+// What a piece costs beside its tiles, in half tiles: to start it, to leave its sums; and to add them: for the launch, and parts that are
+// added in the time of a half tile. The tiles a piece needs. Causal: whether every block in equally many pieces is laid out as well.
+struct ShareCost { int start, leave, merge, parts_per, least; bool alike; };
+// tiles(blk): of each of n_blk blocks; asked: 0 none are shared, > 1 every block in so many pieces, -1 what ends before `percent` of whole blocks
+template <typename Tiles>
+inline DkdvPlan share_blocks(int n_bh, int n_blk, Tiles tiles, bool causal, int asked, int cus, ShareCost price, int percent) {
   DkdvPlan best;
-  const int n_blk = (Sk + kBwdRows - 1) / kBwdRows, n_qt = (Sq + kBwdTile - 1) / kBwdTile;
-  if (asked == 0 || n_blk > kMaxItems || n_bh > cus || (asked < 0 && (int64_t)n_bh * n_blk > 4 * cus)) return best;
-  // (the heads in one group, see launch_bwd)
-  if (2 * ((int64_t)Sq + Sk) * 128 * 2 * n_bh > (256ll << 20)) return best;
-  auto tiles = [&](int blk) { const int first = kBwdRows / kBwdTile * blk; return causal ? (first < n_qt ? n_qt - first : 0) : n_qt; };
   int64_t sum = 0;
   for (int blk = 0; blk < n_blk; ++blk) sum += tiles(blk);
   const int mean = (int)((sum * n_bh + cus - 1) / cus);
@@ -72,7 +72,7 @@ inline DkdvPlan make_dkdv_plan(int n_bh, int Sq, int Sk, bool causal, int asked,
       if (s > 1) plan.merges[plan.n_merges++] = (uint32_t)blk | (uint32_t)s << 12 | (uint32_t)plan.n_parts << 16;
       for (int i = 0; i < s; ++i) {
         const uint32_t item = (uint32_t)blk | (uint32_t)i << 8 | (uint32_t)s << 12 | (s > 1 ? (uint32_t)plan.n_parts++ << 16 : kWholeBlock >> 16 << 16);
-        const int c = 2 * (tiles(blk) * (i + 1) / s - tiles(blk) * i / s) + 4 + (s > 1 ? 2 : 0);    // half tiles
+        const int c = 2 * (tiles(blk) * (i + 1) / s - tiles(blk) * i / s) + price.start + (s > 1 ? price.leave : 0);
         int at = plan.n_items++;
         for (; at > 0 && cost[at - 1] < c; --at) { cost[at] = cost[at - 1]; plan.items[at] = plan.items[at - 1]; }
         cost[at] = c;
@@ -84,16 +84,16 @@ inline DkdvPlan make_dkdv_plan(int n_bh, int Sq, int Sk, bool causal, int asked,
   auto consider = [&](auto pieces_of, bool forced) {
     DkdvPlan plan;
     if (!lay_out(pieces_of, plan) || plan.n_merges == 0) return;
-    const int time = makespan(cost, plan.n_items, n_bh, cus) + plan.n_parts * n_bh / 32 + 4;
+    const int time = makespan(cost, plan.n_items, n_bh, cus) + plan.n_parts * n_bh / price.parts_per + price.merge;
     if (forced || time < best_time) { best_time = time; best = plan; }
   };
   if (asked > 1) {
-    consider([&](int blk) { const int t = tiles(blk); return t < 1 ? 1 : t < asked ? t : asked; }, true);
+    consider([&](int blk) { const int t = tiles(blk) / price.least; return t < 1 ? 1 : t < asked ? t : asked; }, true);
     return best;
   }
   DkdvPlan whole;
   if (!lay_out([](int) { return 1; }, whole)) return best;
-  best_time = makespan(cost, whole.n_items, n_bh, cus) * (causal ? 90 : 82) / 100;
+  best_time = makespan(cost, whole.n_items, n_bh, cus) * percent / 100;
   constexpr int kMinTiles = 4;
   auto fits = [&](int blk, int s) { const int most = tiles(blk) / kMinTiles; return s < most ? s : most > 1 ? most : 1; };
   if (causal) {
@@ -101,6 +101,7 @@ inline DkdvPlan make_dkdv_plan(int n_bh, int Sq, int Sk, bool causal, int asked,
       const int most = mean * f / 4 > kMinTiles ? mean * f / 4 : kMinTiles;
       consider([&](int blk) { const int s = (tiles(blk) + most - 1) / most; return fits(blk, s > kMaxPieces ? kMaxPieces : s); }, false);
     }
+    for (int s = 2; price.alike && s <= kMaxPieces; ++s) consider([&](int blk) { return fits(blk, s); }, false);
   } else {
     const int rest = ((n_bh * n_blk) % cus + n_bh - 1) / n_bh;
     for (int s = 2; s <= kMaxPieces; ++s) {
@@ -109,6 +110,14 @@ inline DkdvPlan make_dkdv_plan(int n_bh, int Sq, int Sk, bool causal, int asked,
     }
   }
   return best;
+}
+inline DkdvPlan make_dkdv_plan(int n_bh, int Sq, int Sk, bool causal, int asked, int cus) {
+  const int n_blk = (Sk + kBwdRows - 1) / kBwdRows, n_qt = (Sq + kBwdTile - 1) / kBwdTile;
+  if (asked == 0 || n_blk > kMaxItems || n_bh > cus || (asked < 0 && (int64_t)n_bh * n_blk > 4 * cus)) return DkdvPlan();
+  // (the heads in one group, see launch_bwd)
+  if (2 * ((int64_t)Sq + Sk) * 128 * 2 * n_bh > (256ll << 20)) return DkdvPlan();
+  auto tiles = [&](int blk) { const int first = kBwdRows / kBwdTile * blk; return causal ? (first < n_qt ? n_qt - first : 0) : n_qt; };
+  return share_blocks(n_bh, n_blk, tiles, causal, asked, cus, {4, 2, 4, 32, 1, false}, causal ? 90 : 82);
 }
 
 }  // namespace fo

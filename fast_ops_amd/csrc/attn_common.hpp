@@ -179,16 +179,16 @@ struct DropRows {
   static __device__ __forceinline__ uint32_t index(const DropoutParams& d, int bh, int Sq, int Sk, int row, int key) {
     return d.offset + ((uint32_t)bh * (uint32_t)Sq + (uint32_t)row) * (uint32_t)Sk + (uint32_t)key;
   }
-  // the state of key tile `tile`, asked for every tile in turn; row0: the wave's first row (block b is 32 b rows further)
+  // the state of key tile `tile` (of those from key0 on), asked for every tile in turn; row0: the wave's first row (block b is 32 b rows further)
   template <typename P>
-  __device__ __forceinline__ void look(const P& d_in, int bh, int Sq, int Sk, int row0, int tile) {
+  __device__ __forceinline__ void look(const P& d_in, int bh, int Sq, int Sk, int row0, int tile, int key0 = 0) {
     if (__builtin_expect(tile % kDropSpanTiles == 0, 0)) {      // (laid out away from the tile loops)
       const DropoutParams d = {d_in.seed, d_in.threshold, d_in.offset, 1.0f, 1.0f, 0.0f};
-      look_at_span(d, bh, Sq, Sk, row0, tile * 64);
+      look_at_span(d, bh, Sq, Sk, row0, key0 + tile * 64);
     }
     if (__builtin_expect(by_tile, 0)) {
       const DropoutParams d = {d_in.seed, d_in.threshold, d_in.offset, 1.0f, 1.0f, 0.0f};
-      look_at_tile(d, bh, Sq, Sk, row0, tile);
+      look_at_tile(d, bh, Sq, Sk, row0, tile % kDropSpanTiles, key0 + tile * 64);
     }
   }
   // The next kDropSpanTiles tiles from key0 on as a whole; where some row is neither kept nor dropped over all of them, every row's
@@ -226,8 +226,8 @@ struct DropRows {
     }
   }
   // one of those tiles; its rows that are neither are hashed
-  __device__ __forceinline__ void look_at_tile(const DropoutParams& d, int bh, int Sq, int Sk, int row0, int tile) {
-    const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5, t = tile % kDropSpanTiles;
+  __device__ __forceinline__ void look_at_tile(const DropoutParams& d, int bh, int Sq, int Sk, int row0, int t, int key0) {
+    const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
     uint64_t mixed_rows = 0, keep_rows = 0, drop_rows = 0;
 #pragma unroll
     for (int b = 0; b < QB; ++b) {
@@ -241,7 +241,7 @@ struct DropRows {
       while (mixed != 0) {
         const int i = __builtin_ctz(mixed);
         mixed &= mixed - 1;
-        const uint64_t k = __builtin_amdgcn_ballot_w64(dropout_keep(index(d, bh, Sq, Sk, row0 + 32 * b + i, tile * 64 + lane), d.seed, d.threshold));
+        const uint64_t k = __builtin_amdgcn_ballot_w64(dropout_keep(index(d, bh, Sq, Sk, row0 + 32 * b + i, key0 + lane), d.seed, d.threshold));
         if (l32 == i) { bits[b][0] = (uint32_t)k >> (4 * hh); bits[b][1] = (uint32_t)(k >> 32) >> (4 * hh); }
       }
     }
@@ -252,9 +252,9 @@ struct DropRows {
   // what the state is.
   typedef uint32_t Words[2][QB][8];
   template <typename P>
-  __device__ __forceinline__ void look(const P& d_in, int bh, int Sq, int Sk, int row0, int tile, Words& words) {
+  __device__ __forceinline__ void look(const P& d_in, int bh, int Sq, int Sk, int row0, int tile, Words& words, int key0) {
     if (__builtin_expect(tile % kDropSpanTiles != 0 && !by_tile, 1)) return;
-    look(d_in, bh, Sq, Sk, row0, tile);
+    look(d_in, bh, Sq, Sk, row0, tile, key0);
     if (state == kMasked) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)

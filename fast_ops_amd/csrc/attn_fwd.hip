@@ -29,6 +29,7 @@
 #include <type_traits>
 
 #include "attn_common.hpp"
+#include "attn_fwd_plan.hpp"
 
 // This file is compiled several times, in parallel: as it stands it is the C ABI and the kernel choice, and holds no
 // kernel; attn_fwd_bf16_d64.hip ... attn_fwd_f16_d128.hip include it with FO_ATTN_UNIT set and instantiate launch<T, D>,
@@ -60,7 +61,16 @@ struct AttnParams {
   uint8_t order_tab[kOrderTab];         // position in an XCD's launch order -> rank of the workgroup (0 = heaviest) that runs there
   DropoutParams drop;                   // used by the kernels instantiated with dropout only
   BiasParams bias;                      // used by the kernels instantiated with bias only
+  // 128-row pipelined form: where the workgroups of a shared query block leave their sums (fwd_part_floats each), part_bytes of room, and
+  // which blocks are shared (make_fwd_plan); n_items 0 = a workgroup per block
+  float* part;
+  int64_t part_bytes;
+  int n_items, n_merges;
+  uint32_t items[kMaxItems], merges[kMaxMerges];
 };
+// a part: a wave's accumulators of O^T, 1 KiB per four registers, for each of four waves; then reference (base 2) and row sum of each row
+constexpr int fwd_part_floats(int D) { return kBM * D + 2 * kBM; }
+__host__ __device__ inline float* fwd_part(float* base, int D, uint32_t part, int n_bh, int bh) { return base + ((int64_t)part * n_bh + bh) * fwd_part_floats(D); }
 
 constexpr int kDecodeMinKeys = 128;
 constexpr int64_t kMaxRowStride = 1ll << 24;   // elements; see attn_fwd_impl
@@ -684,10 +694,12 @@ struct BiasRing {
 };
 
 // TBIAS: bytes per element of a bias with a query stride (128 rows, no dropout; 0: none)
-template <typename T, int D, bool CAUSAL, int QB, int DBG, int BM = kWideBM, bool VBIAS = false, bool DROP = false, int TBIAS = 0>
+// PARTS: workgroups share query blocks (128 rows; make_fwd_plan). A form of its own: what it adds costs a launch of whole blocks 2 %.
+template <typename T, int D, bool CAUSAL, int QB, int DBG, int BM = kWideBM, bool VBIAS = false, bool DROP = false, int TBIAS = 0, bool PARTS = false>
 __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 128 || VBIAS || TBIAS != 0) ? 1 : 2) attn_fwd_wide_kernel(const AttnParams prm_arg) {
   const AttnParams& prm = prm_arg;
   static_assert(TBIAS == 0 || (BM == kBM && QB == 1 && !VBIAS && !DROP), "form with a bias per query");
+  static_assert(!PARTS || BM == kBM, "form that shares blocks");
   // VBIAS: an additive bias that is the same for every query of a head (query stride 0: the reference's "vector" bias,
   // flash_attention_triton.py:176-186, e.g. a key padding mask). The head's row of it, at most kVBiasKeys keys, is put
   // into LDS once per workgroup as fp32 divided by softmax_scale, so that (S + b / scale) * scale * log2 e is the biased
@@ -777,6 +789,18 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   int wg_id = blockIdx.x;
   int bh, item;
   decode(wg_id, bh, item);
+  // PARTS: a workgroup takes the key tiles from tile0 on, up to tile_end; everything below sees those keys only
+  int tile0 = 0, tile_end = 0;
+  uint32_t part = kWholeBlock >> 16;
+  if constexpr (PARTS) {
+    const uint32_t w = prm.items[wg_id / n_bh];
+    bh = wg_id % n_bh;
+    item = (int)(w & 255u);
+    part = w >> 16;
+    const int piece = (int)(w >> 8) & 15, pieces = (int)(w >> 12) & 15, all = fwd_plan_tiles(item, prm.Sk, CAUSAL);
+    tile0 = all * piece / pieces;
+    tile_end = all * (piece + 1) / pieces;
+  }
   if (tail_mode && item * BM >= prm.Sq) return;        // (the second half of a last block that has only one)
   int pass = 0;
   bool first_block = true, prefetched = false;
@@ -828,14 +852,16 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   }
   const int q0 = qblk * BM;
   const int q0w = q0 + wave_s * 32 * QB;
-  const int Sq = prm.Sq, Sk = prm.Sk;
-  const T* __restrict__ kbase = (const T*)prm.k + b * prm.ks[0] + h * prm.ks[1];
-  const T* __restrict__ vbase = (const T*)prm.v + b * prm.vs[0] + h * prm.vs[1];
+  // (of a shared block: the workgroup's own keys, counted from its first one, key0; q0k, where the wave's first row stands among them)
+  const int key0 = PARTS ? tile0 * kBN : 0, q0k = q0w - key0;
+  const int Sq = prm.Sq, Sk = PARTS ? min(prm.Sk, tile_end * kBN) - key0 : prm.Sk;
+  const T* __restrict__ kbase = (const T*)prm.k + b * prm.ks[0] + h * prm.ks[1] + key0 * prm.ks[2];
+  const T* __restrict__ vbase = (const T*)prm.v + b * prm.vs[0] + h * prm.vs[1] + key0 * prm.vs[2];
 
   int n_tiles, n_w;                       // tiles the workgroup walks / tiles in which this wave has unmasked keys
   if constexpr (CAUSAL) {
-    n_tiles = (min(Sk, q0 + BM) + kBN - 1) / kBN;
-    n_w = min(n_tiles, (q0w + 32 * QB - 1) / kBN + 1);
+    n_tiles = (min(Sk, q0 + BM - key0) + kBN - 1) / kBN;
+    n_w = min(n_tiles, (q0k + 32 * QB - 1) / kBN + 1);
   } else {
     n_tiles = (Sk + kBN - 1) / kBN;
     n_w = n_tiles;
@@ -960,7 +986,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
 #pragma unroll
     for (int i = 0; i < BR::DMAS; ++i) {
       const int row = i * BR::ROWS_PER_DMA + lane / BR::PIECES;
-      bias_row[i] = (const BE*)prm.bias.ptr + b * prm.bias.strides[0] + h * prm.bias.strides[1] + (int64_t)min(q0w + row, Sq - 1) * prm.bias.strides[2];
+      bias_row[i] = (const BE*)prm.bias.ptr + b * prm.bias.strides[0] + h * prm.bias.strides[1] + (int64_t)min(q0w + row, Sq - 1) * prm.bias.strides[2] + key0;
     }
   }
   auto issue_bias = [&](int sub, int i) {            // copy i of a half tile, anywhere
@@ -1006,7 +1032,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
       const float per_scale = 1.4426950408889634f / prm.scale_log2e;
       const int n_pad = n_tiles * kBN;                                   // at most kVBiasKeys: the launcher checks
       for (int i = tid; i < n_pad; i += kWideWaves * 64)
-        ((FO_LDS float*)(smem + 2 * kRing * TILE_BYTES))[i] = load_bias<T>(prm.bias, brow + min(i, prm.Sk - 1)) * per_scale;
+        ((FO_LDS float*)(smem + 2 * kRing * TILE_BYTES))[i] = load_bias<T>(prm.bias, brow + key0 + min(i, Sk - 1)) * per_scale;
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                 // (in LDS before the first tile's barrier)
     }
   }
@@ -1159,7 +1185,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
 #pragma unroll
         for (int b2 = 0; b2 < QB; ++b2) {
           int lim = key_base - Sk + 1;
-          if (CAUSAL) lim = max(lim, key_base - (q0w + 32 * b2 + l32));
+          if (CAUSAL) lim = max(lim, key_base - (q0k + 32 * b2 + l32));
 #pragma unroll
           for (int r = 0; r < 16; ++r) S[P][b2][r] = (lim > -((r & 3) + 8 * (r >> 2))) ? -INFINITY : S[P][b2][r];
         }
@@ -1276,7 +1302,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     for (int b2 = 0; b2 < QB; ++b2) l_run[b2] += psum[b2];
   };
   auto drop_look = [&](int j) {
-    if constexpr (DROP) drop.look(prm.drop, bh, Sq, Sk, q0w, j, drop_words);
+    if constexpr (DROP) drop.look(prm.drop, bh, Sq, prm.Sk, q0w, j, drop_words, key0);
   };
   using std::integral_constant;
   typedef integral_constant<int, 0> P0;
@@ -1312,7 +1338,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   // kept free of alternatives: unmasked tiles, then masked tiles, then the last tile, whose second step has no scores
   // left to compute; the first and last tiles always take the masking variant.
   int j_mask = n_w;                                   // first tile that needs the mask
-  if (CAUSAL) j_mask = min(j_mask, (q0w + 1) / kBN);   // smallest j with 64 j + 63 > q0w
+  if (CAUSAL) j_mask = min(j_mask, (q0k + 1) / kBN);   // smallest j with 64 j + 63 > q0k
   if (Sk % kBN != 0) j_mask = min(j_mask, n_tiles - 1);
 
   // first tile: fill the pipeline - S(0) on its own, then a step that has nothing to multiply yet
@@ -1362,7 +1388,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
 #pragma unroll
   for (int b2 = 0; b2 < QB; ++b2) {
     int lim = 4 * hh - Sk + 1;
-    if (CAUSAL) lim = max(lim, 4 * hh - (q0w + 32 * b2 + l32));
+    if (CAUSAL) lim = max(lim, 4 * hh - (q0k + 32 * b2 + l32));
     float mloc = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -1445,6 +1471,22 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   // ---- epilogue: normalise, write O and LSE
 #pragma unroll
   for (int d = 0; d < DBLK; ++d) mfma_result_fence_a(oacc[d]);
+  if constexpr (PARTS) {
+    if (part != kWholeBlock >> 16) {                    // a shared block: the sums as they stand, for the merge
+      float* mine = fwd_part(prm.part, D, part, n_bh, bh);
+#pragma unroll
+      for (int db = 0; db < DBLK; ++db) {
+        f32x16 t = oacc[db][0];
+        asm volatile("" : "+v"(t));
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg)
+          *(f32x4*)(mine + ((wave_s * DBLK + db) * 4 + rg) * 256 + lane * 4) = f32x4{t[4 * rg], t[4 * rg + 1], t[4 * rg + 2], t[4 * rg + 3]};
+      }
+      const float l_tot = l_run[0] + half_swap(l_run[0]);
+      if (hh == 0) *(f32x2*)(mine + kBM * D + 2 * (wave_s * 32 + l32)) = f32x2{TBIAS ? m_run[0] : m_run[0] * c, l_tot};
+      return;
+    }
+  }
   // A lane holds 4 consecutive d of one query row per accumulator register group: written straight to memory that is
   // 8 bytes per lane, 16 per row and instruction. Instead the wave's rows are staged in LDS (the rings are free once
   // every wave is past its last tile; rows padded by 16 bytes against bank conflicts) and leave as whole 16-byte
@@ -1506,6 +1548,70 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   }   // query blocks
 }
 
+// O and LSE of the query blocks that several workgroups shared: their sums brought to the largest of their references and added, in order.
+// One workgroup per 32 rows of a block, a wave per 32 columns; bound by reading the parts, which the caches hold (see make_fwd_plan for what
+// it costs).
+template <typename T, int D>
+__global__ void __launch_bounds__(2 * D) attn_fwd_merge_kernel(const AttnParams prm) {
+  constexpr int OROW = D * 2 + 16, CH = D * 2 / 16;
+  __shared__ __attribute__((aligned(16))) char rows[32 * OROW];
+  const int n_bh = prm.B * prm.H, quarter = blockIdx.x & 3, at = (int)(blockIdx.x >> 2), bh = at % n_bh;
+  const uint32_t w = prm.merges[at / n_bh];
+  const int q0 = (int)(w & 255u) * kBM + 32 * quarter, pieces = (int)(w >> 12) & 15;
+  const int db = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
+  f32x2 ml[kMaxPieces];
+  f32x4 o4[kMaxPieces][4];
+#pragma unroll
+  for (int i = 0; i < kMaxPieces; ++i) {
+    if (i < pieces) {
+      const float* p = fwd_part(prm.part, D, (w >> 16) + i, n_bh, bh);
+      ml[i] = *(const f32x2*)(p + kBM * D + 2 * (32 * quarter + l32));
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) o4[i][rg] = *(const f32x4*)(p + ((quarter * (D / 32) + db) * 4 + rg) * 256 + lane * 4);
+    }
+  }
+  float m = ml[0][0], l = 0.0f;
+#pragma unroll
+  for (int i = 1; i < kMaxPieces; ++i) m = i < pieces ? fmaxf(m, ml[i][0]) : m;
+  f32x4 acc[4];
+#pragma unroll
+  for (int i = 0; i < kMaxPieces; ++i) {
+    if (i < pieces) {
+      const float f = __builtin_amdgcn_exp2f(ml[i][0] - m);      // (no key of a piece counts: 0, and so is its sum)
+      l = i == 0 ? f * ml[i][1] : l + f * ml[i][1];
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[rg][u] = i == 0 ? f * o4[i][rg][u] : acc[rg][u] + f * o4[i][rg][u];
+    }
+  }
+  const float inv = prm.drop.keep_scale / l;
+  typedef __attribute__((ext_vector_type(4))) T vec4;
+#pragma unroll
+  for (int rg = 0; rg < 4; ++rg) {
+    const vec4 out = {(T)(acc[rg][0] * inv), (T)(acc[rg][1] * inv), (T)(acc[rg][2] * inv), (T)(acc[rg][3] * inv)};
+    *(vec4*)(rows + l32 * OROW + (32 * db + 8 * rg + 4 * hh) * 2) = out;
+  }
+  if (db == 0 && hh == 0 && prm.lse != nullptr && q0 + l32 < prm.Sq)
+    prm.lse[(int64_t)bh * prm.Sq + q0 + l32] = (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
+  __syncthreads();
+  T* obase = (T*)prm.o + (bh / prm.H) * prm.os[0] + (bh % prm.H) * prm.os[1];
+  for (int i = threadIdx.x; i < 32 * CH; i += 2 * D) {
+    const int row = i / CH, ch = i % CH;
+    if (q0 + row < prm.Sq) *(i32x4*)(obase + (int64_t)(q0 + row) * prm.os[2] + ch * 8) = *(const i32x4*)(rows + row * OROW + ch * 16);
+  }
+}
+
+// The plan of a launch of the 128-row pipelined form on the current device; a thread's last eight are kept (laying one out takes 10 to 30 us).
+const DkdvPlan& fwd_plan(int n_bh, int Sq, int Sk, bool causal);
+// Whether workgroups of the 128-row pipelined form share query blocks of a call (given p.part_bytes of memory for their sums)
+[[maybe_unused]] static const DkdvPlan* shares_blocks(const AttnParams& p, int D, bool causal) {
+  if (p.part_bytes <= 0) return nullptr;
+  const int n_bh = p.B * p.H;
+  const DkdvPlan& plan = fwd_plan(n_bh, p.Sq, p.Sk, causal);
+  return plan.n_merges > 0 && p.part_bytes >= (int64_t)plan.n_parts * n_bh * fwd_part_floats(D) * 4 ? &plan : nullptr;
+}
+
 // heads per group in the causal order "heaviest query blocks of a group's heads first" of the kernels that take one
 // 128-row query block per workgroup (see launch_one)
 [[maybe_unused]] static int heavy_first_group(const AttnParams& p, int D) {   // (used by the launchers only: not in every unit)
@@ -1544,6 +1650,22 @@ static int launch_wide(AttnParams p, hipStream_t stream) {
   }
   p.heavy_first = (CAUSAL && BM != kWideBM) ? heavy_first_group(p, D) : 0;
   p.order_n = 0;
+  p.n_items = 0;
+  if constexpr (BM != kWideBM) {
+    const DkdvPlan* plan = p.tail_base == 0 ? shares_blocks(p, D, CAUSAL) : nullptr;
+    if (plan != nullptr) {
+      p.n_items = plan->n_items;
+      p.n_merges = plan->n_merges;
+      for (int i = 0; i < plan->n_items; ++i) p.items[i] = plan->items[i];
+      for (int i = 0; i < plan->n_merges; ++i) p.merges[i] = plan->merges[i];
+      static const hipError_t parts_attr = hipFuncSetAttribute((const void*)attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS, DROP, TBIAS, true>,
+                                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (parts_attr != hipSuccess) return FO_ERR_LAUNCH;
+      attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS, DROP, TBIAS, true><<<(unsigned)(plan->n_items * p.B * p.H), BM / (32 * QB) * 64, lds, stream>>>(p);
+      attn_fwd_merge_kernel<T, D><<<(unsigned)(4 * p.n_merges * p.B * p.H), 2 * D, 0, stream>>>(p);
+      return launch_status();
+    }
+  }
   static const hipError_t attr = hipFuncSetAttribute((const void*)attn_fwd_wide_kernel<T, D, CAUSAL, QB, DBG, BM, VBIAS, DROP, TBIAS>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return FO_ERR_LAUNCH;
@@ -1656,7 +1778,9 @@ static int choose_kernel(const AttnParams& p, int D, bool causal, bool dropout, 
     if (p.d != D || dropout || !p.bias.dma_ok || !wide_ok || (D == 128 && p.bias.is_f32)) return FO_ATTN_KERNEL_ROWS128;
     if (forced >= 0) return forced == FO_ATTN_KERNEL_ROWS128_PIPE ? FO_ATTN_KERNEL_ROWS128_PIPE : FO_ATTN_KERNEL_ROWS128;
     const int64_t wgs128 = ((int64_t)p.Sq + kBM - 1) / kBM * p.B * p.H, cus = device_cus();
-    return (int64_t)p.Sq * p.Sk >= kRowBiasPipePairs && wgs128 <= (causal ? cus + cus / 2 : cus) ? FO_ATTN_KERNEL_ROWS128_PIPE : FO_ATTN_KERNEL_ROWS128;
+    // (more of them when several can share the blocks of the last round, not causal: 12 x 3072 119 -> 109)
+    if ((int64_t)p.Sq * p.Sk < kRowBiasPipePairs) return FO_ATTN_KERNEL_ROWS128;
+    return wgs128 <= (causal ? cus + cus / 2 : cus) || (!causal && shares_blocks(p, D, false)) ? FO_ATTN_KERNEL_ROWS128_PIPE : FO_ATTN_KERNEL_ROWS128;
   }
   if ((p.bias.ptr != nullptr && !key_bias) || p.d != D) return FO_ATTN_KERNEL_ROWS128;
   // ... and needs one 256-row workgroup (two query blocks each when causal) per CU to be worth it: below that the
@@ -1708,6 +1832,9 @@ static int choose_kernel(const AttnParams& p, int D, bool causal, bool dropout, 
       const int64_t wgs128 = ((int64_t)p.Sq + kBM - 1) / kBM * p.B * p.H;
       const int64_t slots = (int64_t)n_cu * (D == 64 ? 2 : 1) * (causal ? 2 : 1);
       if (wgs128 <= slots && keys >= (D == 64 ? 2048 : 1024)) v = FO_ATTN_KERNEL_ROWS128_PIPE;
+      // not causal, with a last round that workgroups can share (given the memory for it): plain kernel -> shared, 12 heads x 3072 86 -> 74 us,
+      // with a padding mask and dropout 104 -> 82, 6 heads x 6000 159 -> 129 and 196 -> 145
+      else if (D == 128 && !causal && keys >= 1024 && shares_blocks(p, D, false)) v = FO_ATTN_KERNEL_ROWS128_PIPE;
     }
     // head_dim 128 with many key tiles per query block: four waves x 64 rows. Every K / V^T fragment read from LDS feeds two
     // MFMAs, which costs less energy (at full load the chip's clock is what its power budget leaves) but more cycles per
@@ -1890,6 +2017,43 @@ static bool takes_decode(const AttnParams& p, bool causal, bool dropout, int for
   return (int64_t)p.B * p.H * p.Sq < (1ll << 31);
 }
 
+namespace fo {
+const DkdvPlan& fwd_plan(int n_bh, int Sq, int Sk, bool causal) {
+  struct Place { int n_bh, Sq, Sk, causal, asked, cus; DkdvPlan plan; };
+  constexpr int kPlaces = 8;
+  static thread_local Place places[kPlaces];      // (n_bh 0: empty)
+  static thread_local int oldest = 0;
+  const int asked = tune(g_attn_split), cus = device_cus();
+  for (const Place& p : places)
+    if (p.n_bh == n_bh && p.Sq == Sq && p.Sk == Sk && p.causal == (int)causal && p.asked == asked && p.cus == cus) return p.plan;
+  Place& p = places[oldest];
+  oldest = (oldest + 1) % kPlaces;
+  p.n_bh = n_bh; p.Sq = Sq; p.Sk = Sk; p.causal = (int)causal; p.asked = asked; p.cus = cus;
+  p.plan = make_fwd_plan(n_bh, Sq, Sk, causal, asked, cus);
+  return p.plan;
+}
+}  // namespace fo
+// bytes that the shared blocks of a call leave their sums in, 0 where no block is shared
+static int64_t fwd_part_bytes(const AttnParams& p, bool causal, bool dropout) {
+  const int D = p.d > 64 ? 128 : 64;
+  AttnParams with = p;
+  with.part_bytes = 1ll << 62;                      // (as if there were all the memory in the world)
+  if (choose_kernel(with, D, causal, dropout, tune(g_attn_variant)) != FO_ATTN_KERNEL_ROWS128_PIPE) return 0;
+  const DkdvPlan* plan = shares_blocks(with, D, causal);
+  return plan ? (int64_t)plan->n_parts * p.B * p.H * fwd_part_floats(D) * (int64_t)sizeof(float) : 0;
+}
+static void set_bias(AttnParams& p, const void* bias, const int64_t* strides, int dtype) {
+  p.bias.ptr = bias;
+  for (int i = 0; i < 3; ++i) p.bias.strides[i] = bias ? strides[i] : 0;
+  p.bias.is_f32 = dtype == FO_DTYPE_F32;
+  const int64_t elt = p.bias.is_f32 ? 4 : 2;
+  p.bias.vec_ok = bias && ((uintptr_t)bias % (4 * elt)) == 0 && p.bias.strides[0] % 4 == 0 && p.bias.strides[1] % 4 == 0 && p.bias.strides[2] % 4 == 0;
+  // (a bias that is the same for every query - query stride 0 - is one row per tile: per-element loads of it are
+  // broadcasts, and the kernel keeps its two workgroups per CU without the LDS for bias tiles)
+  p.bias.dma_ok = bias && p.bias.strides[2] != 0 && ((uintptr_t)bias % 16) == 0 && (p.bias.strides[0] * elt) % 16 == 0 &&
+                  (p.bias.strides[1] * elt) % 16 == 0 && (p.bias.strides[2] * elt) % 16 == 0;
+}
+
 static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, float* lse,
                          int B, int H, int Sq, int Sk, int D,
                          const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os,
@@ -1925,17 +2089,10 @@ static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, f
   p.heavy_first = 0; p.order_n = 0; p.id_limit = 0; p.tail_base = 0; p.keep_on = 0;
   const bool drop = dropout_p > 0.0f;
   p.drop = make_dropout(dropout_p, seed, rng_offset);
-  p.bias.ptr = bias;
-  for (int i = 0; i < 3; ++i) p.bias.strides[i] = bias ? bias_strides[i] : 0;
-  p.bias.is_f32 = bias_dtype == FO_DTYPE_F32;
-  {
-    const int64_t elt = p.bias.is_f32 ? 4 : 2;
-    p.bias.vec_ok = bias && ((uintptr_t)bias % (4 * elt)) == 0 && p.bias.strides[0] % 4 == 0 && p.bias.strides[1] % 4 == 0 && p.bias.strides[2] % 4 == 0;
-    // (a bias that is the same for every query - query stride 0 - is one row per tile: per-element loads of it are
-    // broadcasts, and the kernel keeps its two workgroups per CU without the LDS for bias tiles)
-    p.bias.dma_ok = bias && p.bias.strides[2] != 0 && ((uintptr_t)bias % 16) == 0 && (p.bias.strides[0] * elt) % 16 == 0 &&
-                    (p.bias.strides[1] * elt) % 16 == 0 && (p.bias.strides[2] * elt) % 16 == 0;
-  }
+  set_bias(p, bias, bias_strides, bias_dtype);
+  p.n_items = 0; p.n_merges = 0;
+  p.part = (float*)ws;
+  p.part_bytes = ws != nullptr && ((uintptr_t)ws & 15u) == 0 ? ws_bytes : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (takes_decode(p, causal != 0, drop, tune(g_attn_variant))) {
     DecodeParams d;
@@ -1971,13 +2128,28 @@ extern "C" int fo_attn_fwd_kernel(int B, int H, int Sq, int Sk, int D, const int
   return choose_kernel(p, D > 64 ? 128 : 64, causal != 0, has_dropout != 0, tune(g_attn_variant));
 }
 
-extern "C" int64_t fo_attn_fwd_workspace(int B, int H, int Sq, int Sk, int D, const int64_t* ks, const int64_t* vs, int causal) {
+extern "C" int64_t fo_attn_fwd_workspace_ex(int B, int H, int Sq, int Sk, int D, const int64_t* ks, const int64_t* vs, int causal, const fo_attn_extras* extras) {
   if (!ks || !vs || check_sizes(B, H, Sq, Sk, D) || check_strides(ks, D, true) || check_strides(vs, D, true)) return 0;
   AttnParams p = {};
   p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.d = D;
   for (int i = 0; i < 3; ++i) { p.ks[i] = ks[i]; p.vs[i] = vs[i]; }
-  if (!takes_decode(p, causal != 0, false, tune(g_attn_variant))) return 0;
-  return decode_workspace_bytes(B, H, Sq, D, decode_split(B, H, decode_n_kv(p), Sq, Sk, D, device_cus()));
+  const bool dropout = extras && extras->dropout_p > 0.0f;
+  if (extras) set_bias(p, extras->bias, extras->bias_strides, extras->bias_dtype);
+  if (takes_decode(p, causal != 0, dropout, tune(g_attn_variant))) return decode_workspace_bytes(B, H, Sq, D, decode_split(B, H, decode_n_kv(p), Sq, Sk, D, device_cus()));
+  return fwd_part_bytes(p, causal != 0, dropout);
+}
+
+extern "C" int64_t fo_attn_fwd_workspace(int B, int H, int Sq, int Sk, int D, const int64_t* ks, const int64_t* vs, int causal) {
+  return fo_attn_fwd_workspace_ex(B, H, Sq, Sk, D, ks, vs, causal, nullptr);
+}
+
+extern "C" int fo_attn_fwd_ex_ws(const void* q, const void* k, const void* v, void* o, float* lse,
+                                 int B, int H, int Sq, int Sk, int D,
+                                 const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os,
+                                 float softmax_scale, int causal, int dtype, const fo_attn_extras* extras, void* ws, int64_t ws_bytes, void* stream) {
+  if (!extras) return fo_attn_fwd_ws(q, k, v, o, lse, B, H, Sq, Sk, D, qs, ks, vs, os, softmax_scale, causal, dtype, ws, ws_bytes, stream);
+  return attn_fwd_impl(q, k, v, o, lse, B, H, Sq, Sk, D, qs, ks, vs, os, softmax_scale, causal, dtype, extras->dropout_p,
+                       extras->dropout_seed, extras->dropout_offset, extras->bias, extras->bias_strides, extras->bias_dtype, stream, ws, ws_bytes);
 }
 
 extern "C" int fo_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,

@@ -8,6 +8,7 @@ std::atomic<int> g_lion_variant{-1};
 std::atomic<int> g_attn_variant{-1};
 std::atomic<int> g_attn_bwd_variant{-1};
 std::atomic<int> g_attn_order{-1};
+std::atomic<int> g_attn_split{-1};
 std::atomic<int> g_attn_keep_on{-1};
 std::atomic<int> g_attn_decode_split{-1};
 std::atomic<int> g_attn_tail{-1};
@@ -63,6 +64,10 @@ extern "C" int fo_tune_set(const char* key, int value) {
     if (value > 2) return FO_ERR_UNSUPPORTED;
     fo::g_attn_keep_on = value; return FO_OK;
   }
+  if (strcmp(key, "attn.split") == 0) {
+    if (value == 1 || value > 4) return FO_ERR_UNSUPPORTED;      // 0 = never, 2 to 4 = every block in so many pieces
+    fo::g_attn_split = value; return FO_OK;
+  }
   if (strcmp(key, "attn.decode_split") == 0) {
     if (value == 0 || value > 64) return FO_ERR_UNSUPPORTED;
     fo::g_attn_decode_split = value; return FO_OK;
@@ -98,6 +103,7 @@ extern "C" int fo_tune_get(const char* key) {
   if (strcmp(key, "attn_bwd.variant") == 0) return fo::tune(fo::g_attn_bwd_variant);
   if (strcmp(key, "attn.order") == 0) return fo::tune(fo::g_attn_order);
   if (strcmp(key, "attn.keep_on") == 0) return fo::tune(fo::g_attn_keep_on);
+  if (strcmp(key, "attn.split") == 0) return fo::tune(fo::g_attn_split);
   if (strcmp(key, "attn.decode_split") == 0) return fo::tune(fo::g_attn_decode_split);
   if (strcmp(key, "attn.tail") == 0) return fo::tune(fo::g_attn_tail);
   if (strcmp(key, "attn.balance") == 0) return fo::tune(fo::g_attn_balance);

@@ -175,7 +175,7 @@ def dropout_mask(
 class _FwdPlan:
     """What a forward call of one (shapes, strides, dtype, device, layout) needs besides the data pointers: checked once,
     then reused - the checks, the stride arrays for the C ABI and the sizes cost more host time than a small kernel runs."""
-    __slots__ = ("B", "H", "Sq", "Sk", "D", "qs", "ks", "vs", "os", "o_dense_like_q", "dtype_code", "device_index", "lse_shape", "ws_bytes")
+    __slots__ = ("B", "H", "Sq", "Sk", "D", "qs", "ks", "vs", "os", "o_dense_like_q", "dtype_code", "device_index", "lse_shape", "ws_bytes", "ws_bytes_causal", "ws_forms")
 
 
 _FWD_PLANS: dict = {}
@@ -209,19 +209,40 @@ def _fwd_plan(q: Tensor, k: Tensor, v: Tensor, dims: Tuple[int, int, int, int]) 
     plan.dtype_code = _DTYPE_CODE[q.dtype]
     plan.device_index = q.device.index if q.device.index is not None else torch.cuda.current_device()
     plan.lse_shape = (B, H, Sq)
-    with torch.cuda.device(plan.device_index):       # scratch memory of a call without mask, bias and dropout: few queries, many keys
-        plan.ws_bytes = _lib.load().fo_attn_fwd_workspace(B, H, Sq, Sk, D, plan.ks, plan.vs, 0)
+    with torch.cuda.device(plan.device_index):       # scratch memory of a call without bias and dropout, by the mask; other forms: _fwd_workspace
+        plan.ws_bytes, plan.ws_bytes_causal = (_lib.load().fo_attn_fwd_workspace(B, H, Sq, Sk, D, plan.ks, plan.vs, causal) for causal in (0, 1))
+    plan.ws_forms = {}
     if len(_FWD_PLANS) > 4096:
         _FWD_PLANS.clear()
     _FWD_PLANS[key] = plan
     return plan
 
 
+def _fwd_workspace(plan: _FwdPlan, causal: bool, bias: Optional[Tensor], dropout: Optional[Dropout], extras) -> int:
+    """Bytes of scratch memory that a call with a bias or dropout can use, worked out once per plan and form (as _bwd_workspace)."""
+    form = (causal, dropout is not None and dropout[0] > 0.0, None if bias is None else (bias.stride(), bias.data_ptr() % 16, bias.dtype))
+    n = plan.ws_forms.get(form)
+    if n is None:
+        n = _lib.load().fo_attn_fwd_workspace_ex(plan.B, plan.H, plan.Sq, plan.Sk, plan.D, plan.ks, plan.vs, 1 if causal else 0, extras)
+        if len(plan.ws_forms) > 64:
+            plan.ws_forms.clear()
+        plan.ws_forms[form] = n
+    return n
+
+
+def _scratch(n_bytes: int, device) -> Optional[Tensor]:
+    """Scratch memory, or None where there is none to be had (the call then computes the same without)."""
+    try:
+        return torch.empty(n_bytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def attn_fwd_strided(
     q: Tensor, k: Tensor, v: Tensor, dims: Tuple[int, int, int, int], causal: bool, softmax_scale: Optional[float],
     dropout: Optional[Dropout] = None, bias: Optional[Tensor] = None,
 ) -> Tuple[Tensor, Tensor]:
-    """Launches fo_attn_fwd (fo_attn_fwd_dropout when ``dropout`` is given, fo_attn_fwd_ex when ``bias`` is). ``dims`` =
+    """Launches fo_attn_fwd (fo_attn_fwd_ex when ``bias`` or ``dropout`` is given), with scratch memory where it helps. ``dims`` =
     positions of (batch, head, sequence, head_dim) in the tensors' shapes; ``bias`` is [B|1, H|1, Sq|1, Sk] whatever
     ``dims`` says. Returns (O with q's shape, dtype and layout; LSE fp32 [B, H, Sq])."""
     plan = _fwd_plan(q, k, v, dims)
@@ -241,16 +262,21 @@ def attn_fwd_strided(
         args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
                 plan.B, plan.H, plan.Sq, plan.Sk, plan.D, plan.qs, plan.ks, plan.vs, plan.os,
                 scale, 1 if causal else 0, plan.dtype_code)
-        if bias is not None:
-            status = lib.fo_attn_fwd_ex(*args, ctypes.byref(_extras(bias, dropout)), stream)
-        elif dropout is None or dropout[0] == 0.0:
-            if plan.ws_bytes and not causal:
-                ws = torch.empty(plan.ws_bytes, dtype=torch.uint8, device=q.device)
-                status = lib.fo_attn_fwd_ws(*args, ws.data_ptr(), plan.ws_bytes, stream)
+        if bias is None and (dropout is None or dropout[0] == 0.0):
+            n = plan.ws_bytes_causal if causal else plan.ws_bytes
+            ws = _scratch(n, q.device) if n else None
+            if ws is not None:
+                status = lib.fo_attn_fwd_ws(*args, ws.data_ptr(), n, stream)
             else:
                 status = lib.fo_attn_fwd(*args, stream)
         else:
-            status = lib.fo_attn_fwd_dropout(*args, float(dropout[0]), dropout[1] & 0xFFFFFFFF, dropout[2] % (1 << 64), stream)
+            extras = ctypes.byref(_extras(bias, dropout))
+            n = _fwd_workspace(plan, causal, bias, dropout, extras)
+            ws = _scratch(n, q.device) if n else None
+            if ws is not None:
+                status = lib.fo_attn_fwd_ex_ws(*args, extras, ws.data_ptr(), n, stream)
+            else:
+                status = lib.fo_attn_fwd_ex(*args, extras, stream)
     finally:
         if guard is not None:
             guard.__exit__(None, None, None)

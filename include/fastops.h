@@ -84,12 +84,14 @@ int fo_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse
                 const int64_t* v_strides_host, const int64_t* o_strides_host,
                 float softmax_scale, int causal, int dtype, void* stream);
 
-/* fo_attn_fwd with scratch memory for shapes of few query rows and many keys (up to 32 queries per head, not causal), whose
- * keys are then dealt to several workgroups per head: ws points to ws_bytes bytes on the device, 16-byte aligned, used by
- * this call only until the stream has passed it and never needing to be cleared. fo_attn_fwd_workspace answers how many
- * bytes the call of a shape can use on the current device: 0 for every other shape, and where one workgroup per head
- * fills the chip. With less (or ws NULL) the call computes the same with one workgroup per head, as fo_attn_fwd does. No
- * reference counterpart. */
+/* fo_attn_fwd with scratch memory, for calls whose workgroups would leave much of the chip idle: few query rows and many keys (up to
+ * 32 queries per head, not causal), whose keys are then dealt to several workgroups per head, and few heads, or causal ones of which
+ * the longest query blocks keep the others waiting (head_dim 64 and 128), whose keys several workgroups then share; the parts are added in
+ * a fixed order by a second launch. ws points to ws_bytes bytes on the device, 16-byte aligned, used by this call only until the
+ * stream has passed it and never needing to be cleared. fo_attn_fwd_workspace answers how many bytes the call of a shape can use
+ * on the current device: 0 where nothing is shared. With less (or ws NULL) the call computes the same with one workgroup per head or
+ * query block, as fo_attn_fwd does. fo_attn_fwd_workspace_ex and fo_attn_fwd_ex_ws are the same for calls with extras
+ * (fo_attn_fwd_ex; of the bias' pointer only its alignment counts for the answer); extras may be NULL. No reference counterpart. */
 int64_t fo_attn_fwd_workspace(int B, int H, int Sq, int Sk, int D, const int64_t* k_strides_host, const int64_t* v_strides_host, int causal);
 int fo_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
                    int B, int H, int Sq, int Sk, int D,
@@ -208,6 +210,14 @@ int fo_attn_fwd_ex(const void* q, const void* k, const void* v, void* o, float* 
                    const int64_t* q_strides_host, const int64_t* k_strides_host,
                    const int64_t* v_strides_host, const int64_t* o_strides_host,
                    float softmax_scale, int causal, int dtype, const fo_attn_extras* extras_host, void* stream);
+/* with scratch memory: see fo_attn_fwd_ws */
+int64_t fo_attn_fwd_workspace_ex(int B, int H, int Sq, int Sk, int D, const int64_t* k_strides_host, const int64_t* v_strides_host, int causal,
+                                 const fo_attn_extras* extras_host);
+int fo_attn_fwd_ex_ws(const void* q, const void* k, const void* v, void* o, float* lse,
+                      int B, int H, int Sq, int Sk, int D,
+                      const int64_t* q_strides_host, const int64_t* k_strides_host,
+                      const int64_t* v_strides_host, const int64_t* o_strides_host,
+                      float softmax_scale, int causal, int dtype, const fo_attn_extras* extras_host, void* ws, int64_t ws_bytes, void* stream);
 int fo_attn_bwd_ex(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
                    float* delta_ws, void* dq, void* dk, void* dv, int B, int H, int Sq, int Sk, int D,
                    const int64_t* const* strides_host, float softmax_scale, int causal, int dtype,
