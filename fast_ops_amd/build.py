@@ -59,6 +59,8 @@ SOURCES = {
     "dropout_mask.hip": [],
     "bias_rows.hip": [],
 }
+# the host path of ordinary calls, a CPython module of its own that uses torch's C++ interface (nothing of it runs on the GPU)
+HOST_SOURCE, HOST_PATH = os.path.join(CSRC, "host_path.cpp"), os.path.join(HERE, "_host.so")
 # sources that other sources include (a change in one of them makes every object stale, like a header's)
 INCLUDED_SOURCES = ["attn_fwd.hip", "attn_bwd.hip"]
 # sources whose generated assembly is checked by asm_lint: source -> regular expression of the kernel symbols to check
@@ -151,6 +153,27 @@ def _compile_one(hipcc: str, src: str, extra: list, force: bool, verbose: bool) 
 _EXTRA_DEFINES: list = []
 
 
+def build_host(force: bool = False, verbose: bool = True) -> str:
+    """Compiles csrc/host_path.cpp against the installed torch. Returns the module's path."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    deps = [HOST_SOURCE, os.path.join(os.path.dirname(HERE), "include", "fastops.h"), torch.__file__]
+    if not force and os.path.exists(HOST_PATH) and all(os.path.getmtime(d) <= os.path.getmtime(HOST_PATH) for d in deps):
+        return HOST_PATH
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I" + sysconfig.get_paths()["include"], *("-I" + p for p in include_paths()), HOST_SOURCE, "-o", HOST_PATH,
+           *("-L" + p for p in library_paths()), "-lc10", "-ltorch_cpu", "-ltorch_python"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for {HOST_SOURCE}:\n{res.stderr}")
+    return HOST_PATH
+
+
 def build_library(force: bool = False, verbose: bool = True, ablations: bool = False) -> str:
     """Compiles every HIP source for gfx950 and links the shared library. Returns the library path."""
     global _EXTRA_DEFINES
@@ -165,7 +188,9 @@ def build_library(force: bool = False, verbose: bool = True, ablations: bool = F
         with open(stamp, "w") as f:
             f.write(want)
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as ex:
+        host = ex.submit(build_host, force, verbose)
         objs = list(ex.map(lambda kv: _compile_one(hipcc, kv[0], kv[1], force, verbose), SOURCES.items()))
+        host.result()
     need_link = force or not os.path.exists(LIB_PATH) or any(os.path.getmtime(o) > os.path.getmtime(LIB_PATH) for o in objs)
     if need_link:
         cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", LIB_PATH] + objs

@@ -29,6 +29,29 @@ _DTYPE_CODE = {torch.float16: _lib.FO_DTYPE_F16, torch.bfloat16: _lib.FO_DTYPE_B
 # the raw hipStream_t that is current on a device, without building a torch.cuda.Stream object around it
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda dev: torch.cuda.current_stream(dev).cuda_stream)
 _I64x3 = ctypes.c_int64 * 3
+_BHSD, _BSHD = (0, 1, 2, 3), (0, 2, 1, 3)
+_torch_empty = torch.empty
+_host_module = False        # not asked for yet
+
+
+def _host():
+    """The compiled host path of ordinary calls (csrc/host_path.cpp), or None: where it was not built, or while torch.empty is not
+    torch's own (who replaces it, to count or to refuse allocations, sees every one of them)."""
+    global _host_module
+    if _host_module is False:
+        lib = _lib.load()
+        try:
+            from .. import _host as module
+        except ImportError:
+            module = None
+        device = getattr(torch._C, "_cuda_getDevice", None)
+        if module is not None:
+            names = ("fo_attn_fwd_ex_ws", "fo_attn_fwd_workspace_ex", "fo_attn_bwd_ws", "fo_attn_bwd_workspace_ex", "fo_strerror")
+            addresses = {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names}
+            if device is None or not module.init(addresses, device, _raw_stream):
+                module = None
+        _host_module = module
+    return _host_module if torch.empty is _torch_empty else None
 
 
 def _check_inputs(q: Tensor, k: Tensor, v: Tensor) -> None:
@@ -245,6 +268,11 @@ def attn_fwd_strided(
     """Launches fo_attn_fwd (fo_attn_fwd_ex when ``bias`` or ``dropout`` is given), with scratch memory where it helps. ``dims`` =
     positions of (batch, head, sequence, head_dim) in the tensors' shapes; ``bias`` is [B|1, H|1, Sq|1, Sk] whatever
     ``dims`` says. Returns (O with q's shape, dtype and layout; LSE fp32 [B, H, Sq])."""
+    host = _host()
+    if host is not None and (dims == _BHSD or dims == _BSHD):
+        done = host.fwd(q, k, v, dims == _BSHD, causal, softmax_scale, dropout, bias)
+        if done is not None:
+            return done
     plan = _fwd_plan(q, k, v, dims)
     scale = float(softmax_scale) if softmax_scale else 1.0 / math.sqrt(plan.D)        # flash_attention_triton.py:750
     o = torch.empty_like(q) if plan.o_dense_like_q else torch.empty(q.shape, dtype=q.dtype, device=q.device)
@@ -356,6 +384,11 @@ def attn_bwd_strided(
 ) -> Tuple[Tensor, Tensor, Tensor]:
     """Launches fo_attn_bwd_ws. Returns (dQ, dK, dV) with the shapes and dtypes of q, k, v (dense; a K/V whose heads are
     an expanded view gets a full-size gradient, which autograd then reduces)."""
+    host = _host()
+    if host is not None and (dims == _BHSD or dims == _BSHD):
+        done = host.bwd(q, k, v, o, lse, d_o, dims == _BSHD, causal, softmax_scale, dropout, bias)
+        if done is not None:
+            return done
     if d_o.dtype != q.dtype or d_o.shape != q.shape:
         _check_inputs(q, k, v)
         raise RuntimeError(f"dO must have the output's shape and dtype, got {tuple(d_o.shape)} {d_o.dtype}")

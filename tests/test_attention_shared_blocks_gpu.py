@@ -66,6 +66,7 @@ def test_shared_blocks(B, H, Sq, Sk, D, causal, dtype, form, pieces, split):
 def test_without_the_memory_the_blocks_are_whole(monkeypatch):
     q, k, v = (torch.randn(1, 4, 2048, 128, generator=torch.Generator().manual_seed(i)).to(DEV, torch.bfloat16) for i in range(3))
     shared = multi_head_attention(q, k, v, causal=True)
+    monkeypatch.setattr(surface, "_host", lambda: None)
     monkeypatch.setattr(surface, "_scratch", lambda n, device: None)
     whole = multi_head_attention(q, k, v, causal=True)
     _lib.tune_set("attn.split", 0)
