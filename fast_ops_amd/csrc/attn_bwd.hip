@@ -380,6 +380,16 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
     for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
   const float c = prm.scale_log2e, scale = prm.scale;
   DropRows<1> drop;
+  // head_dim 64: the products of dP start from -delta, sixteen registers that hold it, so that an element's dS takes an instruction less:
+  // whole backward, 8 x 12 heads x 1024 causal 77.8 -> 75.5 us, 16 x 16 171 -> 166, 4 x 16 x 2048 233 -> 229. (At head_dim 128 every register
+  // is taken; with dropout, which clears dP before delta joins it, 113 -> 116 us.)
+  constexpr bool DP_FROM_DELTA = D == 64 && !DROP;
+  f32x16 dp_start;
+  if constexpr (DP_FROM_DELTA) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dp_start[r] = delta;
+    asm volatile("" : "+v"(dp_start));
+  }
 
   for (int tile = 0; tile < n_tiles; ++tile) {
     const int buf = tile & 1;
@@ -409,7 +419,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) { sacc[kb][r] = 0.0f; dpacc[kb][r] = 0.0f; }
+      for (int r = 0; r < 16; ++r) { sacc[kb][r] = 0.0f; dpacc[kb][r] = DP_FROM_DELTA ? dp_start[r] : 0.0f; }
     if constexpr (KBIAS) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
@@ -470,7 +480,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) attn_bwd_dq_kernel(const At
             float shift = row_shift;
             if constexpr (BIAS) shift = __builtin_fmaf(b4[u], kLog2e, -lse2);
             const float p = dead ? 0.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][r], c, shift));
-            dsf[kb * 2 + (r >> 3)][r & 7] = (T)(p * (dpacc[kb][r] + delta));
+            dsf[kb * 2 + (r >> 3)][r & 7] = (T)(p * (DP_FROM_DELTA ? dpacc[kb][r] : dpacc[kb][r] + delta));
           }
         };
         // The bias of four keys at a time (few values in flight: this kernel has no registers to spare). From the
