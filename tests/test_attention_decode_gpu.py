@@ -66,6 +66,13 @@ def test_decode_with_keys_that_score_minus_infinity(Sq, Sk, D, dtype, live, spli
     assert float((lse.cpu() - lse_ref).abs().max()) <= LSE_ATOL
 
 
+# The merge takes four splits with the references and eight at a time behind them: the edges of both, and the most there are.
+@pytest.mark.parametrize("split", [3, 4, 5, 12, 13, 20, 64])
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.float16)])
+def test_decode_merges_any_number_of_splits(split, D, dtype):
+    test_decode_against_oracle(1, 3, 2, 65 * 32 + 1, D, dtype, False, split)
+
+
 # a shape's first call may fall into a time when another kernel, or fewer workgroups per row block, were asked for
 @pytest.mark.parametrize("key,value", [("attn.variant", 0), ("attn.decode_split", 1)])
 def test_workspace_follows_what_is_asked_for(key, value):
