@@ -98,13 +98,21 @@ def test_a_workspace_that_does_not_fit(monkeypatch):
     t = [x.requires_grad_(True) for x in (q, k, v)]
     o = multi_head_attention(*t, causal=True)
     want = torch.autograd.grad(o, t, go, retain_graph=True)
-    free, _ = torch.cuda.mem_get_info()
+    rest = []
+    torch.cuda.empty_cache()
     torch.cuda.set_per_process_memory_fraction(1e-4)          # nothing new
     try:
-        torch.cuda.empty_cache()
+        # nor what is left of blocks that other tensors hold a part of
+        size = 1 << 26
+        while size >= 512:
+            try:
+                rest.append(torch.empty(size, dtype=torch.uint8, device=q.device))
+            except torch.OutOfMemoryError:
+                size //= 2
         with pytest.raises(torch.OutOfMemoryError):
             torch.autograd.grad(o, t, go, retain_graph=True)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+        rest.clear()
     for a, b in zip(torch.autograd.grad(o, t, go), want):
         assert torch.allclose(a.float(), b.float(), atol=2e-2, rtol=2e-2)
