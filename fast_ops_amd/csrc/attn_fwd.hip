@@ -1403,7 +1403,10 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     if constexpr (VBIAS || TBIAS != 0) m_run[b2] = fmaxf(m_run[b2], kNoKeyYet);
   }
   drop_look(0);
-  step(0, P0{}, Y{}, N{}, Y{}, N{}, N{}, -1, N{});   // (its reference is its own row maximum: every P <= 1, no recovery)
+  // (its reference is its own row maximum: every P <= 1, no recovery - but what a bias per query holds above the diagonal may be NaN or
+  // infinite, which the recovery path removes with the keys it belongs to)
+  if constexpr (TBIAS != 0) step(0, P0{}, Y{}, N{}, Y{}, N{}, N{}, -1);
+  else step(0, P0{}, Y{}, N{}, Y{}, N{}, N{}, -1, N{});
   if (n_w > 1) step(1, P1{}, Y{}, Y{}, Y{}, N{}, N{}, -1); else step(1, P1{}, N{}, Y{}, Y{}, N{}, N{}, -1);
   // Should the steps above have parked registers in scratch memory (they do not at present), wait here, visibly to
   // the compiler, for any reload still in flight: otherwise it guards the first use inside the loops with a vmcnt(0)
