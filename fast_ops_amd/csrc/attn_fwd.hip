@@ -1378,23 +1378,41 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     for (int j4 = 0; j4 < 4; ++j4) load_key_bias(1, j4);
   }
   if constexpr (TBIAS != 0) {
+    // S(1) too: the reference is that of the plain kernel, over whole first tiles (see below)
+    const uint32_t kb1 = k_lane + sub_base(1), kb2 = k_lane + sub_base(2);
 #pragma unroll
-    for (int j4 = 0; j4 < 4; ++j4) bias_of[0][j4] = load_bias_of(0, j4);
+    for (int f = 0; f < KSTEPS; ++f) {
+      if (f == 0) Mfma::v_init_ba(S[1][0], KF[f % RD], qf[0][f]);
+      else Mfma::v_acc_ba(S[1][0], KF[f % RD], qf[0][f]);
+      KF[f % RD] = (f + RD < KSTEPS) ? k_frag(kb1, f + RD) : k_frag(kb2, f + RD - KSTEPS);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+      for (int j4 = 0; j4 < 4; ++j4) bias_of[sub][j4] = load_bias_of(sub, j4);
+    mfma_result_fence_v(S[1]);
   }
   // The reference of the exponentials starts as the row maximum of the first sub-tile (dead keys left out as the step
   // will mask them: lim as there, sub-tile 0; key 0 is never dead, so the maximum is finite). Started from -inf, the
   // first step takes the recovery path - maxima, every exponential a second time, 64 accumulator registers rescaled -
   // once per query block, 1-2 us each time.
+  // TBIAS: of the first two, as in the plain kernel, which most of these calls run on otherwise. Where the reference is a row's own
+  // maximum its largest P is 1 and is not rounded: from one sub-tile O of 12 heads x 3072 causal was 1.7 % further from float64.
 #pragma unroll
   for (int b2 = 0; b2 < QB; ++b2) {
-    int lim = 4 * hh - Sk + 1;
-    if (CAUSAL) lim = max(lim, 4 * hh - (q0k + 32 * b2 + l32));
     float mloc = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      float sv = S[0][b2][r];
-      if constexpr (TBIAS != 0) sv = __builtin_fmaf(sv, c, (float)bias_of[0][r >> 2][r & 3] * 1.4426950408889634f);
-      mloc = fmaxf(mloc, (lim > -((r & 3) + 8 * (r >> 2))) ? -INFINITY : sv);
+    for (int sub = 0; sub < (TBIAS ? 2 : 1); ++sub) {
+      const int key_base = 32 * sub + 4 * hh;
+      int lim = key_base - Sk + 1;
+      if (CAUSAL) lim = max(lim, key_base - (q0k + 32 * b2 + l32));
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        float sv = S[sub][b2][r];
+        if constexpr (TBIAS != 0) sv = __builtin_fmaf(sv, c, (float)bias_of[sub][r >> 2][r & 3] * 1.4426950408889634f);
+        mloc = fmaxf(mloc, (lim > -((r & 3) + 8 * (r >> 2))) ? -INFINITY : sv);
+      }
     }
     m_run[b2] = fmaxf(mloc, half_swap(mloc));
     // (a bias may have removed every key of the sub-tile: the reference then starts from a large negative number
@@ -1405,7 +1423,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   drop_look(0);
   // (its reference is its own row maximum: every P <= 1, no recovery - but what a bias per query holds above the diagonal may be NaN or
   // infinite, which the recovery path removes with the keys it belongs to)
-  if constexpr (TBIAS != 0) step(0, P0{}, Y{}, N{}, Y{}, N{}, N{}, -1);
+  if constexpr (TBIAS != 0) step(0, P0{}, N{}, N{}, Y{}, N{}, N{}, -1);      // (S(1) is there)
   else step(0, P0{}, Y{}, N{}, Y{}, N{}, N{}, -1, N{});
   if (n_w > 1) step(1, P1{}, Y{}, Y{}, Y{}, N{}, N{}, -1); else step(1, P1{}, N{}, Y{}, Y{}, N{}, N{}, -1);
   // Should the steps above have parked registers in scratch memory (they do not at present), wait here, visibly to

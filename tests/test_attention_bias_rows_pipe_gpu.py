@@ -62,3 +62,27 @@ def test_the_rule():
         assert _kernel(1, 4, 1024, 768, D, True, f32) == pipe and _kernel(1, 4, 1024, 767, D, True, f32) == plain
     assert _kernel(1, 4, 2048, 2048, 128, True, True) == plain                    # fp32 at head_dim 128
     assert _kernel(1, 4, 2048, 2048, 96, True, False) == plain                    # a head_dim off 64 and 128
+
+
+@pytest.mark.parametrize("D,bias_f32", [(128, False), (64, False), (64, True)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_as_exact_as_the_plain_kernel(causal, D, bias_f32):
+    # P is rounded against a row's reference, and not at all where that is its own score: both kernels take it from the first 64 keys. (From
+    # the first 32 the pipelined one's O was 1.7 % further off under a causal mask, over seeds within 0.1 %.)
+    H, S, dtype = 12, 1536, torch.bfloat16
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn(1, S, H, D, generator=g).to(DEV, dtype) for _ in range(3))
+    bias = torch.randn(1, H, S, S, generator=g).to(DEV, torch.float32 if bias_f32 else dtype)
+    x = [t.transpose(1, 2).double().contiguous() for t in (q, k, v)]
+    s = x[0] @ x[1].transpose(2, 3).contiguous() / D ** 0.5 + bias.double()
+    if causal:
+        s.masked_fill_(torch.ones(S, S, dtype=torch.bool, device=DEV).triu(1), float("-inf"))
+    exact = (s.softmax(-1) @ x[2]).transpose(1, 2)
+    off = {}
+    for variant in (_lib.FO_ATTN_KERNEL_ROWS128, _lib.FO_ATTN_KERNEL_ROWS128_PIPE):
+        _lib.tune_set("attn.variant", variant)
+        try:
+            off[variant] = float((flash_attn(q, k, v, bias=bias, causal=causal).double() - exact).norm())
+        finally:
+            _lib.tune_set("attn.variant", -1)
+    assert off[_lib.FO_ATTN_KERNEL_ROWS128_PIPE] <= 1.003 * off[_lib.FO_ATTN_KERNEL_ROWS128], off
