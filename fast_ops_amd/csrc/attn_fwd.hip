@@ -679,6 +679,11 @@ __host__ __device__ inline int wide_items(int n_qblk, bool causal) { return caus
 // keys of a per-key bias the pipelined kernel keeps in LDS (fp32, beside the rings: 128 + 32 of the 160 KiB at head_dim 128)
 constexpr int kVBiasKeys = 8192;
 constexpr float kNoKeyYet = -1.0e30f;   // reference of a row all of whose keys so far a bias of -inf has removed
+// the same in the base-2 domain (bias per query): below every finite score
+constexpr float kNoKeyYetBase2 = -3.4028235e38f;
+// From this reference on (base 2) its own rounding counts: a score is rounded before it becomes the reference and fused with it afterwards,
+// so that the two differ by up to 2^-24 of it where they should be equal - 2^-10 here, and 2^76 for rows masked with -1e30.
+constexpr float kFarReference = 16384.0f;
 
 // A bias with a query stride in the pipelined kernel: each wave copies the 32 rows x 32 keys of a step into a ring of its own, in
 // LDS behind the rings of K and V, four steps ahead, and a lane holds the 16 values of a step in registers a step before it. Rows of a half
@@ -1062,6 +1067,12 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) { m_run[qb] = -INFINITY; l_run[qb] = 0.0f; }
   const float c = prm.scale_log2e;
+  // some row of the wave has a far reference (kFarReference): every step goes through the recovery path, which rounds a score
+  // before it takes the reference off
+  bool far = false;
+  auto look_far = [&]() {
+    if constexpr (TBIAS != 0) far = __builtin_amdgcn_ballot_w64(fabsf(m_run[0]) > kFarReference && m_run[0] != kNoKeyYetBase2) != 0;
+  };
 
   const uint32_t k_lane = (uint32_t)((l32 >> 4) * 1024 + hh * 256 + (l32 & 15) * 16);
   const uint32_t v_lane = (uint32_t)(kRing * TILE_BYTES + lane * 8);
@@ -1255,7 +1266,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     // taken branch, which holds a lone wave up until its instructions are fetched. Four waves x 64 rows: 2 x 16 heads x 8192
     // 464 -> 457 us causal, 849 -> 844 not causal; the 128-row form loses up to 1 % that way, the eight-wave form does not care.)
     constexpr bool RECOVER_FAR = QB == 2;
-    const bool recover = __builtin_amdgcn_ballot_w64(redo) != 0;
+    const bool recover = __builtin_amdgcn_ballot_w64(redo) != 0 || far;
     if (CAN_RECOVER && (RECOVER_FAR ? __builtin_expect(recover, 0) : recover) && !(DBG & 2)) {
       // rare: true row maxima of this sub-tile, new references, P and row sums again, O and l rescaled
 #pragma unroll
@@ -1297,6 +1308,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
 #pragma unroll
         for (int d = 0; d < DBLK; ++d) scale_acc(oacc[d][b2], alpha);
       }
+      look_far();
     }
 #pragma unroll
     for (int b2 = 0; b2 < QB; ++b2) l_run[b2] += psum[b2];
@@ -1418,11 +1430,12 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     // (a bias may have removed every key of the sub-tile: the reference then starts from a large negative number
     // instead of -inf, so that a removed key gives exp2(-inf) = 0 and not exp2(-inf + inf); the first key that counts
     // overflows the row sum and the recovery path moves the reference to it, with O and l multiplied by exp2(-huge) = 0)
-    if constexpr (VBIAS || TBIAS != 0) m_run[b2] = fmaxf(m_run[b2], kNoKeyYet);
+    if constexpr (VBIAS || TBIAS != 0) m_run[b2] = fmaxf(m_run[b2], TBIAS ? kNoKeyYetBase2 : kNoKeyYet);
   }
+  look_far();
   drop_look(0);
   // (its reference is its own row maximum: every P <= 1, no recovery - but what a bias per query holds above the diagonal may be NaN or
-  // infinite, which the recovery path removes with the keys it belongs to)
+  // infinite, which the recovery path removes with the keys it belongs to, and the reference may be far)
   if constexpr (TBIAS != 0) step(0, P0{}, N{}, N{}, Y{}, N{}, N{}, -1);      // (S(1) is there)
   else step(0, P0{}, Y{}, N{}, Y{}, N{}, N{}, -1, N{});
   if (n_w > 1) step(1, P1{}, Y{}, Y{}, Y{}, N{}, N{}, -1); else step(1, P1{}, N{}, Y{}, Y{}, N{}, N{}, -1);
