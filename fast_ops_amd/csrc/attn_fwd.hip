@@ -617,10 +617,6 @@ template <typename T, bool NOP> struct AsmMfma;
   static __device__ __forceinline__ void v_init_ba(f32x16& acc, i32x4 a, i32x4 b) {                                     \
     asm volatile(PRE MNEMONIC " %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "a"(b));                                          \
   }                                                                                                                     \
-  /* acc (VGPRs) = a b + c, B operand in AGPRs */                                                                       \
-  static __device__ __forceinline__ void v_from_ba(f32x16& acc, i32x4 a, i32x4 b, const f32x16& c) {                    \
-    asm volatile(PRE MNEMONIC " %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "a"(b), "v"(c));                                 \
-  }                                                                                                                     \
   /* acc (VGPRs) += a b, B operand in AGPRs */                                                                          \
   static __device__ __forceinline__ void v_acc_ba(f32x16& acc, i32x4 a, i32x4 b) {                                      \
     asm volatile(PRE MNEMONIC " %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));                                          \
@@ -632,7 +628,6 @@ template <typename T, bool NOP> struct AsmMfma;
 #else
 #define FO_MFMA_BODY(PRE, MNEMONIC)                                                                                     \
   static __device__ __forceinline__ void v_init_ba(f32x16&, i32x4, i32x4) {}                                            \
-  static __device__ __forceinline__ void v_from_ba(f32x16&, i32x4, i32x4, const f32x16&) {}                             \
   static __device__ __forceinline__ void v_acc_ba(f32x16&, i32x4, i32x4) {}                                             \
   static __device__ __forceinline__ void a_acc(f32x16&, i32x4, i32x4) {}
 #endif
@@ -709,10 +704,11 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   // flash_attention_triton.py:176-186, e.g. a key padding mask). The head's row of it, at most kVBiasKeys keys, is put
   // into LDS once per workgroup as fp32 divided by softmax_scale, so that (S + b / scale) * scale * log2 e is the biased
   // score in the base-2 domain and the running maximum, the lazily raised reference and LSE keep their meaning with
-  // S + b / scale in the place of S. The first product of a 32-key sub-tile takes its 16 values for a lane's registers (they
-  // depend on the register and the half of the wave only) as what it adds to, so that a score costs no instruction more; they are
-  // read from LDS a step ahead. (Added where the scores are scaled, an instruction per score, 12 heads x 8192 took 379 us instead of
-  // 369, causal 210 instead of 204; x 4096 causal 71.2 instead of 69.2, x 2048 37.2 instead of 35.9.) A bias of -inf removes a key; a row whose keys so far are all removed has the reference
+  // S + b / scale in the place of S. A step reads the 16 values of its 32 keys that a lane's registers hold (they
+  // depend on the register and the half of the wave only) and adds them where the scores are scaled: one more VALU
+  // instruction per score. (Taken as what the first product of a sub-tile adds to they cost none, 2 to 3 % of such calls, but every
+  // product is then rounded at the size of the bias: LSE of rows that see one key, |b| from 500 to 1500, head_dim 128, 8.4e-5 rms
+  // from float64 instead of 5.4e-5, modelled in fp32.) A bias of -inf removes a key; a row whose keys so far are all removed has the reference
   // kNoKeyYet, a large negative number, against which removed keys give 0 and the first key that counts overflows the
   // row sum once (recovery path), which multiplies the row's empty O and l by 0 (left padding: one step per row).
   // TBIAS: the bias joins a score where that is scaled: exp2(S c + (b log2 e - m)), two instructions per score more, with m, the reference,
@@ -1090,14 +1086,6 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     return __builtin_bit_cast(i32x4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
 
-  // VBIAS: bias / scale of a sub-tile's keys as a lane's registers hold them, four at a time (register 4 j + u: key 8 j + 4 hh + u)
-  f32x16 key_bias;
-  auto load_key_bias = [&](int sub, int j4) {
-    const f32x4 v = *(FO_LDS const f32x4*)(vbias + sub * 32 + 8 * j4);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) key_bias[4 * j4 + u] = v[u];
-  };
-
   // ---- one pipeline step for sub-tile s (parity P = s & 1), as micro-groups of one MFMA each:
   //   HAS_QK: S[P^1] = K(s+1) Q^T;   HAS_PV: O += V(s-1)^T PF[P^1]^T;   always: S[P] -> PF[P] = exp2(S c - m c), row sums.
   // On entry KF holds K fragments 0..RD-1 of sub-tile s+1 and VF holds V^T fragments 0..RD-1 of sub-tile s-1; on exit
@@ -1149,6 +1137,17 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
       dma_dst = smem + ((P == 0 ? 0 : kRing) + (dma_tile & (kRing - 1))) * TILE_BYTES + wave_s * DMA_PER_WAVE * 1024;
     }
     float ex[NEL];
+    f32x4 bq[VBIAS ? 4 : 1];                 // bias / scale of the keys of registers 4 j .. 4 j + 3 (keys 32 s + 8 j + 4 hh ..)
+    int lim_v[QB];                           // VBIAS: lim of the mask, see there
+    auto look_lim = [&]() {
+#pragma unroll
+      for (int b2 = 0; b2 < QB; ++b2) {
+        const int key_base = s * 32 + 4 * hh;
+        lim_v[b2] = key_base - Sk + 1;
+        if (CAUSAL) lim_v[b2] = max(lim_v[b2], key_base - (q0k + 32 * b2 + l32));
+      }
+    };
+    if constexpr (VBIAS && MASK) look_lim();
     // score e of NEL: query block, accumulator register (the first 8 registers of every block first: they are the
     // first 16-key step of P V)
     auto el_qb = [](int e) { return QB == 2 ? (e >> 3) & 1 : 0; };
@@ -1161,8 +1160,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
       const int f = i / QB, qb = i % QB;                               // fragment, query block
       if (g >= NMF) {
       } else if (is_qk) {
-        if (f == 0 && VBIAS) Mfma::v_from_ba(S[P ^ 1][qb], KF[f % RD], qf[qb][f], key_bias);
-        else if (f == 0) Mfma::v_init_ba(S[P ^ 1][qb], KF[f % RD], qf[qb][f]);
+        if (f == 0) Mfma::v_init_ba(S[P ^ 1][qb], KF[f % RD], qf[qb][f]);
         else Mfma::v_acc_ba(S[P ^ 1][qb], KF[f % RD], qf[qb][f]);
         if (FO_PIN_MFMA & FORM) __builtin_amdgcn_sched_barrier(0);
         if (qb == QB - 1 && !(DBG & 4)) KF[f % RD] = (f + RD < KSTEPS) ? k_frag(kb1, f + RD) : k_frag(kb2, f + RD - KSTEPS);
@@ -1182,14 +1180,13 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
           dma16_uniform_base(P == 0 ? k_src0[i] : v_src0[i], dma_off, dma_dst + i * 1024);
         }
       }
-      if constexpr (VBIAS && HAS_QK) {
-        // (the products that take the values of this step are issued in the groups up to LAST: two groups on, that operand has been read)
-        constexpr int LAST = HAS_PV ? 2 * (QB - 1) : QB - 1, GB = (G - 4) / 2 > LAST + 2 ? (G - 4) / 2 : LAST + 2;
-        static_assert(GB + 4 <= G, "room for the reads of the bias");
-        if (g >= GB && g < GB + 4) load_key_bias(min(s + 2, 2 * n_tiles - 1), g - GB);
+      if constexpr (VBIAS) {
+        // (the first eight registers of every block are used in the first half of the step, the others in the second)
+        if (g == 0) { bq[0] = *(FO_LDS const f32x4*)(vbias + s * 32); bq[1] = *(FO_LDS const f32x4*)(vbias + s * 32 + 8); }
+        if (g == (GE0 + 1 + NE / 2) - 3) { bq[2] = *(FO_LDS const f32x4*)(vbias + s * 32 + 16); bq[3] = *(FO_LDS const f32x4*)(vbias + s * 32 + 24); }
       }
       // -- this group's share of the softmax arithmetic
-      if (MASK && g == GMASK) {
+      if (MASK && !VBIAS && g == GMASK) {
         // register r holds key key_base + koff(r), koff(r) = (r & 3) + 8 * (r >> 2); dead iff key > q or key >= Sk,
         // i.e. iff lim + koff(r) > 0 with lim = max(key_base - q, key_base - Sk + 1)
         const int key_base = s * 32 + 4 * hh;
@@ -1237,6 +1234,12 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
         }
         if (ge - 1 == g) {
           if constexpr (TBIAS != 0) ex[e] = __builtin_fmaf(S[P][b2][r], c, ex[e]);
+          else if constexpr (VBIAS) {
+            // (masked behind the bias, which may be anything where a key is not seen)
+            float x = S[P][b2][r] + bq[r >> 2][r & 3];
+            if (MASK) x = (lim_v[b2] > -((r & 3) + 8 * (r >> 2))) ? -INFINITY : x;
+            ex[e] = __builtin_fmaf(x, c, -mc[b2]);
+          }
           else ex[e] = (DBG & 2) ? S[P][b2][r] : __builtin_fmaf(S[P][b2][r], c, -mc[b2]);
           asm volatile("" : "+v"(ex[e]));                              // pins the instruction to this micro-group
         }
@@ -1272,6 +1275,20 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
 #pragma unroll
       for (int d = 0; d < DBLK; ++d) mfma_result_fence_a(oacc[d]);
       const float cr = TBIAS ? 1.0f : c;
+      if constexpr (VBIAS) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          f32x4 t4 = *(FO_LDS const f32x4*)(vbias + s * 32 + 8 * j);
+          asm volatile("" : "+v"(t4));                                 // (four values at a time: no registers to spare here)
+#pragma unroll
+          for (int b2 = 0; b2 < QB; ++b2)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const float x = S[P][b2][4 * j + u] + t4[u];
+              S[P][b2][4 * j + u] = (MASK && lim_v[b2] > -(u + 8 * j)) ? -INFINITY : x;
+            }
+        }
+      }
       if constexpr (TBIAS != 0) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -1368,16 +1385,11 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     const uint32_t kb0 = k_lane + sub_base(0), kb1 = k_lane + sub_base(1);
 #pragma unroll
     for (int i = 0; i < RD; ++i) KF[i] = k_frag(kb0, i);
-    if constexpr (VBIAS) {
-#pragma unroll
-      for (int j4 = 0; j4 < 4; ++j4) load_key_bias(0, j4);
-    }
 #pragma unroll
     for (int f = 0; f < KSTEPS; ++f) {
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
-        if (f == 0 && VBIAS) Mfma::v_from_ba(S[0][qb], KF[f % RD], qf[qb][f], key_bias);
-        else if (f == 0) Mfma::v_init_ba(S[0][qb], KF[f % RD], qf[qb][f]);
+        if (f == 0) Mfma::v_init_ba(S[0][qb], KF[f % RD], qf[qb][f]);
         else Mfma::v_acc_ba(S[0][qb], KF[f % RD], qf[qb][f]);
       }
       KF[f % RD] = (f + RD < KSTEPS) ? k_frag(kb0, f + RD) : k_frag(kb1, f + RD - KSTEPS);
@@ -1385,10 +1397,6 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     }
   }
   mfma_result_fence_v(S[0]);
-  if constexpr (VBIAS) {
-#pragma unroll
-    for (int j4 = 0; j4 < 4; ++j4) load_key_bias(1, j4);
-  }
   if constexpr (TBIAS != 0) {
     // S(1) too: the reference is that of the plain kernel, over whole first tiles (see below)
     const uint32_t kb1 = k_lane + sub_base(1), kb2 = k_lane + sub_base(2);
@@ -1422,6 +1430,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         float sv = S[sub][b2][r];
+        if constexpr (VBIAS) sv += vbias[8 * (r >> 2) + (r & 3)];
         if constexpr (TBIAS != 0) sv = __builtin_fmaf(sv, c, (float)bias_of[sub][r >> 2][r & 3] * 1.4426950408889634f);
         mloc = fmaxf(mloc, (lim > -((r & 3) + 8 * (r >> 2))) ? -INFINITY : sv);
       }
