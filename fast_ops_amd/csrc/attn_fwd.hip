@@ -74,6 +74,13 @@ __host__ __device__ inline float* fwd_part(float* base, int D, uint32_t part, in
 
 constexpr int kDecodeMinKeys = 128;
 constexpr int64_t kMaxRowStride = 1ll << 24;   // elements; see attn_fwd_impl
+// From this reference on (base 2) its own rounding counts: a score is rounded before it becomes the reference and fused with it afterwards,
+// so that the two differ by up to 2^-24 of it where they should be equal - 2^-10 here, and 2^76 for rows masked with -1e30. Such rows
+// take the reference off a rounded score.
+constexpr float kFarReference = 16384.0f;
+// Reference of a row all of whose keys so far a bias of -inf has removed, below every finite score (base 2; a reference that is
+// multiplied by scale log2 e > 1 stays in range divided by it)
+constexpr float kNoKeyYet = -3.4e38f;
 constexpr float kLazyLog2 = 8.0f;   // how far (in log2 units) a tile maximum may exceed the reference before a rescale
 
 // KBIAS (without BIAS): a bias that is the same for every query (query stride 0) at no cost per score. The 64 values of a
@@ -471,7 +478,18 @@ __global__ void __launch_bounds__(kWaves * 64, 2) attn_fwd_kernel(const AttnPara
         for (int r = 0; r < 16; ++r) oacc[i][r] *= alpha;
     }
     // a bias may mask every key seen so far (-inf, e.g. left padding): the reference then stays 0 until a key counts
-    const float mc = ((BIAS || KBIAS || TBIAS) && m_run == -INFINITY) ? 0.0f : m_run * c;
+    float mc = ((BIAS || KBIAS || TBIAS) && m_run == -INFINITY) ? 0.0f : m_run * c;
+    if constexpr (KBIAS) {
+      const bool far = fabsf(mc) > kFarReference;
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(far) != 0, 0)) {
+        const float base = far ? m_run : 0.0f;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sacc[kb][r] -= base;
+        if (far) mc = 0.0f;
+      }
+    }
     float psum = 0.0f;
     vec8 pf[4];
 #pragma unroll
@@ -673,12 +691,6 @@ __host__ __device__ inline int wide_items(int n_qblk, bool causal) { return caus
 
 // keys of a per-key bias the pipelined kernel keeps in LDS (fp32, beside the rings: 128 + 32 of the 160 KiB at head_dim 128)
 constexpr int kVBiasKeys = 8192;
-constexpr float kNoKeyYet = -1.0e30f;   // reference of a row all of whose keys so far a bias of -inf has removed
-// the same in the base-2 domain (bias per query): below every finite score
-constexpr float kNoKeyYetBase2 = -3.4028235e38f;
-// From this reference on (base 2) its own rounding counts: a score is rounded before it becomes the reference and fused with it afterwards,
-// so that the two differ by up to 2^-24 of it where they should be equal - 2^-10 here, and 2^76 for rows masked with -1e30.
-constexpr float kFarReference = 16384.0f;
 
 // A bias with a query stride in the pipelined kernel: each wave copies the 32 rows x 32 keys of a step into a ring of its own, in
 // LDS behind the rings of K and V, four steps ahead, and a lane holds the 16 values of a step in registers a step before it. Rows of a half
@@ -1063,11 +1075,18 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) { m_run[qb] = -INFINITY; l_run[qb] = 0.0f; }
   const float c = prm.scale_log2e;
+  const float no_key_yet = TBIAS ? kNoKeyYet : kNoKeyYet / fmaxf(c, 1.0f);
   // some row of the wave has a far reference (kFarReference): every step goes through the recovery path, which rounds a score
   // before it takes the reference off
   bool far = false;
+  auto is_far = [&](float m) { return fabsf(TBIAS ? m : m * c) > kFarReference; };
   auto look_far = [&]() {
-    if constexpr (TBIAS != 0) far = __builtin_amdgcn_ballot_w64(fabsf(m_run[0]) > kFarReference && m_run[0] != kNoKeyYetBase2) != 0;
+    if constexpr (VBIAS || TBIAS != 0) {
+      bool f = false;
+#pragma unroll
+      for (int b2 = 0; b2 < QB; ++b2) f = f || (is_far(m_run[b2]) && m_run[b2] != no_key_yet);
+      far = __builtin_amdgcn_ballot_w64(f) != 0;
+    }
   };
 
   const uint32_t k_lane = (uint32_t)((l32 >> 4) * 1024 + hh * 256 + (l32 & 15) * 16);
@@ -1128,6 +1147,17 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     float mc[QB], psum[QB];
 #pragma unroll
     for (int b2 = 0; b2 < QB; ++b2) { mc[b2] = TBIAS ? m_run[b2] : m_run[b2] * c; psum[b2] = 0.0f; }
+    // (the step without a recovery path does for far references what that path does)
+    constexpr bool FAR_HERE = VBIAS && !CAN_RECOVER;
+    float far_base[QB];
+    if constexpr (FAR_HERE) {
+#pragma unroll
+      for (int b2 = 0; b2 < QB; ++b2) {
+        const bool f = is_far(m_run[b2]);
+        far_base[b2] = f ? m_run[b2] : 0.0f;
+        mc[b2] = f ? 0.0f : mc[b2];
+      }
+    }
     // copies this step issues between its MFMAs (spread): the K blocks of tile dma_tile in the step of an even sub-tile,
     // the V blocks in that of an odd one
     uint32_t dma_off = 0;
@@ -1238,6 +1268,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
             // (masked behind the bias, which may be anything where a key is not seen)
             float x = S[P][b2][r] + bq[r >> 2][r & 3];
             if (MASK) x = (lim_v[b2] > -((r & 3) + 8 * (r >> 2))) ? -INFINITY : x;
+            if constexpr (FAR_HERE) x -= far_base[b2];
             ex[e] = __builtin_fmaf(x, c, -mc[b2]);
           }
           else ex[e] = (DBG & 2) ? S[P][b2][r] : __builtin_fmaf(S[P][b2][r], c, -mc[b2]);
@@ -1307,12 +1338,13 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
         mloc = fmaxf(mloc, half_swap(mloc));
         const float m_new = fmaxf(m_run[b2], mloc);                    // finite: key 0 is never masked (a bias: see kNoKeyYet)
         const float alpha = __builtin_amdgcn_exp2f((m_run[b2] - m_new) * cr);
-        const float mcn = m_new * cr;
+        const bool f = VBIAS && is_far(m_new);
+        const float mcn = f ? 0.0f : m_new * cr, base = f ? m_new : 0.0f;
         float ps = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {
-          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[P][b2][r], cr, -mcn));
-          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[P][b2][r + 1], cr, -mcn));
+          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(VBIAS ? S[P][b2][r] - base : S[P][b2][r], cr, -mcn));
+          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(VBIAS ? S[P][b2][r + 1] - base : S[P][b2][r + 1], cr, -mcn));
           ps += p0;
           ps += p1;
           const vec2 pk = {(T)p0, (T)p1};
@@ -1439,7 +1471,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     // (a bias may have removed every key of the sub-tile: the reference then starts from a large negative number
     // instead of -inf, so that a removed key gives exp2(-inf) = 0 and not exp2(-inf + inf); the first key that counts
     // overflows the row sum and the recovery path moves the reference to it, with O and l multiplied by exp2(-huge) = 0)
-    if constexpr (VBIAS || TBIAS != 0) m_run[b2] = fmaxf(m_run[b2], TBIAS ? kNoKeyYetBase2 : kNoKeyYet);
+    if constexpr (VBIAS || TBIAS != 0) m_run[b2] = fmaxf(m_run[b2], no_key_yet);
   }
   look_far();
   drop_look(0);

@@ -11,7 +11,7 @@ from oracle.attention_oracle import attention_fwd_oracle
 from test_attention_bias_gpu import DEV, _bshd, _check
 
 pytestmark = pytest.mark.gpu
-PLAIN, PIPE = _lib.FO_ATTN_KERNEL_ROWS128, _lib.FO_ATTN_KERNEL_ROWS128_PIPE
+PLAIN, PIPE, W4 = _lib.FO_ATTN_KERNEL_ROWS128, _lib.FO_ATTN_KERNEL_ROWS128_PIPE, _lib.FO_ATTN_KERNEL_ROWS256_W4
 
 
 @pytest.fixture
@@ -80,6 +80,22 @@ def test_left_padding_under_a_causal_mask(D, variant, pieces, value, use):
     bias[1, :, :, :pad] = value
     use(variant, pieces)
     _run(q, k, v, bias.to(dtype), True)
+
+
+# (a bias per key is held divided by softmax_scale: beyond 3.4e38 times that it counts as -inf)
+@pytest.mark.parametrize("value", [-1e9, -1e30, -1e36])
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("variant,pieces", [(PLAIN, -1), (PIPE, 0), (PIPE, 2), (PIPE, 3), (W4, -1)])
+@pytest.mark.parametrize("D,bias_f32,dtype", [(128, False, torch.bfloat16), (64, False, torch.bfloat16), (64, True, torch.float16)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_bias_per_key(causal, D, bias_f32, dtype, variant, pieces, form, value, use):
+    S = 520
+    if causal and form == "behind removed keys":
+        pytest.skip("the first rows would see no key")
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn(4, 1, S, D, generator=g).to(dtype) for _ in range(3))
+    use(variant, pieces)
+    _run(q, k, v, _mask((4, S), S, value, form, torch.float32 if bias_f32 else dtype).view(4, 1, 1, S), causal)
 
 
 @pytest.mark.parametrize("above", [float("nan"), float("inf"), float("-inf"), 3e38])
