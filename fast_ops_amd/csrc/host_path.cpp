@@ -1,8 +1,8 @@
 // The host's share of an attention call, in C++: what flash_attention.py does between its arguments and the C entry points - sizes and
 // strides out of the tensors, outputs and scratch memory allocated, the call itself - for the calls that need nothing else. Whatever
-// is not plainly one of those (other types, shapes, layouts, devices; tensor subclasses; torch's modes and transforms; an allocation
-// that finds no memory) is declined with None, and the Python code does it, or refuses it, as it always has. Nothing is kept between calls
-// but a thread's count of declined backwards (see kRetry).
+// is not plainly one of those (other types, shapes, layouts, devices; tensor subclasses; torch's modes and transforms; a backward whose
+// workspace finds no memory) is declined with None, and the Python code does it, or refuses it, as it always has. Outputs that find no
+// memory raise torch.OutOfMemoryError from here. Nothing is kept between calls but what a thread was last refused (Refusal).
 //
 // Why: a short call is its host time. B=2 H=4 S=128 at head_dim 64, without gradients 9.5 -> 4.7 us of it, of which the launch takes about 2.5
 // and two allocations 1.2; forward and backward 112 -> 77 us (the rest is autograd's: a product by a number takes 42 there).
@@ -28,9 +28,20 @@ decltype(&fo_strerror) p_strerror;
 PyObject* current_device = nullptr;      // torch's functions of these names
 PyObject* raw_stream = nullptr;
 
-// as many backwards of a thread go to the Python code after one whose workspace did not fit: that code keeps to a smaller one for so long
+// Scratch memory that a thread was refused: the next kRetry calls that would ask for as much or more on that device do not (a request
+// that fails makes the caching allocator give its cached blocks back, and the calls after it allocate anew).
 constexpr int kRetry = 256;
-thread_local int declined_backwards = 0;
+struct Refusal {
+  int64_t bytes = 0;
+  int device = -1, calls = 0;
+  bool covers(int dev, int64_t n) {
+    if (calls == 0 || dev != device || n < bytes) return false;
+    --calls;
+    return true;
+  }
+  void note(int dev, int64_t n) { bytes = n; device = dev; calls = kRetry; }
+};
+thread_local Refusal refused_fwd, refused_bwd;
 
 struct Dims { int64_t B, H, Sq, Sk, D; };
 
@@ -160,11 +171,12 @@ PyObject* fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t bytes = p_fwd_workspace((int)d.B, (int)d.H, (int)d.Sq, (int)d.Sk, (int)d.D, ks, vs, causal, any ? &ex : nullptr);
     at::Tensor ws;
     void* room = nullptr;
-    if (bytes > 0) {
+    if (bytes > 0 && !refused_fwd.covers((int)q->get_device(), bytes)) {
       try {
         ws = at::empty({bytes}, q->options().dtype(at::kByte));
         room = ws.data_ptr();
-      } catch (const c10::OutOfMemoryError&) {      // (the call computes the same without)
+      } catch (const c10::OutOfMemoryError&) {      // (the call does without)
+        refused_fwd.note((int)q->get_device(), bytes);
       }
     }
     status = p_fwd_ex_ws(q->data_ptr(), k->data_ptr(), v->data_ptr(), o.data_ptr(), (float*)lse.data_ptr(), (int)d.B, (int)d.H, (int)d.Sq, (int)d.Sk, (int)d.D,
@@ -191,7 +203,6 @@ PyObject* bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
   at::Tensor dq, dk, dv;
   HANDLE_TH_ERRORS
   if (n != 11 || !ready || !plain_mode()) return declined();
-  if (declined_backwards > 0) { --declined_backwards; return declined(); }
   if (!plain(a[0], q) || !plain(a[1], k) || !plain(a[2], v) || !plain(a[3], o) || !plain(a[4], lse) || !plain(a[5], g)) return declined();
   if (!PyBool_Check(a[6]) || !PyBool_Check(a[7])) return declined();
   const bool bshd = a[6] == Py_True, causal = a[7] == Py_True;
@@ -202,13 +213,14 @@ PyObject* bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (g->stride(i) % 8 != 0) return declined();
   if (lse->scalar_type() != at::kFloat || !lse->is_contiguous() || lse->numel() != d.B * d.H * d.Sq || lse->get_device() != q->get_device()) return declined();
   if (!stream_on(q->get_device(), stream)) return declined();
+  const int64_t bytes = p_bwd_workspace((int)d.B, (int)d.H, (int)d.Sq, (int)d.Sk, (int)d.D, causal, any ? &ex : nullptr);
+  if (refused_bwd.covers((int)q->get_device(), bytes)) return declined();      // (the Python code keeps to a smaller one for as long)
   {
     pybind11::gil_scoped_release no_gil;
     dq = at::empty(q->sizes(), q->options());
     dk = at::empty(k->sizes(), q->options());
     dv = at::empty(v->sizes(), q->options());
     const int type = q->scalar_type() == at::kHalf ? FO_DTYPE_F16 : FO_DTYPE_BF16;
-    const int64_t bytes = p_bwd_workspace((int)d.B, (int)d.H, (int)d.Sq, (int)d.Sk, (int)d.D, causal, any ? &ex : nullptr);
     at::Tensor ws;
     try {
       ws = at::empty({bytes}, q->options().dtype(at::kByte));
@@ -224,7 +236,7 @@ PyObject* bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
                         dv.data_ptr(), (int)d.B, (int)d.H, (int)d.Sq, (int)d.Sk, (int)d.D, list, scale, causal, type, any ? &ex : nullptr, ws.data_ptr(), bytes, stream);
     }
   }
-  if (!room) { declined_backwards = kRetry; return declined(); }
+  if (!room) { refused_bwd.note((int)q->get_device(), bytes); return declined(); }
   if (status != 0) return failed("fo_attn_bwd_ws", status);
   PyObject *pq = THPVariable_Wrap(std::move(dq)), *pk = THPVariable_Wrap(std::move(dk)), *pv = THPVariable_Wrap(std::move(dv));
   PyObject* all = PyTuple_Pack(3, pq, pk, pv);

@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import threading
 from typing import Optional, Tuple, Union
 
 import numpy as np
@@ -253,11 +254,21 @@ def _fwd_workspace(plan: _FwdPlan, causal: bool, bias: Optional[Tensor], dropout
     return n
 
 
+_FWD_WS_RETRY = 256                 # as _BWD_WS_RETRY
+_refused = threading.local()        # (.fwd: device, bytes, calls) scratch memory that a thread's forward was refused: see _scratch
+
+
 def _scratch(n_bytes: int, device) -> Optional[Tensor]:
-    """Scratch memory, or None where there is none to be had (the call then computes the same without)."""
+    """Scratch memory of a forward, or None where there is none to be had: the call then does without, and so do the next _FWD_WS_RETRY that
+    would ask for as much on that device."""
+    refused = getattr(_refused, "fwd", None)
+    if refused is not None and refused[2] > 0 and refused[0] == device and n_bytes >= refused[1]:
+        refused[2] -= 1
+        return None
     try:
         return torch.empty(n_bytes, dtype=torch.uint8, device=device)
     except torch.OutOfMemoryError:
+        _refused.fwd = [device, n_bytes, _FWD_WS_RETRY]
         return None
 
 
