@@ -70,8 +70,10 @@ def test_the_same_bits(layout, B, H, Sq, Sk, D, dtype, surface_of, form, monkeyp
     for a, b in zip(*_both(monkeypatch, run)):
         assert a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride() and a.device == b.device and not a.requires_grad
         assert torch.equal(a, b)
-    # the host path itself took the forward
-    assert surface._host().fwd(q, k, v, bshd, False, None, None, None) is not None
+    # the host path itself took both
+    extras = [kw["causal"], kw.get("softmax_scale"), (kw["dropout_p"], *kw["dropout_state"]) if "dropout" in form else None, kw.get("bias")]
+    taken = surface._host().fwd(q, k, v, bshd, *extras)
+    assert taken is not None and surface._host().bwd(q, k, v, *taken, go, bshd, *extras) is not None
 
 
 def test_refused_with_the_same_words(monkeypatch):
@@ -92,8 +94,8 @@ def test_refused_with_the_same_words(monkeypatch):
     assert here == there
 
 
-def test_a_workspace_that_does_not_fit(monkeypatch):
-    # the backward's allocation fails in the host path: the Python code takes this call and those after it, which keep to a smaller workspace
+def test_a_backward_without_any_memory():
+    # its outputs find none: that is refused with torch's own error, and the next call is as ever (less than all: test_scratch_memory.py)
     q, k, v, go = _tensors("dense", 1, 4, 2048, 2048, 128, torch.bfloat16, False)
     t = [x.requires_grad_(True) for x in (q, k, v)]
     o = multi_head_attention(*t, causal=True)
