@@ -18,7 +18,7 @@ FO_ATTN_BWD_STATIC_ROWS = 1 << 20
 ABI_MAJOR = 2            # fo_version() // 1000 the signatures below belong to
 FO_DTYPE_F16, FO_DTYPE_BF16, FO_DTYPE_F32 = 0, 1, 2
 FO_ATTN_KERNEL_ROWS128, FO_ATTN_KERNEL_ROWS128_EXACT, FO_ATTN_KERNEL_ROWS128_PIPE, FO_ATTN_KERNEL_ROWS256_W8, FO_ATTN_KERNEL_ROWS256_W4 = 0, 1, 8, 16, 32
-FO_ATTN_KERNEL_DECODE = 64
+FO_ATTN_KERNEL_DECODE, FO_ATTN_KERNEL_SHARED_BLOCKS = 64, 65536
 
 
 class FoLionConsts(ctypes.Structure):
@@ -46,6 +46,7 @@ SIGNATURES = {
     "fo_attn_bias_rows": (ctypes.c_int, [ctypes.c_void_p, _I64P] + [ctypes.c_int] * 5 + [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]),
     "fo_dropout_mask": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int64, ctypes.c_float, ctypes.c_uint32, ctypes.c_uint64, ctypes.c_void_p]),
     "fo_attn_fwd_ex": (ctypes.c_int, [ctypes.c_void_p] * 5 + [ctypes.c_int] * 5 + [_I64P] * 4 + [ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]),
+    "fo_attn_fwd_kernel_ex": (ctypes.c_int, [ctypes.c_int] * 5 + [_I64P] * 2 + [ctypes.c_int, ctypes.c_void_p, ctypes.c_int64]),
     "fo_attn_fwd_workspace_ex": (ctypes.c_int64, [ctypes.c_int] * 5 + [_I64P] * 2 + [ctypes.c_int, ctypes.c_void_p]),
     "fo_attn_fwd_ex_ws": (ctypes.c_int, [ctypes.c_void_p] * 5 + [ctypes.c_int] * 5 + [_I64P] * 4 + [ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]),
     "fo_attn_bwd_ex": (ctypes.c_int, [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.POINTER(_I64P), ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]),

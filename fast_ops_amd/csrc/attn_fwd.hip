@@ -2207,13 +2207,33 @@ extern "C" int fo_attn_fwd_kernel(int B, int H, int Sq, int Sk, int D, const int
   return choose_kernel(p, D > 64 ? 128 : 64, causal != 0, has_dropout != 0, tune(g_attn_variant));
 }
 
-extern "C" int64_t fo_attn_fwd_workspace_ex(int B, int H, int Sq, int Sk, int D, const int64_t* ks, const int64_t* vs, int causal, const fo_attn_extras* extras) {
-  if (!ks || !vs || check_sizes(B, H, Sq, Sk, D) || check_strides(ks, D, true) || check_strides(vs, D, true)) return 0;
+// a call's shape, strides of K and V and extras, for the queries
+static AttnParams asked_params(int B, int H, int Sq, int Sk, int D, const int64_t* ks, const int64_t* vs, const fo_attn_extras* extras) {
   AttnParams p = {};
   p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.d = D;
   for (int i = 0; i < 3; ++i) { p.ks[i] = ks[i]; p.vs[i] = vs[i]; }
-  const bool dropout = extras && extras->dropout_p > 0.0f;
   if (extras) set_bias(p, extras->bias, extras->bias_strides, extras->bias_dtype);
+  return p;
+}
+
+extern "C" int fo_attn_fwd_kernel_ex(int B, int H, int Sq, int Sk, int D, const int64_t* ks, const int64_t* vs, int causal, const fo_attn_extras* extras,
+                                     int64_t ws_bytes) {
+  if (!ks || !vs) return FO_ERR_NULL_POINTER;
+  if (const int rc = check_sizes(B, H, Sq, Sk, D)) return rc;
+  if (const int rc = check_strides(ks, D, true)) return rc;
+  if (const int rc = check_strides(vs, D, true)) return rc;
+  AttnParams p = asked_params(B, H, Sq, Sk, D, ks, vs, extras);
+  p.part_bytes = ws_bytes;
+  const bool dropout = extras && extras->dropout_p > 0.0f;
+  if (takes_decode(p, causal != 0, dropout, tune(g_attn_variant))) return FO_ATTN_KERNEL_DECODE;
+  const int width = D > 64 ? 128 : 64, kernel = choose_kernel(p, width, causal != 0, dropout, tune(g_attn_variant));
+  return kernel == FO_ATTN_KERNEL_ROWS128_PIPE && shares_blocks(p, width, causal != 0) ? kernel + FO_ATTN_KERNEL_SHARED_BLOCKS : kernel;
+}
+
+extern "C" int64_t fo_attn_fwd_workspace_ex(int B, int H, int Sq, int Sk, int D, const int64_t* ks, const int64_t* vs, int causal, const fo_attn_extras* extras) {
+  if (!ks || !vs || check_sizes(B, H, Sq, Sk, D) || check_strides(ks, D, true) || check_strides(vs, D, true)) return 0;
+  const AttnParams p = asked_params(B, H, Sq, Sk, D, ks, vs, extras);
+  const bool dropout = extras && extras->dropout_p > 0.0f;
   if (takes_decode(p, causal != 0, dropout, tune(g_attn_variant))) return decode_workspace_bytes(B, H, Sq, D, decode_split(B, H, decode_n_kv(p), Sq, Sk, D, device_cus()));
   return fwd_part_bytes(p, causal != 0, dropout);
 }

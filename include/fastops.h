@@ -99,8 +99,8 @@ int fo_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* 
                    const int64_t* v_strides_host, const int64_t* o_strides_host,
                    float softmax_scale, int causal, int dtype, void* ws, int64_t ws_bytes, void* stream);
 
-/* Which kernel fo_attn_fwd (or _dropout / _ex, with has_dropout / has_bias non-zero) launches for a call of this shape
- * on the current device with the current "attn.variant": one of the FO_ATTN_KERNEL_* codes below, or a negative
+/* Which kernel fo_attn_fwd (or _dropout / _ex, with has_dropout / has_bias non-zero) launches for a call of this shape without
+ * scratch memory on the current device with the current "attn.variant": one of the FO_ATTN_KERNEL_* codes below, or a negative
  * fo_status where fo_attn_fwd would reject the shape. has_bias: 0 none, 1 a bias with a query stride, 2 a bias that is
  * the same for every query (query stride 0), which the pipelined kernels take as well, and so does dropout (with four
  * waves where the call without it takes the eight-wave form), 3 and 4 a bias with a query stride whose base and strides are
@@ -113,6 +113,7 @@ enum {
   FO_ATTN_KERNEL_ROWS128_PIPE = 8,    /* 128 query rows per workgroup, four waves x 32 rows, in the 256-row kernel's pipeline */
   FO_ATTN_KERNEL_ROWS256_W8 = 16,     /* 256 query rows per workgroup, eight waves x 32 rows */
   FO_ATTN_KERNEL_ROWS256_W4 = 32,     /* 256 query rows per workgroup, four waves x 64 rows */
+  FO_ATTN_KERNEL_SHARED_BLOCKS = 65536, /* fo_attn_fwd_kernel_ex, added to ROWS128_PIPE: workgroups share query blocks */
   FO_ATTN_KERNEL_DECODE = 64          /* up to 32 query rows per workgroup, the keys dealt to its waves and to several workgroups */
 };
 int fo_attn_fwd_kernel(int B, int H, int Sq, int Sk, int D, const int64_t* k_strides_host, const int64_t* v_strides_host,
@@ -218,6 +219,10 @@ int fo_attn_fwd_ex_ws(const void* q, const void* k, const void* v, void* o, floa
                       const int64_t* q_strides_host, const int64_t* k_strides_host,
                       const int64_t* v_strides_host, const int64_t* o_strides_host,
                       float softmax_scale, int causal, int dtype, const fo_attn_extras* extras_host, void* ws, int64_t ws_bytes, void* stream);
+/* fo_attn_fwd_kernel for a call with these extras (NULL: none; of the bias' pointer only its alignment counts) and ws_bytes of scratch memory:
+ * with it some calls take another kernel, and their workgroups share query blocks (see fo_attn_fwd_ws). */
+int fo_attn_fwd_kernel_ex(int B, int H, int Sq, int Sk, int D, const int64_t* k_strides_host, const int64_t* v_strides_host,
+                          int causal, const fo_attn_extras* extras_host, int64_t ws_bytes);
 int fo_attn_bwd_ex(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
                    float* delta_ws, void* dq, void* dk, void* dv, int B, int H, int Sq, int Sk, int D,
                    const int64_t* const* strides_host, float softmax_scale, int causal, int dtype,

@@ -7,15 +7,21 @@ import torch
 
 from fast_ops.flash_attention.flash_attention import flash_attn
 from fast_ops_amd import _lib
+from fast_ops_amd.flash_attention import flash_attention as surface
 from oracle.attention_oracle import attention_fwd_oracle
 from test_attention_bias_gpu import DEV, _bshd, _check
 
 pytestmark = pytest.mark.gpu
 
 
-def _kernel(B, H, Sq, Sk, D, causal, bias_f32):
+def _kernel(B, H, Sq, Sk, D, causal, bias_f32, scratch=True):
+    """The kernel of a call with a bias of this type, of every head, with the scratch memory that it asks for or without any."""
     dense = (_lib.ctypes.c_int64 * 3)(H * Sk * D, Sk * D, D)
-    return _lib.load().fo_attn_fwd_kernel(B, H, Sq, Sk, D, dense, dense, int(causal), 4 if bias_f32 else 3, 0)
+    ex = surface._AttnExtras()
+    ex.bias, ex.bias_dtype = 1 << 20, _lib.FO_DTYPE_F32 if bias_f32 else _lib.FO_DTYPE_BF16
+    ex.bias_strides = (_lib.ctypes.c_int64 * 3)(0, Sq * ((Sk + 7) // 8 * 8), (Sk + 7) // 8 * 8)
+    call, lib, by = (B, H, Sq, Sk, D, dense, dense, int(causal)), _lib.load(), _lib.ctypes.byref(ex)
+    return lib.fo_attn_fwd_kernel_ex(*call, by, lib.fo_attn_fwd_workspace_ex(*call, by) if scratch else 0)
 
 
 @pytest.mark.parametrize("kind", ["noise", "masked", "large rows", "growing"])
@@ -42,7 +48,7 @@ def test_rows_of_bias_in_the_pipelined_kernel(B, H, Sq, Sk, causal, dtype, D, bi
     wide[..., :Sk] = bias.to(DEV)
     _lib.tune_set("attn.variant", _lib.FO_ATTN_KERNEL_ROWS128_PIPE)
     try:
-        assert _kernel(B, H, Sq, Sk, D, causal, bias_f32) == _lib.FO_ATTN_KERNEL_ROWS128_PIPE
+        assert _kernel(B, H, Sq, Sk, D, causal, bias_f32, False) == _lib.FO_ATTN_KERNEL_ROWS128_PIPE
         o, lse = flash_attn(*(_bshd(x.to(DEV)) for x in (q, k, v)), bias=wide[..., :Sk], causal=causal, return_lse=True)
         torch.cuda.synchronize()
     finally:
@@ -52,14 +58,20 @@ def test_rows_of_bias_in_the_pipelined_kernel(B, H, Sq, Sk, causal, dtype, D, bi
 
 
 def test_the_rule():
-    pipe, plain = _lib.FO_ATTN_KERNEL_ROWS128_PIPE, _lib.FO_ATTN_KERNEL_ROWS128
+    pipe, plain, shared = _lib.FO_ATTN_KERNEL_ROWS128_PIPE, _lib.FO_ATTN_KERNEL_ROWS128, _lib.FO_ATTN_KERNEL_SHARED_BLOCKS
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     for D, f32 in [(128, False), (64, False), (64, True)]:
-        assert _kernel(1, cus // 16, 2048, 2048, D, False, f32) == pipe           # one workgroup per unit
-        assert _kernel(1, cus // 16 + 1, 2048, 2048, D, False, f32) == plain
-        assert _kernel(1, cus * 3 // 2 // 16, 2048, 2048, D, True, f32) == pipe   # one and a half when causal
-        assert _kernel(1, cus * 3 // 2 // 16 + 1, 2048, 2048, D, True, f32) == plain
-        assert _kernel(1, 4, 1024, 768, D, True, f32) == pipe and _kernel(1, 4, 1024, 767, D, True, f32) == plain
+        for scratch in (False, True):
+            assert _kernel(1, cus // 16, 2048, 2048, D, False, f32, scratch) == pipe           # one workgroup per unit
+            assert _kernel(1, cus * 3 // 2 // 16, 2048, 2048, D, True, f32, scratch) == pipe   # one and a half when causal
+            assert _kernel(1, cus * 3 // 2 // 16 + 1, 2048, 2048, D, True, f32, scratch) == plain
+            assert _kernel(1, 4, 1024, 767, D, True, f32, scratch) == plain
+        # one more than a unit each, not causal: only where workgroups can share the last round
+        assert _kernel(1, cus // 16 + 1, 2048, 2048, D, False, f32, False) == plain
+        assert _kernel(1, cus // 16 + 1, 2048, 2048, D, False, f32) in (plain, pipe + shared)
+        assert _kernel(1, 12, 3072, 3072, D, False, f32, False) == plain and _kernel(1, 4, 1024, 768, D, True, f32, False) == pipe
+        if cus == 256:
+            assert _kernel(1, 12, 3072, 3072, D, False, f32) == pipe + shared and _kernel(1, 4, 4096, 4096, D, True, f32) == pipe + shared
     assert _kernel(1, 4, 2048, 2048, 128, True, True) == plain                    # fp32 at head_dim 128
     assert _kernel(1, 4, 2048, 2048, 96, True, False) == plain                    # a head_dim off 64 and 128
 

@@ -24,9 +24,13 @@ def split():
     _lib.tune_set("attn.variant", -1)
 
 
-def _workspace(q, k, causal):
-    plan = surface._fwd_plan(q, k, k, (0, 2, 1, 3))
-    return plan.ws_bytes_causal if causal else plan.ws_bytes
+def _kernel(q, k, v, bias, causal, drop):
+    """The kernel of this call with the scratch memory that it asks for."""
+    plan = surface._fwd_plan(q, k, v, (0, 2, 1, 3))
+    if bias is not None:
+        bias = surface._expand_bias(bias, q, plan.B, plan.H, plan.Sq, plan.Sk)
+    call = (plan.B, plan.H, plan.Sq, plan.Sk, plan.D, plan.ks, plan.vs, int(causal), _lib.ctypes.byref(surface._extras(bias, drop)))
+    return _lib.load().fo_attn_fwd_kernel_ex(*call, _lib.load().fo_attn_fwd_workspace_ex(*call))
 
 
 @pytest.mark.parametrize("pieces", [2, 3, 4])
@@ -59,8 +63,7 @@ def test_shared_blocks(B, H, Sq, Sk, D, causal, dtype, form, pieces, split):
     o, lse = flash_attn(*t, bias=dev_bias, causal=causal, return_lse=True, **kw)
     torch.cuda.synchronize()
     _check(_bshd(o), lse, [], o_ref, lse_ref, [])
-    if form == "none":
-        assert _workspace(t[0], t[1], causal) > 0                    # blocks were shared
+    assert _kernel(*t, dev_bias, causal, drop) == _lib.FO_ATTN_KERNEL_ROWS128_PIPE + _lib.FO_ATTN_KERNEL_SHARED_BLOCKS
 
 
 def test_without_the_memory_the_blocks_are_whole(monkeypatch):

@@ -192,6 +192,20 @@ def test_tune_hook_accepts_only_kernels_that_compute_the_function():
     assert lib.fo_tune_set(b"attn_bwd.dq_teams", 0) == -8 and lib.fo_tune_set(b"attn_bwd.dq_teams", 3) == -8
 
 
+def test_attn_kernel_query_with_scratch_memory():
+    # 12 heads x 3072: 288 workgroups on 256 units (assumed where there is no device) are shared where there is memory for their sums
+    lib = _lib.load()
+    strides = (ctypes.c_int64 * 3)(12 * 3072 * 128, 3072 * 128, 128)
+    need = lib.fo_attn_fwd_workspace(1, 12, 3072, 3072, 128, strides, strides, 0)
+    k = lambda D, causal, ws, ex=None: lib.fo_attn_fwd_kernel_ex(1, 12, 3072, 3072, D, strides, strides, causal, ex, ws)
+    if lib.fo_attn_fwd_kernel(1, 13, 2560, 2560, 128, strides, strides, 0, 0, 0) == _lib.FO_ATTN_KERNEL_ROWS128:      # (260 of 256)
+        assert need > 0 and k(128, 0, need) == _lib.FO_ATTN_KERNEL_ROWS128_PIPE + _lib.FO_ATTN_KERNEL_SHARED_BLOCKS
+    assert k(128, 0, need - 1) == k(128, 0, 0) == lib.fo_attn_fwd_kernel(1, 12, 3072, 3072, 128, strides, strides, 0, 0, 0)
+    assert k(76, 0, 0) == -3 and lib.fo_attn_fwd_kernel_ex(1, 1, 1, 1, 64, None, strides, 0, None, 0) == -1
+    for bad in (1, 5):
+        assert lib.fo_tune_set(b"attn.split", bad) == -8
+
+
 def test_attn_kernel_query_and_stride_limit_without_device_work():
     lib = _lib.load()
     I3 = ctypes.c_int64 * 3
