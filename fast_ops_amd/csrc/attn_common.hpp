@@ -336,6 +336,7 @@ struct BiasParams {
   int64_t strides[3];
   int is_f32;
   int dma_ok;   // forward: base and the three strides are multiples of 16 bytes, tiles may be copied with 16-byte pieces
+  int lines;    // forward: those are multiples of 128 bytes, a cache line
   int vec_ok;   // base and the three strides are multiples of 4 elements: 4 consecutive keys may be read with one load
 };
 template <typename T>

@@ -1843,20 +1843,29 @@ static int choose_kernel(const AttnParams& p, int D, bool causal, bool dropout, 
   if (p.bias.ptr != nullptr && p.bias.strides[2] != 0) {
     // A bias with a query stride whose tiles can be copied, without dropout: the 128-row pipelined form as well (at head_dim 128 not an
     // fp32 one: the rings leave 32 KiB of LDS, two of the four half tiles a wave's ring needs), where there are few workgroups for the
-    // chip, as below; its two instructions per score more are why the line lies nearer. Plain -> pipelined, us, bf16 bias that the
-    // memory-side cache holds (in brackets one read from memory): head_dim 128 12 heads x 1024 32.0 -> 26.4, x 2048 56 -> 43 (57 -> 51),
-    // 8 x 1536 42 -> 32, causal 12 x 1024 30.6 -> 26.1, x 2048 56 -> 43 (56 -> 45), x 3072 83 -> 60 (84 -> 72), x 4096 (384 workgroups)
-    // 114 -> 91 (114 -> 103); not: 12 x 3072 (288) 111 -> 122, 64 x 1024 causal (512) 37.0 -> 39.4; head_dim 64 12 x 2048 44 -> 36 (fp32
-    // 48 -> 45), causal 12 x 3072 63 -> 47 (fp32 74 -> 62), x 4096 84 -> 63 (fp32 128 -> 119); not: 12 x 3072 86 -> 90, 64 x 1024 causal
-    // 26.8 -> 29.5. (From so many (query, key) pairs on: 12 x 512 gains 18.7 -> 17.3 us, and up to there a bias whose rows lie off
-    // 16-byte boundaries is read in place, by the plain kernel, so that both give the same bits.)
+    // chip, as below; its instructions per score are why the line lies nearer. Plain -> pipelined, us, bf16 bias that the
+    // memory-side cache holds (in brackets one read from memory): head_dim 128 12 heads x 1024 31.7 -> 26.5 (31.0 -> 29.6), x 2048 57 -> 44 (57 -> 52),
+    // 8 x 1536 43 -> 34 (43 -> 39), causal 12 x 1024 30.5 -> 26.9 (31.0 -> 29.5), x 2048 55 -> 43 (56 -> 51), x 3072 83 -> 60 (84 -> 72), x 4096 (384
+    // workgroups) 112 -> 87 (114 -> 101); not: 12 x 4096 169 -> 183 (166 -> 191), 64 x 1024 causal (512) 37.0 -> 39.4; head_dim 64 12 x 2048 43 -> 36 (44 -> 39; fp32
+    // 47 -> 46, 55 -> 53), causal 12 x 3072 63 -> 50 (66 -> 53; fp32 74 -> 61, 87 -> 78), x 4096 85 -> 64 (91 -> 75; fp32 142 -> 126, 137 -> 121); not: 12 x 4096
+    // 123 -> 130 (121 -> 136), 64 x 1024 causal 26.8 -> 29.5. (From so many (query, key) pairs on: 12 x 512 gains 18.7 -> 17.3 us, and up to there a bias whose
+    // rows lie off 16-byte boundaries is read in place, by the plain kernel, so that both give the same bits.)
     constexpr int64_t kRowBiasPipePairs = 3 << 18;
     if (p.d != D || dropout || !p.bias.dma_ok || !wide_ok || (D == 128 && p.bias.is_f32)) return FO_ATTN_KERNEL_ROWS128;
     if (forced >= 0) return forced == FO_ATTN_KERNEL_ROWS128_PIPE ? FO_ATTN_KERNEL_ROWS128_PIPE : FO_ATTN_KERNEL_ROWS128;
     const int64_t wgs128 = ((int64_t)p.Sq + kBM - 1) / kBM * p.B * p.H, cus = device_cus();
-    // (more of them when several can share the blocks of the last round, not causal: 12 x 3072 119 -> 109)
     if ((int64_t)p.Sq * p.Sk < kRowBiasPipePairs) return FO_ATTN_KERNEL_ROWS128;
-    return wgs128 <= (causal ? cus + cus / 2 : cus) || (!causal && shares_blocks(p, D, false)) ? FO_ATTN_KERNEL_ROWS128_PIPE : FO_ATTN_KERNEL_ROWS128;
+    const bool shared = shares_blocks(p, D, causal) != nullptr;
+    // Rows off the cache lines: each 64-byte piece of a row lies in two of them, which a bias from memory pays for. Where workgroups share
+    // blocks the launch still gains (head_dim 128, from memory: 4 x 3000 80 -> 57, 8 x 1800 52 -> 42, causal 8 x 3000 79 -> 60, 8 x 4200
+    // 112 -> 92), otherwise not (8 x 3000 81 -> 91, 12 x 1800 53 -> 60, causal 51 -> 57, 12 x 3000 121 -> 127, causal 83 -> 91; head_dim 64 8 x 2200 51 ->
+    // 54, 12 x 3000 88 -> 92, fp32 8 x 3000 87 -> 94; but causal 12 x 1800 42 -> 41, 10 x 3000 67 -> 62, fp32 51 -> 51, 82 -> 81).
+    if (!p.bias.lines && !(D == 64 && causal)) return shared && wgs128 <= (causal ? cus + cus / 2 : cus) ? FO_ATTN_KERNEL_ROWS128_PIPE : FO_ATTN_KERNEL_ROWS128;
+    // (more workgroups when several can share the blocks of the last round, not causal: 12 x 3072 from memory 116 -> 104, fp32 at head_dim 64 120 -> 112;
+    // fp32 not quite a round: 8 x 4096, 256 workgroups, 131 -> 136, 16 x 2048 66 -> 71, but 7 x 4096 126 -> 123, 12 x 2560 75 -> 69; causal
+    // 16 x 2048 loses from memory what it gains from the cache, 59 -> 62 and 49 -> 38)
+    const int64_t most = causal ? cus + cus / 2 : p.bias.is_f32 ? cus - cus / 16 : cus;
+    return wgs128 <= most || (!causal && shared) ? FO_ATTN_KERNEL_ROWS128_PIPE : FO_ATTN_KERNEL_ROWS128;
   }
   if ((p.bias.ptr != nullptr && !key_bias) || p.d != D) return FO_ATTN_KERNEL_ROWS128;
   // ... and needs one 256-row workgroup (two query blocks each when causal) per CU to be worth it: below that the
@@ -2131,6 +2140,8 @@ static void set_bias(AttnParams& p, const void* bias, const int64_t* strides, in
   // broadcasts, and the kernel keeps its two workgroups per CU without the LDS for bias tiles)
   p.bias.dma_ok = bias && p.bias.strides[2] != 0 && ((uintptr_t)bias % 16) == 0 && (p.bias.strides[0] * elt) % 16 == 0 &&
                   (p.bias.strides[1] * elt) % 16 == 0 && (p.bias.strides[2] * elt) % 16 == 0;
+  p.bias.lines = p.bias.dma_ok && ((uintptr_t)bias % 128) == 0 && (p.bias.strides[0] * elt) % 128 == 0 && (p.bias.strides[1] * elt) % 128 == 0 &&
+                 (p.bias.strides[2] * elt) % 128 == 0;
 }
 
 static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, float* lse,
@@ -2201,7 +2212,7 @@ extern "C" int fo_attn_fwd_kernel(int B, int H, int Sq, int Sk, int D, const int
   for (int i = 0; i < 3; ++i) { p.ks[i] = ks[i]; p.vs[i] = vs[i]; }
   p.bias.ptr = has_bias ? (const void*)ks : nullptr;   // (only tested against NULL)
   p.bias.strides[2] = has_bias == 2 ? 0 : 1;
-  p.bias.dma_ok = has_bias >= 3;
+  p.bias.dma_ok = p.bias.lines = has_bias >= 3;
   p.bias.is_f32 = has_bias == 4;
   if (takes_decode(p, causal != 0, has_dropout != 0, tune(g_attn_variant))) return FO_ATTN_KERNEL_DECODE;
   return choose_kernel(p, D > 64 ? 128 : 64, causal != 0, has_dropout != 0, tune(g_attn_variant));

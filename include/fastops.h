@@ -104,7 +104,7 @@ int fo_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* 
  * fo_status where fo_attn_fwd would reject the shape. has_bias: 0 none, 1 a bias with a query stride, 2 a bias that is
  * the same for every query (query stride 0), which the pipelined kernels take as well, and so does dropout (with four
  * waves where the call without it takes the eight-wave form), 3 and 4 a bias with a query stride whose base and strides are
- * multiples of 16 bytes, of the operand type and of fp32. Launches nothing. The choice
+ * multiples of 128 bytes, of the operand type and of fp32. Launches nothing. The choice
  * depends on the number of compute units of the current device. No reference counterpart:
  * the reference has one kernel (flash_attention_fwd.cu:164-177); tests use this to assert which code they covered. */
 enum {

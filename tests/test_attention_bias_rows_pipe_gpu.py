@@ -14,12 +14,13 @@ from test_attention_bias_gpu import DEV, _bshd, _check
 pytestmark = pytest.mark.gpu
 
 
-def _kernel(B, H, Sq, Sk, D, causal, bias_f32, scratch=True):
+def _kernel(B, H, Sq, Sk, D, causal, bias_f32, scratch=True, row=None):
     """The kernel of a call with a bias of this type, of every head, with the scratch memory that it asks for or without any."""
     dense = (_lib.ctypes.c_int64 * 3)(H * Sk * D, Sk * D, D)
     ex = surface._AttnExtras()
     ex.bias, ex.bias_dtype = 1 << 20, _lib.FO_DTYPE_F32 if bias_f32 else _lib.FO_DTYPE_BF16
-    ex.bias_strides = (_lib.ctypes.c_int64 * 3)(0, Sq * ((Sk + 7) // 8 * 8), (Sk + 7) // 8 * 8)
+    row = row or (Sk + 7) // 8 * 8
+    ex.bias_strides = (_lib.ctypes.c_int64 * 3)(0, Sq * row, row)
     call, lib, by = (B, H, Sq, Sk, D, dense, dense, int(causal)), _lib.load(), _lib.ctypes.byref(ex)
     return lib.fo_attn_fwd_kernel_ex(*call, by, lib.fo_attn_fwd_workspace_ex(*call, by) if scratch else 0)
 
@@ -61,17 +62,29 @@ def test_the_rule():
     pipe, plain, shared = _lib.FO_ATTN_KERNEL_ROWS128_PIPE, _lib.FO_ATTN_KERNEL_ROWS128, _lib.FO_ATTN_KERNEL_SHARED_BLOCKS
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     for D, f32 in [(128, False), (64, False), (64, True)]:
+        line = 32 if f32 else 64
         for scratch in (False, True):
-            assert _kernel(1, cus // 16, 2048, 2048, D, False, f32, scratch) == pipe           # one workgroup per unit
+            full = cus // 16 - 1 if f32 else cus // 16                                         # one workgroup per unit (fp32: nearly)
+            assert _kernel(1, full, 2048, 2048, D, False, f32, scratch) == pipe
             assert _kernel(1, cus * 3 // 2 // 16, 2048, 2048, D, True, f32, scratch) == pipe   # one and a half when causal
             assert _kernel(1, cus * 3 // 2 // 16 + 1, 2048, 2048, D, True, f32, scratch) == plain
-            assert _kernel(1, 4, 1024, 767, D, True, f32, scratch) == plain
+            assert _kernel(1, 4, 1024, 767, D, True, f32, scratch, 768) == plain
         # one more than a unit each, not causal: only where workgroups can share the last round
         assert _kernel(1, cus // 16 + 1, 2048, 2048, D, False, f32, False) == plain
         assert _kernel(1, cus // 16 + 1, 2048, 2048, D, False, f32) in (plain, pipe + shared)
         assert _kernel(1, 12, 3072, 3072, D, False, f32, False) == plain and _kernel(1, 4, 1024, 768, D, True, f32, False) == pipe
+        # rows off the cache lines: where workgroups share blocks, and at head_dim 64 under a causal mask
+        off = dict(row=1800 + line // 2)
+        assert _kernel(1, 12, 1800, 1800, D, False, f32, **off) == plain
+        assert _kernel(1, 12, 1800, 1800, D, True, f32, **off) == (pipe if D == 64 else plain)
+        assert _kernel(1, 4, 1800, 1800, D, True, f32, False, **off) == (pipe if D == 64 else plain)
         if cus == 256:
             assert _kernel(1, 12, 3072, 3072, D, False, f32) == pipe + shared and _kernel(1, 4, 4096, 4096, D, True, f32) == pipe + shared
+            assert _kernel(1, 12, 3072, 3072, D, False, f32, row=3072 + line // 2) == plain
+            assert _kernel(1, 12, 1800, 1800, D, False, f32, row=1792 + 2 * line) == pipe
+            for causal in (False, True):
+                assert _kernel(1, 4, 1800, 1800, D, causal, f32, **off) == pipe + shared
+            assert (_kernel(1, 16, 2048, 2048, D, False, f32) == pipe) == (not f32)
     assert _kernel(1, 4, 2048, 2048, 128, True, True) == plain                    # fp32 at head_dim 128
     assert _kernel(1, 4, 2048, 2048, 96, True, False) == plain                    # a head_dim off 64 and 128
 
