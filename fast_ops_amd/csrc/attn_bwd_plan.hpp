@@ -24,7 +24,8 @@ constexpr uint32_t kWholeBlock = 0xFFFF1000u;
 //   4 heads x 4096 causal, key bias, dropout 158 -> 109 (0.52); 6 x 3000 the same 131 -> 96 (0.60); 6 x 2500, dropout 120 -> 95 (0.68)
 //   12 x 3072 237 -> 201, with a bf16 bias with a query stride 298 -> 253 (0.69); 8 x 3072 causal with one 121 -> 111 (0.73); 8 x 4096
 //   causal 147 -> 138 (0.77); 12 x 6144 709 -> 661 (0.80); 12 x 3072 causal 134 -> 125, with a bias 152 -> 150 (0.89)
-//   not taken: 12 x 4096 335 -> 348, with key bias and dropout 360 -> 352 (0.84); 6 x 4096 165 -> 158 in 4 pieces (1.1)
+//   not taken: 12 x 4096 335 -> 348, with key bias and dropout 360 -> 352 (0.84: one line for all forms of a call, which these two lie on either
+//   side of); 6 x 4096 165 -> 158 in 4 pieces (1.1)
 constexpr int kMaxPieces = 4;
 struct DkdvPlan {
   int n_items = 0, n_merges = 0, n_parts = 0;

@@ -725,6 +725,7 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
   // row sum once (recovery path), which multiplies the row's empty O and l by 0 (left padding: one step per row).
   // TBIAS: the bias joins a score where that is scaled: exp2(S c + (b log2 e - m)), two instructions per score more, with m, the reference,
   // in the base-2 domain (so that a row whose bias is large as a whole loses nothing to it).
+  // Rows whose reference is far (kFarReference: all keys masked with a large finite value) take the recovery path in every step.
   // BM = 256: the form described above. BM = 128 (QB = 1): the same pipeline with four waves x 32 rows, one query block
   // per workgroup in the 128-row kernel's order (heaviest causal blocks first), for shapes that give the chip too few
   // 256-row workgroups: a workgroup's time per key tile is what bounds those, and this pipeline's is less than half the
@@ -1297,8 +1298,9 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
 #pragma unroll
     for (int b2 = 0; b2 < QB; ++b2) redo = redo || !(psum[b2] <= kLargeRowSum);
     // (RECOVER_FAR: the compiler is told that the path is rare and lays it out behind the loops, so that a step ends without a
-    // taken branch, which holds a lone wave up until its instructions are fetched. Four waves x 64 rows: 2 x 16 heads x 8192
-    // 464 -> 457 us causal, 849 -> 844 not causal; the 128-row form loses up to 1 % that way, the eight-wave form does not care.)
+    // taken branch, which holds a lone wave up until its instructions are fetched. Four waves x 64 rows: 2 x 16 heads x 8192 causal
+    // 464 -> 457 us on one card, 466 -> 464 and 467 -> 468 on others, where runs of one side differ by 0.3 to 0.6 %; the 128-row form loses up to
+    // 1 % that way, the eight-wave form does not care.)
     constexpr bool RECOVER_FAR = QB == 2;
     const bool recover = __builtin_amdgcn_ballot_w64(redo) != 0 || far;
     if (CAN_RECOVER && (RECOVER_FAR ? __builtin_expect(recover, 0) : recover) && !(DBG & 2)) {

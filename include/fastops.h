@@ -89,8 +89,8 @@ int fo_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse
  * the longest query blocks keep the others waiting (head_dim 64 and 128), whose keys several workgroups then share; the parts are added in
  * a fixed order by a second launch. ws points to ws_bytes bytes on the device, 16-byte aligned, used by this call only until the
  * stream has passed it and never needing to be cleared. fo_attn_fwd_workspace answers how many bytes the call of a shape can use
- * on the current device: 0 where nothing is shared. With less (or ws NULL) the call computes the same with one workgroup per head or
- * query block, as fo_attn_fwd does. fo_attn_fwd_workspace_ex and fo_attn_fwd_ex_ws are the same for calls with extras
+ * on the current device: 0 where nothing is shared. With less (or ws NULL) one workgroup per head or query block does the work, as in
+ * fo_attn_fwd: the same sums in another order, so that results agree to their rounding and not to the bit. fo_attn_fwd_workspace_ex and fo_attn_fwd_ex_ws are the same for calls with extras
  * (fo_attn_fwd_ex; of the bias' pointer only its alignment counts for the answer); extras may be NULL. No reference counterpart. */
 int64_t fo_attn_fwd_workspace(int B, int H, int Sq, int Sk, int D, const int64_t* k_strides_host, const int64_t* v_strides_host, int causal);
 int fo_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
