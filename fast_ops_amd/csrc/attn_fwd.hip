@@ -1302,7 +1302,8 @@ __global__ void __launch_bounds__(BM / (32 * QB) * 64, (BM == kWideBM || D == 12
     // 464 -> 457 us on one card, 466 -> 464 and 467 -> 468 on others, where runs of one side differ by 0.3 to 0.6 %; the 128-row form loses up to
     // 1 % that way, the eight-wave form does not care.)
     constexpr bool RECOVER_FAR = QB == 2;
-    const bool recover = __builtin_amdgcn_ballot_w64(redo) != 0 || far;
+    bool recover = __builtin_amdgcn_ballot_w64(redo) != 0;
+    if constexpr (VBIAS || TBIAS != 0) recover = recover || far;
     if (CAN_RECOVER && (RECOVER_FAR ? __builtin_expect(recover, 0) : recover) && !(DBG & 2)) {
       // rare: true row maxima of this sub-tile, new references, P and row sums again, O and l rescaled
 #pragma unroll
